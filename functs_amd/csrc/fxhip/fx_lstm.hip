@@ -34,6 +34,7 @@
 #ifndef FX_LSTM_STAMP
 #define FX_LSTM_STAMP(k)
 #define FX_LSTM_PSTAMP(k)
+#define FX_LSTM_POLLS(n)
 #define FX_LSTM_STAMP_END()
 #define FX_LSTM_STAMP_DECL
 #endif
@@ -342,48 +343,391 @@ __global__ __launch_bounds__(FX_LSTM_BLOCK * UPW, HPT >= 32 ? 4 : 2) void fx_lst
     fx_lstm_leave<DevAtomics>(a.ctl, gridDim.x, base, (uint32_t)n_steps, a.hbuf, (uint32_t)(2 * L * B * H));
 }
 
+// ---- several sequences at once ----------------------------------------------------------------
+// The kernel above walks the batch rows of a step one after the other, and every row pays the whole
+// hand-over of its vectors: 2.0 us a row and step, 1 670 us for T = 100, B = 8, H = 256, L = 3.  Here
+// a step's products for four rows are one set of matrix instructions and a step costs ONE hand-over.
+//   rows     groups of four (v_mfma_f32_4x4x1: tiles of four rows, fp32 in and out).  A group has
+//            workgroups of its own, which hold the weights again but wait for, and read, the vectors of
+//            their own rows only: what all workgroups read in a step is what the step waits for.
+//            H = 512 from nine rows on: two tiles a workgroup, since the device does not hold the
+//            workgroups of more groups at once.
+//   columns  four hidden units a workgroup.  A vector h_j is multiplied by layer j's recurrent and
+//            layer j + 1's input matrix: 16 + 16 gate columns, the 32 columns of a half-wave.
+//   depth    the inner dimension is dealt to eight waves in runs of 16: lane l fetches element l / 4
+//            of row l % 4 and keeps, in registers for the whole sequence, its column's weights of the
+//            eight elements of a run that its half of the wave multiplies (cbsz = 3: a block of four
+//            lanes feeds the eight blocks of its half-wave), so a wave sums nothing but its two halves.
+//   waves    up to four more finish the cells (gate x unit x row: 64 lanes a layer and tile), store
+//            them, clear the words of the step after next and bring x into LDS two steps ahead.  A wave
+//            that did both would queue its next loads up behind the acknowledgements of its stores.
+// Values travel as words (fx_lstm_sched.h): half the bytes of tagged ones.
+// T = 100, B = 8, H = 256, L = 3: 273 us, 2.7 us a step, of which 1.6 us pass from the stores to the
+// last word seen, 0.25 us are products, 0.7 us cells.  T = 64, H = 512, L = 2: 810 -> 234 us for eight
+// rows, 1 620 -> 369 for sixteen, 213 -> 199 for two.
+// How long a wave sleeps behind a step's barrier before it first looks at the step's vectors.  A look
+// that comes too early costs a whole trip, and its reads slow down the stores they wait for; how long
+// the stores take depends on the sizes, so every wave finds its own time: 64 clocks later after an
+// early look, 2 clocks sooner after every other one (an early look costs about 30 times 64 clocks).
+// T = 100, B = 8, H = 256, L = 3: a fixed 512 clocks 407 us, 1 024: 326, 1 280: 302; this: 277 - 285.
+struct FxLook {
+  int at = 24 * 32;   // 32nds of 64 clocks
+  __device__ __forceinline__ void wait() const {
+    for (int n = at >> 5; n > 0; --n) __builtin_amdgcn_s_sleep(1);
+  }
+  __device__ __forceinline__ void seen(uint32_t polls) { at = polls == 0u ? max(at - 1, 0) : min(at + 32, 64 * 32); }
+};
+// every store of the wave has been performed at the memory side of the caches
+__device__ __forceinline__ void fx_stores_acknowledged() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+typedef float fx_f32x4 __attribute__((ext_vector_type(4)));
+template <int Q> struct fx_const { static constexpr int value = Q; };
+template <class F>
+__device__ __forceinline__ void fx_each8(F&& f) {
+  f(fx_const<0>()); f(fx_const<1>()); f(fx_const<2>()); f(fx_const<3>());
+  f(fx_const<4>()); f(fx_const<5>()); f(fx_const<6>()); f(fx_const<7>());
+}
+
+template <int L, int HPT, int MT>
+struct FxLstmRows {
+  static constexpr int HH = HPT * 32;                   // H
+  static constexpr int NW = HPT >= 4 ? 8 : 2 * HPT;     // waves that multiply
+  static constexpr int CW = L * MT < 4 ? L * MT : 4;    // waves that finish cells, and bring x
+  static constexpr int threads = (NW + CW) * 64;
+};
+template <int L, int HPT, int MT>
+__global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_rows_kernel(const FxLstmArgs a) {
+  using C = FxLstmRows<L, HPT, MT>;
+  constexpr int HH = C::HH, NW = C::NW, CW = C::CW, NT = C::threads;
+  constexpr int KW = HH / NW, KI = KW / 16;             // inner elements of a wave, in runs of 16
+  constexpr int S = L + 1;                              // vectors of a step: x and every layer's h
+  constexpr int NV = S * MT * 4;                        // partial sums a lane: [vector][tile][row of the tile]
+  constexpr int CI = (L * MT + CW - 1) / CW;            // (layer, tile) pairs a wave finishes
+  constexpr int XS = HH + 8;                            // distance of x's rows in LDS: the four rows a wave reads lie in different banks
+  constexpr int XP = (MT * HH + CW * 64 - 1) / (CW * 64);   // 16-byte groups of x a lane brings in
+  __shared__ float s_part[2][NW][NV * 32];              // by parity of the step: [(vector, tile)][column half][row][16]
+  __shared__ float s_x[3][4 * MT * XS];                 // x of a step and of the two behind it
+  __shared__ uint32_t s_abort;
+  FX_LSTM_STAMP_DECL
+  const int B = a.B, T = a.T;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int n_wg = HH / 4;                          // workgroups of a group of rows
+  const int group = (int)blockIdx.x / n_wg, gi = (int)blockIdx.x % n_wg;
+  // as above: the workgroups of a die take neighbouring hidden units
+  const int wg = (n_wg % 8 == 0) ? (gi % 8) * (n_wg / 8) + gi / 8 : gi;
+  const int u0 = wg * 4;
+  const int b0 = group * 4 * MT, nb = min(4 * MT, B - b0);
+  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) ? 1u : 0u;
+  const uint32_t base = DevAtomics::load(a.ctl + FX_LSTM_W_BASE);
+  const int n_steps = fx_lstm_steps(T, L);
+  const uint32_t BH = (uint32_t)(B * HH);               // elements of one vector of all rows
+  const int c_ul = (lane >> 2) & 3, c_gate = lane & 3;
+
+  if (wave < NW) {
+    // ---- products.  This lane's column: lanes 0-15 of a half-wave the recurrent matrix of the vector's own
+    // layer, lanes 16-31 the input matrix of the layer above; unit (lane >> 2) & 3, gate lane & 3.
+    // Element of a wave's run that block `blk` (four lanes) fetches: pairs of neighbours where there is a
+    // second run.
+    const int half = (lane >> 4) & 1;
+    auto k_of = [&](int i, int blk) { return wave * KW + (KI == 1 ? blk : 32 * (i / 2) + 2 * blk + (i & 1)); };
+    float w[S][KI][8];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int jc = half ? s : s - 1;                  // the layer whose gates the column belongs to
+      const bool live = jc >= 0 && jc < L;              // (x has no recurrent matrix, the last h no layer above)
+      const int j = min(max(jc, 0), L - 1);
+      const float* m = half ? a.wih : a.whh;
+#pragma unroll
+      for (int i = 0; i < KI; ++i)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const float v = m[((size_t)(j * 4 + c_gate) * HH + k_of(i, 8 * (lane >> 5) + q)) * HH + u0 + c_ul];
+          w[s][i][q] = live ? v : 0.0f;
+        }
+    }
+    // word (row, k) of a vector that this lane fetches, per tile; rows past the batch repeat its last one
+    // (their sums are not used)
+    uint32_t at[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) at[mt] = (uint32_t)((b0 + min(mt * 4 + (lane & 3), nb - 1)) * HH + k_of(0, lane >> 2));
+    const int xat = (lane & 3) * XS + k_of(0, lane >> 2);
+    __syncthreads();
+    if (s_abort != 0u) {   // uniform: written once, ahead of the barrier
+      if (tid == 0 && a.err_host) __hip_atomic_store(a.err_host, (uint32_t)FX_ASYNC_BARRIER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      fx_lstm_poison(a, L, (uint32_t)tid, (uint32_t)(NW * 64));
+      return;
+    }
+    FxLook look;
+    for (int d = 0; d < n_steps; ++d) {
+      FX_LSTM_STAMP(0);
+      fx_f32x4 acc[S][MT];
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[s][mt] = fx_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      // one matrix instruction: element 8 * (half-wave) + Q of a run, for every column of a vector.  Its
+      // callers go round the vectors before they come back to an accumulator: a dependent one waits.
+      auto multiply = [&](auto q, int s, int mt, int i, float v) {
+        constexpr int Q = decltype(q)::value;
+        acc[s][mt] = __builtin_amdgcn_mfma_f32_4x4x1f32(v, w[s][i][Q], acc[s][mt], 3, Q, 0);
+      };
+      // x is known ahead: its products fill the time in which the other workgroups' values travel
+      {
+        float xv[MT][KI];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int i = 0; i < KI; ++i) xv[mt][i] = s_x[d % 3][mt * 4 * XS + xat + (KI == 1 ? 0 : 32 * (i / 2) + (i & 1))];
+#pragma unroll
+        for (int i = 0; i < KI; ++i)
+          fx_each8([&](auto q) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) multiply(q, 0, mt, i, xv[mt][i]);
+          });
+      }
+      FX_LSTM_STAMP(1);
+      // the h vectors, as above: words of the step before, h0 at a layer's first step
+      float hv[L][MT][KI];
+      bool need[L];
+#pragma unroll
+      for (int j = 0; j < L; ++j) {
+        const int tj = fx_lstm_time(d, j, T);
+        need[j] = tj != 0 && (tj > 0 || (j + 1 < L && fx_lstm_time(d, j + 1, T) >= 0));
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int i = 0; i < KI; ++i)
+            hv[j][mt][i] = (tj == 0 && a.h0) ? (a.h0 + (size_t)j * BH)[at[mt] + (KI == 1 ? 0 : 32 * (i / 2) + (i & 1))] : 0.0f;
+      }
+      const uint32_t* src = (const uint32_t*)a.hbuf + (size_t)fx_lstm_slot(base, d - 1) * (L * BH);
+      uint32_t polls = 0;
+      if (d > 0) look.wait();
+      for (;;) {
+        bool ready = true;
+        uint32_t el[L][MT][KI];
+#pragma unroll
+        for (int j = 0; j < L; ++j)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) {
+            if constexpr (KI == 1) {
+              el[j][mt][0] = __hip_atomic_load(src + (size_t)j * BH + at[mt], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+#pragma unroll
+              for (int i = 0; i < KI; i += 2) {
+                const uint64_t two = __hip_atomic_load((const uint64_t*)(src + (size_t)j * BH + at[mt] + 16 * i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                el[j][mt][i] = (uint32_t)two;
+                el[j][mt][i + 1] = (uint32_t)(two >> 32);
+              }
+            }
+          }
+#pragma unroll
+        for (int j = 0; j < L; ++j)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < KI; ++i) {
+              ready = ready && (!need[j] || el[j][mt][i] != 0u);
+              hv[j][mt][i] = need[j] ? __uint_as_float(fx_lstm_word_value(el[j][mt][i])) : hv[j][mt][i];
+            }
+        if (!wave_any(!ready)) break;   // (a matrix instruction reads its operands from all lanes)
+        if (++polls > a.spin_limit || ((polls & 255u) == 0u && DevAtomics::load(a.ctl + FX_LSTM_W_ERR) != 0u)) {
+          // given up (or somebody else has): the workgroup leaves behind this step's barrier
+          DevAtomics::store(a.ctl + FX_LSTM_W_ERR, 1u);
+          if (a.err_host) __hip_atomic_store(a.err_host, (uint32_t)FX_ASYNC_BARRIER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          s_abort = 1u;
+          break;
+        }
+      }
+      look.seen(polls);
+      FX_LSTM_POLLS(polls);
+      FX_LSTM_STAMP(2);
+#pragma unroll
+      for (int i = 0; i < KI; ++i)
+        fx_each8([&](auto q) {
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int j = 0; j < L; ++j) multiply(q, j + 1, mt, i, hv[j][mt][i]);
+        });
+      FX_LSTM_STAMP(3);
+      // the two halves of the wave: the lower keeps the first half of the values, the upper the second
+      float* dst = s_part[d & 1][wave];
+#pragma unroll
+      for (int i = 0; i < NV / 2; ++i) {
+        const float lo = acc[(i >> 2) / MT][(i >> 2) % MT][i & 3];
+        const float hi = acc[((i + NV / 2) >> 2) / MT][((i + NV / 2) >> 2) % MT][(i + NV / 2) & 3];
+        const fx_u32x2v t = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+        const int v = i + (lane >> 5) * (NV / 2);
+        dst[(((v >> 2) * 2 + half) * 4 + (v & 3)) * 16 + (lane & 15)] = __uint_as_float(t.x) + __uint_as_float(t.y);
+      }
+      FX_LSTM_STAMP(4);
+      __syncthreads();
+      FX_LSTM_STAMP(5);
+      if (s_abort != 0u) {   // the results are not to be used: say so in the data
+        fx_lstm_poison(a, L, (uint32_t)tid, (uint32_t)(NW * 64));
+        return;
+      }
+    }
+    FX_LSTM_STAMP_END();
+    __syncthreads();   // the last step's values
+    return;
+  }
+
+  // ---- cells: lane = row of the tile * 16 + unit * 4 + gate; pair jt = layer * MT + tile ----
+  const int cw = wave - NW, f_m = lane >> 4;
+  float bias_ih[CI], bias_hh[CI], cell[CI];
+#pragma unroll
+  for (int ci = 0; ci < CI; ++ci) {
+    const int jt = min(cw + CW * ci, L * MT - 1), j = jt / MT, b = b0 + min((jt % MT) * 4 + f_m, nb - 1);
+    bias_ih[ci] = a.bih[(size_t)(j * 4 + c_gate) * HH + u0 + c_ul];
+    bias_hh[ci] = a.bhh[(size_t)(j * 4 + c_gate) * HH + u0 + c_ul];
+    cell[ci] = a.c0 ? a.c0[((size_t)j * B + b) * HH + u0 + c_ul] : 0.0f;
+  }
+  fx_u32x4_a4 xr[XP];
+  auto fetch_x = [&](int d) {   // (unconditional: what a step without its first layer reads is not used)
+    const float* src = a.x + (size_t)min(d, T - 1) * BH;
+#pragma unroll
+    for (int e = 0; e < XP; ++e) {
+      const int g = min(cw * 64 + lane + CW * 64 * e, MT * HH - 1), r = g / (HH / 4), c = g % (HH / 4);
+      xr[e] = *(const fx_u32x4_a4*)(src + (size_t)(b0 + min(r, nb - 1)) * HH + 4 * c);
+    }
+  };
+  auto park_x = [&](int d) {
+#pragma unroll
+    for (int e = 0; e < XP; ++e) {
+      const int g = min(cw * 64 + lane + CW * 64 * e, MT * HH - 1), r = g / (HH / 4), c = g % (HH / 4);
+      *(fx_u32x4*)(s_x[d % 3] + r * XS + 4 * c) = xr[e];
+    }
+  };
+  fetch_x(0);
+  park_x(0);
+  fetch_x(1);
+  park_x(1);
+  fetch_x(2);
+  __syncthreads();
+  if (s_abort != 0u) return;
+  for (int d = 0; d < n_steps; ++d) {
+    __syncthreads();
+    FX_LSTM_STAMP(5);
+    const uint32_t aborted = s_abort;
+    const uint32_t out_slot = fx_lstm_slot(base, d) * (uint32_t)(L * BH), clear_slot = fx_lstm_slot(base, d + 2) * (uint32_t)(L * BH);
+    if (aborted != 0u) return;   // uniform, ahead of every store of the step
+#pragma unroll
+    for (int ci = 0; ci < CI; ++ci) {
+      const int jt = cw + CW * ci, j = jt / MT, mt = jt % MT;
+      const int t = jt < L * MT ? fx_lstm_time(d, j, T) : -1;
+      if (t < 0) continue;   // uniform in the wave
+      float ih[NW], hh[NW];
+#pragma unroll
+      for (int g = 0; g < NW; ++g) {
+        ih[g] = s_part[d & 1][g][((j * MT + mt) * 2 + 1) * 64 + lane];
+        hh[g] = s_part[d & 1][g][(((j + 1) * MT + mt) * 2) * 64 + lane];
+      }
+#pragma unroll
+      for (int g = 0; g < NW; ++g) ih[g] += hh[g];
+#pragma unroll
+      for (int span = 1; span < NW; span *= 2)
+#pragma unroll
+        for (int g = 0; g + span < NW; g += 2 * span) ih[g] += ih[g + span];
+      const float pre = (ih[0] + bias_ih[ci]) + bias_hh[ci];
+      const float act = c_gate == 2 ? fx_tanh(pre) : fx_sigmoid(pre);
+      const float fg = quad_lane<1>(act), gg = quad_lane<2>(act), og = quad_lane<3>(act);
+      const int r = mt * 4 + f_m;
+      if (c_gate == 0 && r < nb) {
+        const float c = (fg * cell[ci]) + (act * gg);
+        cell[ci] = c;
+        const float h = og * fx_tanh(c);
+        const int b = b0 + r, u = u0 + c_ul;
+        DevAtomics::store((uint32_t*)a.hbuf + out_slot + (uint32_t)((j * B + b) * HH + u), fx_lstm_word(__float_as_uint(h)));
+        if (j == L - 1) a.out[((size_t)t * B + b) * HH + u] = h;
+        if (t == T - 1) {
+          a.state_h[((size_t)j * B + b) * HH + u] = h;
+          a.state_c[((size_t)j * B + b) * HH + u] = c;
+        }
+      }
+    }
+    FX_LSTM_STAMP(6);
+    // between the barriers of steps d and d + 1 the others read x of step d + 1; the slot of step d + 2
+    // was last read in step d - 1
+    park_x(d + 2);
+#pragma unroll
+    for (int ci = 0; ci < CI; ++ci) {
+      const int jt = cw + CW * ci, r = (jt % MT) * 4 + f_m;
+      if (jt < L * MT && c_gate == 0 && r < nb)
+        DevAtomics::store((uint32_t*)a.hbuf + clear_slot + (uint32_t)(((jt / MT) * B + b0 + r) * HH + u0 + c_ul), 0u);
+    }
+    fx_stores_acknowledged();   // ahead of the next barrier (the others are busy until then)
+    fetch_x(d + 3);
+    FX_LSTM_STAMP(7);
+  }
+  FX_LSTM_STAMP_END();
+  __syncthreads();   // every wave's values are at the memory side before the workgroup checks out
+  if (cw == 0 && lane == 0) fx_lstm_leave_slots<DevAtomics>(a.ctl, gridDim.x, base, (uint32_t)n_steps);
+}
+
 typedef void (*fx_lstm_kernel_t)(const FxLstmArgs);
-template <int L, int UPW>
-static fx_lstm_kernel_t pick_hpt(int hpt) {
-  switch (hpt) {
-    case 1: return fx_lstm_stack_kernel<L, 1, UPW>;
-    case 2: return fx_lstm_stack_kernel<L, 2, UPW>;
-    case 4: return fx_lstm_stack_kernel<L, 4, UPW>;
-    case 8: return fx_lstm_stack_kernel<L, 8, UPW>;
-    case 16: return fx_lstm_stack_kernel<L, 16, UPW>;
-    case 32: return fx_lstm_stack_kernel<L, 32, UPW>;
+template <int L>
+static fx_lstm_kernel_t pick_rows(int hpt, int tiles) {
+  switch (hpt * 4 + tiles) {
+    case 4 + 1: return fx_lstm_rows_kernel<L, 1, 1>;
+    case 8 + 1: return fx_lstm_rows_kernel<L, 2, 1>;
+    case 16 + 1: return fx_lstm_rows_kernel<L, 4, 1>;
+    case 32 + 1: return fx_lstm_rows_kernel<L, 8, 1>;
+    case 64 + 1: if constexpr (L <= 3) return fx_lstm_rows_kernel<L, 16, 1>; else return nullptr;
+    case 64 + 2: if constexpr (L <= 3) return fx_lstm_rows_kernel<L, 16, 2>; else return nullptr;
     default: return nullptr;
   }
 }
-template <int UPW>
-static fx_lstm_kernel_t pick_layers(int L, int hpt) {
-  switch (L) {
-    case 1: return pick_hpt<1, UPW>(hpt);
-    case 2: return pick_hpt<2, UPW>(hpt);
-    case 3: return pick_hpt<3, UPW>(hpt);
-    case 4: return pick_hpt<4, UPW>(hpt);
+// one row, or rows one after the other: the sizes for which four units' weights and a tile of rows are
+// more than the registers hold (1024 units; four layers of 512: 725 us with spilled weights against 630
+// for T = 32, B = 8)
+template <int L>
+static fx_lstm_kernel_t pick_serial(int hpt) {
+  constexpr int U = FX_LSTM_UPW;
+  switch (hpt) {
+    case 1: return fx_lstm_stack_kernel<L, 1, U>;
+    case 2: return fx_lstm_stack_kernel<L, 2, U>;
+    case 4: return fx_lstm_stack_kernel<L, 4, U>;
+    case 8: return fx_lstm_stack_kernel<L, 8, U>;
+    case 16: return fx_lstm_stack_kernel<L, 16, U>;
+    case 32: if constexpr (L <= 2) return fx_lstm_stack_kernel<L, 32, U>;
     default: return nullptr;
   }
+}
+struct LstmLaunch { fx_lstm_kernel_t kernel; int grid, threads; };
+template <int L>
+static LstmLaunch pick_launch(const FxLstmArgs& a) {
+  const int hpt = a.H / 32;
+  LstmLaunch r{};
+  if (a.B > 1) {
+    // One tile of four rows a workgroup while all groups of rows together make at most one workgroup
+    // for each of the 256 CUs (the weights fill a CU's registers), else two.
+    const int tiles = (a.H / 4) * ((a.B + 3) / 4) > 256 ? 2 : 1, groups = (a.B + 4 * tiles - 1) / (4 * tiles);
+    const int cells = L * tiles < 4 ? L * tiles : 4;   // FxLstmRows
+    r = LstmLaunch{pick_rows<L>(hpt, tiles), (a.H / 4) * groups, ((a.H >= 128 ? 8 : a.H / 16) + cells) * 64};
+  }
+  // two hidden units per workgroup: every workgroup fetches the step's vectors from the memory
+  // side once, so fewer, larger workgroups fetch less, and sixteen gate sums fill the butterfly
+  if (!r.kernel) r = LstmLaunch{pick_serial<L>(hpt), a.H / FX_LSTM_UPW, FX_LSTM_BLOCK * FX_LSTM_UPW};
+  return r;
 }
 
 // 0: launched; 1: shape outside what the kernel is built for; 2: the grid would not be resident
 // all at once (every workgroup waits for values that all the others write); otherwise a HIP error code + 100.
 int fx_launch_lstm_stack(const FxLstmArgs& a, int L, hipStream_t stream) {
-  if (a.H < 32 || a.H % 32 != 0 || a.B < 1 || a.B > FX_LSTM_MAXB || L * a.B > FX_LSTM_BLOCK) return 1;
-  // two hidden units per workgroup: every workgroup fetches the step's vectors from the memory
-  // side once, so fewer, larger workgroups fetch less, and sixteen gate sums fill the butterfly
-  constexpr int upw = FX_LSTM_UPW;
-  fx_lstm_kernel_t k = pick_layers<FX_LSTM_UPW>(L, a.H / 32);
-  if (!k) return 1;
+  if (a.H < 32 || a.H % 32 != 0 || a.B < 1 || a.B > FX_LSTM_MAXB || L < 1 || L * a.B > FX_LSTM_BLOCK) return 1;
+  const LstmLaunch l = L == 1 ? pick_launch<1>(a) : L == 2 ? pick_launch<2>(a) : L == 3 ? pick_launch<3>(a) : L == 4 ? pick_launch<4>(a) : LstmLaunch{};
+  if (!l.kernel) return 1;
   int dev = 0, per_cu = 0, cus = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const size_t lds = 0;
-  const int threads = FX_LSTM_BLOCK * upw, grid = a.H / upw;
-  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, threads, lds);
+  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)l.kernel, l.threads, 0);
   if (e != hipSuccess) return 100 + (int)e;
-  if ((long)per_cu * cus < grid) return 2;
+  if ((long)per_cu * cus < l.grid) return 2;
   void* args[1] = {(void*)&a};
-  e = hipLaunchKernel((const void*)k, dim3((uint32_t)grid), dim3((uint32_t)threads), args, lds, stream);
+  e = hipLaunchKernel((const void*)l.kernel, dim3((uint32_t)l.grid), dim3((uint32_t)l.threads), args, 0, stream);
   return e == hipSuccess ? 0 : 100 + (int)e;
 }

@@ -34,6 +34,23 @@
 #define FX_LSTM_CTL_WORDS (3u * FX_LSTM_LINE)
 #define FX_LSTM_TAG_WRAP 0x80000000u              // the base starts over (and the tags are cleared) beyond this
 
+// The second hand-over, of the kernels for one sequence and for groups of rows: an element is ONE
+// 32-bit word, its value with all bits inverted, and 0 says that it has not been written yet (the
+// word that would be 0, a NaN of all ones, is written as another NaN).  Half the bytes of a value with
+// its tag, and what all workgroups read in a step is what a step waits for.
+//   Four slots of [L][B][H] words, used in turn: step d writes slot (base + d) & 3, reads slot
+//   (base + d - 1) & 3, and its owners clear their words of slot (base + d + 2) & 3.
+//   Clearing is safe: behind the barrier of step d a workgroup has seen every value of step d - 1, so
+//   every workgroup is past its reads of step d - 1, which were reads of slot d - 2, the one cleared.
+//   A cleared word is seen in time: a workgroup lets its clears of step d be acknowledged before its
+//   barrier of step d + 1, ahead of its values of step d + 1; who reads slot d + 2 (in step d + 3) has
+//   seen those values.
+//   base is a word of the workspace, advanced by the steps of every launch: slots base and base + 1 are
+//   clear when a launch begins (all four in a zeroed workspace), and stay so from launch to launch.
+FX_LSTM_HD inline uint32_t fx_lstm_slot(uint32_t base, int d) { return (base + (uint32_t)d) & 3u; }
+FX_LSTM_HD inline uint32_t fx_lstm_word(uint32_t value_bits) { return value_bits == 0xffffffffu ? ~0x7fc00000u : ~value_bits; }
+FX_LSTM_HD inline uint32_t fx_lstm_word_value(uint32_t word) { return ~word; }
+
 // arguments of the kernel (contiguous fp32 tensors; see fx_lstm_stack in include/fxhip.h)
 struct FxLstmArgs {
   const float *x, *wih, *whh, *bih, *bhh;
@@ -99,5 +116,13 @@ FX_LSTM_HD inline void fx_lstm_leave(uint32_t* ctl, uint32_t n_wg, uint32_t base
     next = 0u;
   }
   A::store(ctl + FX_LSTM_W_BASE, next);
+  A::store(ctl + FX_LSTM_W_LEAVE, 0u);
+}
+
+// The same for the hand-over through words: the slots are as the next launch expects them.
+template <class A>
+FX_LSTM_HD inline void fx_lstm_leave_slots(uint32_t* ctl, uint32_t n_wg, uint32_t base, uint32_t n_steps) {
+  if (A::add(ctl + FX_LSTM_W_LEAVE) + 1u != n_wg) return;
+  A::store(ctl + FX_LSTM_W_BASE, (base + n_steps) & 3u);
   A::store(ctl + FX_LSTM_W_LEAVE, 0u);
 }

@@ -423,16 +423,17 @@ int fx_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* co
  * persistent kernel: a workgroup per two hidden units keeps their columns of the weights in
  * registers for the whole sequence (thread k row k of them, and element k of the step's vectors);
  * the diagonals t + j follow each other without a barrier between workgroups, every h value
- * travels with the tag of the step that wrote it and readers poll for the tag they expect, with
- * bounded waits.  A wait that is given up reports FX_ASYNC_BARRIER through fx_async_error, fills
+ * travels with the tag of the step that wrote it (a batch of several rows: as a word that is clear
+ * until it is written) and readers poll for it, with bounded waits.  A wait that is given up reports FX_ASYNC_BARRIER through fx_async_error, fills
  * out / state_h / state_c with NaN and ends the kernel; its workspace stays marked, and every
  * later launch on it does no step, reports the error again and returns NaN, until the caller has
  * cleared the workspace.  A caller must therefore look at fx_async_error after synchronising and
  * before it uses the results (or test them for NaN), and clear the workspace after an error.
  * Contiguous fp32: x [T, B, H]; wih, whh [L, 4, H, H]; bih, bhh [L, 4, 1, H]; h0, c0, state_h,
  * state_c [L, B, H]; out [T, B, H]; h0 / c0 may be null (zero initial state).  H is 32, 64, ...
- * 1024 (a power of two), L <= 4, B <= 16 (FX_E_UNSUPPORTED otherwise), and H / 2 workgroups of
- * 512 threads must be resident together (FX_E_LIMIT).
+ * 1024 (a power of two), L <= 4, B <= 16 (FX_E_UNSUPPORTED otherwise), and the
+ * workgroups (H / 2 of 512 threads, or H / 4 of up to 768 for every four rows) must be resident
+ * together (FX_E_LIMIT).
  * workspace: fx_lstm_stack_workspace_bytes() of device memory, 256-byte aligned, all zero when it
  * is used for the first time.  A launch that ends without error leaves it ready for the next one,
  * so one workspace, cleared once, serves launch after launch on one stream as long as batch,

@@ -33,6 +33,8 @@ def lstm_emul():
     fp = ctypes.c_void_p
     so.fx_lstm_emul.restype = ctypes.c_int
     so.fx_lstm_emul.argtypes = [fp] * 10 + [ctypes.c_int] * 4 + [ctypes.c_uint32, ctypes.c_int, ctypes.c_int, ctypes.c_uint32]
+    so.fx_lstm_emul_words.restype = ctypes.c_int
+    so.fx_lstm_emul_words.argtypes = [fp] * 10 + [ctypes.c_int] * 4 + [ctypes.c_uint32, ctypes.c_int, ctypes.c_int]
     so.fx_lstm_emul_give_up.restype = ctypes.c_int
     so.fx_lstm_emul_give_up.argtypes = [fp] * 10 + [ctypes.c_int] * 4 + [ctypes.c_uint32, ctypes.c_int]
     return so

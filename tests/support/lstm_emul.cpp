@@ -46,8 +46,22 @@ bool read_tagged(const FxLstmArgs& a, int L, const uint64_t* p, uint32_t want, f
   }
 }
 
-// what one workgroup (hidden unit u) does; skip_wg: that workgroup stops writing after step 0
-void workgroup(const FxLstmArgs& a, int L, int u, int n_wg, int skip_wg) {
+// the same for a word of the second hand-over
+bool read_word(const FxLstmArgs& a, int L, const uint32_t* p, float* out) {
+  for (uint32_t polls = 0;; ++polls) {
+    const uint32_t e = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+    if (e != 0u) { *out = bits_to_float(fx_lstm_word_value(e)); return true; }
+    if (polls > a.spin_limit || ((polls & 255u) == 255u && HostAtomics::load(a.ctl + FX_LSTM_W_ERR) != 0u)) {
+      HostAtomics::store(a.ctl + FX_LSTM_W_ERR, 1u);
+      fx_lstm_poison(a, L, 0u, 1u);
+      return false;
+    }
+    std::this_thread::yield();
+  }
+}
+
+// what one workgroup (hidden unit u) does, with tags or with words; skip_wg: that workgroup stops writing after step 0
+void workgroup(const FxLstmArgs& a, int L, int u, int n_wg, int skip_wg, bool words) {
   const int H = a.H, B = a.B, T = a.T;
   if (fx_lstm_refused<HostAtomics>(a.ctl)) {   // the workspace carries a given-up wait
     fx_lstm_poison(a, L, (uint32_t)u, (uint32_t)n_wg);
@@ -62,6 +76,12 @@ void workgroup(const FxLstmArgs& a, int L, int u, int n_wg, int skip_wg) {
     if (u == skip_wg && d > 0) return;
     const int rp = (d + 1) & 1;
     const uint32_t want = fx_lstm_tag_read(base, d);
+    uint32_t* slots = (uint32_t*)a.hbuf;
+    auto word_at = [&](int step, int j, int b, int i) { return slots + (size_t)fx_lstm_slot(base, step) * L * B * H + ((size_t)j * B + b) * H + i; };
+    auto read = [&](int j, int b, int i, float* v) {
+      return words ? read_word(a, L, word_at(d - 1, j, b, i), v)
+                   : read_tagged(a, L, a.hbuf + fx_lstm_hoff(rp, j, b, i, L, B, H), want, v);
+    };
     // all reads of the step, then all its writes (as the kernel: dot products, barrier, owners)
     for (int j = 0; j < L; ++j) {
       const int t = fx_lstm_time(d, j, T);
@@ -69,9 +89,9 @@ void workgroup(const FxLstmArgs& a, int L, int u, int n_wg, int skip_wg) {
       for (int b = 0; b < B; ++b) {
         for (int i = 0; i < H; ++i) {
           if (j == 0) cur[i] = a.x[((size_t)t * B + b) * H + i];
-          else if (!read_tagged(a, L, a.hbuf + fx_lstm_hoff(rp, j - 1, b, i, L, B, H), want, &cur[i])) return;
+          else if (!read(j - 1, b, i, &cur[i])) return;
           if (t == 0) hp[i] = a.h0 ? a.h0[((size_t)j * B + b) * H + i] : 0.0f;
-          else if (!read_tagged(a, L, a.hbuf + fx_lstm_hoff(rp, j, b, i, L, B, H), want, &hp[i])) return;
+          else if (!read(j, b, i, &hp[i])) return;
         }
         float g[4];
         for (int k = 0; k < 4; ++k) {
@@ -89,12 +109,16 @@ void workgroup(const FxLstmArgs& a, int L, int u, int n_wg, int skip_wg) {
         hnew[j * B + b] = sigmoidf(g[3]) * tanhf(cc);
       }
     }
+    if (words)   // every layer's words, active or not
+      for (int j = 0; j < L; ++j)
+        for (int b = 0; b < B; ++b) HostAtomics::store(word_at(d + 2, j, b, u), 0u);
     for (int j = 0; j < L; ++j) {
       const int t = fx_lstm_time(d, j, T);
       if (t < 0) continue;
       for (int b = 0; b < B; ++b) {
         const float h = hnew[j * B + b];
-        HostAtomics::store64(a.hbuf + fx_lstm_hoff(d & 1, j, b, u, L, B, H), fx_lstm_pack(float_to_bits(h), fx_lstm_tag_written(base, d)));
+        if (words) HostAtomics::store(word_at(d, j, b, u), fx_lstm_word(float_to_bits(h)));
+        else HostAtomics::store64(a.hbuf + fx_lstm_hoff(d & 1, j, b, u, L, B, H), fx_lstm_pack(float_to_bits(h), fx_lstm_tag_written(base, d)));
         if (j == L - 1) a.out[((size_t)t * B + b) * H + u] = h;
         if (t == T - 1) {
           a.state_h[((size_t)j * B + b) * H + u] = h;
@@ -103,7 +127,8 @@ void workgroup(const FxLstmArgs& a, int L, int u, int n_wg, int skip_wg) {
       }
     }
   }
-  fx_lstm_leave<HostAtomics>(a.ctl, (uint32_t)n_wg, base, (uint32_t)n_steps, a.hbuf, (uint32_t)(2 * L * B * H));
+  if (words) fx_lstm_leave_slots<HostAtomics>(a.ctl, (uint32_t)n_wg, base, (uint32_t)n_steps);
+  else fx_lstm_leave<HostAtomics>(a.ctl, (uint32_t)n_wg, base, (uint32_t)n_steps, a.hbuf, (uint32_t)(2 * L * B * H));
 }
 }  // namespace
 
@@ -131,7 +156,7 @@ extern "C" int fx_lstm_emul(const float* x, const float* wih, const float* whh, 
       std::fill(state_c, state_c + (size_t)L * B * H, NAN);
     }
     std::vector<std::thread> th;
-    for (int u = 0; u < H; ++u) th.emplace_back(workgroup, std::cref(a), L, u, H, skip_wg);
+    for (int u = 0; u < H; ++u) th.emplace_back(workgroup, std::cref(a), L, u, H, skip_wg, false);
     for (auto& t : th) t.join();
     const int err = (int)ctl[FX_LSTM_W_ERR];
     if (err) return err;
@@ -142,6 +167,39 @@ extern "C" int fx_lstm_emul(const float* x, const float* wih, const float* whh, 
         if (e != 0ull) return -1;
     }
     if (ctl[FX_LSTM_W_BASE] != expect_base || ctl[FX_LSTM_W_LEAVE] != 0u) return -1;
+  }
+  return 0;
+}
+
+// The same with the second hand-over (words in four slots).  Returns the error word, or -1 when a run
+// without error did not leave the base, the counter and the two slots behind it as the next launch
+// needs them.
+extern "C" int fx_lstm_emul_words(const float* x, const float* wih, const float* whh, const float* bih, const float* bhh,
+                                  const float* h0, const float* c0, float* out, float* state_h, float* state_c, int T, int B,
+                                  int H, int L, uint32_t spin_limit, int skip_wg, int launches) {
+  std::vector<uint32_t> ctl(FX_LSTM_CTL_WORDS, 0u);
+  std::vector<uint64_t> hbuf((size_t)2 * L * B * H, 0ull);
+  FxLstmArgs a;
+  a.x = x; a.wih = wih; a.whh = whh; a.bih = bih; a.bhh = bhh; a.h0 = h0; a.c0 = c0;
+  a.out = out; a.state_h = state_h; a.state_c = state_c;
+  a.hbuf = hbuf.data(); a.ctl = ctl.data(); a.err_host = nullptr;
+  a.T = T; a.B = B; a.H = H; a.spin_limit = spin_limit;
+  uint32_t expect_base = 0u;
+  const uint32_t* slots = (const uint32_t*)hbuf.data();
+  for (int n = 0; n < launches; ++n) {
+    std::fill(out, out + (size_t)T * B * H, NAN);
+    std::fill(state_h, state_h + (size_t)L * B * H, NAN);
+    std::fill(state_c, state_c + (size_t)L * B * H, NAN);
+    std::vector<std::thread> th;
+    for (int u = 0; u < H; ++u) th.emplace_back(workgroup, std::cref(a), L, u, H, skip_wg, true);
+    for (auto& t : th) t.join();
+    const int err = (int)ctl[FX_LSTM_W_ERR];
+    if (err) return err;
+    expect_base = (expect_base + (uint32_t)fx_lstm_steps(T, L)) & 3u;
+    if (ctl[FX_LSTM_W_BASE] != expect_base || ctl[FX_LSTM_W_LEAVE] != 0u) return -1;
+    for (uint32_t s = 0; s < 2u; ++s)
+      for (size_t i = 0; i < (size_t)L * B * H; ++i)
+        if (slots[((expect_base + s) & 3u) * (size_t)L * B * H + i] != 0u) return -1;
   }
   return 0;
 }
@@ -170,7 +228,7 @@ extern "C" int fx_lstm_emul_give_up(const float* x, const float* wih, const floa
     std::fill(state_h, state_h + n_state, 0.5f);
     std::fill(state_c, state_c + n_state, 0.5f);
     std::vector<std::thread> th;
-    for (int u = 0; u < H; ++u) th.emplace_back(workgroup, std::cref(a), L, u, H, skip);
+    for (int u = 0; u < H; ++u) th.emplace_back(workgroup, std::cref(a), L, u, H, skip, false);
     for (auto& t : th) t.join();
   };
   // every element NaN, except (when given) those of hidden unit `but`

@@ -143,6 +143,22 @@ def test_after_a_given_up_wait_the_workspace_refuses_work_until_it_is_cleared():
     _close((out, sh, sc), _reference(*args), "launch on the cleared workspace")
 
 
+@pytest.mark.parametrize("T,H,L,B,launches", [(1, 32, 1, 2, 5), (1, 32, 4, 2, 3), (2, 32, 2, 2, 4), (7, 32, 3, 3, 3), (6, 64, 2, 2, 2)])
+def test_words_are_cleared_two_steps_ahead_on_host_threads(T, H, L, B, launches):
+    """The hand-over of the rows kernel: values without tags in four slots, cleared two steps ahead,
+    launches in a row (of fewer steps than slots as well) on one workspace that is cleared once."""
+    from tests.support import emul
+    so = emul.lstm_emul()
+    args = _inputs(T * 5 + L, T, H, L, B)
+    out, sh, sc = torch.zeros(T, B, H), torch.zeros(L, B, H), torch.zeros(L, B, H)
+    ts = [t.contiguous() for t in args]
+    err = so.fx_lstm_emul_words(*[t.data_ptr() for t in ts], out.data_ptr(), sh.data_ptr(), sc.data_ptr(), T, B, H, L, 1 << 30, -1, launches)
+    assert err == 0
+    _close((out, sh, sc), _reference(*args), "words T=%d H=%d L=%d B=%d" % (T, H, L, B))
+    if T > 1:   # a workgroup that stops writing: the others give up
+        assert so.fx_lstm_emul_words(*[t.data_ptr() for t in ts], out.data_ptr(), sh.data_ptr(), sc.data_ptr(), T, B, H, L, 2000, 5, 1) == 1
+
+
 def _gpu(x, wih, whh, bih, bhh, h0, c0, launches=1):
     """`launches` calls in a row on one workspace that is cleared once; the last call's results."""
     from functs_amd._lib import check, lib
@@ -171,6 +187,17 @@ def _gpu(x, wih, whh, bih, bhh, h0, c0, launches=1):
 def test_kernel_against_the_oracle(T, H, L, B):
     args = _inputs(T + H + L, T, H, L, B)
     _close(_gpu(*args), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,L,B", [(1, 64, 1, 16), (3, 32, 1, 2), (4, 32, 4, 5), (5, 64, 2, 4), (4, 128, 4, 3), (7, 256, 3, 8),
+                                     (3, 256, 2, 16), (3, 256, 4, 13), (5, 512, 2, 9), (4, 512, 3, 16), (3, 512, 4, 7), (3, 512, 1, 16)])
+def test_rows_of_a_batch_share_a_step(T, H, L, B):
+    """The form for several sequences: groups of four rows, full and ragged, one and two tiles of rows
+    a workgroup, every depth, two to eight waves, more finishing (layer, tile) pairs than waves; two
+    launches on one workspace."""
+    args = _inputs(T + H + L + B, T, H, L, B)
+    _close(_gpu(*args, launches=2), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
 
 
 @pytest.mark.gpu
