@@ -145,10 +145,18 @@ Batched launch(const char* op, int mode, const Tensor& boxes_, const Tensor& sco
   d.n_out = (uint32_t*)r.n.data_ptr<int32_t>();
   if (T > 0) {
     auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
-    Tensor ws = nmsWorkspaces().get(dev, (void*)stream.stream(), T, d.key_capacity);
-    d.workspace = ws.data_ptr();
-    d.workspace_bytes = (size_t)ws.numel();
-    FX_OK_OR_THROW(fx_sort_nms(&d, (void*)stream.stream()));
+    const size_t pairs = mode == 0 && !counts.defined() && T <= 65535 && K >= FX_NMS_PAIRS_MIN_ROWS && K <= FX_NMS_PAIRS_MAX_ROWS ? fx_nms_pairs_workspace_bytes((int)T, (uint32_t)K) : 0;
+    if (pairs > 0) {   // every box is a candidate: ranking and overlap tests over the whole chip
+      const Tensor ws = at::empty({(int64_t)pairs}, at::TensorOptions().dtype(at::kByte).device(dev));
+      d.workspace = ws.data_ptr();
+      d.workspace_bytes = pairs;
+      FX_OK_OR_THROW(fx_nms_pairs(&d, (void*)stream.stream()));
+    } else {
+      const Tensor ws = nmsWorkspaces().get(dev, (void*)stream.stream(), T, d.key_capacity);
+      d.workspace = ws.data_ptr();
+      d.workspace_bytes = (size_t)ws.numel();
+      FX_OK_OR_THROW(fx_sort_nms(&d, (void*)stream.stream()));
+    }
     // pinned blocks must not be handed out again before the launch has read / written them
     if (counts.defined() && counts.is_pinned())
       at::getHostAllocator(at::kCUDA)->record_event(counts.data_ptr(), counts.storage().data_ptr().get_context(), stream.unwrap());

@@ -50,6 +50,8 @@ uint32_t fx_cmap_chunk_rows();
 #include "fx_lstm_sched.h"
 int fx_launch_lstm_stack(const FxLstmArgs& a, int L, hipStream_t stream);
 int fx_launch_sort_nms(const fx_nms_desc& d, uint32_t key_cap, void* workspace, uint32_t* err_host, hipStream_t stream);
+size_t fx_nms_pairs_ws_bytes(int n_tasks, uint32_t rows);
+int fx_launch_nms_pairs(const fx_nms_desc& d, hipStream_t stream);
 size_t fx_nms_workspace_bytes(int n_tasks, uint32_t key_cap);
 size_t fx_nms_workspace_clear_bytes(int n_tasks);
 hipError_t fx_launch_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* cols, void* const* outs,
@@ -1608,6 +1610,32 @@ int fx_sort_nms(const fx_nms_desc* desc, void* stream_) {
   if (rc != 0) return fail(FX_E_HIP, std::string("fx_sort_nms: ") + hipGetErrorString((hipError_t)(rc - 100)));
   g_launches.fetch_add(1, std::memory_order_relaxed);
   g_spec_launches.fetch_add(1, std::memory_order_relaxed);
+  return FX_OK;
+}
+
+size_t fx_nms_pairs_workspace_bytes(int n_tasks, uint32_t rows) {
+  return n_tasks < 1 || rows < 1 || rows > FX_NMS_PAIRS_MAX_ROWS ? 0 : fx_nms_pairs_ws_bytes(n_tasks, rows);
+}
+
+int fx_nms_pairs(const fx_nms_desc* desc, void* stream_) {
+  if (!desc) return fail(FX_E_INVALID, "fx_nms_pairs: null descriptor");
+  const fx_nms_desc& d = *desc;
+  if (d.mode != 0 || d.counts) return fail(FX_E_INVALID, "fx_nms_pairs: mode 0 without counts only");
+  if (d.n_tasks < 0 || d.n_tasks > 65535) return fail(FX_E_LIMIT, "fx_nms_pairs: 0..65535 tasks");
+  if (!d.boxes || !d.scores || !d.dets || !d.out_labels || !d.n_out) return fail(FX_E_INVALID, "fx_nms_pairs: null argument");
+  if (((uintptr_t)d.boxes & 15u) != 0 || (d.boxes_task_stride & 3) != 0)
+    return fail(FX_E_INVALID, "fx_nms_pairs: boxes must be 16-byte aligned and their task stride a multiple of 4");
+  if (d.max_num < 1 || d.max_num > FX_NMS_MAX_OUT)
+    return fail(FX_E_LIMIT, "fx_nms_pairs: max_num must be 1.." + std::to_string(FX_NMS_MAX_OUT));
+  if (d.n_tasks == 0) return FX_OK;
+  const size_t need = fx_nms_pairs_workspace_bytes(d.n_tasks, d.rows);
+  if (need == 0) return fail(FX_E_LIMIT, "fx_nms_pairs: rows must be 1.." + std::to_string(FX_NMS_PAIRS_MAX_ROWS));
+  if (!d.workspace || ((uintptr_t)d.workspace & 255u) != 0 || d.workspace_bytes < need)
+    return fail(FX_E_INVALID, "fx_nms_pairs: workspace must be 256-byte aligned and hold fx_nms_pairs_workspace_bytes()");
+  const int rc = fx_launch_nms_pairs(d, (hipStream_t)stream_);
+  if (rc != 0) return fail(FX_E_HIP, std::string("fx_nms_pairs: ") + hipGetErrorString((hipError_t)(rc - 100)));
+  g_launches.fetch_add(3, std::memory_order_relaxed);
+  g_spec_launches.fetch_add(3, std::memory_order_relaxed);
   return FX_OK;
 }
 

@@ -1,0 +1,41 @@
+// What the kernels of the detection tail share (fx_nms.hip, fx_nms_pairs.hip): the order of the keys
+// and the overlap test.
+#pragma once
+#include "fx_device.h"
+
+namespace {
+
+__device__ __forceinline__ uint32_t orderable(float f) {   // monotone map float -> uint32
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float from_orderable(uint32_t o) {
+  return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
+}
+
+struct Box { float x1, y1, x2, y2; };
+
+__device__ __forceinline__ bool overlaps(const Box& a, float area_a, const Box& b, float area_b, float thr) {
+  const float xx1 = fmaxf(a.x1, b.x1), yy1 = fmaxf(a.y1, b.y1);
+  const float xx2 = fminf(a.x2, b.x2), yy2 = fminf(a.y2, b.y2);
+  const float w = fmaxf(0.0f, xx2 - xx1), h = fmaxf(0.0f, yy2 - yy1);
+  const float inter = w * h;
+  const float iou = inter / ((area_a + area_b) - inter);
+  return iou > thr;
+}
+
+// The same decision without the division, where that is certain: inter / union > thr is settled by
+// comparing inter with thr * union unless the two are within 2e-6 of each other (the product and the
+// quotient are off by at most 2^-24 relative each, 2e-6 is 2^-19), or the product is not an ordinary
+// number (thr <= 0, boxes of no or infinite area, NaN).
+__device__ __forceinline__ void overlaps_fast(const Box& a, float area_a, const Box& b, float area_b, float thr, bool& over, bool& sure) {
+  const float xx1 = fmaxf(a.x1, b.x1), yy1 = fmaxf(a.y1, b.y1);
+  const float xx2 = fminf(a.x2, b.x2), yy2 = fminf(a.y2, b.y2);
+  const float w = fmaxf(0.0f, xx2 - xx1), h = fmaxf(0.0f, yy2 - yy1);
+  const float inter = w * h;
+  const float t = thr * ((area_a + area_b) - inter);
+  over = inter > t * 1.000002f;
+  sure = t > 1e-30f && t < 1e30f && (over || inter < t * 0.999998f);
+}
+
+}  // namespace

@@ -30,7 +30,7 @@
 #include <mutex>
 
 #include "../../../include/fxhip.h"
-#include "fx_device.h"
+#include "fx_nms.h"
 
 // a hook for timing the phases of a task's last workgroup from a test program; nothing in the library
 #ifndef FX_NMS_STAMP
@@ -42,14 +42,6 @@
 
 namespace {
 
-__device__ __forceinline__ uint32_t orderable(float f) {   // monotone map float -> uint32
-  const uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float from_orderable(uint32_t o) {
-  return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
-}
-
 // one stage of the bitonic network on a key a lane, partners J lanes apart: the lower lane keeps
 // the smaller key where the run ascends
 template <uint32_t J>
@@ -57,17 +49,6 @@ __device__ __forceinline__ uint64_t bitonic_step(uint64_t key, bool up, uint32_t
   const uint64_t other = ((uint64_t)fx_lane_xor<J>((uint32_t)(key >> 32), lane) << 32) | (uint64_t)fx_lane_xor<J>((uint32_t)key, lane);
   const bool keep_min = ((lane & J) == 0u) == up;
   return ((key < other) == keep_min) ? key : other;
-}
-
-struct Box { float x1, y1, x2, y2; };
-
-__device__ __forceinline__ bool overlaps(const Box& a, float area_a, const Box& b, float area_b, float thr) {
-  const float xx1 = fmaxf(a.x1, b.x1), yy1 = fmaxf(a.y1, b.y1);
-  const float xx2 = fminf(a.x2, b.x2), yy2 = fminf(a.y2, b.y2);
-  const float w = fmaxf(0.0f, xx2 - xx1), h = fmaxf(0.0f, yy2 - yy1);
-  const float inter = w * h;
-  const float iou = inter / ((area_a + area_b) - inter);
-  return iou > thr;
 }
 
 // workspace: per task FX_NMS_WS_WORDS counters (candidates, finished slices, largest coordinate,

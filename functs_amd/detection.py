@@ -94,11 +94,18 @@ def _launch(mode, boxes, scores, factors, labels, counts, n_classes, score_thr, 
     d.key_capacity = key_capacity
     d.dets, d.out_labels, d.out_index, d.n_out = dets.data_ptr(), out_labels.data_ptr(), out_index.data_ptr(), n_out.data_ptr()
     stream = torch.cuda.current_stream(dev)
-    if T > 0:
+    # every box a candidate: ranking and overlap tests over the whole chip
+    pairs = 0
+    if mode == 0 and counts is None and 0 < T <= 65535 and C["FX_NMS_PAIRS_MIN_ROWS"] <= rows <= min(C["FX_NMS_PAIRS_MAX_ROWS"], key_capacity):
+        pairs = lib.fx_nms_pairs_workspace_bytes(T, rows)
+    if pairs > 0:
+        ws = torch.empty(pairs, dtype=torch.uint8, device=dev)
+        d.workspace, d.workspace_bytes = ws.data_ptr(), pairs
+    elif T > 0:
         ws = _workspace(dev, stream, T, key_capacity)
         d.workspace, d.workspace_bytes = ws.data_ptr(), ws.numel()
     with torch.cuda.device(dev):
-        check(lib.fx_sort_nms(ctypes.byref(d), ctypes.c_void_p(stream.cuda_stream)))
+        check((lib.fx_nms_pairs if pairs > 0 else lib.fx_sort_nms)(ctypes.byref(d), ctypes.c_void_p(stream.cuda_stream)))
     return NmsResult(dets, out_labels, out_index, n_out, stream)
 
 

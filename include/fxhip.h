@@ -511,6 +511,15 @@ typedef struct fx_nms_desc {
 size_t fx_sort_nms_workspace_bytes(int n_tasks, uint32_t key_capacity);
 size_t fx_sort_nms_workspace_clear_bytes(int n_tasks);
 int fx_sort_nms(const fx_nms_desc* desc, void* stream);
+/* The same results for boxes that are all candidates (mode 0, counts null), up to FX_NMS_PAIRS_MAX_ROWS
+ * rows, as three launches that spread the ranking and the overlap tests over the chip.  Below
+ * FX_NMS_PAIRS_MIN_ROWS fx_sort_nms is as fast: two chunks of boxes are too little to spread (a call,
+ * 64 rows: 27.0 us against 25.6; 100: 28.1 against 27.7; 200: 29.3 against 33.9; 2 000: 47 against 157).  Its workspace is
+ * scratch memory (256-byte aligned, nothing is expected in it or left in it); key_capacity is not read. */
+#define FX_NMS_PAIRS_MIN_ROWS 129
+#define FX_NMS_PAIRS_MAX_ROWS 4096 /* 64 chunks of 64 */
+size_t fx_nms_pairs_workspace_bytes(int n_tasks, uint32_t rows); /* 0: more rows than that, or none */
+int fx_nms_pairs(const fx_nms_desc* desc, void* stream);
 
 /* ---- device utilities ---- */
 int fx_device_count(void);

@@ -286,3 +286,36 @@ def test_compaction_feeds_the_tail_without_the_host():
         dets, labels, index = onms.multiclass_nms(boxes[t].cpu(), cls[t].cpu(), obj[t].cpu())
         assert got[t][2].cpu().tolist() == index.tolist() and torch.equal(got[t][0].cpu(), dets) and torch.equal(got[t][1].cpu(), labels)
     assert int(res.n.sum()) > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,classes,max_num", [(1, 1, 5), (128, 3, 64), (129, 1, 7), (192, 1, 1024), (193, 2, 1), (1000, 80, 1024), (1025, 1, 300),
+                                               (2048, 5, 1024), (3000, 60, 100), (4095, 1, 1024), (4096, 9, 1024), (4097, 3, 1024)])
+def test_boxes_that_are_all_candidates_take_three_launches_with_the_same_result(n, classes, max_num):
+    """fx_nms_pairs against fx_sort_nms (which a call with counts takes) bit for bit, three images: ties,
+    scores that are no candidates (NaN, -inf), boxes without area, with infinite and NaN corners, and
+    overlaps exactly at the threshold; one row more than it takes goes to fx_sort_nms."""
+    from functs_amd import aot, detection
+    g = torch.Generator().manual_seed(n)
+    T = 3
+    b = torch.stack([_boxes(g, n, span=100.0 + 400.0 * t) for t in range(T)])
+    b[2, : n // 2] = b[2, : n // 2].round()                       # whole corners: many overlaps are simple fractions
+    s = torch.rand(T, n, generator=g)
+    s[1, n // 2:] = s[1, : n - n // 2].clone()
+    lab = torch.randint(0, classes, (T, n), generator=g)
+    if n >= 64:
+        s[0, 3], s[0, 17], s[0, 40] = float("nan"), float("-inf"), -2.0
+        b[0, 5, 2:] = b[0, 5, :2]
+        b[0, 9, 0] -= 500.0
+        b[1, 11, 1] = float("nan")
+    dev = torch.device("cuda:0")
+    args = (b.to(dev), s.to(dev), lab.to(dev))
+    for thr in (0.5, 0.0):
+        print("fx_nms_pairs n=%d classes=%d max_num=%d thr=%g" % (n, classes, max_num, thr), flush=True)
+        l0, _ = aot.launch_stats()
+        got = detection.batched_nms_batched(*args, iou_threshold=thr, max_num=max_num)
+        l1, _ = aot.launch_stats()
+        assert l1 - l0 == (3 if 128 < n <= 4096 else 1)
+        want = detection.batched_nms_batched(*args, counts=torch.full((T,), n, dtype=torch.int32, device=dev), iou_threshold=thr, max_num=max_num)
+        assert torch.equal(got.n, want.n) and torch.equal(got.index, want.index) and torch.equal(got.labels, want.labels)
+        assert torch.equal(got.dets.view(torch.int32), want.dets.view(torch.int32))
