@@ -285,6 +285,11 @@ static const FxSpecKernels* spec_of(const fx::Plan* p) {
   return fx_spec_find(p->spec_key);
 }
 
+static const bool g_spec_linked_set = [] {
+  fx::spec_linked = [](uint64_t key) { return g_specialize.load(std::memory_order_relaxed) && key != 0 && fx_spec_find(key) != nullptr; };
+  return true;
+}();
+
 // With a dump directory set, every plan that has no specialised kernels linked in leaves
 // the translation unit that would specialise it there (one file per key).
 static void dump_spec_source(const fx::Plan* p) {

@@ -206,7 +206,9 @@ struct FxOut {
                                   // immediate operands follow: FX_K items are interpreted as one batch
   uint32_t rowseg;                // rowwave: lanes per row (16, 32 or 64); a wave holds 64 / rowseg rows and
                                   // FX_WMAX / FX_WSUM reduce inside each segment of rowseg lanes
-  uint32_t pad[2];
+  uint32_t box;                   // dense: 0, or 1 + the affine record of the element offsets in the output (a program
+                                  // for a box of the output's elements: dim, numel, inner ... are those of the box)
+  uint32_t pad[1];
 };
 
 

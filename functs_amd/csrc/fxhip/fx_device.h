@@ -1229,6 +1229,8 @@ __global__ __launch_bounds__(FX_BLOCK, 4) void fx_region_dense(const uint32_t* _
     const uint32_t n_items = rowwave ? (n_rows_w + rows_per_item - 1) / rows_per_item : (n_groups + 63u) / 64u;
     if (item0 >= n_items) continue;
 
+    const uint32_t box = uni(od[FX_W(FxOut, box)]);   // elements of a box: their offsets are an affine map of their coordinates
+    bool contig = true;
     auto make_item = [&](uint32_t k, uint32_t (&e)[FX_V], uint32_t& M, FxCoord<R>& q) {
       uint32_t row, col0;
       bool live;
@@ -1257,6 +1259,12 @@ __global__ __launch_bounds__(FX_BLOCK, 4) void fx_region_dense(const uint32_t* _
       q.step = 1;
       const uint32_t rem = fx_unflatten<R>(row, vd, dk, mk, sk, q.c0);
       q.c0[0] = vd == 0 ? 0 : (int32_t)rem;
+      if (box) {
+        int32_t off[FX_V];
+        contig = fx_affine<R>(cx, q, (int32_t)box - 1, 0, 0, off);
+#pragma unroll
+        for (int j = 0; j < FX_V; ++j) e[j] = (uint32_t)off[j];
+      }
     };
 
     if (uni(od[FX_W(FxOut, pure)]) && kmax == FX_K && item0 + FX_K <= n_items) {
@@ -1303,7 +1311,7 @@ __global__ __launch_bounds__(FX_BLOCK, 4) void fx_region_dense(const uint32_t* _
           A[j] = lead ? v : 0u;
         }
         S::template run<R>(cx, lead ? pb + 1 : pb, pe, q, M, A);
-        fx_store_vec(op, obase, e, M, true, odt, ovt, A);
+        fx_store_vec(op, obase, e, M, contig, odt, ovt, A);
       }
     }
   }

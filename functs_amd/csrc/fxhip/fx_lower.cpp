@@ -233,6 +233,16 @@ struct SlotAlloc {
 
 struct Prog { uint32_t begin, end, vt; bool rowwave; bool wide; };
 
+// A box of an output's elements: first coordinate and extent per dimension.
+struct Box {
+  Shape lo, n;
+  static Box whole(const Shape& s) { Box b; b.lo.assign(s.size(), 0); b.n = s; return b; }
+};
+// Where a program's first condition on one output coordinate changes its answer: the box is cut
+// there, and each part's program no longer asks.
+struct Cut { int dim = -1; std::vector<int64_t> at; };   // coordinates inside the box, ascending
+#define FX_MAX_BOXES 24
+
 class Lowerer {
  public:
   Lowerer(const Region& R, const std::vector<const fx_arg*>& in, int n_tasks, SlotAlloc& slots)
@@ -250,6 +260,18 @@ class Lowerer {
   // says that the low-word program moved int64 data as it is, so that the high words need a
   // program of their own; otherwise the result fits 32 bits and its store sign-extends.
   Prog lower(int vid, const Shape& rootShape, int half = 0);
+  // The program of the elements of one box; its root coordinates are those of the box whose extent
+  // is not 1 (boxDims).  cut (may be null) receives the first place where the box can be cut.
+  Prog lowerBox(int vid, const Box& b, Cut* cut, int half = 0);
+  // The boxes an output is computed in: one (the whole output) unless cutting pays.
+  std::vector<Box> boxesOf(int vid, const Shape& s, const Prog& whole);
+  static Shape boxDims(const Box& b) {
+    Shape r;
+    for (int64_t n : b.n) if (n != 1) r.push_back(n);
+    if (r.empty()) r.push_back(1);
+    return r;
+  }
+  int boxAffine(const Box& b, const Shape& s);   // affine record: element offset in the output of a box's element
 
  private:
   const Region& R_;
@@ -269,6 +291,10 @@ class Lowerer {
   bool loopVarBound_ = false;
   IdxExpr loopVar_;
   bool usedRowWave_ = false;
+  Cut* cut_ = nullptr;        // while a program is tried: where its output could be cut
+  int cutDim_[FX_MAXR];       // output dimension of every root coordinate
+  Prog lowerFrame(int vid, const Shape& rootShape, const Frame& f, int half);
+  void noteCut(const IdxExpr& x, int64_t lo, int64_t hi, int64_t step);
   // int64 outputs: while only movement operators (views, *_rev merges, cat, index, where ...)
   // lie between a value and the output, the value travels word by word and is exact
   bool moveCtx_ = false;
@@ -1230,6 +1256,7 @@ void Lowerer::emitBinary(uint16_t op, const Operand& l, const Operand& r, uint32
 void Lowerer::emitCond(const IdxExpr& x, int64_t lo, int64_t hi, int64_t step, const std::function<void()>& thenFn,
                        const std::function<void()>& elseFn) {
   FX_CHECK(maskDepth_ + 1 <= FX_MASK_DEPTH, FX_E_LIMIT, "predicated regions nested deeper than " << FX_MASK_DEPTH);
+  if (cut_ && cut_->dim < 0) noteCut(x, lo, hi, step);
   const size_t before = code.size();
   emitIdx(x);
   auto fit = [](int64_t v) { return (int32_t)std::min<int64_t>(std::max<int64_t>(v, std::numeric_limits<int32_t>::min()), std::numeric_limits<int32_t>::max()); };
@@ -1711,6 +1738,113 @@ bool Lowerer::rowWaveFrame(const Frame& f, int d, int64_t extent) const {
 
 Prog Lowerer::lower(int vid, const Shape& rootShape, int half) {
   FX_CHECK(rootShape.size() <= FX_MAXR, FX_E_UNSUPPORTED, "region outputs above rank " << FX_MAXR << " are not supported");
+  Frame f(rootShape.size());
+  for (size_t i = 0; i < f.size(); ++i) f[i] = IdxExpr::root((int)i);
+  return lowerFrame(vid, rootShape, f, half);
+}
+
+Prog Lowerer::lowerBox(int vid, const Box& b, Cut* cut, int half) {
+  Frame f(b.n.size());
+  int k = 0;
+  for (size_t i = 0; i < f.size(); ++i) {
+    if (b.n[i] == 1) { f[i] = IdxExpr(b.lo[i]); continue; }
+    cutDim_[k] = (int)i;
+    f[i] = IdxExpr::root(k++) + IdxExpr(b.lo[i]);
+  }
+  cut_ = cut;
+  Prog p = lowerFrame(vid, boxDims(b), f, half);
+  cut_ = nullptr;
+  return p;
+}
+
+// lo <= x < hi (x - lo a multiple of step) with x = +-(one root coordinate) + constant: the root
+// coordinates where the answer changes.  A lattice of a step above 1 is cut into single
+// coordinates while the dimension is short (the columns of a box table).
+void Lowerer::noteCut(const IdxExpr& x, int64_t lo, int64_t hi, int64_t step) {
+  if (!x.affine() || x.ct != 0) return;
+  for (auto c : x.rc) if (c) return;
+  int k = -1;
+  for (int i = 0; i < FX_MAXR; ++i) {
+    if (!x.c[i]) continue;
+    if (k >= 0 || (x.c[i] != 1 && x.c[i] != -1)) return;
+    k = i;
+  }
+  if (k < 0 || k >= rootRank_) return;
+  const int64_t n = rootDim_[k];
+  std::vector<int64_t> at;
+  if (step == 1) {
+    // x = r + k0: r in [lo - k0, hi - k0); x = k0 - r: r in [k0 - hi + 1, k0 - lo + 1)
+    const int64_t a = x.c[k] == 1 ? lo - x.k : x.k - hi + 1, e = x.c[k] == 1 ? hi - x.k : x.k - lo + 1;
+    if (a > 0 && a < n) at.push_back(a);
+    if (e > 0 && e < n && e > a) at.push_back(e);
+  } else if (n <= 8) {
+    for (int64_t i = 1; i < n; ++i) at.push_back(i);
+  }
+  if (at.empty()) return;
+  cut_->dim = cutDim_[k];
+  cut_->at = at;
+}
+
+// Long programs are long because every element carries the code of every element: nested range
+// tests for the parts of cat / stack / in-place slices (the corners of a box table, the levels of a
+// pyramid), each with the whole computation of its part behind it.  Cut where those tests change
+// their answer, a part's program is its own computation only (box regression: 1 553 instructions
+// of 17 predicates deep against four straight ones).  Kept whole: programs short enough to be bound by
+// their launch, rows reduced across a wave (their lanes must hold the whole row), int64 outputs
+// (two programs a word pair), and cuts that do not halve the instructions an element stands for.
+// Interpreted, MI355X: box regression of 8 732 x 21 boxes 518 -> 60 us (1 553 instructions -> four times
+// 103), the YOLO head of four 608 x 608 images with its NMS 743 -> 270 us (18 boxes).
+std::vector<Box> Lowerer::boxesOf(int vid, const Shape& s, const Prog& whole) {
+  const std::vector<Box> one{Box::whole(s)};
+  const size_t len = whole.end - whole.begin;
+  const int64_t numel = numel_of(s);
+  if (s.empty() || len < 32 || whole.rowwave || V(vid).dtype == FX_DT_I64 || numel == 0 || numel >= ((int64_t)1 << 31)) return one;
+  const std::vector<FxInsn> code0 = code;
+  const std::vector<FxAffine> affs0 = affs;
+  const int temps0 = maxTemps;
+  std::vector<Box> todo = one, done;
+  size_t total = 0;
+  double work = 0;
+  while (!todo.empty()) {
+    Box b = todo.back();
+    todo.pop_back();
+    Cut cut;
+    const Prog p = lowerBox(vid, b, &cut);
+    if (cut.dim >= 0 && done.size() + todo.size() + cut.at.size() + 1 <= FX_MAX_BOXES) {
+      const int64_t lo = b.lo[(size_t)cut.dim], n = b.n[(size_t)cut.dim];
+      cut.at.push_back(n);
+      for (size_t i = cut.at.size(); i-- > 0;) {
+        Box q = b;
+        const int64_t from = i ? cut.at[i - 1] : 0;
+        q.lo[(size_t)cut.dim] = lo + from;
+        q.n[(size_t)cut.dim] = cut.at[i] - from;
+        todo.push_back(q);   // (the first part on top: boxes come out in output order)
+      }
+    } else {
+      done.push_back(b);
+      total += p.end - p.begin;
+      work += (double)(p.end - p.begin) * (double)numel_of(b.n);
+    }
+  }
+  code = code0;
+  affs = affs0;
+  maxTemps = temps0;
+  if (done.size() < 2 || total > len || work * 2 > (double)len * (double)numel) return one;
+  return done;
+}
+
+int Lowerer::boxAffine(const Box& b, const Shape& s) {
+  const Shape st = contiguous_strides(s);
+  IdxExpr e(0);
+  int k = 0;
+  for (size_t i = 0; i < s.size(); ++i) {
+    e.k += b.lo[i] * st[i];
+    if (b.n[i] != 1) e.c[k++] = st[i];
+  }
+  return addAffine(e);
+}
+
+Prog Lowerer::lowerFrame(int vid, const Shape& rootShape, const Frame& f, int half) {
   rootRank_ = (int)rootShape.size();
   for (int i = 0; i < FX_MAXR; ++i) rootDim_[i] = i < rootRank_ ? rootShape[i] : 1;
   tempTop_ = 0;
@@ -1720,8 +1854,6 @@ Prog Lowerer::lower(int vid, const Shape& rootShape, int half) {
   moveCtx_ = V(vid).kind == VK_TENSOR && V(vid).dtype == FX_DT_I64;
   half_ = moveCtx_ ? half : 0;
   sawWide_ = false;
-  Frame f(rootRank_);
-  for (int i = 0; i < rootRank_; ++i) f[i] = IdxExpr::root(i);
   Prog p;
   p.begin = (uint32_t)code.size();
   emit(vid, f);
@@ -1853,13 +1985,25 @@ static bool findWindow(const ClassBuild& cb, StreamInfo* si, std::vector<WinPick
 // ---------------------------------------------------------------------------
 // plan construction
 // ---------------------------------------------------------------------------
-static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args);
+bool (*spec_linked)(uint64_t) = nullptr;
+
+static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args, bool boxed, bool* could_box);
 
 const Plan* plan_region(Region& R, const fx_arg* args, int n_args) {
   R.index_ints.resize(R.inputs.size(), 0);
   for (;;) {
     try {
-      return plan_region_once(R, args, n_args);
+      // Outputs are computed whole where the region has compiled kernels for that (one store of whole
+      // groups an item, temporaries in registers; the lean kernel), in boxes otherwise if that pays
+      // (Lowerer::boxesOf) and the descriptor still fits.
+      bool could_box = false;
+      const Plan* whole = plan_region_once(R, args, n_args, false, &could_box);
+      if (!could_box || (spec_linked && spec_linked(whole->spec_key))) return whole;
+      try {
+        return plan_region_once(R, args, n_args, true, nullptr);
+      } catch (const Error&) {
+        return whole;
+      }
     } catch (const NeedIndexInt& need) {
       FX_CHECK(need.input >= 0 && need.input < (int)R.index_ints.size() && !R.index_ints[need.input], FX_E_INVALID,
                "per-task int input " << need.input << " cannot be resolved");
@@ -1868,7 +2012,8 @@ const Plan* plan_region(Region& R, const fx_arg* args, int n_args) {
   }
 }
 
-static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args) {
+// boxed: outputs in boxes, in the place of the plan of whole outputs that could_box was set for
+static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args, bool boxed_outs, bool* could_box) {
   FX_CHECK(R.finalized, FX_E_INVALID, "region is not finalized");
   const int T = R.degree;
   // argument layout
@@ -1900,7 +2045,7 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args) {
     }
   }
   auto it = R.plans.find(key);
-  if (it != R.plans.end()) return it->second.get();
+  if (it != R.plans.end() && !boxed_outs) return it->second.get();
 
   std::unique_ptr<Plan> P(new Plan());
   P->region = &R;
@@ -1996,22 +2141,36 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args) {
                "output " << o << " is 4 GiB or larger; split the region");
       for (int t : cb.tasks) P->out_shape[o][t] = s;
       // an int64 output that moves int64 data is two records, one per 32-bit word
+      const size_t code0 = L.code.size(), affs0 = L.affs.size();
+      const int temps0 = L.maxTemps;
       Prog p0 = L.lower(R.outputs[o], s);
-      for (int half = 0; half < (p0.wide ? 2 : 1); ++half) {
-      Prog p = half == 0 ? p0 : L.lower(R.outputs[o], s, 1);
+      std::vector<Box> boxes(1);
+      if (P->mode == FX_MODE_DENSE) boxes = L.boxesOf(R.outputs[o], s, p0);
+      if (!boxed_outs && boxes.size() > 1) { *could_box = true; boxes.resize(1); }
+      if (boxes.size() > 1) {   // the boxes' programs stand in the place of the whole one
+        L.code.resize(code0);
+        L.affs.resize(affs0);
+        L.maxTemps = temps0;
+      }
+      for (int part = 0; part < (boxes.size() > 1 ? (int)boxes.size() : p0.wide ? 2 : 1); ++part) {
+      const bool boxed = boxes.size() > 1;
+      const int half = boxed ? 0 : part;
+      const Prog p = boxed ? L.lowerBox(R.outputs[o], boxes[(size_t)part], nullptr) : half == 0 ? p0 : L.lower(R.outputs[o], s, 1);
+      const Shape dims = boxed ? Lowerer::boxDims(boxes[(size_t)part]) : s;
       FxOut od;
       memset(&od, 0, sizeof(od));
       od.prog_begin = p.begin;
       od.prog_end = p.end;
       od.vt = p.vt;
-      fillDims(od, s);
-      od.numel = (uint32_t)numel_of(s);
+      fillDims(od, dims);
+      od.numel = (uint32_t)numel_of(dims);
+      if (boxed) od.box = 1u + (uint32_t)L.boxAffine(boxes[(size_t)part], s);
       od.dtype = p0.wide ? (half ? FX_I64HI : FX_I64LO) : storage_dt(P->out_dtype[o]);
       od.ptr_slot = (uint32_t)out_slot[o];
       od.task_stride = 0;
       if (p.rowwave) {
         od.rowwave = 1;
-        od.rowlen = (uint32_t)s.back();
+        od.rowlen = (uint32_t)dims.back();
         const uint32_t lanes = (od.rowlen + FX_V - 1) / FX_V;
         od.rowseg = lanes <= 16 ? 16u : (lanes <= 32 ? 32u : 64u);
       }
@@ -2019,7 +2178,7 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args) {
         // leading load: unconditional, affine, not inside a reduction loop
         const FxInsn& i0 = L.code[p.begin];
         od.lead = (p.end > p.begin && i0.op == FX_LDA) ? 1u : 0u;
-        bool pure = od.lead != 0 && !p.rowwave;
+        bool pure = od.lead != 0 && !p.rowwave && !boxed;
         for (uint32_t pc = p.begin + 1; pure && pc < p.end; ++pc) {
           const FxInsn& in = L.code[pc];
           pure = fx_op_is_pure_unary(in.op) || (fx_op_is_pure_binary(in.op) && (in.flags & FX_F_IMM));
@@ -2040,7 +2199,7 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args) {
         fx_fastdiv_make(std::max<uint32_t>(od.gprow, 1), &od.gr_magic, &od.gr_shift);
         if (od.colmajor) od.pure = 0;
       }
-      max_rank = std::max<int>(max_rank, (int)s.size());
+      max_rank = std::max<int>(max_rank, (int)dims.size());
       cb.outs.push_back(od);
       }
     }
@@ -2272,7 +2431,7 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args) {
     bool fits = taskmap.size() == (size_t)T;
     for (size_t i = 0; fits && i < taskmap.size(); ++i) fits = taskmap[i] == (uint32_t)i;
     for (const FxOut& od : cb.outs)
-      fits = fits && ((od.dtype == FX_F32 && od.vt == FX_VT_F) || (od.dtype == FX_I32 && od.vt == FX_VT_I));
+      fits = fits && od.box == 0 && ((od.dtype == FX_F32 && od.vt == FX_VT_F) || (od.dtype == FX_I32 && od.vt == FX_VT_I));
     if (fits) {
       FxLeanArgs& f = P->lean;
       f.blob_words = (uint32_t)blob.size();

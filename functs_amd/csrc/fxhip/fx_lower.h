@@ -150,6 +150,8 @@ void match_head(Plan* p);
 // Fills p->cmap: does the plan compute the decode + per-class score filter of an SSD-style head (fx_cmap_match.cpp)?
 void match_classmap(Plan* p);
 
+// Whether compiled kernels are at hand for a spec_hash (set by the library; null: none are).
+extern bool (*spec_linked)(uint64_t key);
 // Builds (or fetches from the cache) the plan of `r` for these arguments.
 const Plan* plan_region(Region& r, const fx_arg* args, int n_args);
 std::string disasm(const Plan& p);

@@ -320,6 +320,18 @@ extern "C" int fx_emul_run_tables(const uint32_t* sb, size_t n_words, const uint
         for (uint32_t oi = 0; oi < cl.n_outs; ++oi) {
           const FxOut& od = outs[oi];
           void* op = (void*)ptr_of(cx, (int32_t)od.ptr_slot);
+          // element of the output that element e of the record's coordinate space is
+          auto place = [&](uint32_t e) -> int64_t {
+            int64_t off = e;
+            if (od.box) {
+              const FxAffine& a = cx.aff[od.box - 1];
+              int32_t c[FX_MAXR];
+              decompose(od, e, c);
+              off = a.base;
+              for (int k = 0; k < FX_MAXR; ++k) off += (int64_t)fx_aff_coef(&a, k) * c[k];
+            }
+            return (int64_t)od.task_stride * task + off;
+          };
           if (od.rowwave) {
             const uint32_t rows = od.rowlen ? od.numel / od.rowlen : 0;
             for (uint32_t r = 0; r < rows; ++r) {
@@ -327,7 +339,7 @@ extern "C" int fx_emul_run_tables(const uint32_t* sb, size_t n_words, const uint
               for (uint32_t k = 0; k < od.rowlen; ++k) decompose(od, r * od.rowlen + k, L[k].c);
               run(cx, (int)od.prog_begin, (int)od.prog_end, L);
               for (uint32_t k = 0; k < od.rowlen; ++k)
-                store_elem(op, (int64_t)od.task_stride * task + r * od.rowlen + k, od.dtype, od.vt, L[k].A);
+                store_elem(op, place(r * od.rowlen + k), od.dtype, od.vt, L[k].A);
             }
             continue;
           }
@@ -335,7 +347,7 @@ extern "C" int fx_emul_run_tables(const uint32_t* sb, size_t n_words, const uint
             int32_t c[FX_MAXR];
             decompose(od, e, c);
             uint32_t v = run1(cx, (int)od.prog_begin, (int)od.prog_end, c);
-            store_elem(op, (int64_t)od.task_stride * task + e, od.dtype, od.vt, v);
+            store_elem(op, place(e), od.dtype, od.vt, v);
           }
         }
       } else {

@@ -1,0 +1,114 @@
+"""Outputs computed in boxes of their elements (fx_lower.cpp, Lowerer::boxesOf): one program per box,
+cut where the range tests of cat / stack / in-place slices change their answer.  Values against
+stock PyTorch at extents around lane groups and work items, for the emulator and the GPU."""
+import re
+
+import pytest
+import torch
+
+from functs_amd import Region
+from tests.util import assert_close, assert_exact, run_region
+
+# a corner is the difference of a centre and half a size of at most e^4 / 2 = 27.3, whose exponentials
+# differ by a few units in the last place: four of them (2^-23 * 27.3 each) whatever the difference is
+CANCELLED = 4 * 27.3 * 2.0 ** -23
+BACKENDS = ["emul", pytest.param("hip", marks=pytest.mark.gpu)]
+
+
+def corners(x, a):
+    """x [n, 4], a [m, 4]: a cat over rows of two corner decodes, then in-place edits of columns."""
+    def decode(t, scale):
+        xy, wh = t[:, :2] * scale, t[:, 2:].clamp(-4.0, 4.0).exp() * 0.5
+        return torch.cat([xy - wh, xy + wh], 1)
+    r = torch.cat([decode(x, 0.1), decode(a, 0.2)], 0)
+    r[:, 0::2] = r[:, 0::2].clamp(0.0, 9.0)
+    r[:, 3] = r[:, 1] + 1.0
+    return r
+
+
+def corners_region(n, m, per_task=0):
+    r = Region(max(per_task, 1), per_task > 0)
+    x, a = r.tensor_input(rank=2, per_task=per_task > 0), r.tensor_input(rank=2)
+
+    def decode(t, scale):
+        xy, wh = t.slice(1, 0, 2) * scale, t.slice(1, 2, 4).clamp(-4.0, 4.0).exp() * 0.5
+        return r.cat([xy - wh, xy + wh], 1)
+    v = r.cat([decode(x, 0.1), decode(a, 0.2)], 0)
+    v = v.slice_rev(v.slice(1, 0, 4, 2).clamp(0.0, 9.0), 1, 0, 4, 2)
+    v = v.select_rev(v.select(1, 1) + 1.0, 1, 3)
+    r.output(v)
+    r.finalize()
+    return r
+
+
+def n_programs(region, *args):
+    return int(re.search(r"n_entries = (\d+)", region.spec_source(*args)).group(1))
+
+
+@pytest.mark.parametrize("backend", BACKENDS)
+@pytest.mark.parametrize("n,m", [(1, 1), (3, 5), (64, 1), (63, 193), (257, 300), (1025, 2)])
+def test_rows_and_columns(backend, n, m):
+    g = torch.Generator().manual_seed(n)
+    x, a = torch.randn(n, 4, generator=g) * 30, torch.randn(4, m, generator=g).t()   # (a: strides 1, m)
+    r = corners_region(n, m)
+    (got,) = run_region(backend, r, x, a)
+    assert_close(got, corners(x, a), atol=CANCELLED)
+    assert n_programs(r, x, a) == 8   # two parts of four columns
+
+
+@pytest.mark.parametrize("backend", BACKENDS)
+def test_tasks_of_a_map(backend):
+    g = torch.Generator().manual_seed(7)
+    xs, a = [torch.randn(n, 4, generator=g) for n in (65, 65, 30)], torch.randn(9, 4, generator=g)   # two task classes
+    r = corners_region(65, 9, per_task=3)
+    (got,) = run_region(backend, r, xs, a)
+    for o, x in zip(got, xs):
+        assert_close(o, corners(x, a), atol=CANCELLED)
+
+
+@pytest.mark.parametrize("backend", BACKENDS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16, torch.int32, torch.int64])
+@pytest.mark.parametrize("dims", [(5, 7), (2, 3, 131)])
+def test_types_and_whole_groups(backend, dtype, dims):
+    """Many narrow parts along the last dimension, odd widths: boxes that end inside a lane group."""
+    if backend == "emul" and dtype == torch.float16:
+        pytest.skip("the emulator has no fp16")
+    g = torch.Generator().manual_seed(3)
+    parts = [torch.randint(-9, 9, dims[:-1] + (w,), generator=g).to(dtype) for w in (dims[-1], 1, 2, 4, 6)]
+    r = Region()
+    ins = [r.tensor_input(dtype, len(dims)) for _ in parts]
+    last = len(dims) - 1
+    r.output(r.cat([(v + 1) * 2 if i % 2 else v * 3 - 1 for i, v in enumerate(ins)] + [v + 5 - 2 for v in ins], last))
+    r.finalize()
+    ref = torch.cat([(v + 1) * 2 if i % 2 else v * 3 - 1 for i, v in enumerate(parts)] + [v + 5 - 2 for v in parts], last)
+    (got,) = run_region(backend, r, *parts)
+    assert_exact(got, ref)
+    assert (n_programs(r, *parts) > 2) == (dtype != torch.int64)
+
+
+@pytest.mark.parametrize("backend", BACKENDS)
+@pytest.mark.parametrize("w", [8, 33, 200])
+def test_a_reduction_inside_a_box(backend, w):
+    """A softmax whose rows are one box of the output: its rows are reduced across a wave."""
+    g = torch.Generator().manual_seed(w)
+    x, y = torch.randn(37, w, generator=g), torch.randn(37, 3, generator=g)
+    r = Region()
+    a, b = r.tensor_input(rank=2), r.tensor_input(rank=2)
+    r.output(r.cat([b * 2.0 + 1.0, b.sigmoid(), a.softmax(1), b.exp() - 1.0, (b + 3.0) * 0.5, b.tanh()], 1))
+    r.finalize()
+    (got,) = run_region(backend, r, x, y)
+    assert_close(got, torch.cat([y * 2 + 1, y.sigmoid(), x.softmax(1), y.exp() - 1, (y + 3) * 0.5, y.tanh()], 1), rtol=2e-6, atol=1e-6)
+
+
+def test_what_stays_whole():
+    # a triangle's test moves with two coordinates, an index's with data: no box answers them
+    r = Region()
+    a = r.tensor_input(rank=2)
+    r.output(r.op("TRIU", a.exp() + a.sigmoid() * 2.0 - 1.0, 0))
+    r.finalize()
+    assert n_programs(r, torch.randn(9, 9)) == 1
+    r = Region()
+    a = r.tensor_input(rank=2)
+    r.output(r.cat([a, a + 1.0], 0))   # short
+    r.finalize()
+    assert n_programs(r, torch.randn(9, 9)) == 1
