@@ -14,6 +14,7 @@ namespace {
 #define FX_AS1 __attribute__((address_space(1)))
 #define FX_AS4 __attribute__((address_space(4)))
 typedef uint32_t fx_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t fx_u16x4_a2 __attribute__((ext_vector_type(4), aligned(2)));  // 64 bits, 2-byte aligned
 typedef uint32_t fx_u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // 128 bits, 4-byte aligned
 
 // word offset of a field inside a blob structure
@@ -83,6 +84,19 @@ __device__ __forceinline__ void fx_load_vec(uint64_t base_, const int32_t (&off)
     }
     return;
   }
+  // the same for 16-bit elements: one 64-bit load per lane, 2-byte alignment
+  if (consecutive && (dt == FX_F16 || dt == FX_BF16) && !wave_any(M != 0u && M != VM) && wave_any(M == VM)) {
+    const uint32_t o0 = M ? (uint32_t)off[0] : 0u;
+    const fx_u16x4_a2 v = *(const FX_AS1 fx_u16x4_a2*)(base + (o0 << 1));
+    if (dt == FX_F16) {
+#pragma unroll
+      for (int j = 0; j < FX_V; ++j) out[j] = f2u(__half2float(__ushort_as_half(v[j])));
+    } else {
+#pragma unroll
+      for (int j = 0; j < FX_V; ++j) out[j] = (uint32_t)v[j] << 16;
+    }
+    return;
+  }
   uint32_t o[FX_V];
 #pragma unroll
   for (int j = 0; j < FX_V; ++j) o[j] = ((M >> j) & 1u) ? (uint32_t)off[j] : 0u;
@@ -135,6 +149,12 @@ __device__ __forceinline__ void fx_load_vec(uint64_t base_, const int32_t (&off)
   }
 }
 
+// round to nearest even, every NaN the quiet one
+__device__ __forceinline__ uint16_t fx_bf16(float f) {
+  const uint32_t u = f2u(f);
+  return f != f ? (uint16_t)0x7fc0u : (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+
 __device__ __forceinline__ void fx_store(uint64_t base_, uint32_t o, uint32_t dt, uint32_t vt, uint32_t v) {
   FX_AS1 uint8_t* base = (FX_AS1 uint8_t*)base_;
   switch (dt) {
@@ -152,10 +172,7 @@ __device__ __forceinline__ void fx_store(uint64_t base_, uint32_t o, uint32_t dt
     } break;
     case FX_BF16: {
       float f = vt == FX_VT_F ? u2f(v) : (float)(int32_t)v;
-      uint32_t u = f2u(f);
-      uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-      if (f != f) r = 0x7fc0u;
-      *(FX_AS1 uint16_t*)(base + (o << 1)) = (uint16_t)r;
+      *(FX_AS1 uint16_t*)(base + (o << 1)) = fx_bf16(f);
     } break;
     default: break;
   }
@@ -381,6 +398,17 @@ __device__ __forceinline__ void fx_store_vec(uint64_t base_, uint32_t obase, con
       for (int j = 0; j < FX_V; ++j)
         if ((M >> j) & 1u) *(FX_AS1 uint32_t*)(base + ((obase + e[0] + j) << 2)) = A[j];
     }
+  } else if (contig && M == (1u << FX_V) - 1u && (dt == FX_F16 || dt == FX_BF16) && vt == FX_VT_F) {
+    // one 64-bit store, 2-byte alignment
+    fx_u16x4_a2 v;
+    if (dt == FX_F16) {
+#pragma unroll
+      for (int j = 0; j < FX_V; ++j) v[j] = __half_as_ushort(__float2half(u2f(A[j])));
+    } else {
+#pragma unroll
+      for (int j = 0; j < FX_V; ++j) v[j] = fx_bf16(u2f(A[j]));
+    }
+    *(FX_AS1 fx_u16x4_a2*)((FX_AS1 uint8_t*)base_ + ((obase + e[0]) << 1)) = v;
   } else {
 #pragma unroll
     for (int j = 0; j < FX_V; ++j)
@@ -939,8 +967,8 @@ __device__ __forceinline__ void fx_lead_load(const FxLead& ld, const FxCoord<R>&
 }
 
 // Leading loads of a batch of KP items, all in flight together.  When every item of the
-// batch is a run of FX_V consecutive 32-bit elements in each of its live lanes (decided
-// for the whole batch, wave-uniform), the loads are KP unconditional 128-bit loads with
+// batch is a run of FX_V consecutive 32-bit (16-bit) elements in each of its live lanes (decided
+// for the whole batch, wave-uniform), the loads are KP unconditional 128-bit (64-bit) loads with
 // no branch between them; otherwise each item goes through fx_lead_load.
 // make_item(k, e, M, q) sets up item k.
 template <int R, int KP, class MI>
@@ -948,7 +976,8 @@ __device__ __forceinline__ void fx_lead_batch(const FxLead& ld, MI&& make_item, 
                                               uint32_t (&e0)[KP], uint32_t (&Mk)[KP]) {
   const uint32_t VM = (1u << FX_V) - 1u;
   uint32_t o0[KP];
-  bool fast = ld.dt == FX_F32 || ld.dt == FX_I32;
+  const bool half = ld.dt == FX_F16 || ld.dt == FX_BF16;
+  bool fast = ld.dt == FX_F32 || ld.dt == FX_I32 || (half && !ld.lds);
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
     uint32_t e[FX_V], M;
@@ -970,6 +999,19 @@ __device__ __forceinline__ void fx_lead_batch(const FxLead& ld, MI&& make_item, 
     if (ld.cvt) {
 #pragma unroll
       for (int j = 0; j < KP * FX_V; ++j) X[j] = f2u((float)(int32_t)X[j]);
+    }
+  } else if (fast && half) {
+    const FX_AS1 uint8_t* base = (const FX_AS1 uint8_t*)ld.p;
+    fx_u16x4_a2 v[KP];
+#pragma unroll
+    for (int k = 0; k < KP; ++k) v[k] = *(const FX_AS1 fx_u16x4_a2*)(base + (o0[k] << 1));
+    asm volatile("" ::: "memory");   // (the conversions behind a branch of their own: see fx_load_vec)
+    if (ld.dt == FX_F16) {
+#pragma unroll
+      for (int j = 0; j < KP * FX_V; ++j) X[j] = f2u(__half2float(__ushort_as_half(v[j / FX_V][j % FX_V])));
+    } else {
+#pragma unroll
+      for (int j = 0; j < KP * FX_V; ++j) X[j] = (uint32_t)v[j / FX_V][j % FX_V] << 16;
     }
   } else if (fast) {
     const FX_AS1 uint8_t* base = (const FX_AS1 uint8_t*)ld.p;
