@@ -233,14 +233,36 @@ struct SlotAlloc {
 
 struct Prog { uint32_t begin, end, vt; bool rowwave; bool wide; };
 
-// A box of an output's elements: first coordinate and extent per dimension.
+// A box of an output's elements: first coordinate per output dimension, and the coordinates that
+// move inside it.  Output coordinate d is lo[d] + sum of coef * root coordinate over the roots of d
+// (none: one element; two: a dimension taken apart, r = q * r1 + r2).
 struct Box {
-  Shape lo, n;
-  static Box whole(const Shape& s) { Box b; b.lo.assign(s.size(), 0); b.n = s; return b; }
+  struct Root { int dim; int64_t coef, n; };
+  Shape lo;
+  std::vector<Root> roots;
+  static Box whole(const Shape& s) {
+    Box b;
+    b.lo.assign(s.size(), 0);
+    for (size_t i = 0; i < s.size(); ++i) if (s[i] != 1) b.roots.push_back({(int)i, 1, s[i]});
+    return b;
+  }
+  Shape dims() const {
+    Shape r;
+    for (const Root& q : roots) r.push_back(q.n);
+    if (r.empty()) r.push_back(1);
+    return r;
+  }
 };
-// Where a program's first condition on one output coordinate changes its answer: the box is cut
-// there, and each part's program no longer asks.
-struct Cut { int dim = -1; std::vector<int64_t> at; };   // coordinates inside the box, ascending
+// What a try of a box's program found: the first condition on one root coordinate that changes its
+// answer inside the box (cut there, each part's program no longer asks), and the first division of
+// an index by s that one root coordinate keeps from being exact (taken apart, every part of the
+// index is affine).
+struct Cut {
+  int root = -1;
+  std::vector<int64_t> at;   // root coordinates, ascending
+  int frac = -1;             // root to take apart into (r / by, r % by)
+  int64_t by = 0;
+};
 #define FX_MAX_BOXES 24
 
 class Lowerer {
@@ -260,17 +282,9 @@ class Lowerer {
   // says that the low-word program moved int64 data as it is, so that the high words need a
   // program of their own; otherwise the result fits 32 bits and its store sign-extends.
   Prog lower(int vid, const Shape& rootShape, int half = 0);
-  // The program of the elements of one box; its root coordinates are those of the box whose extent
-  // is not 1 (boxDims).  cut (may be null) receives the first place where the box can be cut.
-  Prog lowerBox(int vid, const Box& b, Cut* cut, int half = 0);
-  // The boxes an output is computed in: one (the whole output) unless cutting pays.
+  Prog lowerBox(int vid, const Box& b, Cut* cut);   // the program of the elements of one box
+  // The boxes an output is computed in; none: whole, as lower() has it.
   std::vector<Box> boxesOf(int vid, const Shape& s, const Prog& whole);
-  static Shape boxDims(const Box& b) {
-    Shape r;
-    for (int64_t n : b.n) if (n != 1) r.push_back(n);
-    if (r.empty()) r.push_back(1);
-    return r;
-  }
   int boxAffine(const Box& b, const Shape& s);   // affine record: element offset in the output of a box's element
 
  private:
@@ -291,8 +305,10 @@ class Lowerer {
   bool loopVarBound_ = false;
   IdxExpr loopVar_;
   bool usedRowWave_ = false;
-  Cut* cut_ = nullptr;        // while a program is tried: where its output could be cut
-  int cutDim_[FX_MAXR];       // output dimension of every root coordinate
+  bool boxed_ = false;        // a box's program: index divisions that are exact need no code
+  Cut* cut_ = nullptr;        // while a program is tried: how its box could be divided
+  bool divExact(const IdxExpr& e, int64_t s, IdxExpr* quot, IdxExpr* rem) const;
+  void noteFactor(const IdxExpr& e, int64_t s);
   Prog lowerFrame(int vid, const Shape& rootShape, const Frame& f, int half);
   void noteCut(const IdxExpr& x, int64_t lo, int64_t hi, int64_t step);
   // int64 outputs: while only movement operators (views, *_rev merges, cat, index, where ...)
@@ -795,6 +811,24 @@ Frame Lowerer::viewFrame(const Frame& f, const Shape& outShape, const Shape& inS
       continue;
     }
     // split: dim_k = (flat / stride_k) % size_k
+    if (boxed_) {
+      int64_t st_k = 1;
+      for (size_t q = 1; q < nonunit.size(); ++q) st_k *= inShape[nonunit[q]];
+      IdxExpr rem = flat, quot;
+      std::vector<IdxExpr> parts;
+      for (size_t q = 0; q < nonunit.size(); ++q) {
+        IdxExpr next;
+        if (!divExact(rem, st_k, &quot, &next)) { noteFactor(rem, st_k); break; }
+        parts.push_back(quot);
+        rem = next;
+        if (q + 1 < nonunit.size()) st_k /= inShape[nonunit[q + 1]];
+      }
+      if (parts.size() == nonunit.size()) {
+        for (size_t q = 0; q < nonunit.size(); ++q) r[nonunit[q]] = parts[q];
+        continue;
+      }
+    }
+    if (!temps) return Frame();
     int64_t stride = 1;
     for (size_t q = nonunit.size(); q-- > 0;) {
       size_t k = nonunit[q];
@@ -932,7 +966,13 @@ Lowerer::Res Lowerer::resolve(int vid, Frame f) {
             }
           }
         }
-        if (needs_code) break;  // RK_OP
+        if (needs_code) {
+          const Frame exact = boxed_ ? viewFrame(f, os, is, nullptr) : Frame();
+          if (exact.empty()) break;  // RK_OP
+          f = exact;
+          vid = arg(0);
+          continue;
+        }
         std::vector<int> none;
         f = viewFrame(f, os, is, &none);
         vid = arg(0);
@@ -1256,7 +1296,7 @@ void Lowerer::emitBinary(uint16_t op, const Operand& l, const Operand& r, uint32
 void Lowerer::emitCond(const IdxExpr& x, int64_t lo, int64_t hi, int64_t step, const std::function<void()>& thenFn,
                        const std::function<void()>& elseFn) {
   FX_CHECK(maskDepth_ + 1 <= FX_MASK_DEPTH, FX_E_LIMIT, "predicated regions nested deeper than " << FX_MASK_DEPTH);
-  if (cut_ && cut_->dim < 0) noteCut(x, lo, hi, step);
+  if (cut_ && cut_->root < 0) noteCut(x, lo, hi, step);
   const size_t before = code.size();
   emitIdx(x);
   auto fit = [](int64_t v) { return (int32_t)std::min<int64_t>(std::max<int64_t>(v, std::numeric_limits<int32_t>::min()), std::numeric_limits<int32_t>::max()); };
@@ -1601,7 +1641,9 @@ void Lowerer::emitOpBody(const Res& r) {
         if (in[i] == 1) fi[i] = IdxExpr(0);
         else if (hi < in[i]) fi[i] = x;
         else if (x.isConst()) fi[i] = IdxExpr(x.k % in[i]);
+        else if (IdxExpr quot; boxed_ && divExact(x, in[i], &quot, &fi[i])) {}
         else {
+          if (boxed_) noteFactor(x, in[i]);
           emitIdx(x);
           emitI(FX_ITMOD, 0, 0, (uint32_t)(int32_t)in[i], FX_F_IMM);
           int t = allocTemp();
@@ -1743,18 +1785,47 @@ Prog Lowerer::lower(int vid, const Shape& rootShape, int half) {
   return lowerFrame(vid, rootShape, f, half);
 }
 
-Prog Lowerer::lowerBox(int vid, const Box& b, Cut* cut, int half) {
-  Frame f(b.n.size());
-  int k = 0;
-  for (size_t i = 0; i < f.size(); ++i) {
-    if (b.n[i] == 1) { f[i] = IdxExpr(b.lo[i]); continue; }
-    cutDim_[k] = (int)i;
-    f[i] = IdxExpr::root(k++) + IdxExpr(b.lo[i]);
+Prog Lowerer::lowerBox(int vid, const Box& b, Cut* cut) {
+  Frame f(b.lo.size());
+  for (size_t i = 0; i < f.size(); ++i) f[i] = IdxExpr(b.lo[i]);
+  for (size_t k = 0; k < b.roots.size(); ++k) {
+    IdxExpr& x = f[(size_t)b.roots[k].dim];
+    x = x + IdxExpr::root((int)k) * b.roots[k].coef;
   }
   cut_ = cut;
-  Prog p = lowerFrame(vid, boxDims(b), f, half);
-  cut_ = nullptr;
-  return p;
+  boxed_ = true;
+  struct Done { Lowerer& l; ~Done() { l.cut_ = nullptr; l.boxed_ = false; } } done{*this};
+  return lowerFrame(vid, b.dims(), f, 0);
+}
+
+// e = s * quot + rem with 0 <= rem < s for every element of the box: both are affine
+bool Lowerer::divExact(const IdxExpr& e, int64_t s, IdxExpr* quot, IdxExpr* rem) const {
+  if (!e.affine() || e.ct != 0 || s < 1) return false;
+  for (auto c : e.rc) if (c) return false;
+  IdxExpr q, r;
+  auto part = [s](int64_t c, int64_t* cq, int64_t* cr) { *cr = ((c % s) + s) % s; *cq = (c - *cr) / s; };
+  for (int i = 0; i < FX_MAXR; ++i) part(e.c[i], &q.c[i], &r.c[i]);
+  part(e.k, &q.k, &r.k);
+  int64_t lo, hi;
+  range(r, &lo, &hi);
+  if (lo < 0 || hi >= s) return false;
+  *quot = q;
+  *rem = r;
+  return true;
+}
+
+// The root coordinate that keeps e / s from being exact, and what it has to be taken apart by: c * r
+// with r = by * r1 + r2 is a multiple of s in r1.  Its extent has to be a multiple of that.
+void Lowerer::noteFactor(const IdxExpr& e, int64_t s) {
+  if (!cut_ || cut_->frac >= 0 || !e.affine()) return;
+  for (int i = 0; i < rootRank_; ++i) {
+    const int64_t c = e.c[i] < 0 ? -e.c[i] : e.c[i];
+    if (c == 0 || c % s == 0 || c * (rootDim_[i] - 1) < s) continue;
+    int64_t a = c, b = s;
+    while (b) { const int64_t t = a % b; a = b; b = t; }
+    const int64_t by = s / a;
+    if (by > 1 && by < rootDim_[i] && rootDim_[i] % by == 0) { cut_->frac = i; cut_->by = by; return; }
+  }
 }
 
 // lo <= x < hi (x - lo a multiple of step) with x = +-(one root coordinate) + constant: the root
@@ -1781,7 +1852,7 @@ void Lowerer::noteCut(const IdxExpr& x, int64_t lo, int64_t hi, int64_t step) {
     for (int64_t i = 1; i < n; ++i) at.push_back(i);
   }
   if (at.empty()) return;
-  cut_->dim = cutDim_[k];
+  cut_->root = k;
   cut_->at = at;
 }
 
@@ -1792,55 +1863,64 @@ void Lowerer::noteCut(const IdxExpr& x, int64_t lo, int64_t hi, int64_t step) {
 // of 17 predicates deep against four straight ones).  Kept whole: programs short enough to be bound by
 // their launch, rows reduced across a wave (their lanes must hold the whole row), int64 outputs
 // (two programs a word pair), and cuts that do not halve the instructions an element stands for.
-// Interpreted, MI355X: box regression of 8 732 x 21 boxes 518 -> 60 us (1 553 instructions -> four times
-// 103), the YOLO head of four 608 x 608 images with its NMS 743 -> 270 us (18 boxes).
+// A root coordinate that only keeps an index division from being exact is taken apart
+// (n = cells * anchors: the row of a flattened map), which turns the division and the load behind it
+// into one affine load; an integer division is 40 instructions an element on this device.
+// Interpreted, MI355X: box regression of 8 732 x 21 boxes 518 us whole, 60 in four boxes, 24 with the
+// divisions gone (1 553 instructions, four times 103, four times 30); the YOLO head of four 608 x 608
+// images with its NMS 743, 270, 122 us (18 boxes).
 std::vector<Box> Lowerer::boxesOf(int vid, const Shape& s, const Prog& whole) {
-  const std::vector<Box> one{Box::whole(s)};
   const size_t len = whole.end - whole.begin;
   const int64_t numel = numel_of(s);
-  if (s.empty() || len < 32 || whole.rowwave || V(vid).dtype == FX_DT_I64 || numel == 0 || numel >= ((int64_t)1 << 31)) return one;
+  if (s.empty() || len < 32 || whole.rowwave || V(vid).dtype == FX_DT_I64 || numel == 0 || numel >= ((int64_t)1 << 31)) return {};
   const std::vector<FxInsn> code0 = code;
   const std::vector<FxAffine> affs0 = affs;
   const int temps0 = maxTemps;
-  std::vector<Box> todo = one, done;
+  std::vector<Box> todo{Box::whole(s)}, done;
   size_t total = 0;
   double work = 0;
   while (!todo.empty()) {
-    Box b = todo.back();
+    const Box b = todo.back();
     todo.pop_back();
     Cut cut;
     const Prog p = lowerBox(vid, b, &cut);
-    if (cut.dim >= 0 && done.size() + todo.size() + cut.at.size() + 1 <= FX_MAX_BOXES) {
-      const int64_t lo = b.lo[(size_t)cut.dim], n = b.n[(size_t)cut.dim];
-      cut.at.push_back(n);
+    if (cut.root >= 0 && done.size() + todo.size() + cut.at.size() + 1 <= FX_MAX_BOXES) {
+      const Box::Root r = b.roots[(size_t)cut.root];
+      cut.at.push_back(r.n);
       for (size_t i = cut.at.size(); i-- > 0;) {
         Box q = b;
-        const int64_t from = i ? cut.at[i - 1] : 0;
-        q.lo[(size_t)cut.dim] = lo + from;
-        q.n[(size_t)cut.dim] = cut.at[i] - from;
+        const int64_t from = i ? cut.at[i - 1] : 0, n = cut.at[i] - from;
+        q.lo[(size_t)r.dim] += r.coef * from;
+        q.roots[(size_t)cut.root].n = n;
+        if (n == 1) q.roots.erase(q.roots.begin() + cut.root);
         todo.push_back(q);   // (the first part on top: boxes come out in output order)
       }
+    } else if (cut.frac >= 0 && b.roots.size() < FX_MAXR) {
+      Box q = b;
+      Box::Root& r = q.roots[(size_t)cut.frac];
+      const Box::Root inner{r.dim, r.coef, cut.by};
+      r.coef *= cut.by;
+      r.n /= cut.by;
+      q.roots.insert(q.roots.begin() + cut.frac + 1, inner);
+      todo.push_back(q);
     } else {
       done.push_back(b);
       total += p.end - p.begin;
-      work += (double)(p.end - p.begin) * (double)numel_of(b.n);
+      work += (double)(p.end - p.begin) * (double)numel_of(b.dims());
     }
   }
   code = code0;
   affs = affs0;
   maxTemps = temps0;
-  if (done.size() < 2 || total > len || work * 2 > (double)len * (double)numel) return one;
+  if (total > len || work * 2 > (double)len * (double)numel) return {};
   return done;
 }
 
 int Lowerer::boxAffine(const Box& b, const Shape& s) {
   const Shape st = contiguous_strides(s);
   IdxExpr e(0);
-  int k = 0;
-  for (size_t i = 0; i < s.size(); ++i) {
-    e.k += b.lo[i] * st[i];
-    if (b.n[i] != 1) e.c[k++] = st[i];
-  }
+  for (size_t i = 0; i < s.size(); ++i) e.k += b.lo[i] * st[i];
+  for (size_t k = 0; k < b.roots.size(); ++k) e.c[k] = b.roots[k].coef * st[(size_t)b.roots[k].dim];
   return addAffine(e);
 }
 
@@ -2144,19 +2224,19 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args, b
       const size_t code0 = L.code.size(), affs0 = L.affs.size();
       const int temps0 = L.maxTemps;
       Prog p0 = L.lower(R.outputs[o], s);
-      std::vector<Box> boxes(1);
+      std::vector<Box> boxes;
       if (P->mode == FX_MODE_DENSE) boxes = L.boxesOf(R.outputs[o], s, p0);
-      if (!boxed_outs && boxes.size() > 1) { *could_box = true; boxes.resize(1); }
-      if (boxes.size() > 1) {   // the boxes' programs stand in the place of the whole one
+      if (!boxed_outs && !boxes.empty()) { *could_box = true; boxes.clear(); }
+      const bool boxed = !boxes.empty();
+      if (boxed) {   // the boxes' programs stand in the place of the whole one
         L.code.resize(code0);
         L.affs.resize(affs0);
         L.maxTemps = temps0;
       }
-      for (int part = 0; part < (boxes.size() > 1 ? (int)boxes.size() : p0.wide ? 2 : 1); ++part) {
-      const bool boxed = boxes.size() > 1;
+      for (int part = 0; part < (boxed ? (int)boxes.size() : p0.wide ? 2 : 1); ++part) {
       const int half = boxed ? 0 : part;
       const Prog p = boxed ? L.lowerBox(R.outputs[o], boxes[(size_t)part], nullptr) : half == 0 ? p0 : L.lower(R.outputs[o], s, 1);
-      const Shape dims = boxed ? Lowerer::boxDims(boxes[(size_t)part]) : s;
+      const Shape dims = boxed ? boxes[(size_t)part].dims() : s;
       FxOut od;
       memset(&od, 0, sizeof(od));
       od.prog_begin = p.begin;

@@ -112,3 +112,37 @@ def test_what_stays_whole():
     r.output(r.cat([a, a + 1.0], 0))   # short
     r.finalize()
     assert n_programs(r, torch.randn(9, 9)) == 1
+
+
+@pytest.mark.parametrize("backend", BACKENDS)
+@pytest.mark.parametrize("batch,a,w,hw", [(1, 1, 5, (1, 1)), (2, 3, 7, (5, 3)), (1, 3, 85, (7, 6)), (3, 2, 6, (1, 9))])
+def test_divisions_that_come_out_even(backend, batch, a, w, hw):
+    """Flattened maps of two levels and repeated rows: the row number is taken apart into the map's
+    coordinates (n = (y * w + x) * a + anchor), and the divisions of the views need no code."""
+    g = torch.Generator().manual_seed(w)
+    maps = [torch.randn(batch, a * w, h, v, generator=g) for h, v in (hw, (2 * hw[0], hw[1] + 1))]
+    rois = torch.randn(sum(m.size(2) * m.size(3) for m in maps), 4, generator=g)
+    r = Region()
+    ins, ri = [r.tensor_input(rank=4) for _ in maps], r.tensor_input(rank=2)
+    flat = []
+    for v, m in zip(ins, maps):
+        flat.append(v.permute(0, 2, 3, 1).view(batch, m.size(2) * m.size(3) * a, w))
+    p = r.cat(flat, 1)
+    p = p.slice_rev(p.slice(2, 0, 2).sigmoid(), 2, 0, 2)
+    rep = ri.repeat(1, a).view(rois.size(0) * a, 4)
+    xy, wh = p.slice(2, 0, 2) + rep.slice(1, 0, 2), (rep.slice(1, 2, 4) - rep.slice(1, 0, 2)) * p.slice(2, 2, 4).exp()
+    r.output(p)
+    r.output(r.cat([xy - wh * 0.5, xy + wh * 0.5], 2))
+    r.finalize()
+
+    q = torch.cat([m.permute(0, 2, 3, 1).reshape(batch, -1, w) for m in maps], 1)
+    q[..., :2] = q[..., :2].sigmoid()
+    ref = rois.repeat(1, a).view(-1, 4)
+    rxy, rwh = q[..., :2] + ref[:, :2], (ref[:, 2:] - ref[:, :2]) * q[..., 2:4].exp()
+    got = run_region(backend, r, *maps, rois)
+    assert_close(got[0], q)
+    # sums of two halves that may cancel: a few units in the last place of the larger one
+    top = max(1.0, float(rxy.abs().max()), float(rwh.abs().max()))
+    assert_close(got[1], torch.cat([rxy - rwh * 0.5, rxy + rwh * 0.5], 2), atol=4 * top * 2.0 ** -23)
+    assert n_programs(r, *maps, rois) >= 8
+    assert "ITDIV" not in r.disasm(*maps, rois) and "ITMOD" not in r.disasm(*maps, rois)
