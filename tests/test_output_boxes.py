@@ -146,3 +146,21 @@ def test_divisions_that_come_out_even(backend, batch, a, w, hw):
     assert_close(got[1], torch.cat([rxy - rwh * 0.5, rxy + rwh * 0.5], 2), atol=4 * top * 2.0 ** -23)
     assert n_programs(r, *maps, rois) >= 8
     assert "ITDIV" not in r.disasm(*maps, rois) and "ITMOD" not in r.disasm(*maps, rois)
+
+
+@pytest.mark.parametrize("backend", BACKENDS)
+@pytest.mark.parametrize("c,n", [(8, 8), (9, 64), (10, 33), (23, 70), (64, 260)])
+def test_transposed_boxes(backend, c, n):
+    """Boxes that turn a matrix over: lane groups along the columns, lanes along the rows, and what is
+    left of the last group in a box of its own."""
+    g = torch.Generator().manual_seed(c)
+    x, y = torch.randn(2, c, n, generator=g), torch.randn(2, 3, n, generator=g)
+    r = Region()
+    a, b = r.tensor_input(rank=3), r.tensor_input(rank=3)
+    parts = [b.sigmoid() * 2.0 - 1.0, a, b.exp() + 1.0, a * 0.5 + 2.0, b.tanh() - 1.0, (b + 1.0) * (b - 1.0)]
+    r.output(r.cat([v.transpose(1, 2) for v in parts], 2))
+    r.finalize()
+    (got,) = run_region(backend, r, x, y)
+    ref = torch.cat([y.sigmoid() * 2 - 1, x, y.exp() + 1, x * 0.5 + 2, y.tanh() - 1, (y + 1) * (y - 1)], 1).transpose(1, 2)
+    assert_close(got, ref, atol=2.0 ** -22)   # (differences of values near 1)
+    assert n_programs(r, x, y) >= 6 + (2 if c % 4 else 0)
