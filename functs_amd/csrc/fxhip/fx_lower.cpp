@@ -1884,7 +1884,16 @@ std::vector<Box> Lowerer::boxesOf(int vid, const Shape& s, const Prog& whole) {
     const Box b = todo.back();
     todo.pop_back();
     Cut cut;
-    const Prog p = lowerBox(vid, b, &cut);
+    Prog p;
+    try {
+      p = lowerBox(vid, b, &cut);
+    } catch (const Error&) {   // (a box's index record may exceed 32 bits where the whole program's steps do not)
+      loopVarBound_ = false;
+      code = code0;
+      affs = affs0;
+      maxTemps = temps0;
+      return {};
+    }
     if (cut.root >= 0 && done.size() + todo.size() + cut.at.size() + 1 <= FX_MAX_BOXES) {
       const Box::Root r = b.roots[(size_t)cut.root];
       cut.at.push_back(r.n);
