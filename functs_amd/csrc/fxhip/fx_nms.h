@@ -27,7 +27,9 @@ __device__ __forceinline__ bool overlaps(const Box& a, float area_a, const Box& 
 // The same decision without the division, where that is certain: inter / union > thr is settled by
 // comparing inter with thr * union unless the two are within 2e-6 of each other (the product and the
 // quotient are off by at most 2^-24 relative each, 2e-6 is 2^-19), or the product is not an ordinary
-// number (thr <= 0, boxes of no or infinite area, NaN).
+// number (boxes of no or infinite area, NaN) or thr is not positive (boxes with swapped corners may make the
+// union negative, and dividing by it turns the comparison round: with thr < 0 the product would be an
+// ordinary number all the same).
 __device__ __forceinline__ void overlaps_fast(const Box& a, float area_a, const Box& b, float area_b, float thr, bool& over, bool& sure) {
   const float xx1 = fmaxf(a.x1, b.x1), yy1 = fmaxf(a.y1, b.y1);
   const float xx2 = fminf(a.x2, b.x2), yy2 = fminf(a.y2, b.y2);
@@ -35,7 +37,7 @@ __device__ __forceinline__ void overlaps_fast(const Box& a, float area_a, const 
   const float inter = w * h;
   const float t = thr * ((area_a + area_b) - inter);
   over = inter > t * 1.000002f;
-  sure = t > 1e-30f && t < 1e30f && (over || inter < t * 0.999998f);
+  sure = thr > 0.0f && t > 1e-30f && t < 1e30f && (over || inter < t * 0.999998f);
 }
 
 }  // namespace

@@ -319,3 +319,18 @@ def test_boxes_that_are_all_candidates_take_three_launches_with_the_same_result(
         want = detection.batched_nms_batched(*args, counts=torch.full((T,), n, dtype=torch.int32, device=dev), iou_threshold=thr, max_num=max_num)
         assert torch.equal(got.n, want.n) and torch.equal(got.index, want.index) and torch.equal(got.labels, want.labels)
         assert torch.equal(got.dets.view(torch.int32), want.dets.view(torch.int32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("thr", [-0.5, -1e-3, 0.0, 0.3])
+def test_thresholds_below_zero_and_corners_in_any_order(thr):
+    """fx_nms_pairs against fx_sort_nms bit for bit where the union of two boxes may be negative (corners
+    in any order): dividing by it turns the comparison round, so the product cannot stand in for it."""
+    from functs_amd import detection
+    g = torch.Generator().manual_seed(5)
+    n, dev = 300, torch.device("cuda:0")
+    b, s = (torch.rand(1, n, 4, generator=g) * 20).to(dev), torch.rand(1, n, generator=g).to(dev)
+    print("fx_nms_pairs n=%d thr=%g" % (n, thr), flush=True)
+    got = detection.batched_nms_batched(b, s, None, iou_threshold=thr)
+    want = detection.batched_nms_batched(b, s, None, counts=torch.full((1,), n, dtype=torch.int32, device=dev), iou_threshold=thr)
+    assert torch.equal(got.n, want.n) and torch.equal(got.index, want.index) and torch.equal(got.dets.view(torch.int32), want.dets.view(torch.int32))
