@@ -18,10 +18,18 @@
 // value travels with the tag of the step that wrote it and readers poll for the tag they expect
 // (fx_lstm_sched.h), with bounded waits.
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
+
+#include <map>
+#include <mutex>
+#include <set>
+#include <thread>
+#include <utility>
 
 #define FX_LSTM_HD __host__ __device__
 #include "../../../include/fxhip.h"
 #include "fx_device.h"
+#include "fx_lstm_groups.h"
 #include "fx_lstm_sched.h"
 
 #define FX_LSTM_BLOCK 256
@@ -127,7 +135,7 @@ __global__ __launch_bounds__(FX_LSTM_BLOCK * UPW, HPT >= 32 ? 4 : 2) void fx_lst
   const int wg = (n_wg % 8 == 0) ? ((int)blockIdx.x % 8) * (n_wg / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
   const int u0 = wg * UPW;
   // a workspace that still carries a given-up wait is refused (below, behind the first barrier)
-  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) ? 1u : 0u;
+  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) ? 1u : 0u;
   // tags of this launch start behind those of every launch before it
   const uint32_t base = DevAtomics::load(a.ctl + FX_LSTM_W_BASE);
 
@@ -351,7 +359,7 @@ __global__ __launch_bounds__(FX_LSTM_BLOCK * UPW, HPT >= 32 ? 4 : 2) void fx_lst
 //            workgroups of its own, which hold the weights again but wait for, and read, the vectors of
 //            their own rows only: what all workgroups read in a step is what the step waits for.
 //            H = 512 from nine rows on: two tiles a workgroup, since the device does not hold the
-//            workgroups of more groups at once.
+//            workgroups of more groups at once.  (The choice of the form is lstm_forms and what fits.)
 //   columns  four hidden units a workgroup.  A vector h_j is multiplied by layer j's recurrent and
 //            layer j + 1's input matrix: 16 + 16 gate columns, the 32 columns of a half-wave.
 //   depth    the inner dimension is dealt to eight waves in runs of 16: lane l fetches element l / 4
@@ -420,7 +428,7 @@ __global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_row
   const int wg = (n_wg % 8 == 0) ? (gi % 8) * (n_wg / 8) + gi / 8 : gi;
   const int u0 = wg * 4;
   const int b0 = group * 4 * MT, nb = min(4 * MT, B - b0);
-  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) ? 1u : 0u;
+  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) ? 1u : 0u;
   const uint32_t base = DevAtomics::load(a.ctl + FX_LSTM_W_BASE);
   const int n_steps = fx_lstm_steps(T, L);
   const uint32_t BH = (uint32_t)(B * HH);               // elements of one vector of all rows
@@ -697,37 +705,85 @@ static fx_lstm_kernel_t pick_serial(int hpt) {
     default: return nullptr;
   }
 }
-struct LstmLaunch { fx_lstm_kernel_t kernel; int grid, threads; };
+struct LstmLaunch { fx_lstm_kernel_t kernel; int grid, threads, tiles; };   // tiles of rows a workgroup; 0: row by row
+// the forms that serve these sizes, the fastest first
 template <int L>
-static LstmLaunch pick_launch(const FxLstmArgs& a) {
+static int lstm_forms(const FxLstmArgs& a, LstmLaunch (&f)[3]) {
   const int hpt = a.H / 32;
-  LstmLaunch r{};
-  if (a.B > 1) {
-    // One tile of four rows a workgroup while all groups of rows together make at most one workgroup
-    // for each of the 256 CUs (the weights fill a CU's registers), else two.
-    const int tiles = (a.H / 4) * ((a.B + 3) / 4) > 256 ? 2 : 1, groups = (a.B + 4 * tiles - 1) / (4 * tiles);
-    const int cells = L * tiles < 4 ? L * tiles : 4;   // FxLstmRows
-    r = LstmLaunch{pick_rows<L>(hpt, tiles), (a.H / 4) * groups, ((a.H >= 128 ? 8 : a.H / 16) + cells) * 64};
-  }
+  int n = 0;
+  if (a.B > 1)
+    for (int tiles = 1; tiles <= 2; ++tiles) {
+      const int groups = (a.B + 4 * tiles - 1) / (4 * tiles), cells = L * tiles < 4 ? L * tiles : 4;   // FxLstmRows
+      if (fx_lstm_kernel_t k = pick_rows<L>(hpt, tiles)) f[n++] = LstmLaunch{k, (a.H / 4) * groups, ((a.H >= 128 ? 8 : a.H / 16) + cells) * 64, tiles};
+    }
   // two hidden units per workgroup: every workgroup fetches the step's vectors from the memory
   // side once, so fewer, larger workgroups fetch less, and sixteen gate sums fill the butterfly
-  if (!r.kernel) r = LstmLaunch{pick_serial<L>(hpt), a.H / FX_LSTM_UPW, FX_LSTM_BLOCK * FX_LSTM_UPW};
-  return r;
+  if (fx_lstm_kernel_t k = pick_serial<L>(hpt)) f[n++] = LstmLaunch{k, a.H / FX_LSTM_UPW, FX_LSTM_BLOCK * FX_LSTM_UPW, 0};
+  return n;
 }
+
+static std::mutex g_lstm_mu;
+static std::map<int, FxLstmGroups> g_lstm_groups;   // by device
+static std::set<int> g_lstm_captured;               // devices on which a launch has been captured
 
 // 0: launched; 1: shape outside what the kernel is built for; 2: the grid would not be resident
 // all at once (every workgroup waits for values that all the others write); otherwise a HIP error code + 100.
-int fx_launch_lstm_stack(const FxLstmArgs& a, int L, hipStream_t stream) {
+int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uint64_t* words_hbuf, hipStream_t stream) {
+  FxLstmArgs a = args;
   if (a.H < 32 || a.H % 32 != 0 || a.B < 1 || a.B > FX_LSTM_MAXB || L < 1 || L * a.B > FX_LSTM_BLOCK) return 1;
-  const LstmLaunch l = L == 1 ? pick_launch<1>(a) : L == 2 ? pick_launch<2>(a) : L == 3 ? pick_launch<3>(a) : L == 4 ? pick_launch<4>(a) : LstmLaunch{};
-  if (!l.kernel) return 1;
-  int dev = 0, per_cu = 0, cus = 0;
+  LstmLaunch f[3];
+  const int n = L == 1 ? lstm_forms<1>(a, f) : L == 2 ? lstm_forms<2>(a, f) : L == 3 ? lstm_forms<3>(a, f) : L == 4 ? lstm_forms<4>(a, f) : 0;
+  if (n == 0) return 1;
+  int dev = 0, cus = 0;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)l.kernel, l.threads, 0);
   if (e != hipSuccess) return 100 + (int)e;
-  if ((long)per_cu * cus < l.grid) return 2;
-  void* args[1] = {(void*)&a};
-  e = hipLaunchKernel((const void*)l.kernel, dim3((uint32_t)l.grid), dim3((uint32_t)l.threads), args, 0, stream);
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    cap = hipStreamCaptureStatusNone;
+  }
+  const bool capturing = cap != hipStreamCaptureStatusNone;
+  std::lock_guard<std::mutex> lock(g_lstm_mu);
+  if (capturing) g_lstm_captured.insert(dev);
+  // A captured launch is replayed whenever the program likes, beside any other: from the first one on,
+  // every launch leaves half of the device free where a form of it can.
+  const uint32_t device = (uint32_t)cus * FX_LSTM_CU / (g_lstm_captured.count(dev) ? 2u : 1u);
+  const LstmLaunch* l = nullptr;
+  uint32_t need = 0;
+  for (int i = 0; i < n; ++i) {
+    // one tile of four rows a workgroup while that makes at most one workgroup for each CU, whose registers the
+    // weights fill
+    if (f[i].tiles == 1 && f[i].grid > cus) continue;
+    int per_cu = 0;
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)f[i].kernel, f[i].threads, 0);
+    if (e != hipSuccess) return 100 + (int)e;
+    if ((long)per_cu * cus < f[i].grid) continue;
+    const uint32_t want = fx_lstm_need((uint32_t)f[i].grid, (uint32_t)per_cu);
+    if (l && want >= need) continue;
+    l = &f[i];
+    need = want;
+    if (need <= device) break;
+  }
+  if (!l) return 2;
+  if (l->tiles > 0) {   // the hand-over through words
+    std::swap(a.ctl, words_ctl);
+    a.hbuf = words_hbuf;
+  }
+  a.ctl_other = words_ctl;
+  void* kargs[1] = {(void*)&a};
+  const dim3 grid((uint32_t)l->grid), block((uint32_t)l->threads);
+  if (capturing) {
+    e = hipLaunchKernel((const void*)l->kernel, grid, block, kargs, 0, stream);
+    return e == hipSuccess ? 0 : 100 + (int)e;
+  }
+  std::vector<void*> wait_for;
+  const uint64_t thread = stream == hipStreamPerThread ? (uint64_t)std::hash<std::thread::id>()(std::this_thread::get_id()) : 0u;
+  FxLstmGroups::Member& m = g_lstm_groups[dev].admit((uint64_t)(uintptr_t)stream, thread, need, device, &wait_for);
+  for (void* w : wait_for)
+    if (w && e == hipSuccess) e = hipStreamWaitEvent(stream, (hipEvent_t)w, 0);
+  if (e == hipSuccess && !m.done) e = hipEventCreateWithFlags((hipEvent_t*)&m.done, hipEventDisableTiming);
+  // (the event is the kernel's own completion: a record behind it costs a launch 1.3 - 2.5 us)
+  if (e == hipSuccess) e = hipExtLaunchKernel((const void*)l->kernel, grid, block, kargs, 0, stream, nullptr, (hipEvent_t)m.done, 0);
   return e == hipSuccess ? 0 : 100 + (int)e;
 }

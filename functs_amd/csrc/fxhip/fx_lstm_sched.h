@@ -58,6 +58,7 @@ struct FxLstmArgs {
   float *out, *state_h, *state_c;
   uint64_t* hbuf;      // [2][L][B][H] (value, tag): h of the cells of the last two steps
   uint32_t* ctl;       // FX_LSTM_CTL_WORDS control words
+  uint32_t* ctl_other; // those of the other hand-over: a wait that was given up in either refuses both
   uint32_t* err_host;  // pinned word that a given-up wait reports to as well (may be null)
   int T, B, H;
   uint32_t spin_limit;

@@ -432,8 +432,12 @@ int fx_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* co
  * Contiguous fp32: x [T, B, H]; wih, whh [L, 4, H, H]; bih, bhh [L, 4, 1, H]; h0, c0, state_h,
  * state_c [L, B, H]; out [T, B, H]; h0 / c0 may be null (zero initial state).  H is 32, 64, ...
  * 1024 (a power of two), L <= 4, B <= 16 (FX_E_UNSUPPORTED otherwise), and the
- * workgroups (H / 2 of 512 threads, or H / 4 of up to 768 for every four rows) must be resident
- * together (FX_E_LIMIT).
+ * workgroups (H / 2 of 512 threads, or H / 4 of up to 768 for every four or eight rows) must be resident
+ * together (FX_E_LIMIT if no form's are).  Launches on several streams of a device overlap when all their
+ * workgroups find places together (two stacks of 512 units with one sequence each, for instance);
+ * one that does not fit waits, in its stream, for the launches before it.  A captured launch cannot be
+ * made to wait: it, and from then on every launch on that device, takes a form for half of the device
+ * where there is one, so that ONE replay and the calls, or two replays, may run at the same time.
  * workspace: fx_lstm_stack_workspace_bytes() of device memory, 256-byte aligned, all zero when it
  * is used for the first time.  A launch that ends without error leaves it ready for the next one,
  * so one workspace, cleared once, serves launch after launch on one stream as long as batch,

@@ -26,7 +26,8 @@ def build():
 
 def lstm_emul():
     """ctypes handle of the CPU build of the persistent LSTM kernel's schedule and barrier."""
-    sources = [os.path.join(_HERE, "lstm_emul.cpp"), os.path.join(_HERE, "..", "..", "functs_amd", "csrc", "fxhip", "fx_lstm_sched.h")]
+    csrc = os.path.join(_HERE, "..", "..", "functs_amd", "csrc", "fxhip")
+    sources = [os.path.join(_HERE, "lstm_emul.cpp"), os.path.join(csrc, "fx_lstm_sched.h"), os.path.join(csrc, "fx_lstm_groups.h")]
     if not os.path.exists(_LSTM_SO) or any(os.path.exists(s) and os.path.getmtime(s) > os.path.getmtime(_LSTM_SO) for s in sources):
         build()
     so = ctypes.CDLL(_LSTM_SO)
@@ -35,6 +36,11 @@ def lstm_emul():
     so.fx_lstm_emul.argtypes = [fp] * 10 + [ctypes.c_int] * 4 + [ctypes.c_uint32, ctypes.c_int, ctypes.c_int, ctypes.c_uint32]
     so.fx_lstm_emul_words.restype = ctypes.c_int
     so.fx_lstm_emul_words.argtypes = [fp] * 10 + [ctypes.c_int] * 4 + [ctypes.c_uint32, ctypes.c_int, ctypes.c_int]
+    so.fx_lstm_groups_emul.restype = ctypes.c_uint64
+    so.fx_lstm_groups_emul.argtypes = [ctypes.c_uint32, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_uint32), ctypes.c_int, ctypes.c_uint32,
+                                       ctypes.POINTER(ctypes.c_int)]
+    so.fx_lstm_need_of.restype = ctypes.c_uint32
+    so.fx_lstm_need_of.argtypes = [ctypes.c_uint32, ctypes.c_uint32]
     so.fx_lstm_emul_give_up.restype = ctypes.c_int
     so.fx_lstm_emul_give_up.argtypes = [fp] * 10 + [ctypes.c_int] * 4 + [ctypes.c_uint32, ctypes.c_int]
     return so

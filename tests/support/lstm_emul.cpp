@@ -14,9 +14,12 @@
 
 #include <algorithm>
 #include <atomic>
+#include <random>
 #include <thread>
+#include <utility>
 #include <vector>
 
+#include "../../functs_amd/csrc/fxhip/fx_lstm_groups.h"
 #include "../../functs_amd/csrc/fxhip/fx_lstm_sched.h"
 
 namespace {
@@ -256,3 +259,40 @@ extern "C" int fx_lstm_emul_give_up(const float* x, const float* wih, const floa
   if (ctl[FX_LSTM_W_ERR] == 0u) bits |= 16;
   return bits;
 }
+
+// A random program of launches on several streams (FxLstmGroups): every launch starts when its stream is
+// free and the events that it waits for have happened, and takes a random time.  Returns the most that
+// ran at one time, in the units of `needs`; *waits: launches that waited for another stream.
+extern "C" uint64_t fx_lstm_groups_emul(uint32_t seed, int streams, int launches, const uint32_t* needs, int n_needs, uint32_t device, int* waits) {
+  std::mt19937 rng(seed);
+  FxLstmGroups groups;
+  std::vector<double> free_at(streams, 0.0);       // end of the stream's last launch
+  std::vector<double> events;                      // time of the last record of every event (handle - 1)
+  std::vector<std::pair<double, int64_t>> edges;   // (time, + need / - need)
+  *waits = 0;
+  double clock = 0.0;
+  for (int i = 0; i < launches; ++i) {
+    const int s = (int)(rng() % (uint32_t)streams);
+    const uint32_t need = needs[rng() % (uint32_t)n_needs];
+    clock += (double)(rng() % 100) * 0.01;         // when the host issues it
+    std::vector<void*> wait_for;
+    FxLstmGroups::Member& m = groups.admit((uint64_t)s, 0u, need, device, &wait_for);
+    double start = std::max(clock, free_at[(size_t)s]);
+    for (void* w : wait_for) start = std::max(start, events[(size_t)(uintptr_t)w - 1]);
+    *waits += wait_for.empty() ? 0 : 1;
+    if (!m.done) {
+      events.push_back(0.0);
+      m.done = (void*)(uintptr_t)events.size();
+    }
+    const double end = start + 0.01 + (double)(rng() % 300) * 0.01;
+    free_at[(size_t)s] = end;
+    events[(size_t)(uintptr_t)m.done - 1] = end;
+    edges.push_back({start, (int64_t)need});
+    edges.push_back({end, -(int64_t)need});
+  }
+  std::sort(edges.begin(), edges.end());           // (an end sorts ahead of a start at the same time)
+  int64_t sum = 0, most = 0;
+  for (auto& e : edges) most = std::max(most, sum += e.second);
+  return (uint64_t)most;
+}
+extern "C" uint32_t fx_lstm_need_of(uint32_t grid, uint32_t per_cu) { return fx_lstm_need(grid, per_cu); }

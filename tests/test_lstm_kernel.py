@@ -159,6 +159,26 @@ def test_words_are_cleared_two_steps_ahead_on_host_threads(T, H, L, B, launches)
         assert so.fx_lstm_emul_words(*[t.data_ptr() for t in ts], out.data_ptr(), sh.data_ptr(), sc.data_ptr(), T, B, H, L, 2000, 5, 1) == 1
 
 
+@pytest.mark.parametrize("seed", range(12))
+def test_launches_that_may_overlap_fit_the_device_together(seed):
+    """A workgroup waits for all others of its launch, so launches on several streams may only run at the
+    same time when all their workgroups get places: random programs over the grids of the kernel's forms."""
+    import ctypes
+    from tests.support import emul
+    so = emul.lstm_emul()
+    device = so.fx_lstm_need_of(256, 1)
+    assert device == so.fx_lstm_need_of(512, 2) == so.fx_lstm_need_of(512, 3) and so.fx_lstm_need_of(8, 16) * 512 == device
+    forms = [(256, 1), (128, 1), (256, 2), (192, 1), (128, 3), (64, 1), (32, 2), (8, 8)]
+    forms = forms[seed % 3:] if seed % 2 else forms[: 3 + seed % 4]
+    needs = (ctypes.c_uint32 * len(forms))(*[so.fx_lstm_need_of(*f) for f in forms])
+    waits = ctypes.c_int()
+    assert so.fx_lstm_groups_emul(seed, 1, 200, needs, len(forms), device, ctypes.byref(waits)) <= device and waits.value == 0   # one stream never waits
+    for streams in (2, 3, 7):
+        assert so.fx_lstm_groups_emul(seed, streams, 300, needs, len(forms), device, ctypes.byref(waits)) <= device and waits.value > 0
+    halves = (ctypes.c_uint32 * 1)(so.fx_lstm_need_of(256, 2))
+    assert so.fx_lstm_groups_emul(seed, 2, 100, halves, 1, device, ctypes.byref(waits)) == device and waits.value == 0   # two halves overlap
+
+
 def _gpu(x, wih, whh, bih, bhh, h0, c0, launches=1):
     """`launches` calls in a row on one workspace that is cleared once; the last call's results."""
     from functs_amd._lib import check, lib
@@ -242,3 +262,82 @@ def test_sizes_the_kernel_is_built_for():
     assert lib.fx_lstm_stack_fits(1, 512, 2) == 1 and lib.fx_lstm_stack_fits(16, 512, 4) == 1
     assert lib.fx_lstm_stack_fits(1, 1024, 2) == 1 and lib.fx_lstm_stack_fits(1, 1024, 3) == 0
     assert lib.fx_lstm_stack_fits(1, 96, 2) == 0 and lib.fx_lstm_stack_fits(17, 64, 2) == 0 and lib.fx_lstm_stack_fits(1, 64, 5) == 0
+
+
+class _Stack:
+    """One stack's operands and workspace on the device."""
+
+    def __init__(self, T, H, L, B):
+        from functs_amd._lib import lib
+        self.dev, self.T, self.H, self.L, self.B = torch.device("cuda:0"), T, H, L, B
+        args = _inputs(T + H + L + B, T, H, L, B)
+        self.want = _reference(*args)
+        self.args = [t.contiguous().to(self.dev) for t in args]
+        self.ws = torch.zeros(lib.fx_lstm_stack_workspace_bytes(B, H, L), dtype=torch.uint8, device=self.dev)
+        self.out = [torch.empty(T, B, H, device=self.dev)] + [torch.empty(L, B, H, device=self.dev) for _ in range(2)]
+
+    def launch(self):
+        from functs_amd._lib import check, lib
+        check(lib.fx_lstm_stack(*[t.data_ptr() for t in self.args + self.out], self.T, self.B, self.H, self.L, self.ws.data_ptr(),
+                                self.ws.numel(), ctypes.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream)))
+
+    def check(self, what):
+        _close(tuple(t.cpu() for t in self.out), self.want, what)
+
+
+@pytest.fixture
+def short_waits():
+    """Waits that are given up after a fraction of a second."""
+    from functs_amd._lib import lib
+    lib.fx_set_lstm_spin_limit(100000)
+    yield lib
+    lib.fx_set_lstm_spin_limit(1000000)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[(12, 512, 2, 8), (9, 512, 2, 8)], [(12, 512, 2, 8), (12, 512, 2, 1), (12, 256, 1, 16)], [(12, 512, 2, 1)] * 4])
+def test_launches_on_several_streams_take_turns_where_they_do_not_fit_together(sizes, short_waits):
+    """Stacks that take the whole device, or together more than it, on a stream each: none starves."""
+    stacks = [_Stack(*s) for s in sizes]
+    streams = [torch.cuda.Stream() for _ in stacks]
+    torch.cuda.synchronize()
+    print("fx_lstm_stack on %d streams: %s" % (len(sizes), sizes), flush=True)
+    for _ in range(4):
+        for st, s in zip(stacks, streams):
+            with torch.cuda.stream(s):
+                st.launch()
+                st.launch()
+    torch.cuda.synchronize()
+    assert short_waits.fx_async_error(1) == 0
+    for st, s in zip(stacks, sizes):
+        st.check("streams %r" % (s,))
+
+
+@pytest.mark.gpu
+def test_a_captured_launch_leaves_room_for_another(short_waits):
+    """A graph's launch is replayed whenever the program likes: it and every later launch keep to half of
+    the device, so a replay and a call on another stream run side by side; one workspace serves both forms."""
+    a, b = _Stack(12, 512, 2, 8), _Stack(9, 512, 2, 8)
+    side = torch.cuda.Stream()
+    print("fx_lstm_stack captured", flush=True)
+    a.launch()   # (the whole device, words)
+    torch.cuda.synchronize()
+    a.check("before the capture")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        a.launch()
+    for _ in range(4):
+        for t in a.out + b.out:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        with torch.cuda.stream(side):
+            b.launch()
+        torch.cuda.synchronize()
+        assert short_waits.fx_async_error(1) == 0
+        a.check("replay")
+        b.check("beside a replay")
+    a.launch()
+    torch.cuda.synchronize()
+    a.check("a call on the graph's workspace")
+    assert short_waits.fx_async_error(1) == 0
