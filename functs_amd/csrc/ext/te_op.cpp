@@ -1251,7 +1251,12 @@ void runLstmStack(Stack& stack) {
     checkAsyncError();
     TORCH_CHECK(T <= INT32_MAX && B <= INT32_MAX && H <= INT32_MAX, "fx::lstm_stack: sizes beyond 32 bits");
     auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.device().index());
-    at::Tensor ws = lstmWorkspaces().get(x.device(), (void*)stream.stream(), B, H, L);
+    // a captured launch takes a workspace of its graph's memory, cleared in every replay: another graph's may
+    // not have been cleared yet, and replays of two graphs may overlap
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream.stream(), &capture) != hipSuccess) (void)hipGetLastError();
+    at::Tensor ws = capture == hipStreamCaptureStatusNone ? lstmWorkspaces().get(x.device(), (void*)stream.stream(), B, H, L)
+                                                          : at::zeros({(int64_t)fx_lstm_stack_workspace_bytes((int)B, (int)H, (int)L)}, opts.dtype(at::kByte));
     TORCH_CHECK(((uintptr_t)ws.data_ptr() & 255u) == 0, "fx::lstm_stack: workspace is not 256-byte aligned");
     FX_OK_OR_THROW(fx_lstm_stack(x.data_ptr<float>(), wih.data_ptr<float>(), whh.data_ptr<float>(), bih.data_ptr<float>(),
                                  bhh.data_ptr<float>(), h0.defined() ? h0.data_ptr<float>() : nullptr,

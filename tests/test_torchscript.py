@@ -485,6 +485,31 @@ def test_c4_lstm_as_hip_graph():
         assert_close(g_.cpu(), r, "graphed c4", rtol=1e-4, atol=1e-6)
 
 
+@pytest.mark.gpu
+def test_every_captured_lstm_clears_a_workspace_of_its_own():
+    """Two graphs of one function, of which only the second is replayed, in memory that held other values."""
+    from functs_amd.benchmark import PROGRAMS
+    args = _cuda(oc.c4_inputs(3, 12, 64, 2, 1))
+    f = fj.build(fj.script(PROGRAMS["c4"]), list(oc.c4_inputs(3, 12, 64, 2, 1)))
+    want = f(*args)
+    torch.cuda.synchronize()
+    pool, g0 = torch.cuda.graph_pool_handle(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g0, pool=pool):
+        junk = [torch.full((8192,), 255, dtype=torch.uint8, device="cuda") for _ in range(600)]
+    g0.replay()
+    torch.cuda.synchronize()
+    del junk
+    graphs, outs = [torch.cuda.CUDAGraph() for _ in range(2)], []
+    for g in graphs:
+        with torch.cuda.graph(g, pool=pool):
+            outs.append(f(*args))
+    for _ in range(3):
+        graphs[1].replay()
+        torch.cuda.synchronize()
+        for got, w in zip(outs[1], want):
+            assert torch.equal(got, w)
+
+
 def test_hip_graph_refuses_row_compaction():
     args = oc.c2_inputs(0, SMALL_GRIDS)
     with pytest.raises(ValueError, match="row-compacting"):
