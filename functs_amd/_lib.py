@@ -194,6 +194,7 @@ _sig("fx_async_error_report", None, _i)
 _fp = ctypes.c_void_p
 _sig("fx_sort_nms", ctypes.c_int, ctypes.POINTER(FxNmsDesc), ctypes.c_void_p)
 _sig("fx_nms_pairs", ctypes.c_int, ctypes.POINTER(FxNmsDesc), ctypes.c_void_p)
+_sig("fx_nms_pairs_pays", ctypes.c_int, ctypes.c_int, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_float)
 _sig("fx_nms_pairs_workspace_bytes", ctypes.c_size_t, ctypes.c_int, ctypes.c_uint32)
 _sig("fx_sort_nms_workspace_bytes", ctypes.c_size_t, ctypes.c_int, ctypes.c_uint32)
 _sig("fx_sort_nms_workspace_clear_bytes", ctypes.c_size_t, ctypes.c_int)

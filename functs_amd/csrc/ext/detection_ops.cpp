@@ -145,7 +145,8 @@ Batched launch(const char* op, int mode, const Tensor& boxes_, const Tensor& sco
   d.n_out = (uint32_t*)r.n.data_ptr<int32_t>();
   if (T > 0) {
     auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
-    const size_t pairs = mode == 0 && !counts.defined() && T <= 65535 && K >= FX_NMS_PAIRS_MIN_ROWS && K <= FX_NMS_PAIRS_MAX_ROWS ? fx_nms_pairs_workspace_bytes((int)T, (uint32_t)K) : 0;
+    const bool pays = mode == 0 && !counts.defined() && fx_nms_pairs_pays((int)T, (uint32_t)K, d.max_num, d.score_thr);
+    const size_t pairs = pays ? fx_nms_pairs_workspace_bytes((int)T, (uint32_t)K) : 0;
     if (pairs > 0) {   // every box is a candidate: ranking and overlap tests over the whole chip
       const Tensor ws = at::empty({(int64_t)pairs}, at::TensorOptions().dtype(at::kByte).device(dev));
       d.workspace = ws.data_ptr();

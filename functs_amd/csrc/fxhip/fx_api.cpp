@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <limits>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -1631,6 +1632,13 @@ size_t fx_nms_pairs_workspace_bytes(int n_tasks, uint32_t rows) {
   return n_tasks < 1 || rows < 1 || rows > FX_NMS_PAIRS_MAX_ROWS ? 0 : fx_nms_pairs_ws_bytes(n_tasks, rows);
 }
 
+int fx_nms_pairs_pays(int n_tasks, uint32_t rows, uint32_t max_num, float score_thr) {
+  if (n_tasks < 1 || rows < FX_NMS_PAIRS_MIN_ROWS || rows > FX_NMS_PAIRS_MAX_ROWS) return 0;
+  if (!(score_thr == -std::numeric_limits<float>::infinity()) || (rows < 320 && n_tasks > 4)) return 0;
+  const uint64_t keys = (uint64_t)n_tasks * rows, kept = std::min(max_num, rows);
+  return keys <= 20000 && keys * rows <= (2048 + kept) << 14 ? 1 : 0;
+}
+
 int fx_nms_pairs(const fx_nms_desc* desc, void* stream_) {
   if (!desc) return fail(FX_E_INVALID, "fx_nms_pairs: null descriptor");
   const fx_nms_desc& d = *desc;
@@ -1642,6 +1650,8 @@ int fx_nms_pairs(const fx_nms_desc* desc, void* stream_) {
   if (d.max_num < 1 || d.max_num > FX_NMS_MAX_OUT)
     return fail(FX_E_LIMIT, "fx_nms_pairs: max_num must be 1.." + std::to_string(FX_NMS_MAX_OUT));
   if (d.n_tasks == 0) return FX_OK;
+  if ((uint64_t)d.n_tasks * ((d.rows + 63u) / 64u) * 4096u >= (1ull << 32))
+    return fail(FX_E_LIMIT, "fx_nms_pairs: " + std::to_string(d.n_tasks) + " tasks of " + std::to_string(d.rows) + " rows are more threads than a launch holds");
   const size_t need = fx_nms_pairs_workspace_bytes(d.n_tasks, d.rows);
   if (need == 0) return fail(FX_E_LIMIT, "fx_nms_pairs: rows must be 1.." + std::to_string(FX_NMS_PAIRS_MAX_ROWS));
   if (!d.workspace || ((uintptr_t)d.workspace & 255u) != 0 || d.workspace_bytes < need)

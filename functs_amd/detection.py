@@ -1,5 +1,6 @@
 """The step behind row compaction in the reference's detection programs - score threshold, sort by
-descending score, class-aware greedy NMS, top-k - as ONE launch for all images (fx_sort_nms).
+descending score, class-aware greedy NMS, top-k - as ONE launch for all images (fx_sort_nms), or as three
+that use the whole chip where all boxes are candidates and few images are to be done (fx_nms_pairs).
 
 Same names and argument meaning as the reference's Python
 (functs/benchmark/ai_model/yolov3/yolov3_bbox.py:104-179, functs/benchmark/ai_model/ssd/ssd_bbox.py:175-214),
@@ -94,9 +95,9 @@ def _launch(mode, boxes, scores, factors, labels, counts, n_classes, score_thr, 
     d.key_capacity = key_capacity
     d.dets, d.out_labels, d.out_index, d.n_out = dets.data_ptr(), out_labels.data_ptr(), out_index.data_ptr(), n_out.data_ptr()
     stream = torch.cuda.current_stream(dev)
-    # every box a candidate: ranking and overlap tests over the whole chip
+    # every box a candidate: ranking and overlap tests over the whole chip where that pays
     pairs = 0
-    if mode == 0 and counts is None and 0 < T <= 65535 and C["FX_NMS_PAIRS_MIN_ROWS"] <= rows <= min(C["FX_NMS_PAIRS_MAX_ROWS"], key_capacity):
+    if mode == 0 and counts is None and rows <= key_capacity <= MAX_CANDIDATES and lib.fx_nms_pairs_pays(T, rows, max_num, score_thr):
         pairs = lib.fx_nms_pairs_workspace_bytes(T, rows)
     if pairs > 0:
         ws = torch.empty(pairs, dtype=torch.uint8, device=dev)

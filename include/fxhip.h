@@ -516,14 +516,30 @@ size_t fx_sort_nms_workspace_bytes(int n_tasks, uint32_t key_capacity);
 size_t fx_sort_nms_workspace_clear_bytes(int n_tasks);
 int fx_sort_nms(const fx_nms_desc* desc, void* stream);
 /* The same results for boxes that are all candidates (mode 0, counts null), up to FX_NMS_PAIRS_MAX_ROWS
- * rows, as three launches that spread the ranking and the overlap tests over the chip.  Below
- * FX_NMS_PAIRS_MIN_ROWS fx_sort_nms is as fast: two chunks of boxes are too little to spread (a call,
- * 64 rows: 27.0 us against 25.6; 100: 28.1 against 27.7; 200: 29.3 against 33.9; 2 000: 47 against 157).  Its workspace is
- * scratch memory (256-byte aligned, nothing is expected in it or left in it); key_capacity is not read. */
+ * rows, as three launches that spread the ranking and the overlap tests over the chip.  Its workspace is
+ * scratch memory (256-byte aligned, nothing is expected in it or left in it); key_capacity is not read.
+ * FX_E_LIMIT: more rows, more than 65535 tasks, or a ranking of 2^32 threads and more (tasks * rows / 64
+ * rounded up * 4096).  n_out, like the other results, is valid in stream order: a host that polls it in
+ * pinned memory may see it before the rows are there. */
 #define FX_NMS_PAIRS_MIN_ROWS 129
 #define FX_NMS_PAIRS_MAX_ROWS 4096 /* 64 chunks of 64 */
 size_t fx_nms_pairs_workspace_bytes(int n_tasks, uint32_t rows); /* 0: more rows than that, or none */
 int fx_nms_pairs(const fx_nms_desc* desc, void* stream);
+/* 1: a call is better served by fx_nms_pairs than by fx_sort_nms.  The work of fx_nms_pairs is tasks * rows^2
+ * overlap tests and tasks * rows^2 / 16 keys read, whatever is kept; fx_sort_nms gives every task a CU of its
+ * own (up to 256 tasks take the time of one) and walks what it keeps, at most max_num boxes, and only a call's
+ * candidates: a score threshold is its case (16 tasks of 4 096 rows, 1 in 10 above it: 32 us, fx_nms_pairs 206).
+ * Microseconds a call, launches back to back, fx_sort_nms (300 kept; max_num and as many kept 1 024) : fx_nms_pairs
+ *     rows     1 task          4 tasks          8 tasks          16 tasks         32 tasks         128 tasks
+ *     200      24 : 30         24 : 29          24 : 29          25 : 30          25 : 30          25 : 34
+ *     500      40 : 30         40 : 29          40 : 30          40 : 29          41 : 29          38 : 56
+ *     1 000    39, 117 : 30    38, 118 : 29     39, 118 : 29     39, 119 : 31     39, 119 : 46     41 : 139
+ *     2 000    44, 199 : 29    44, 211 : 29     44, 211 : 41-51  44, 211 : 67-76  45, 223 : 117-127
+ *     4 096    53, 194 : 30    54, 195 : 64-76  54, 196 : 111+   54, 196 : 204+   54, 198 : 391+
+ * Hence bounds on tasks * rows and on tasks * rows^2, the latter moved by what may be kept.  Few rows are
+ * bound by three launches against one when nobody waits for them; a caller of one image that does is served
+ * faster from FX_NMS_PAIRS_MIN_ROWS on (129 rows 33 : 31, 200: 39 : 31, 400: 56 : 33; 64: 25.6 : 27.0). */
+int fx_nms_pairs_pays(int n_tasks, uint32_t rows, uint32_t max_num, float score_thr);
 
 /* ---- device utilities ---- */
 int fx_device_count(void);

@@ -334,3 +334,54 @@ def test_thresholds_below_zero_and_corners_in_any_order(thr):
     got = detection.batched_nms_batched(b, s, None, iou_threshold=thr)
     want = detection.batched_nms_batched(b, s, None, counts=torch.full((1,), n, dtype=torch.int32, device=dev), iou_threshold=thr)
     assert torch.equal(got.n, want.n) and torch.equal(got.index, want.index) and torch.equal(got.dets.view(torch.int32), want.dets.view(torch.int32))
+
+
+def test_three_launches_where_they_pay():
+    """The rule of fx_nms_pairs_pays: all boxes are candidates, and not more images and rows than one pass over
+    all pairs is cheaper for; its scratch memory stays small with it."""
+    from functs_amd._lib import lib
+    inf = float("inf")
+    assert all(lib.fx_nms_pairs_pays(1, n, m, -inf) for n in (129, 200, 500, 2000, 4096) for m in (1, 300, 1024))
+    assert not any(lib.fx_nms_pairs_pays(1, n, 1024, -inf) for n in (0, 1, 128, 4097))
+    assert not any(lib.fx_nms_pairs_pays(t, n, 1024, thr) for t in (1, 16) for n in (200, 4096) for thr in (0.05, 0.0, -1.0, inf, float("nan")))
+    assert lib.fx_nms_pairs_pays(4, 200, 300, -inf) and not lib.fx_nms_pairs_pays(5, 200, 300, -inf)
+    assert lib.fx_nms_pairs_pays(8, 2000, 300, -inf) and not lib.fx_nms_pairs_pays(16, 2000, 1024, -inf)
+    assert lib.fx_nms_pairs_pays(32, 500, 300, -inf) and not lib.fx_nms_pairs_pays(128, 500, 300, -inf) and not lib.fx_nms_pairs_pays(0, 500, 300, -inf)
+    assert all(lib.fx_nms_pairs_workspace_bytes(t, n) < 16 << 20 for t in range(1, 156) for n in (129, 500, 1000, 4096) if lib.fx_nms_pairs_pays(t, n, 1024, -inf))
+
+
+def test_a_ranking_of_too_many_threads_is_refused():
+    from functs_amd._lib import C, FxNmsDesc, lib
+    import ctypes
+    d = FxNmsDesc()
+    d.mode, d.n_tasks, d.rows, d.max_num = 0, 16384, 4096, 100
+    d.boxes = d.scores = d.dets = d.out_labels = d.n_out = d.workspace = 256   # (refused ahead of any use)
+    d.workspace_bytes = 1 << 62
+    assert lib.fx_nms_pairs(ctypes.byref(d), None) == C["FX_E_LIMIT"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,n,kw", [(1, 4096, {"score_thr": 0.9}), (16, 600, {"score_thr": 0.5}), (64, 1000, {}), (5, 200, {}), (40, 500, {})])
+def test_other_calls_keep_to_one_launch_or_agree_with_it(T, n, kw):
+    """A score threshold and many images: the route and its result against the call with counts."""
+    from functs_amd import aot, detection
+    from functs_amd._lib import lib
+    g = torch.Generator().manual_seed(T)
+    dev = torch.device("cuda:0")
+    b, s = torch.stack([_boxes(g, n, span=600.0) for _ in range(T)]).to(dev), torch.rand(T, n, generator=g).to(dev)
+    print("batched_nms_batched T=%d n=%d %s" % (T, n, kw), flush=True)
+    l0, _ = aot.launch_stats()
+    got = detection.batched_nms_batched(b, s, None, max_num=300, **kw)
+    l1, _ = aot.launch_stats()
+    assert l1 - l0 == (3 if lib.fx_nms_pairs_pays(T, n, 300, kw.get("score_thr", float("-inf"))) else 1) == (3 if (T, n) == (40, 500) else 1)
+    want = detection.batched_nms_batched(b, s, None, counts=torch.full((T,), n, dtype=torch.int32, device=dev), max_num=300, **kw)
+    assert torch.equal(got.n, want.n) and torch.equal(got.index, want.index) and torch.equal(got.dets.view(torch.int32), want.dets.view(torch.int32))
+
+
+@pytest.mark.gpu
+def test_a_key_capacity_out_of_range_is_refused_on_either_route():
+    from functs_amd import detection
+    from functs_amd._lib import FxError
+    b, s = torch.rand(1, 500, 4, device="cuda"), torch.rand(1, 500, device="cuda")
+    with pytest.raises(FxError):
+        detection.batched_nms_batched(b, s, None, key_capacity=20000)
