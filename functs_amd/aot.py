@@ -55,12 +55,13 @@ SPEC_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc", "fxh
 
 
 @contextlib.contextmanager
-def capture(directory: str = SPEC_DIR, program_tables: bool = True, rowstream: bool = True):
+def capture(directory: str = SPEC_DIR, program_tables: bool = True, rowstream: bool = True, boxes: bool = False):
     """Every region planned inside the block that has no compiled kernels linked in writes
     ``fx_spec_<key>.hip`` (its programs as a table for the generic kernels) and, when it has a
-    row-stream form, ``fx_rs_<key>.hip`` into ``directory``."""
+    row-stream form, ``fx_rs_<key>.hip`` into ``directory``; with ``boxes`` also the program table of
+    the form with its outputs in boxes, when it has one."""
     os.makedirs(directory, exist_ok=True)
-    _lib.lib.fx_spec_dump_what((1 if program_tables else 0) | (2 if rowstream else 0))
+    _lib.lib.fx_spec_dump_what((1 if program_tables else 0) | (2 if rowstream else 0) | (4 if boxes else 0))
     _lib.check(_lib.lib.fx_spec_dump_dir(directory.encode()))
     try:
         yield directory
@@ -120,6 +121,27 @@ def load_cached_kernels() -> int:
     return len(_loaded)
 
 
+def _units_to_compile(directory: str, tables: str):
+    """Names of the units in `directory` that compile_sources takes.  Of a region with a form in boxes one
+    is enough: the whole form if it is taken (a region runs it wherever it is at hand), else the boxes."""
+    names, boxes_of = [], {}
+    for src in sorted(glob.glob(os.path.join(directory, "fx_*.hip"))):
+        name = os.path.splitext(os.path.basename(src))[0]
+        if name.startswith("fx_spec_"):
+            with open(src) as fh:
+                text = fh.read()
+            dense = "FX_SPEC_DENSE" in text
+            m = re.search(r"FxInsn code\[(\d+)\]", text)
+            n_insn = int(m.group(1)) if m else 1 << 30
+            if tables == "none" or (tables == "dense" and not dense) or (tables == "auto" and not (dense and n_insn <= AUTO_TABLE_INSNS)):
+                continue
+            m = re.search(r"in boxes \(whole: ([0-9a-f]{16})\)", text)
+            if m:
+                boxes_of[name] = "fx_spec_" + m.group(1)
+        names.append(name)
+    return [n for n in names if boxes_of.get(n) not in names]
+
+
 def compile_sources(directory: str, verbose: bool = False, tables: str = "auto"):
     """Compiles the generated units of `directory` that have no object in the cache yet into
     shared objects there and loads them.  Every row-stream unit (``fx_rs_*.hip``: straight-line
@@ -136,16 +158,8 @@ def compile_sources(directory: str, verbose: bool = False, tables: str = "auto")
     os.makedirs(out_dir, exist_ok=True)
     lib_dir = os.path.dirname(_lib.LIB_PATH)
     done = []
-    for src in sorted(glob.glob(os.path.join(directory, "fx_*.hip"))):
-        name = os.path.splitext(os.path.basename(src))[0]
-        if name.startswith("fx_spec_"):
-            with open(src) as fh:
-                text = fh.read()
-            dense = "FX_SPEC_DENSE" in text
-            m = re.search(r"FxInsn code\[(\d+)\]", text)
-            n_insn = int(m.group(1)) if m else 1 << 30
-            if tables == "none" or (tables == "dense" and not dense) or (tables == "auto" and not (dense and n_insn <= AUTO_TABLE_INSNS)):
-                continue
+    for name in _units_to_compile(directory, tables):
+        src = os.path.join(directory, name + ".hip")
         obj = os.path.join(out_dir, name + ".so")
         if not os.path.isfile(obj):
             tmp = obj + ".%d.tmp" % os.getpid()
@@ -169,7 +183,7 @@ def compile_missing(fn=None, planner=None, verbose: bool = False, tables: str = 
     Returns the names of the units compiled now."""
     tmp = tempfile.mkdtemp(prefix="functs_amd_src_")
     try:
-        with capture(tmp):
+        with capture(tmp, boxes=True):
             if fn is not None:
                 plan(fn)
             if planner is not None:

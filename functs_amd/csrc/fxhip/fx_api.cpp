@@ -64,8 +64,8 @@ hipError_t fx_launch_compact_rows(const uint8_t* mask, int64_t n, const void* co
 
 struct fx_region {
   fx::Region r;
-  std::mutex mu;  // plan cache + device upload (the reference serialises extent
-                  // evaluation the same way, cuda_codegen_tssa.cpp:1207)
+  std::mutex& mu = r.mu;  // plan cache + device upload (the reference serialises extent
+                          // evaluation the same way, cuda_codegen_tssa.cpp:1207)
 };
 struct fx_plan {
   fx::Plan p;
@@ -118,11 +118,13 @@ int fx_region_create(int parallel_degree, int is_parallel_map, fx_region** out) 
 
 void fx_region_destroy(fx_region* r) {
   if (!r) return;
-  for (auto& kv : r->r.plans) {
-    if (kv.second->dev_blob) (void)hipFree(kv.second->dev_blob);
-    for (auto& st : kv.second->status)
-      if (st.ptr) (void)hipFree(st.ptr);
-  }
+  for (auto& kv : r->r.plans)
+    for (fx::Plan* p : {kv.second.get(), kv.second->boxed.get()}) {
+      if (!p) continue;
+      if (p->dev_blob) (void)hipFree(p->dev_blob);
+      for (auto& st : p->status)
+        if (st.ptr) (void)hipFree(st.ptr);
+    }
   delete r;
 }
 
@@ -277,7 +279,7 @@ static std::atomic<uint32_t> g_totals_spin_us{2000u};   // microseconds that fx_
 static std::atomic<uint32_t> g_lstm_spin{1000000u};   // polls of a wait of fx_lstm_stack before it is given up
 static std::mutex g_dump_mu;
 static std::string g_dump_dir;
-static int g_dump_what = 3;   // bit 0: program tables (fx_spec_*), bit 1: row-stream units (fx_rs_*)
+static int g_dump_what = 3;   // bit 0: program tables (fx_spec_*), bit 1: row-stream units (fx_rs_*), bit 2: program tables of outputs in boxes
 
 static std::atomic<uint64_t> g_launches{0}, g_spec_launches{0};
 
@@ -286,14 +288,10 @@ static const FxSpecKernels* spec_of(const fx::Plan* p) {
   return fx_spec_find(p->spec_key);
 }
 
-static const bool g_spec_linked_set = [] {
-  fx::spec_linked = [](uint64_t key) { return g_specialize.load(std::memory_order_relaxed) && key != 0 && fx_spec_find(key) != nullptr; };
-  return true;
-}();
-
 // With a dump directory set, every plan that has no specialised kernels linked in leaves
-// the translation unit that would specialise it there (one file per key).
-static void dump_spec_source(const fx::Plan* p) {
+// the translation unit that would specialise it there (one file per key); bit 2: a plan that has a form
+// in boxes leaves that form's as well (whole: the plan it is a form of).
+static void dump_spec_source(const fx::Plan* p, const fx::Plan* whole = nullptr) {
   std::string dir;
   int what = 3;
   {
@@ -301,6 +299,7 @@ static void dump_spec_source(const fx::Plan* p) {
     dir = g_dump_dir;
     what = g_dump_what;
   }
+  if (p->boxed && (what & 4) && !fx_spec_find(p->spec_key)) dump_spec_source(p->boxed.get(), p);
   if (!dir.empty() && (what & 2) && p->rs.ok && !fx_rs_find(p->rs.key)) {
     char rname[64];
     snprintf(rname, sizeof(rname), "/fx_rs_%016llx.hip", (unsigned long long)p->rs.key);
@@ -336,6 +335,10 @@ static void dump_spec_source(const fx::Plan* p) {
     for (size_t d = 0; d < sh.size(); ++d) label += (d ? "," : "") + std::to_string(sh[d]);
     label += "]";
   }
+  if (whole) {
+    snprintf(name, sizeof(name), ", in boxes (whole: %016llx)", (unsigned long long)whole->spec_key);
+    label += name;
+  }
   const std::string src = fx::spec_source(*p, label);
   if (FILE* f = fopen(path.c_str(), "w")) {
     fwrite(src.data(), 1, src.size(), f);
@@ -348,13 +351,27 @@ int fx_region_plan(fx_region* reg, const fx_arg* args, int n_args, const fx_plan
   FX_TRY
   std::lock_guard<std::mutex> g(reg->mu);
   const fx::Plan* p = fx::plan_region(reg->r, args, n_args);
+  if (!spec_of(p)) (void)fx::boxed_form(p);
   *plan = reinterpret_cast<const fx_plan*>(p);
   dump_spec_source(p);
   return FX_OK;
   FX_CATCH
 }
 
-static const fx::Plan* P(const fx_plan* p) { return reinterpret_cast<const fx::Plan*>(p); }
+// The plan that a handle stands for now: outputs are computed whole where the region has compiled kernels
+// for that (one store of whole groups an item, temporaries in registers; the lean kernel), in boxes
+// otherwise.  Kernels may be switched off and on or loaded later, so a handle keeps both forms.
+static const fx::Plan* P(const fx_plan* p) {
+  const fx::Plan* whole = reinterpret_cast<const fx::Plan*>(p);
+  if (whole->box_args.empty() || spec_of(whole)) return whole;
+  std::lock_guard<std::mutex> g(whole->region->mu);
+  const fx::Plan* boxed = nullptr;
+  try {
+    boxed = fx::boxed_form(whole);
+  } catch (...) {   // (fx_region_plan has reported it; this may be any entry point)
+  }
+  return boxed ? boxed : whole;
+}
 
 void fx_set_specialization(int on) { g_specialize.store(on ? 1 : 0, std::memory_order_relaxed); }
 int fx_specialization_count(void) { return fx_spec_count(); }
@@ -385,7 +402,7 @@ int fx_spec_dump_dir(const char* dir) {
 int fx_spec_dump_what(int what) {
   std::lock_guard<std::mutex> g(g_dump_mu);
   const int before = g_dump_what;
-  g_dump_what = what & 3;
+  g_dump_what = what & 7;
   return before;
 }
 

@@ -1887,7 +1887,8 @@ std::vector<Box> Lowerer::boxesOf(int vid, const Shape& s, const Prog& whole) {
     Prog p;
     try {
       p = lowerBox(vid, b, &cut);
-    } catch (const Error&) {   // (a box's index record may exceed 32 bits where the whole program's steps do not)
+    } catch (const Error& e) {   // (a box's index record may exceed 32 bits where the whole program's steps do not)
+      if (e.code != FX_E_LIMIT && e.code != FX_E_UNSUPPORTED) throw;
       loopVarBound_ = false;
       code = code0;
       affs = affs0;
@@ -2114,42 +2115,16 @@ static bool findWindow(const ClassBuild& cb, StreamInfo* si, std::vector<WinPick
 // ---------------------------------------------------------------------------
 // plan construction
 // ---------------------------------------------------------------------------
-bool (*spec_linked)(uint64_t) = nullptr;
-
-static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args, bool boxed, bool* could_box);
-
-const Plan* plan_region(Region& R, const fx_arg* args, int n_args) {
-  R.index_ints.resize(R.inputs.size(), 0);
-  for (;;) {
-    try {
-      // Outputs are computed whole where the region has compiled kernels for that (one store of whole
-      // groups an item, temporaries in registers; the lean kernel), in boxes otherwise if that pays
-      // (Lowerer::boxesOf) and the descriptor still fits.
-      bool could_box = false;
-      const Plan* whole = plan_region_once(R, args, n_args, false, &could_box);
-      if (!could_box || (spec_linked && spec_linked(whole->spec_key))) return whole;
-      try {
-        return plan_region_once(R, args, n_args, true, nullptr);
-      } catch (const Error&) {
-        return whole;
-      }
-    } catch (const NeedIndexInt& need) {
-      FX_CHECK(need.input >= 0 && need.input < (int)R.index_ints.size() && !R.index_ints[need.input], FX_E_INVALID,
-               "per-task int input " << need.input << " cannot be resolved");
-      R.index_ints[need.input] = 1;
-    }
-  }
-}
-
-// boxed: outputs in boxes, in the place of the plan of whole outputs that could_box was set for
-static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args, bool boxed_outs, bool* could_box) {
+// What a plan depends on: the arguments' layouts and the int values that shapes or programs are made of.
+// arg_base: first argument of every input.
+static std::vector<int64_t> plan_key(const Region& R, const fx_arg* args, int n_args, std::vector<int>* arg_base) {
   FX_CHECK(R.finalized, FX_E_INVALID, "region is not finalized");
   const int T = R.degree;
   // argument layout
-  std::vector<int> arg_base(R.inputs.size());
+  arg_base->assign(R.inputs.size(), 0);
   int expect = 0;
   for (size_t i = 0; i < R.inputs.size(); ++i) {
-    arg_base[i] = expect;
+    (*arg_base)[i] = expect;
     expect += R.vals[R.inputs[i]].per_task ? T : 1;
   }
   FX_CHECK(n_args == expect, FX_E_INVALID, "expected " << expect << " arguments, got " << n_args);
@@ -2160,21 +2135,66 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args, b
     const Value& v = R.vals[R.inputs[i]];
     int n = v.per_task ? T : 1;
     for (int t = 0; t < n; ++t) {
-      const fx_arg& a = args[arg_base[i] + t];
+      const fx_arg& a = args[(*arg_base)[i] + t];
       if (v.kind == VK_TENSOR) {
-        FX_CHECK(a.kind == 0, FX_E_INVALID, "argument " << arg_base[i] + t << " must be a tensor");
+        FX_CHECK(a.kind == 0, FX_E_INVALID, "argument " << (*arg_base)[i] + t << " must be a tensor");
         FX_CHECK(a.rank >= 0 && a.rank <= FX_ARG_MAX_RANK, FX_E_INVALID, "bad tensor rank");
         key.push_back(a.dtype); key.push_back(a.rank);
         for (int d = 0; d < a.rank; ++d) { key.push_back(a.sizes[d]); key.push_back(a.strides[d]); }
       } else {
-        FX_CHECK(a.kind != 0, FX_E_INVALID, "argument " << arg_base[i] + t << " must be a scalar");
+        FX_CHECK(a.kind != 0, FX_E_INVALID, "argument " << (*arg_base)[i] + t << " must be a scalar");
         key.push_back(-7);
         if ((v.kind == VK_INT || v.kind == VK_BOOL) && (!v.per_task || R.index_ints[i])) key.push_back(a.ival);
       }
     }
   }
-  auto it = R.plans.find(key);
-  if (it != R.plans.end() && !boxed_outs) return it->second.get();
+  return key;
+}
+
+static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_args, const std::vector<int>& arg_base, bool boxed_outs, bool* could_box);
+
+const Plan* plan_region(Region& R, const fx_arg* args, int n_args) {
+  R.index_ints.resize(R.inputs.size(), 0);
+  for (;;) {
+    try {
+      std::vector<int> arg_base;
+      const std::vector<int64_t> key = plan_key(R, args, n_args, &arg_base);
+      auto it = R.plans.find(key);
+      if (it != R.plans.end()) return it->second.get();
+      bool could_box = false;
+      std::unique_ptr<Plan> whole = build_plan(R, args, n_args, arg_base, false, &could_box);
+      if (could_box) whole->box_args.assign(args, args + n_args);
+      const Plan* res = whole.get();
+      R.plans[key] = std::move(whole);
+      return res;
+    } catch (const NeedIndexInt& need) {
+      FX_CHECK(need.input >= 0 && need.input < (int)R.index_ints.size() && !R.index_ints[need.input], FX_E_INVALID,
+               "per-task int input " << need.input << " cannot be resolved");
+      R.index_ints[need.input] = 1;
+    }
+  }
+}
+
+const Plan* boxed_form(const Plan* whole) {
+  Plan& w = *const_cast<Plan*>(whole);
+  if (w.box_args.empty() || w.box_tried) return w.boxed.get();
+  std::unique_ptr<Plan> p;
+  try {
+    p = build_plan(*const_cast<Region*>(w.region), w.box_args.data(), w.n_args, w.arg_base, true, nullptr);
+  } catch (const Error& e) {   // the boxes' descriptor does not fit
+    if (e.code != FX_E_LIMIT && e.code != FX_E_UNSUPPORTED) throw;
+  }
+  w.box_tried = true;
+  // (nor do an interpreter's temporaries beside it; and the caller's memory is laid out for the whole form)
+  if (p && (w.needs_compiled || !p->needs_compiled) && p->scratch_bytes == w.scratch_bytes && p->sptr.size() == w.sptr.size() &&
+      p->tptr.size() == w.tptr.size() && p->sscal.size() == w.sscal.size() && p->tscal.size() == w.tscal.size())
+    w.boxed = std::move(p);
+  return w.boxed.get();
+}
+
+// boxed_outs: outputs in boxes (Lowerer::boxesOf), for a plan of whole outputs that could_box was set for
+static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_args, const std::vector<int>& arg_base, bool boxed_outs, bool* could_box) {
+  const int T = R.degree;
 
   std::unique_ptr<Plan> P(new Plan());
   P->region = &R;
@@ -2307,6 +2327,8 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args, b
         // leading load: unconditional, affine, not inside a reduction loop
         const FxInsn& i0 = L.code[p.begin];
         od.lead = (p.end > p.begin && i0.op == FX_LDA) ? 1u : 0u;
+        // (the batches of pure programs keep one output offset an item and store whole groups behind it: the
+        // elements of a box may lie apart)
         bool pure = od.lead != 0 && !p.rowwave && !boxed;
         for (uint32_t pc = p.begin + 1; pure && pc < p.end; ++pc) {
           const FxInsn& in = L.code[pc];
@@ -2656,9 +2678,7 @@ static const Plan* plan_region_once(Region& R, const fx_arg* args, int n_args, b
     match_classmap(P.get());
   }
   rs_analyze(P.get());
-  const Plan* res = P.get();
-  R.plans[key] = std::move(P);
-  return res;
+  return P;
 }
 
 // ---------------------------------------------------------------------------

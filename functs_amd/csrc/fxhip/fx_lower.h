@@ -11,6 +11,7 @@
 
 #include <map>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -60,6 +61,7 @@ struct Region {
   // into classes (all other per-task scalars are plain run-time data)
   std::vector<char> index_ints;
   std::map<std::vector<int64_t>, std::unique_ptr<Plan>> plans;
+  mutable std::mutex mu;     // plans and what is filled in after they were made
 
   int add(const Value& v) {
     vals.push_back(v);
@@ -130,6 +132,11 @@ struct Plan {
   int n_args = 0;
   // device copy of blob, created on first run
   uint64_t spec_key = 0;       // spec_hash of this plan
+  // The same outputs in boxes (Lowerer::boxesOf), where that pays for an interpreter: built when it is
+  // first asked for (boxed_form), from the layouts that this plan was made for (empty: it does not pay).
+  std::vector<fx_arg> box_args;
+  bool box_tried = false;
+  std::unique_ptr<Plan> boxed;
   void* dev_blob = nullptr;
   int dev_id = -1;
   // streaming compaction: tile status words, one buffer per launch stream (zero when allocated,
@@ -150,10 +157,10 @@ void match_head(Plan* p);
 // Fills p->cmap: does the plan compute the decode + per-class score filter of an SSD-style head (fx_cmap_match.cpp)?
 void match_classmap(Plan* p);
 
-// Whether compiled kernels are at hand for a spec_hash (set by the library; null: none are).
-extern bool (*spec_linked)(uint64_t key);
 // Builds (or fetches from the cache) the plan of `r` for these arguments.
 const Plan* plan_region(Region& r, const fx_arg* args, int n_args);
+// The form of a plan with its outputs in boxes; null: there is none.  As plan_region, under the region's lock.
+const Plan* boxed_form(const Plan* whole);
 std::string disasm(const Plan& p);
 // Rank the region kernels are instantiated for (1, 2, 3, 4 or FX_MAXR).
 int kernel_rank(int rank);

@@ -287,7 +287,7 @@ void fx_launch_stats(uint64_t* total, uint64_t* specialised); /* region kernel l
 int fx_plan_dense_lean(const fx_plan*);
 void fx_set_dense_lean(int on);
 int fx_spec_dump_dir(const char* dir);          /* plans without specialised kernels leave their source in dir (NULL: stop) */
-int fx_spec_dump_what(int what);                /* which sources: 1 program tables (fx_spec_*), 2 row-stream units (fx_rs_*), 3 both (default), 0 none; returns the setting before */
+int fx_spec_dump_what(int what);                /* which sources: 1 program tables (fx_spec_*), 2 row-stream units (fx_rs_*), 3 both (default), 4 also the tables of outputs in boxes, 0 none; returns the setting before */
 
 /* ---- execution (replaces CudaCodeGenTssa::call_raw, cuda_codegen_tssa.cpp:1167-1290) ----
  * out_ptrs[out_idx * parallel_degree + task] = device buffer of that output.

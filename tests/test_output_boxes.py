@@ -1,6 +1,7 @@
 """Outputs computed in boxes of their elements (fx_lower.cpp, Lowerer::boxesOf): one program per box,
 cut where the range tests of cat / stack / in-place slices change their answer.  Values against
 stock PyTorch at extents around lane groups and work items, for the emulator and the GPU."""
+import os
 import re
 
 import pytest
@@ -164,3 +165,66 @@ def test_transposed_boxes(backend, c, n):
     ref = torch.cat([y.sigmoid() * 2 - 1, x, y.exp() + 1, x * 0.5 + 2, y.tanh() - 1, (y + 1) * (y - 1)], 1).transpose(1, 2)
     assert_close(got, ref, atol=2.0 ** -22)   # (differences of values near 1)
     assert n_programs(r, x, y) >= 6 + (2 if c % 4 else 0)
+
+
+def _decode_args():
+    from functs_amd.benchmark.inputs import INPUTS
+    return INPUTS["c3"](0)
+
+
+@pytest.mark.parametrize("first", [True, False])
+def test_a_plan_does_not_remember_the_switch_it_was_made_under(first):
+    """A region whose whole form is linked runs that whenever compiled kernels are on, in boxes while they
+    are off, whatever held when it was planned first."""
+    from functs_amd import aot, configs
+    r, args = configs.build_c3_decode(), _decode_args()
+    try:
+        seen = {}
+        for on in (first, not first, first, not first):
+            aot.enable(on)
+            seen.setdefault(on, set()).add((r.spec_key(*args), r.specialized(*args), n_programs(r, *args)))
+    finally:
+        aot.enable(True)
+    assert [len(v) for v in seen.values()] == [1, 1]
+    (key_on, linked, whole), (key_off, off, boxes) = seen[True].pop(), seen[False].pop()
+    assert linked and whole == 2 and not off and boxes > 2 and key_on != key_off
+
+
+@pytest.mark.gpu
+def test_both_forms_of_a_linked_region_on_the_device():
+    from functs_amd import aot, configs
+    r, args = configs.build_c3_decode(), [t.cuda() for t in _decode_args()]
+    outs, ran = [], []
+    try:
+        for on in (False, True, False):
+            aot.enable(on)
+            before = aot.launch_stats()
+            outs.append([t.clone() for t in r(*args)])
+            ran.append(aot.launch_stats()[1] - before[1])
+    finally:
+        aot.enable(True)
+    assert ran == [0, 1, 0]
+    for got in outs[1:]:
+        for a, b in zip(got, outs[0]):
+            assert torch.equal(a, b)
+
+
+def test_a_capture_leaves_the_whole_form_and_on_request_the_boxes(tmp_path):
+    from functs_amd import aot
+    x, a = torch.randn(50, 4), torch.randn(20, 4)
+    entries = lambda d: sorted(int(re.search(r"n_entries = (\d+)", (d / f).read_text()).group(1)) for f in os.listdir(d))
+    with aot.capture(str(tmp_path / "whole")):
+        aot._plan_region(corners_region(50, 20), x, a)
+    assert entries(tmp_path / "whole") == [1]
+    with aot.capture(str(tmp_path / "both"), boxes=True):
+        aot._plan_region(corners_region(50, 20), x, a)
+    assert entries(tmp_path / "both") == [1, 8] and set(os.listdir(tmp_path / "whole")) < set(os.listdir(tmp_path / "both"))
+    # one of the two is compiled: the whole form where it is short enough, else the boxes
+    whole = os.listdir(tmp_path / "whole")[0][:-4]
+    assert aot._units_to_compile(str(tmp_path / "both"), "dense") == [whole] == aot._units_to_compile(str(tmp_path / "both"), "auto")
+    limit, aot.AUTO_TABLE_INSNS = aot.AUTO_TABLE_INSNS, 100
+    try:
+        (boxes,) = aot._units_to_compile(str(tmp_path / "both"), "auto")
+    finally:
+        aot.AUTO_TABLE_INSNS = limit
+    assert boxes != whole
