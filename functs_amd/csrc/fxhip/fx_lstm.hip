@@ -755,11 +755,15 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     // one tile of four rows a workgroup while that makes at most one workgroup for each CU, whose registers the
     // weights fill
     if (f[i].tiles == 1 && f[i].grid > cus) continue;
-    int per_cu = 0;
+    int per_cu = 0, sure = 0;
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)f[i].kernel, f[i].threads, 0);
     if (e != hipSuccess) return 100 + (int)e;
     if ((long)per_cu * cus < f[i].grid) continue;
-    const uint32_t want = fx_lstm_need((uint32_t)f[i].grid, (uint32_t)per_cu);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&sure, (const void*)f[i].kernel, (int)fx_lstm_block((uint32_t)f[i].threads), 0) != hipSuccess) {
+      (void)hipGetLastError();
+      sure = 1;
+    }
+    const uint32_t want = fx_lstm_need((uint32_t)f[i].grid, (uint32_t)sure);
     if (l && want >= need) continue;
     l = &f[i];
     need = want;

@@ -4,7 +4,10 @@
 // text builds for the CPU as well, where a test runs it (tests/support/lstm_emul.cpp).
 //
 // A launch needs grid / r compute units, r = how many of its workgroups fit one, rounded down to a power
-// of two (unit: FX_LSTM_CU-ths).  Launches whose needs together are at most the device all get their
+// of two (unit: FX_LSTM_CU-ths).  r counts every workgroup as a whole number of waves for each of the
+// compute unit's four SIMDs (fx_lstm_block): which SIMD gets the odd waves is the hardware's choice, and two
+// workgroups of ten waves of 96 registers, which would fit with five waves on each, do not with six on one.
+// Launches whose needs together are at most the device all get their
 // places, whatever the order in which the workgroups arrive: take the smallest of those that still have
 // workgroups without a place (smaller ones end by themselves).  If no compute unit had room for one more,
 // every one would be full, for what the others take of it is a multiple of what this one takes; but one
@@ -20,6 +23,7 @@
 
 #define FX_LSTM_CU 64u
 
+inline uint32_t fx_lstm_block(uint32_t threads) { return (threads + 255u) & ~255u; }
 inline uint32_t fx_lstm_need(uint32_t grid, uint32_t per_cu) {
   uint32_t r = 1u;
   while (2u * r <= per_cu && 2u * r <= FX_LSTM_CU) r *= 2u;

@@ -39,6 +39,8 @@ def lstm_emul():
     so.fx_lstm_groups_emul.restype = ctypes.c_uint64
     so.fx_lstm_groups_emul.argtypes = [ctypes.c_uint32, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_uint32), ctypes.c_int, ctypes.c_uint32,
                                        ctypes.POINTER(ctypes.c_int)]
+    so.fx_lstm_block_of.restype = ctypes.c_uint32
+    so.fx_lstm_block_of.argtypes = [ctypes.c_uint32]
     so.fx_lstm_need_of.restype = ctypes.c_uint32
     so.fx_lstm_need_of.argtypes = [ctypes.c_uint32, ctypes.c_uint32]
     so.fx_lstm_emul_give_up.restype = ctypes.c_int

@@ -295,4 +295,5 @@ extern "C" uint64_t fx_lstm_groups_emul(uint32_t seed, int streams, int launches
   for (auto& e : edges) most = std::max(most, sum += e.second);
   return (uint64_t)most;
 }
+extern "C" uint32_t fx_lstm_block_of(uint32_t threads) { return fx_lstm_block(threads); }
 extern "C" uint32_t fx_lstm_need_of(uint32_t grid, uint32_t per_cu) { return fx_lstm_need(grid, per_cu); }

@@ -179,6 +179,25 @@ def test_launches_that_may_overlap_fit_the_device_together(seed):
     assert so.fx_lstm_groups_emul(seed, 2, 100, halves, 1, device, ctypes.byref(waits)) == device and waits.value == 0   # two halves overlap
 
 
+@pytest.mark.parametrize("waves,registers", [(5, 40), (5, 72), (7, 72), (8, 92), (8, 120), (10, 64), (10, 96), (11, 112), (12, 104), (12, 152)])
+def test_workgroups_that_share_a_compute_unit_fit_however_their_waves_are_dealt(waves, registers):
+    """The share of a compute unit that a launch is counted with is enough when the odd waves of all
+    workgroups go to the same SIMD: (waves, registers) of a workgroup beside every other kind."""
+    from tests.support import emul
+    so = emul.lstm_emul()
+    kinds = [(5, 40), (7, 72), (8, 92), (10, 96), (11, 112), (12, 152)] + [(waves, registers)]
+    unit = so.fx_lstm_need_of(1, 1)
+
+    def share(w, v):   # resident workgroups as the runtime counts them: waves of the whole unit
+        per_cu = 4 * min(8, 512 // v) // (so.fx_lstm_block_of(64 * w) // 64)
+        return so.fx_lstm_need_of(1, per_cu)
+    for w, v in kinds:
+        for n in range(unit // share(waves, registers) + 1):
+            m = (unit - n * share(waves, registers)) // share(w, v)   # the rest of the unit, filled up
+            most = [n * -(-waves // 4), m * -(-w // 4)]               # waves on the fullest SIMD
+            assert sum(most) <= 8 and most[0] * registers + most[1] * v <= 512, (w, v, n, m)
+
+
 def _gpu(x, wih, whh, bih, bhh, h0, c0, launches=1):
     """`launches` calls in a row on one workspace that is cleared once; the last call's results."""
     from functs_amd._lib import check, lib
