@@ -2163,7 +2163,10 @@ const Plan* plan_region(Region& R, const fx_arg* args, int n_args) {
       if (it != R.plans.end()) return it->second.get();
       bool could_box = false;
       std::unique_ptr<Plan> whole = build_plan(R, args, n_args, arg_base, false, &could_box);
-      if (could_box) whole->box_args.assign(args, args + n_args);
+      if (could_box) {
+        whole->box_args.assign(args, args + n_args);
+        for (fx_arg& a : whole->box_args) a.ptr = nullptr;   // (layouts only: the tensors are the caller's)
+      }
       const Plan* res = whole.get();
       R.plans[key] = std::move(whole);
       return res;
