@@ -1870,6 +1870,12 @@ void Lowerer::noteCut(const IdxExpr& x, int64_t lo, int64_t hi, int64_t step) {
 // Interpreted, MI355X: box regression of 8 732 x 21 boxes 518 us whole, 60 in four boxes, 24 with the
 // divisions gone (1 553 instructions, four times 103, four times 30); the YOLO head of four 608 x 608
 // images with its NMS 743, 270, 122 us (18 boxes).
+// Only instructions are weighed.  Boxes that are columns of a row-major output write parts of lines, which costs
+// less than what they save also where the output is beyond the caches (whole : boxes, us): corner decode of
+// 20 M rows of four fp32 3 244 : 827, of bf16 3 348 : 605; four in-place column edits of 20 M rows 1 322 : 794,
+// of bf16 1 402 : 403; eight tables of one column joined, 10 M rows 2 579 : 928, bf16 2 615 : 524, of three
+// columns, 4 M rows 3 081 : 1 349; box regression of 1 M x 21 boxes 45 300 : 1 686; 2 x 1 024 x 65 536 turned
+// over 2 883 : 1 395.
 std::vector<Box> Lowerer::boxesOf(int vid, const Shape& s, const Prog& whole) {
   const size_t len = whole.end - whole.begin;
   const int64_t numel = numel_of(s);

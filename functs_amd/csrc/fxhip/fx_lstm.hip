@@ -366,6 +366,9 @@ __global__ __launch_bounds__(FX_LSTM_BLOCK * UPW, HPT >= 32 ? 4 : 2) void fx_lst
 //            of row l % 4 and keeps, in registers for the whole sequence, its column's weights of the
 //            eight elements of a run that its half of the wave multiplies (cbsz = 3: a block of four
 //            lanes feeds the eight blocks of its half-wave), so a wave sums nothing but its two halves.
+//            (Three sizes of H = 512 need more than the 168 registers a lane of a workgroup of this size has
+//            and fetch some weights again every step: 6 registers' worth for L = 2 on two tiles, 12 and 52
+//            for L = 3 on one and two.  They are no slower than row by row all the same: figures below.)
 //   waves    up to four more finish the cells (gate x unit x row: 64 lanes a layer and tile), store
 //            them, clear the words of the step after next and bring x into LDS two steps ahead.  A wave
 //            that did both would queue its next loads up behind the acknowledgements of its stores.
@@ -689,9 +692,11 @@ static fx_lstm_kernel_t pick_rows(int hpt, int tiles) {
     default: return nullptr;
   }
 }
-// one row, or rows one after the other: the sizes for which four units' weights and a tile of rows are
+// one row, or rows one after the other: the sizes for which four units' weights and a tile of rows are far
 // more than the registers hold (1024 units; four layers of 512: 725 us with spilled weights against 630
-// for T = 32, B = 8)
+// for T = 32, B = 8).  Three layers of 512, T = 64, which spill less, row by row : one tile : two tiles, us:
+//   B = 2 281 : 279 : 482, 4 551 : 321 : 518, 8 1 090 : 336 : 602, 9 1 260 : - : 740, 16 2 174 : - : 866
+// two layers: B = 2 209 : 191 : 285, 8 804 : 228 : 346, 16 1 597 : - : 366.
 template <int L>
 static fx_lstm_kernel_t pick_serial(int hpt) {
   constexpr int U = FX_LSTM_UPW;

@@ -34,7 +34,7 @@
 #define FX_LSTM_CTL_WORDS (3u * FX_LSTM_LINE)
 #define FX_LSTM_TAG_WRAP 0x80000000u              // the base starts over (and the tags are cleared) beyond this
 
-// The second hand-over, of the kernels for one sequence and for groups of rows: an element is ONE
+// The second hand-over, of the kernel for groups of rows (one row at a time goes by tags): an element is ONE
 // 32-bit word, its value with all bits inverted, and 0 says that it has not been written yet (the
 // word that would be 0, a NaN of all ones, is written as another NaN).  Half the bytes of a value with
 // its tag, and what all workgroups read in a step is what a step waits for.

@@ -470,7 +470,9 @@ void fx_set_lstm_spin_limit(uint32_t polls); /* barrier polls before a wait is g
  * Outputs have fixed shapes; rows from n_out[task] on are zero.  out_index is the candidate's
  * position in the input (mode 0: row, mode 1: row * n_classes + class).
  * `counts` (valid rows per task) and `n_out` may be device memory or pinned host memory: a count
- * that a compaction wrote is read by the kernel, not by the host.
+ * that a compaction wrote is read by the kernel, not by the host, and a host may poll n_out in pinned
+ * memory to learn how many rows there are.  The rows themselves, and all results in device memory,
+ * are valid in stream order only, wherever they lie (rows in pinned memory arrive with the kernel's end).
  * Limits: at most FX_NMS_MAX_CANDIDATES candidates per task - `key_capacity` says how many the
  * launch is sized for (rounded up to a power of two >= 128); a task with more returns zeros, sets
  * its n_out to FX_NMS_OVERFLOW and reports FX_ASYNC_NMS_CAPACITY through fx_async_error - and
@@ -519,8 +521,7 @@ int fx_sort_nms(const fx_nms_desc* desc, void* stream);
  * rows, as three launches that spread the ranking and the overlap tests over the chip.  Its workspace is
  * scratch memory (256-byte aligned, nothing is expected in it or left in it); key_capacity is not read.
  * FX_E_LIMIT: more rows, more than 65535 tasks, or a ranking of 2^32 threads and more (tasks * rows / 64
- * rounded up * 4096).  n_out, like the other results, is valid in stream order: a host that polls it in
- * pinned memory may see it before the rows are there. */
+ * rounded up * 4096).  n_out and the rows: as with fx_sort_nms. */
 #define FX_NMS_PAIRS_MIN_ROWS 129
 #define FX_NMS_PAIRS_MAX_ROWS 4096 /* 64 chunks of 64 */
 size_t fx_nms_pairs_workspace_bytes(int n_tasks, uint32_t rows); /* 0: more rows than that, or none */
