@@ -18,7 +18,6 @@
 // value travels with the tag of the step that wrote it and readers poll for the tag they expect
 // (fx_lstm_sched.h), with bounded waits.
 #include <hip/hip_runtime.h>
-#include <hip/hip_ext.h>
 
 #include <map>
 #include <mutex>
@@ -730,6 +729,26 @@ static int lstm_forms(const FxLstmArgs& a, LstmLaunch (&f)[3]) {
 static std::mutex g_lstm_mu;
 static std::map<int, FxLstmGroups> g_lstm_groups;   // by device
 static std::set<int> g_lstm_captured;               // devices on which a launch has been captured
+// Workgroups of a form that a CU holds, and that it holds however their waves are dealt (fx_lstm_groups.h):
+// facts of the code and the device, asked for once.
+struct LstmFit { int per_cu, sure; };
+static std::map<std::pair<int, const void*>, LstmFit> g_lstm_fit;
+static hipError_t lstm_fit(int dev, const LstmLaunch& f, LstmFit* fit) {
+  const void* k = (const void*)f.kernel;
+  auto it = g_lstm_fit.find({dev, k});
+  if (it == g_lstm_fit.end()) {
+    LstmFit v{};
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&v.per_cu, k, f.threads, 0);
+    if (e != hipSuccess) return e;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v.sure, k, (int)fx_lstm_block((uint32_t)f.threads), 0) != hipSuccess) {
+      (void)hipGetLastError();
+      v.sure = 1;
+    }
+    it = g_lstm_fit.emplace(std::make_pair(dev, k), v).first;
+  }
+  *fit = it->second;
+  return hipSuccess;
+}
 
 // 0: launched; 1: shape outside what the kernel is built for; 2: the grid would not be resident
 // all at once (every workgroup waits for values that all the others write); otherwise a HIP error code + 100.
@@ -760,15 +779,11 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     // one tile of four rows a workgroup while that makes at most one workgroup for each CU, whose registers the
     // weights fill
     if (f[i].tiles == 1 && f[i].grid > cus) continue;
-    int per_cu = 0, sure = 0;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)f[i].kernel, f[i].threads, 0);
+    LstmFit fit;
+    e = lstm_fit(dev, f[i], &fit);
     if (e != hipSuccess) return 100 + (int)e;
-    if ((long)per_cu * cus < f[i].grid) continue;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&sure, (const void*)f[i].kernel, (int)fx_lstm_block((uint32_t)f[i].threads), 0) != hipSuccess) {
-      (void)hipGetLastError();
-      sure = 1;
-    }
-    const uint32_t want = fx_lstm_need((uint32_t)f[i].grid, (uint32_t)sure);
+    if ((long)fit.per_cu * cus < f[i].grid) continue;
+    const uint32_t want = fx_lstm_need((uint32_t)f[i].grid, (uint32_t)fit.sure);
     if (l && want >= need) continue;
     l = &f[i];
     need = want;
@@ -786,13 +801,30 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     e = hipLaunchKernel((const void*)l->kernel, grid, block, kargs, 0, stream);
     return e == hipSuccess ? 0 : 100 + (int)e;
   }
-  std::vector<void*> wait_for;
+  const bool legacy = stream == nullptr || stream == hipStreamLegacy;
+  const uint64_t id = legacy ? 0u : (uint64_t)(uintptr_t)stream;
   const uint64_t thread = stream == hipStreamPerThread ? (uint64_t)std::hash<std::thread::id>()(std::this_thread::get_id()) : 0u;
-  FxLstmGroups::Member& m = g_lstm_groups[dev].admit((uint64_t)(uintptr_t)stream, thread, need, device, &wait_for);
-  for (void* w : wait_for)
-    if (w && e == hipSuccess) e = hipStreamWaitEvent(stream, (hipEvent_t)w, 0);
-  if (e == hipSuccess && !m.done) e = hipEventCreateWithFlags((hipEvent_t*)&m.done, hipEventDisableTiming);
-  // (the event is the kernel's own completion: a record behind it costs a launch 1.3 - 2.5 us)
-  if (e == hipSuccess) e = hipExtLaunchKernel((const void*)l->kernel, grid, block, kargs, 0, stream, nullptr, (hipEvent_t)m.done, 0);
+  FxLstmGroups& groups = g_lstm_groups[dev];
+  auto record = [&](FxLstmGroups::Member& m) {
+    if (!m.done) m.done = groups.event_to_use();
+    if (!m.done) e = hipEventCreateWithFlags((hipEvent_t*)&m.done, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord((hipEvent_t)m.done, (hipStream_t)(uintptr_t)m.stream);
+    return e == hipSuccess;
+  };
+  auto wait_for = [&](void* event) {
+    e = hipStreamWaitEvent(stream, (hipEvent_t)event, 0);
+    return e == hipSuccess;
+  };
+  bool joins = false;
+  FxLstmGroups::Member& m = groups.admit(id, thread, need, device, legacy, &joins);
+  if (joins && !(groups.close_late(record) && groups.wait(id, thread, wait_for))) {
+    groups.withdraw();
+    (void)hipGetLastError();
+    return 100 + (int)e;
+  }
+  e = hipLaunchKernel((const void*)l->kernel, grid, block, kargs, 0, stream);
+  // (a record costs launches in a row 1.3 - 2.5 us each; a completion event given to the kernel itself costs them
+  // nothing, but some thousand such launches make every later call of the program, torch's as well, 5 us slower)
+  if (e == hipSuccess && !m.late) (void)record(m);
   return e == hipSuccess ? 0 : 100 + (int)e;
 }

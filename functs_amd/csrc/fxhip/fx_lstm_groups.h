@@ -16,6 +16,9 @@
 // stream's first launch of a group waits for the last launches of the group before (events, on the
 // device).  A program with one stream never waits; on two streams two stacks of 512 units, one sequence
 // each, run at the same time, and two that take the whole device run one after the other.
+// Events: the legacy default stream always exists and is never captured, so its event is recorded when a group
+// closes, from whichever thread that is, and launches on it cost nothing.  On any other stream an event is
+// recorded behind every launch: when it is wanted the stream may be gone, or capturing.
 #pragma once
 #include <stdint.h>
 
@@ -34,39 +37,62 @@ struct FxLstmGroups {
   struct Member {
     uint64_t stream, thread;   // (thread: for the streams that every thread has of its own)
     uint32_t need;             // the largest of the stream's launches in the group: one of them runs at a time
-    void* done;                // event behind the last of them
+    void* done;                // event behind the last of them (null: none was made yet)
+    bool late;                 // ... which is recorded when the group has closed (close_late), not behind every launch
   };
   std::vector<Member> now, before;
   std::vector<void*> spare;    // events to use again
 
-  // The member that a launch belongs to.  wait_for: events that its stream has to wait for ahead of it.
-  // `done` is null for a new member that got no spare event.
-  Member& admit(uint64_t stream, uint64_t thread, uint32_t need, uint32_t device, std::vector<void*>* wait_for) {
-    wait_for->clear();
-    auto same = [&](const Member& m) { return m.stream == stream && m.thread == thread; };
+  static bool same(const Member& m, uint64_t stream, uint64_t thread) { return m.stream == stream && m.thread == thread; }
+  // The member that a launch belongs to.  *joins: its stream has to wait for the others' events of the group
+  // before (wait) ahead of it, once close_late has recorded the late ones.
+  Member& admit(uint64_t stream, uint64_t thread, uint32_t need, uint32_t device, bool late, bool* joins) {
     uint64_t total = need;
     Member* mine = nullptr;
     for (Member& m : now) {
-      if (same(m)) mine = &m;
-      total += same(m) ? (m.need > need ? m.need - need : 0u) : m.need;
+      if (same(m, stream, thread)) mine = &m;
+      total += same(m, stream, thread) ? (m.need > need ? m.need - need : 0u) : m.need;
     }
     if (total > device && !(mine && now.size() == 1)) {   // (alone there is nobody to wait for)
-      for (const Member& m : before) spare.push_back(m.done);
+      for (const Member& m : before)
+        if (m.done) spare.push_back(m.done);
       before.swap(now);
       now.clear();
       mine = nullptr;
     }
+    *joins = !mine;
     if (mine) {
       if (mine->need < need) mine->need = need;
       return *mine;
     }
-    for (const Member& m : before)
-      if (!same(m)) wait_for->push_back(m.done);
-    now.push_back(Member{stream, thread, need, nullptr});
-    if (!spare.empty()) {
-      now.back().done = spare.back();
-      spare.pop_back();
-    }
+    now.push_back(Member{stream, thread, need, nullptr, late});
     return now.back();
+  }
+  void* event_to_use() {
+    if (spare.empty()) return nullptr;
+    void* e = spare.back();
+    spare.pop_back();
+    return e;
+  }
+  // record(Member&): gives the member its event and records it on its stream; false: it could not
+  template <class F>
+  bool close_late(F&& record) {
+    for (Member& m : before)
+      if (m.late) {
+        if (!record(m)) return false;
+        m.late = false;
+      }
+    return true;
+  }
+  template <class F>
+  bool wait(uint64_t stream, uint64_t thread, F&& wait_for) {
+    for (const Member& m : before)
+      if (m.done && !same(m, stream, thread) && !wait_for(m.done)) return false;   // (no event: its launch failed)
+    return true;
+  }
+  // the launch that joined last did not get as far as that
+  void withdraw() {
+    if (now.back().done) spare.push_back(now.back().done);
+    now.pop_back();
   }
 };

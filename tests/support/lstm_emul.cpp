@@ -261,7 +261,8 @@ extern "C" int fx_lstm_emul_give_up(const float* x, const float* wih, const floa
 }
 
 // A random program of launches on several streams (FxLstmGroups): every launch starts when its stream is
-// free and the events that it waits for have happened, and takes a random time.  Returns the most that
+// free and the events that it waits for have happened, and takes a random time; stream 0 is the one whose
+// events are recorded late.  Returns the most that
 // ran at one time, in the units of `needs`; *waits: launches that waited for another stream.
 extern "C" uint64_t fx_lstm_groups_emul(uint32_t seed, int streams, int launches, const uint32_t* needs, int n_needs, uint32_t device, int* waits) {
   std::mt19937 rng(seed);
@@ -275,18 +276,32 @@ extern "C" uint64_t fx_lstm_groups_emul(uint32_t seed, int streams, int launches
     const int s = (int)(rng() % (uint32_t)streams);
     const uint32_t need = needs[rng() % (uint32_t)n_needs];
     clock += (double)(rng() % 100) * 0.01;         // when the host issues it
-    std::vector<void*> wait_for;
-    FxLstmGroups::Member& m = groups.admit((uint64_t)s, 0u, need, device, &wait_for);
-    double start = std::max(clock, free_at[(size_t)s]);
-    for (void* w : wait_for) start = std::max(start, events[(size_t)(uintptr_t)w - 1]);
-    *waits += wait_for.empty() ? 0 : 1;
-    if (!m.done) {
-      events.push_back(0.0);
-      m.done = (void*)(uintptr_t)events.size();
+    auto record = [&](FxLstmGroups::Member& m) {   // behind all that its stream has been given so far
+      if (!m.done) m.done = groups.event_to_use();
+      if (!m.done) {
+        events.push_back(0.0);
+        m.done = (void*)(uintptr_t)events.size();
+      }
+      events[(size_t)(uintptr_t)m.done - 1] = free_at[(size_t)m.stream];
+      return true;
+    };
+    if (streams > 2 && i % 7 == 3) {               // a launch that fails ahead of its waits holds nobody up
+      bool joins = false;
+      groups.admit((uint64_t)streams, 0u, need, device, true, &joins);
+      groups.withdraw();
     }
+    bool joins = false, waited = false;
+    FxLstmGroups::Member& m = groups.admit((uint64_t)s, 0u, need, device, s == 0, &joins);
+    double start = std::max(clock, free_at[(size_t)s]);
+    auto wait_for = [&](void* w) {
+      start = std::max(start, events[(size_t)(uintptr_t)w - 1]);
+      return waited = true;
+    };
+    if (joins && !(groups.close_late(record) && groups.wait((uint64_t)s, 0u, wait_for))) return ~0ull;
+    *waits += waited ? 1 : 0;
     const double end = start + 0.01 + (double)(rng() % 300) * 0.01;
     free_at[(size_t)s] = end;
-    events[(size_t)(uintptr_t)m.done - 1] = end;
+    if (!m.late) record(m);
     edges.push_back({start, (int64_t)need});
     edges.push_back({end, -(int64_t)need});
   }

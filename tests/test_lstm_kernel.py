@@ -333,6 +333,25 @@ def test_launches_on_several_streams_take_turns_where_they_do_not_fit_together(s
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("order", [(0, 1), (1, 0), (0, 1, 2, 0, 2, 1)])
+def test_the_default_stream_takes_turns_with_others(order, short_waits):
+    """The default stream's event is recorded when a launch on another one has to wait for it."""
+    stacks = [_Stack(12, 512, 2, 8), _Stack(9, 512, 2, 8), _Stack(5, 512, 1, 16)]
+    streams = [torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    print("fx_lstm_stack on the default stream and others: %r" % (order,), flush=True)
+    for _ in range(5):
+        for i in order:
+            with torch.cuda.stream(streams[i]):
+                stacks[i].launch()
+                stacks[i].launch()
+    torch.cuda.synchronize()
+    assert short_waits.fx_async_error(1) == 0
+    for i in set(order):
+        stacks[i].check("stream %d" % i)
+
+
+@pytest.mark.gpu
 def test_a_captured_launch_leaves_room_for_another(short_waits):
     """A graph's launch is replayed whenever the program likes: it and every later launch keep to half of
     the device, so a replay and a call on another stream run side by side; one workspace serves both forms."""
