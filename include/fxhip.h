@@ -435,7 +435,8 @@ int fx_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* co
  * workgroups (H / 2 of 512 threads, or H / 4 of up to 768 for every four or eight rows) must be resident
  * together (FX_E_LIMIT if no form's are).  Launches on several streams of a device overlap when all their
  * workgroups find places together (two stacks of 512 units with one sequence each, for instance);
- * one that does not fit waits, in its stream, for the launches before it.  A captured launch cannot be
+ * one that does not fit waits, in its stream, for the launches before it (a launch on another stream than the
+ * legacy default one records an event behind it for that).  A captured launch cannot be
  * made to wait: it, and from then on every launch on that device, takes a form for half of the device
  * where there is one, so that ONE replay and the calls, or two replays, may run at the same time.
  * workspace: fx_lstm_stack_workspace_bytes() of device memory, 256-byte aligned, all zero when it
