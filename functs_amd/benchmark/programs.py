@@ -200,8 +200,8 @@ def yolov3_head_nms(pred_maps: List[Tensor], base_anchors: List[Tensor]):
 
 def attention_steps(x: Tensor, k: Tensor, v: Tensor, wq: Tensor, wk: Tensor, wv: Tensor, wo: Tensor, start_len: int):
     """Single-query attention over a growing key / value cache (attention.py:38-58): every step
-    writes one row of both caches at a position that the loop carries, the products stay library
-    GEMMs, scale and softmax fuse.  x [B, H, 1, D]; k, v [B, H, L, D], filled up to start_len;
+    writes one row of both caches at a position that the loop carries.  Built for tensors on a GPU the
+    loop is one kernel; otherwise the products stay library GEMMs, scale and softmax fuse.  x [B, H, 1, D]; k, v [B, H, L, D], filled up to start_len;
     wq, wk, wv, wo [H, D, D]."""
     k = k + 0.0
     v = v + 0.0

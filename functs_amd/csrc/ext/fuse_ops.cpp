@@ -1106,6 +1106,10 @@ bool FaitPipeline(std::shared_ptr<Graph> graph, std::vector<c10::TypePtr> input_
   HoistLoopInvariants(graph);   // parallelize_loops.cpp:130
   EliminateCommonSubexpression(graph);
   if (CollapseRecurrentLoops(graph)) EliminateDeadCode(graph);   // buffers the collapsed node no longer reads
+  if (CollapseAttentionLoops(graph)) {   // (only for these shapes on a GPU: others build their loop again)
+    EliminateDeadCode(graph);
+    specialized = true;
+  }
   CollapseAssignLoops(graph);
   trace("canonicalisation");
   ParallelizeLoops(graph);

@@ -165,6 +165,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("_jit_pass_fait_canonicalize_fusable_maps", CanonicalizeFusableMaps);
   m.def("_jit_pass_collapse_assign_loops", CollapseAssignLoops);
   m.def("_jit_pass_collapse_recurrent_loops", CollapseRecurrentLoops);
+  m.def("_jit_pass_collapse_attention_loops", CollapseAttentionLoops);
   m.def("_jit_pass_canonicalize_ops", CanonicalizeOps);
   m.def("_jit_pass_fold_static_type_queries", FoldStaticTypeQueries);
   m.def("_jit_pass_uniform_constants_to_fills", UniformConstantsToFills);

@@ -27,6 +27,11 @@ void CollapseAssignLoops(std::shared_ptr<torch::jit::Graph> graph);
 // persistent kernel; true if the graph changed.
 bool CollapseRecurrentLoops(std::shared_ptr<torch::jit::Graph> graph);
 
+// A decoding loop of single-query attention over a growing key / value cache
+// (functs/benchmark/simpleops/attention/attention.py:38-58) becomes one fx::attention_steps node when
+// the static shapes fit the kernel and the example lies on a GPU; true if the graph changed.
+bool CollapseAttentionLoops(std::shared_ptr<torch::jit::Graph> graph);
+
 // fait/passes/canonicalize.cpp:148-157 (on a functionalized graph): one spelling per meaning
 // (arange(end), max.other, new_zeros, pow with a constant exponent, empty slices, t(), to.dtype /
 // to.other, view).

@@ -49,6 +49,8 @@ FUNCTS_SYM(ParallelMap, "prim::ParallelMap")
 FUNCTS_SYM(ForallSelectRev, "fx::forall_select_rev")
 // the (time, layer) loop nest of a stacked LSTM collapsed to one node (recurrent.cpp)
 FUNCTS_SYM(LstmStack, "fx::lstm_stack")
+// a decoding loop of single-query attention collapsed to one node (attention.cpp)
+FUNCTS_SYM(AttentionSteps, "fx::attention_steps")
 // attributes of tssa::ParallelFunctor
 FUNCTS_SYM(parallel_degree, "attr::parallel_degree")
 FUNCTS_SYM(is_parallel_args, "attr::is_parallel_args")

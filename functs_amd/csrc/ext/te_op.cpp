@@ -14,6 +14,7 @@
 // pops the arguments, pushes one IValue per output; outputs are freshly
 // allocated, inputs are never written.
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
@@ -164,9 +165,12 @@ Node* functorFromMap(Node* mapNode, Node* group) {
   return f;
 }
 
-// fx::lstm_stack (the collapsed loop nest of a stacked LSTM, recurrent.cpp) as a region of one
-// node: its tensor and int operands are the arguments, its None operands stay constants.
-Node* functorFromLstmStack(Node* n) {
+// loops collapsed to one node with a kernel of its own (recurrent.cpp, attention.cpp)
+bool isLoopKernel(const Node* n) { return n->kind() == sym::LstmStack() || n->kind() == sym::AttentionSteps(); }
+
+// such a node as a region of one node: its tensor and int operands are the arguments, its constant
+// operands (None among them) stay constants.
+Node* functorFromLoopKernel(Node* n) {
   Graph* g = n->owningGraph();
   Node* f = g->createWithSubgraph(sym::ParallelFunctor());
   auto sub = f->g(c10::attr::Subgraph);
@@ -184,7 +188,7 @@ Node* functorFromLstmStack(Node* n) {
     types.push_back(in->type());
     operands.push_back(sub->addInput()->copyMetadata(in));
   }
-  Node* k = sub->create(sym::LstmStack(), operands, n->outputs().size());
+  Node* k = sub->create(n->kind(), operands, n->outputs().size());
   sub->appendNode(k);
   for (size_t i = 0; i < n->outputs().size(); ++i) {
     k->output(i)->copyMetadata(n->output(i));
@@ -253,8 +257,8 @@ void toFunctorIn(Block* b) {
   for (auto it = b->nodes().begin(); it != b->nodes().end();) {
     Node* n = *it;
     ++it;
-    if (n->kind() == c10::prim::FusionGroup || n->kind() == sym::LstmStack()) {
-      Node* f = n->kind() == sym::LstmStack() ? functorFromLstmStack(n) : functorFromGroup(n);
+    if (n->kind() == c10::prim::FusionGroup || isLoopKernel(n)) {
+      Node* f = isLoopKernel(n) ? functorFromLoopKernel(n) : functorFromGroup(n);
       f->insertBefore(n);
       for (size_t k = 0; k < n->outputs().size(); ++k) n->output(k)->replaceAllUsesWith(f->output(k));
       n->destroy();
@@ -1270,12 +1274,83 @@ void runLstmStack(Stack& stack) {
   push(stack, std::move(sc));
 }
 
-// the region of a functor made by functorFromLstmStack: one fx::lstm_stack node over the arguments
-const Node* loneLstmStack(const Graph& sub) {
+// --- fx::attention_steps --------------------------------------------------------
+// fx::attention_steps(x, k, v, wq, wk, wv, wo, start, stop, scale, k_add?, v_add?) -> (k, v, x) is the loop
+//   k = k + k_add; v = v + v_add
+//   for row in range(start, stop):
+//     k[:, :, row] = x @ wk; v[:, :, row] = x @ wv
+//     x = softmax((k @ (x @ wq)^T)^T * scale) @ v @ wo
+// in functional form: the results are new tensors.  Operands that the kernel is not made for (a
+// gradient wanted, autocast, other types or sizes than the graph was built for) run it as ATen's operators.
+void runAttentionSteps(Stack& stack) {
+  auto in = last(stack, 12);
+  at::Tensor t[7];
+  for (size_t i = 0; i < 7; ++i) {
+    TORCH_CHECK(in[i].isTensor(), "fx::attention_steps: operand ", i, " must be a tensor");
+    t[i] = in[i].toTensor();
+    TORCH_CHECK(t[i].is_cuda(), "fx::attention_steps runs on the GPU only; operand ", i, " is a ", t[i].device(), " tensor");
+  }
+  const int64_t start = in[7].toInt(), stop = in[8].toInt();
+  const double scale = in[9].toDouble();
+  const at::Tensor &x0 = t[0], &k0 = t[1];
+  bool kernel = x0.dim() == 4 && x0.size(2) == 1 && k0.dim() == 4 && !at::autocast::is_autocast_enabled(at::kCUDA);
+  if (kernel) {
+    const int64_t B = x0.size(0), H = x0.size(1), D = x0.size(3), rows = k0.size(2);
+    const std::vector<int64_t> cache{B, H, rows, D}, weight{H, D, D};
+    for (size_t i = 0; i < 7; ++i) {
+      kernel = kernel && t[i].scalar_type() == at::kFloat && t[i].device() == x0.device() && !t[i].is_neg() && !(at::GradMode::is_enabled() && t[i].requires_grad());
+      if (i > 0) kernel = kernel && t[i].sizes() == at::IntArrayRef(i < 3 ? cache : weight);
+    }
+    kernel = kernel && D <= INT32_MAX && rows <= INT32_MAX && fx_attention_steps_fits((int)D, (int)rows) && B * H <= INT32_MAX / 512;
+    if (stop > start)   // (as select reports it)
+      for (int64_t row : {start, stop - 1})
+        TORCH_CHECK_INDEX(row >= -rows && row < rows, "select(): index ", row, " out of range for tensor of size ", k0.sizes(), " at dimension 2");
+  }
+  at::Tensor k, v, x;
+  if (kernel) {
+    c10::DeviceGuard guard(x0.device());
+    for (at::Tensor& a : t) {   // (the kernel reads 16 bytes at a time)
+      a = a.contiguous();
+      if (((uintptr_t)a.data_ptr() & 15u) != 0) a = a.clone();
+    }
+    const auto opts = x0.options();
+    k = at::empty(k0.sizes(), opts);
+    v = at::empty(k0.sizes(), opts);
+    x = at::empty(x0.sizes(), opts);
+    checkAsyncError();
+    auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x0.device().index());
+    auto number = [&](size_t i) { return in[i].isNone() ? -0.0f : (float)in[i].toDouble(); };   // (-0 changes no number)
+    FX_OK_OR_THROW(fx_attention_steps(x0.data_ptr<float>(), t[1].data_ptr<float>(), t[2].data_ptr<float>(), t[3].data_ptr<float>(),
+                                      t[4].data_ptr<float>(), t[5].data_ptr<float>(), t[6].data_ptr<float>(), k.data_ptr<float>(),
+                                      v.data_ptr<float>(), x.data_ptr<float>(), (int)x0.size(0), (int)x0.size(1), (int)x0.size(3),
+                                      (int)k0.size(2), (int)start, (int)std::max<int64_t>(stop - start, 0), (float)scale, number(10), number(11),
+                                      (void*)stream.stream()));
+  } else {
+    k = in[10].isNone() ? k0.clone() : at::add(k0, in[10].toScalar());
+    v = in[11].isNone() ? t[2].clone() : at::add(t[2], in[11].toScalar());
+    x = start < stop ? x0 : x0.clone();
+    for (int64_t row = start; row < stop; ++row) {
+      const at::Tensor q = at::matmul(x, t[3]);
+      const std::vector<int64_t> sizes{x.size(0), x.size(1), x.size(-1)};
+      k = at::select_scatter(k, at::matmul(x, t[4]).reshape(sizes).to(k.scalar_type()), 2, row);
+      v = at::select_scatter(v, at::matmul(x, t[5]).reshape(sizes).to(v.scalar_type()), 2, row);
+      at::Tensor p = at::matmul(k, q.transpose(2, 3)).transpose(2, 3);
+      p = at::softmax(at::mul(p, scale), 3);
+      x = at::matmul(at::matmul(p, v), t[6]);
+    }
+  }
+  drop(stack, 12);
+  push(stack, std::move(k));
+  push(stack, std::move(v));
+  push(stack, std::move(x));
+}
+
+// the region of a functor made by functorFromLoopKernel: one node over the arguments
+const Node* loneLoopKernel(const Graph& sub) {
   const Node* found = nullptr;
   for (const Node* n : sub.nodes()) {
     if (n->kind() == c10::prim::Constant) continue;
-    if (n->kind() != sym::LstmStack() || found) return nullptr;
+    if (!isLoopKernel(n) || found) return nullptr;
     found = n;
   }
   return found;
@@ -1283,7 +1358,7 @@ const Node* loneLstmStack(const Graph& sub) {
 
 Operation createParallelFunctor(const Node* node) {
   auto sub = node->g(c10::attr::Subgraph);
-  if (const Node* k = loneLstmStack(*sub)) {
+  if (const Node* k = loneLoopKernel(*sub)) {
     // operand i of the node: argument number (position among the functor's inputs) or a constant
     struct Operand { int arg; c10::IValue constant; };
     std::vector<Operand> operands;
@@ -1294,16 +1369,17 @@ Operation createParallelFunctor(const Node* node) {
       }
       size_t pos = 0;
       while (pos < sub->inputs().size() && sub->inputs()[pos] != v) ++pos;
-      TORCH_CHECK(pos >= 1 && pos < sub->inputs().size(), "ParallelFunctor: fx::lstm_stack operand is not an argument");
+      TORCH_CHECK(pos >= 1 && pos < sub->inputs().size(), "ParallelFunctor: an operand of ", k->kind().toQualString(), " is not an argument");
       operands.push_back({(int)pos - 1, c10::IValue()});
     }
     const size_t n_args = sub->inputs().size() - 1;
-    return [operands, n_args](Stack& stack) {
+    void (*const run)(Stack&) = k->kind() == sym::LstmStack() ? runLstmStack : runAttentionSteps;
+    return [operands, n_args, run](Stack& stack) {
       std::vector<c10::IValue> args;
       for (const c10::IValue& v : last(stack, n_args)) args.push_back(v);
       drop(stack, n_args);
       for (const Operand& o : operands) stack.push_back(o.arg < 0 ? o.constant : args[(size_t)o.arg]);
-      runLstmStack(stack);
+      run(stack);
     };
   }
   auto runner = std::make_shared<RegionRunner>(node);
@@ -1317,6 +1393,9 @@ RegisterOperators registerFunctor({
     Operator("fx::lstm_stack(Tensor x, Tensor wih, Tensor whh, Tensor bih, Tensor bhh, Tensor? out, Tensor? state_h, "
              "Tensor? state_c, int T, int L) -> (Tensor, Tensor, Tensor)",
              [](Stack& stack) { runLstmStack(stack); }, c10::AliasAnalysisKind::PURE_FUNCTION),
+    Operator("fx::attention_steps(Tensor x, Tensor k, Tensor v, Tensor wq, Tensor wk, Tensor wv, Tensor wo, int start, int stop, "
+             "float scale, float? k_add, float? v_add) -> (Tensor, Tensor, Tensor)",
+             [](Stack& stack) { runAttentionSteps(stack); }, c10::AliasAnalysisKind::PURE_FUNCTION),
 });
 
 
@@ -1393,7 +1472,7 @@ bool trySinkProducer(Node* f2, Node* f1) {
   const auto par2 = f2->is(sym::is_parallel_args());
   const size_t first2 = f2->i(sym::parallel_degree()) < 0 ? 1 : 0;
   for (Node* n : f1->g(c10::attr::Subgraph)->nodes())
-    if (n->kind() == sym::LstmStack() || n->kind() == sym::ForallSelectRev()) return false;
+    if (isLoopKernel(n) || n->kind() == sym::ForallSelectRev()) return false;
   // F1's results may only feed F2 and size queries with a constant dimension
   for (Value* o : f1->outputs())
     for (const Use& u : o->uses()) {
@@ -1663,7 +1742,7 @@ bool inferNode(Node* n) {
 bool inferFunctor(Node* n) {
   if (n->i(sym::parallel_degree()) < 0) return false;
   for (Node* k : n->g(c10::attr::Subgraph)->nodes())
-    if (k->kind() == sym::LstmStack()) return false;
+    if (isLoopKernel(k)) return false;
   const bool is_map = n->i(sym::is_parallel_map()) != 0;
   const auto par = n->is(sym::is_parallel_args());
   auto types = n->tys(sym::input_refine_types());
@@ -1736,10 +1815,13 @@ void planIn(Block* b, std::vector<std::string>* report) {
     if (n->kind() != sym::ParallelFunctor()) continue;
     std::ostringstream line;
     const auto sub = n->g(c10::attr::Subgraph);
-    bool special = false;
+    const Node* special = nullptr;
     for (Node* k : sub->nodes())
-      if (k->kind() == sym::LstmStack()) special = true;
-    if (special) { report->push_back("lstm_stack functor: a kernel of its own, nothing to plan"); continue; }
+      if (isLoopKernel(k)) special = k;
+    if (special) {
+      report->push_back(std::string(special->kind().toUnqualString()) + " functor: a kernel of its own, nothing to plan");
+      continue;
+    }
     const auto types = n->tys(sym::input_refine_types());
     const auto par = n->is(sym::is_parallel_args());
     const int64_t degree = n->i(sym::parallel_degree());

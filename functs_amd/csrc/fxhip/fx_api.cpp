@@ -48,6 +48,7 @@ hipError_t fx_launch_classmap_head(const FxCmapLaunch& hl, const FxDyn* dyn, boo
 hipError_t fx_cmap_resident(uint32_t lds_bytes, uint32_t* wide, uint32_t* narrow);
 uint32_t fx_cmap_lds_bytes(const FxCmapLaunch& hl);
 uint32_t fx_cmap_chunk_rows();
+#include "fx_attn.h"
 #include "fx_lstm_sched.h"
 int fx_launch_lstm_stack(const FxLstmArgs& a, int L, uint32_t* words_ctl, uint64_t* words_hbuf, hipStream_t stream);
 int fx_launch_sort_nms(const fx_nms_desc& d, uint32_t key_cap, void* workspace, uint32_t* err_host, hipStream_t stream);
@@ -1604,6 +1605,33 @@ int fx_lstm_stack(const float* x, const float* wih, const float* whh, const floa
 }
 void fx_set_totals_spin_us(uint32_t us) { g_totals_spin_us.store(us, std::memory_order_relaxed); }
 void fx_set_lstm_spin_limit(uint32_t polls) { g_lstm_spin.store(polls, std::memory_order_relaxed); }
+
+// ---- attention over a growing cache (fx_attn.hip) ----
+int fx_attention_steps_fits(int depth, int rows) {
+  return depth == FX_ATTN_DEPTH && rows >= 1 && rows <= FX_ATTN_MAX_ROWS ? 1 : 0;
+}
+
+int fx_attention_steps(const float* x, const float* k, const float* v, const float* wq, const float* wk, const float* wv,
+                       const float* wo, float* k_out, float* v_out, float* x_out, int batch, int heads, int depth, int rows,
+                       int start, int steps, float scale, float k_add, float v_add, void* stream) {
+  if (batch < 0 || heads < 0 || steps < 0) return fail(FX_E_INVALID, "fx_attention_steps: negative size");
+  if (!fx_attention_steps_fits(depth, rows))
+    return fail(FX_E_UNSUPPORTED, "fx_attention_steps: depth must be " + std::to_string(FX_ATTN_DEPTH) + " and rows 1.." + std::to_string(FX_ATTN_MAX_ROWS) +
+                                      " (got " + std::to_string(depth) + ", " + std::to_string(rows) + ")");
+  if (steps > 0 && (start < -rows || (int64_t)start + steps > rows))
+    return fail(FX_E_INVALID, "fx_attention_steps: rows " + std::to_string(start) + " to " + std::to_string((int64_t)start + steps - 1) +
+                                  " are out of range of a cache of " + std::to_string(rows));
+  if (batch == 0 || heads == 0) return FX_OK;
+  if ((int64_t)batch * heads > INT32_MAX / 512) return fail(FX_E_LIMIT, "fx_attention_steps: more heads than a launch holds");
+  for (const void* p : {(const void*)x, (const void*)k, (const void*)v, (const void*)wq, (const void*)wk, (const void*)wv, (const void*)wo,
+                        (const void*)k_out, (const void*)v_out, (const void*)x_out})
+    if (!p || ((uintptr_t)p & 15u) != 0) return fail(FX_E_INVALID, "fx_attention_steps: null or not 16-byte aligned argument");
+  const FxAttnArgs a{x, k, v, wq, wk, wv, wo, k_out, v_out, x_out, heads, rows, start, steps, scale, k_add, v_add};
+  HIP_OK(fx_launch_attention_steps(a, batch * heads, (hipStream_t)stream));
+  g_launches.fetch_add(1, std::memory_order_relaxed);
+  g_spec_launches.fetch_add(1, std::memory_order_relaxed);
+  return FX_OK;
+}
 
 // ---- detection tail (fx_nms.hip) ----
 

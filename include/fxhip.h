@@ -455,6 +455,25 @@ int fx_lstm_stack(const float* x, const float* wih, const float* whh, const floa
                   int layers, void* workspace, size_t workspace_bytes, void* stream);
 void fx_set_lstm_spin_limit(uint32_t polls); /* barrier polls before a wait is given up (default 1000000; tests) */
 
+/* ---- single-query attention over a growing cache as one launch ----
+ * The decoding loop of functs/benchmark/simpleops/attention/attention.py:38-58
+ *   k_out = k + k_add; v_out = v + v_add          (pass -0.0f to take the caches as they are)
+ *   for s in [0, steps): row = start + s          (a row below zero counts from the end)
+ *     q = x @ wq; k_out[row] = x @ wk; v_out[row] = x @ wv
+ *     x = softmax(scale * (k_out @ q)) @ v_out @ wo      (over all rows of the cache)
+ * which the reference runs on the host, six library products and their glue a step (the loop
+ * carries x, the caches and the position: fait/passes/parallelize_loops.cpp:17), as ONE kernel: a
+ * workgroup per (batch row, head) keeps the head's weights and caches in registers through all steps.
+ * Contiguous fp32, 16-byte aligned: x, x_out [batch, heads, depth]; k, v, k_out, v_out [batch, heads,
+ * rows, depth]; wq, wk, wv, wo [heads, depth, depth].  The results may not overlap the operands.
+ * depth is 64 and rows 1..512 (FX_E_UNSUPPORTED otherwise; fx_attention_steps_fits tells, for a
+ * compiler pass that decides whether to emit the call); every row written must lie in [-rows, rows)
+ * (FX_E_INVALID).  steps may be 0: the caches and x are copied. */
+int fx_attention_steps_fits(int depth, int rows);
+int fx_attention_steps(const float* x, const float* k, const float* v, const float* wq, const float* wk, const float* wv,
+                       const float* wo, float* k_out, float* v_out, float* x_out, int batch, int heads, int depth, int rows,
+                       int start, int steps, float scale, float k_add, float v_add, void* stream);
+
 /* ---- detection tail: score threshold + sort + class-aware greedy NMS + top-k, one launch ----
  * The step behind row compaction in the reference's detection programs, which it runs as ATen /
  * torchvision kernels with host synchronisations in between:
