@@ -3,8 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#define FX_ATTN_DEPTH 64      // elements of a head: 64 x 64 weights are 32 registers a lane of eight waves
-#define FX_ATTN_MAX_ROWS 512  // rows of a cache: with it, both caches of a head are 128 registers more
+#define FX_ATTN_DEPTH 64      // elements of a head: its four 64 x 64 weights are 64 registers a lane of four waves
+#define FX_ATTN_MAX_ROWS 512  // rows of a cache: both caches of a head are then 128 registers a lane of eight waves
 
 // contiguous fp32 tensors, 16-byte aligned; see fx_attention_steps in include/fxhip.h
 struct FxAttnArgs {
