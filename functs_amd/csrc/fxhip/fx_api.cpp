@@ -50,7 +50,7 @@ uint32_t fx_cmap_lds_bytes(const FxCmapLaunch& hl);
 uint32_t fx_cmap_chunk_rows();
 #include "fx_attn.h"
 #include "fx_lstm_sched.h"
-int fx_launch_lstm_stack(const FxLstmArgs& a, int L, uint32_t* words_ctl, uint64_t* words_hbuf, hipStream_t stream);
+int fx_launch_lstm_stack(const FxLstmArgs& a, int L, uint32_t* words_ctl, uint32_t* die_ctl, hipStream_t stream);
 int fx_launch_sort_nms(const fx_nms_desc& d, uint32_t key_cap, void* workspace, uint32_t* err_host, hipStream_t stream);
 size_t fx_nms_pairs_ws_bytes(int n_tasks, uint32_t rows);
 int fx_launch_nms_pairs(const fx_nms_desc& d, hipStream_t stream);
@@ -1560,14 +1560,15 @@ int fx_lstm_stack_fits(int batch, int hidden, int layers) {
   if (hidden == 1024 && layers * (hidden / 32) > 64) return 0;
   return 1;
 }
-// A workspace is two areas, one for each hand-over (tags, words): which form a launch takes depends on what
-// else may run, and a form finds only what its own launches left.
+// A workspace is an area for each hand-over (tags, words, a sequence on one die): which form a launch takes
+// depends on what else may run, and a form finds only what its own launches left.
 static size_t lstm_area_bytes(int batch, int hidden, int layers) {
   return ((size_t)FX_LSTM_CTL_WORDS * 4 + (size_t)2 * layers * batch * hidden * 8 + 255) & ~(size_t)255;
 }
 size_t fx_lstm_stack_workspace_bytes(int batch, int hidden, int layers) {
   if (batch < 1 || hidden < 1 || layers < 1) return 0;
-  return 2 * lstm_area_bytes(batch, hidden, layers);
+  const size_t die = fx_lstm_die_fits(batch, hidden, layers) ? (size_t)FX_LSTM_CTL_WORDS * 4 + (size_t)fx_lstm_die_area(batch, hidden, layers).words * 8 : 0;
+  return 2 * lstm_area_bytes(batch, hidden, layers) + die;
 }
 
 int fx_lstm_stack(const float* x, const float* wih, const float* whh, const float* bih, const float* bhh, const float* h0,
@@ -1590,10 +1591,11 @@ int fx_lstm_stack(const float* x, const float* wih, const float* whh, const floa
   a.err_host = err_word(true);
   a.T = seq_len; a.B = batch; a.H = hidden;
   a.spin_limit = g_lstm_spin.load(std::memory_order_relaxed);
-  a.ctl_other = nullptr;   // (the launcher's choice)
+  a.ctl_other = a.ctl_third = nullptr;   // (the launcher's choice)
   FX_TRY
   uint32_t* words_ctl = (uint32_t*)((char*)workspace + lstm_area_bytes(batch, hidden, layers));
-  const int rc = fx_launch_lstm_stack(a, layers, words_ctl, (uint64_t*)(words_ctl + FX_LSTM_CTL_WORDS), (hipStream_t)stream_);
+  uint32_t* die_ctl = fx_lstm_die_fits(batch, hidden, layers) ? (uint32_t*)((char*)workspace + 2 * lstm_area_bytes(batch, hidden, layers)) : nullptr;
+  const int rc = fx_launch_lstm_stack(a, layers, words_ctl, die_ctl, (hipStream_t)stream_);
   if (rc == 1) return fail(FX_E_UNSUPPORTED, "fx_lstm_stack: no kernel for these sizes");
   if (rc == 2)
     return fail(FX_E_LIMIT, "fx_lstm_stack: the workgroups for hidden " + std::to_string(hidden) + " and batch " + std::to_string(batch) + " would not be resident together on this device");

@@ -134,7 +134,7 @@ __global__ __launch_bounds__(FX_LSTM_BLOCK * UPW, HPT >= 32 ? 4 : 2) void fx_lst
   const int wg = (n_wg % 8 == 0) ? ((int)blockIdx.x % 8) * (n_wg / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
   const int u0 = wg * UPW;
   // a workspace that still carries a given-up wait is refused (below, behind the first barrier)
-  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) ? 1u : 0u;
+  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) || fx_lstm_refused<DevAtomics>(a.ctl_third) ? 1u : 0u;
   // tags of this launch start behind those of every launch before it
   const uint32_t base = DevAtomics::load(a.ctl + FX_LSTM_W_BASE);
 
@@ -393,6 +393,23 @@ __device__ __forceinline__ void fx_stores_acknowledged() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
+// the die that the wave runs on (hardware register XCC_ID, four bits)
+__device__ __forceinline__ uint32_t fx_die_of_wave() { return (uint32_t)__builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)); }
+// N consecutive floats of any alignment that floats have
+template <int N>
+__device__ __forceinline__ void fx_die_load(const float* p, float (&v)[N]) {
+  typedef float chunk __attribute__((ext_vector_type(N < 4 ? N : 4), aligned(4)));
+#pragma unroll
+  for (int i = 0; i < N; i += 4) {
+    if constexpr (N == 1) {
+      v[0] = *p;
+    } else {
+      const chunk c = *(const chunk*)(p + i);
+#pragma unroll
+      for (int k = 0; k < (N < 4 ? N : 4); ++k) v[i + k] = c[k];
+    }
+  }
+}
 typedef float fx_f32x4 __attribute__((ext_vector_type(4)));
 template <int Q> struct fx_const { static constexpr int value = Q; };
 template <class F>
@@ -430,7 +447,7 @@ __global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_row
   const int wg = (n_wg % 8 == 0) ? (gi % 8) * (n_wg / 8) + gi / 8 : gi;
   const int u0 = wg * 4;
   const int b0 = group * 4 * MT, nb = min(4 * MT, B - b0);
-  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) ? 1u : 0u;
+  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) || fx_lstm_refused<DevAtomics>(a.ctl_third) ? 1u : 0u;
   const uint32_t base = DevAtomics::load(a.ctl + FX_LSTM_W_BASE);
   const int n_steps = fx_lstm_steps(T, L);
   const uint32_t BH = (uint32_t)(B * HH);               // elements of one vector of all rows
@@ -678,6 +695,383 @@ __global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_row
   if (cw == 0 && lane == 0) fx_lstm_leave_slots<DevAtomics>(a.ctl, gridDim.x, base, (uint32_t)n_steps);
 }
 
+// ---- a sequence on one die ---------------------------------------------------------------------
+// What the kernels above spend most of a step on is the hand-over: a value goes to the memory side of the
+// caches and comes back from there, 0.45 us one way at its quickest and 0.9 to 1.6 with every workgroup of the
+// chip reading.  The compute units of one die share a cache: a store that stays in it is seen by a load of
+// another unit after 0.2 us.  A die's registers hold the weights of one layer of 512 units, or of all layers
+// of fewer, so here a sequence's layers (a stage of them, fx_lstm_sched.h) run on the 32 units of a die and
+// sequences on dies of their own; only h between stages crosses, and nothing waits for that.
+//   columns  a workgroup has 2 E of the 64 E hidden units, 8 E gate columns a layer.
+//   depth    dealt to eight waves in runs of 8 E.  Lane (kl, cl) = (lane >> 3, lane & 7) multiplies E elements
+//            by E columns: gate cl >> 1 of E units.  A lane fetches ONE element and has the others of its
+//            group of E lanes by lane-crossing moves; sums are taken over kl only.
+//   shadow   the products with the layer's input (x, or h of the layer below, two steps old) come first: they
+//            fill the time in which the layer's own h travels.
+//   cells    one or two more waves: a lane a gate column, four lanes a cell; they bring the stage's input into
+//            LDS two steps ahead.
+// Where a workgroup runs is the hardware's choice (dies in turn).  Loads are device-scope either way; whether a
+// value may be stored to the die's cache only, the workgroups of a stage find out while they load their
+// weights: each publishes its die, and unless all agree they store to the memory side.
+// us a launch, T = 64, this : the forms above: 512 units, one sequence, one to three layers 80 : 110, 92 : 119, 98 : 188;
+// two layers, four sequences 98 : 219; 256 units, four layers, four sequences 89 : 207; 128, three, eight 71 : 125;
+// 64, one, one 47 : 105.  T = 100, 256 units, three layers, eight sequences 131 : 269.  T = 8: 27 : 28 (512, two
+// layers), 12 : 16 (64, one), 20 : 20 (64, three, eight sequences).  A step of two layers of 512 units is 1.1 us:
+// 0.3 from the barrier to the cells' stores, 0.3 until they are seen, 0.35 products, 0.1 sums (on the SIMD that also
+// finishes cells, the others wait for it); of 64 units 0.65.
+template <int CTRL>
+__device__ __forceinline__ float fx_dpp(float v) { return dpp_get<CTRL>(v); }
+// element e of the lane's group of E lanes; E = 8: the upper four in mirrored order (fx_die_element)
+template <int E>
+__device__ __forceinline__ void fx_die_spread(float h, float (&v)[E]) {
+  if constexpr (E == 1) v[0] = h;
+  if constexpr (E == 2) {
+    v[0] = fx_dpp<0xA0>(h);   // quad_perm [0, 0, 2, 2]
+    v[1] = fx_dpp<0xF5>(h);   // quad_perm [1, 1, 3, 3]
+  }
+  if constexpr (E >= 4) {
+    v[0] = quad_lane<0>(h); v[1] = quad_lane<1>(h); v[2] = quad_lane<2>(h); v[3] = quad_lane<3>(h);
+  }
+  if constexpr (E == 8) {
+    const float m = fx_dpp<0x141>(h);   // row_half_mirror: the other four of the group
+    v[4] = quad_lane<0>(m); v[5] = quad_lane<1>(m); v[6] = quad_lane<2>(m); v[7] = quad_lane<3>(m);
+  }
+}
+template <int E>
+__device__ __forceinline__ int fx_die_element(int cl, int e) {   // which element of the group spread's v[e] is
+  return E < 8 ? e : e < 4 ? 4 * (cl >> 2) + e : 11 - 4 * (cl >> 2) - e;
+}
+// V values a lane, summed over the lanes that differ in bits 3, 4 and 5 of their number; where the count is even
+// a stage keeps half of the values in each lane.  Left: fx_die_left(V) values from *first on.
+constexpr int fx_die_left(int v) {
+  for (int i = 0; i < 3; ++i) v = v % 2 == 0 ? v / 2 : v;
+  return v;
+}
+template <int V, int BIT>
+__device__ __forceinline__ void fx_die_sum(float (&p)[V], int lane, int* first, float* out) {
+  constexpr bool halve = V % 2 == 0;
+  constexpr int N = halve ? V / 2 : V;
+  float q[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float a = p[i], b = halve ? p[(i + N) % V] : p[i];
+    if constexpr (BIT == 3) {
+      const bool up = halve && (lane & 8) != 0;
+      const float keep = up ? b : a, send = up ? a : b;
+      q[i] = keep + fx_dpp<0x128>(send);   // row_ror:8: from lane l ^ 8
+    } else {
+      const fx_u32x2v t = BIT == 5 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+                                   : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+      q[i] = __uint_as_float(t.x) + __uint_as_float(t.y);
+    }
+  }
+  if (halve) *first += ((lane >> BIT) & 1) * N;
+  if constexpr (BIT > 3) {
+    fx_die_sum<N, BIT - 1>(q, lane, first, out);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = q[i];
+  }
+}
+
+// The activation of a gate: tanh for the cell gate, sigmoid for the others, by way of one exponential
+// (fx_sigmoid's; lanes of both kinds are in one wave, which would go through two).
+__device__ __forceinline__ float fx_die_gate(float x, bool cell_gate) {
+  const float l2e_hi = 1.44269502e+00f, l2e_lo = 1.92596299e-08f, ln2 = 6.93147182e-01f;
+  const float ax = fabsf(x), arg = cell_gate ? 2.0f * ax : -x;
+  const float th = arg * l2e_hi;
+  const float tl = __builtin_fmaf(arg, l2e_hi, -th) + arg * l2e_lo;
+  float e = __builtin_amdgcn_exp2f(th);
+  e = __builtin_fmaf(e, tl * ln2, e);
+  float r = __builtin_amdgcn_rcpf(1.0f + e);
+  r = (th > 128.0f) ? 0.0f : r;
+  r = (th < -150.0f) ? 1.0f : r;
+  const float z = x * x;   // as fx_tanh: a polynomial where 1 - 2 r would cancel
+  float p = -5.70498872745e-3f;
+  p = __builtin_fmaf(p, z, 2.06390887954e-2f);
+  p = __builtin_fmaf(p, z, -5.37397155531e-2f);
+  p = __builtin_fmaf(p, z, 1.33314422036e-1f);
+  p = __builtin_fmaf(p, z, -3.33332819422e-1f);
+  const float small = __builtin_fmaf(p * z, x, x);
+  const float t = ax < 0.625f ? small : copysignf(1.0f - 2.0f * r, x);
+  return cell_gate ? t : r;
+}
+
+template <int E, int NL>
+struct FxLstmDie {
+  static constexpr int HH = 64 * E, C = 8 * E, U = 2 * E;   // units; gate columns a layer and units of a workgroup
+  static constexpr int NW = 8, CW = (NL * C + 63) / 64;     // waves that multiply, waves that finish cells
+  static constexpr int threads = (NW + CW) * 64;
+  // Units of 64 clocks that a wave sleeps ahead of its first look: values are there some 1 100 clocks behind the
+  // barrier, and looks slow down the stores that they wait for.  Longer products are long enough.  (One layer of 64
+  // units, T = 64: 0 to 4 units 52 us, 6 48, 8 46.7, 9 47; 128 units: 2 to 9 within 4 %.)
+  static constexpr int sleep = E == 1 ? 9 - NL : E == 2 ? 2 : E * NL == 4 ? 1 : 0;
+};
+template <int E, int NL>
+__global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kernel(const FxLstmArgs a, int L) {
+  using K = FxLstmDie<E, NL>;
+  constexpr int HH = K::HH, C = K::C, NW = K::NW, NC = NL * C;
+  __shared__ float s_part[2][NW][NC];   // the waves' sums, by parity of the step: [layer][unit][gate]
+  __shared__ __align__(16) float s_in[3][HH];   // the stage's input of a step and of the two behind it
+  __shared__ uint32_t s_abort;
+  const int B = a.B, T = a.T;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int slot = (int)blockIdx.x % FX_LSTM_DIES, gi = (int)blockIdx.x / FX_LSTM_DIES;
+  const int stages = L / NL, b = slot / stages, stage = slot % stages, j0 = stage * NL;
+  const int u0 = gi * K::U;
+  const int n_steps = fx_lstm_stage_steps(T, NL);
+  const uint32_t advance = (uint32_t)n_steps + 1u;   // tags that a launch uses
+  const FxLstmDieArea area = fx_lstm_die_area(B, HH, L);
+  const uint32_t parity = (uint32_t)(L * B * HH);   // from one half of the h buffer to the other
+  const uint32_t base = DevAtomics::load(a.ctl + FX_LSTM_W_BASE);
+  if (b >= B) {   // no sequence for this die
+    if (tid == 0) fx_lstm_leave<DevAtomics>(a.ctl, gridDim.x, base, advance, a.hbuf, area.words);
+    return;
+  }
+  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) || fx_lstm_refused<DevAtomics>(a.ctl_third) ? 1u : 0u;
+  uint64_t* const where = a.hbuf + area.where + slot * FX_LSTM_DIE_WG;
+  if (tid == 0) DevAtomics::store64(where + gi, fx_lstm_pack(fx_die_of_wave(), base + 1u));
+  auto give_up = [&]() {   // the workgroup leaves behind the next barrier
+    DevAtomics::store(a.ctl + FX_LSTM_W_ERR, 1u);
+    if (a.err_host) __hip_atomic_store(a.err_host, (uint32_t)FX_ASYNC_BARRIER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    s_abort = 1u;
+  };
+  // polls so far of a wait: is it to be given up?
+  auto too_long = [&](uint32_t polls) {
+    return polls > a.spin_limit || ((polls & 255u) == 0u && DevAtomics::load(a.ctl + FX_LSTM_W_ERR) != 0u);
+  };
+
+  if (wave < NW) {
+    const int kl = lane >> 3, cl = lane & 7;
+    float w_ih[NL][E][E], w_hh[NL][E][E];   // [layer][element][column]
+#pragma unroll
+    for (int k = 0; k < NL; ++k)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const size_t at = ((size_t)((j0 + k) * 4 + (cl >> 1)) * HH + wave * 8 * E + kl * E + fx_die_element<E>(cl, e)) * HH + u0 + (cl & 1) * E;
+        fx_die_load<E>(a.wih + at, w_ih[k][e]);
+        fx_die_load<E>(a.whh + at, w_hh[k][e]);
+      }
+    const int own = wave * 8 * E + kl * E + cl % E;   // the element that this lane fetches
+    float below[NL] = {};                              // h of the layer below, read in the step before
+    const uint64_t* from[NL];
+#pragma unroll
+    for (int k = 0; k < NL; ++k) from[k] = a.hbuf + fx_lstm_hoff(0, j0 + k, b, own, L, B, HH);
+    __builtin_amdgcn_s_waitcnt(0);   // (the weights are here: otherwise the loop waits for them, and for looks behind them)
+    __syncthreads();
+    if (s_abort != 0u) {   // uniform: written ahead of the barrier
+      if (tid == 0 && a.err_host) __hip_atomic_store(a.err_host, (uint32_t)FX_ASYNC_BARRIER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      fx_lstm_poison(a, L, (uint32_t)tid, (uint32_t)(NW * 64));
+      return;
+    }
+    // Step d; all: every layer is in the middle of the sequence, and nothing is asked about one.
+    // What this lane's products are multiplied by comes through s_in[place] and from the die's cache.
+    uint32_t aborted = 0u;
+    auto step = [&](auto every, int d, int place) {
+      constexpr bool all = decltype(every)::value != 0;
+      float acc[NL * E];
+#pragma unroll
+      for (int i = 0; i < NL * E; ++i) acc[i] = 0.0f;
+      // Sums of E = 8: chains of four products, added up in a tree.  A chain of sixteen loses what the sums over the
+      // lanes keep (T = 64, 512 units, two layers, mean of eight inputs against 64 bits: 2.11e-7; so 1.83e-7, row by row
+      // 1.86e-7).
+      auto multiply = [&](float h, const float (&w)[E][E], int k) {
+        float v[E];
+        fx_die_spread<E>(h, v);
+        if constexpr (E < 8) {
+#pragma unroll
+          for (int e = 0; e < E; ++e)
+#pragma unroll
+            for (int c = 0; c < E; ++c) acc[k * E + c] = __builtin_fmaf(w[e][c], v[e], acc[k * E + c]);
+        } else {
+          float sum[2][E];
+#pragma unroll
+          for (int e = 0; e < E; ++e)
+#pragma unroll
+            for (int c = 0; c < E; ++c) sum[e / 4][c] = e % 4 == 0 ? w[e][c] * v[e] : __builtin_fmaf(w[e][c], v[e], sum[e / 4][c]);
+#pragma unroll
+          for (int c = 0; c < E; ++c) acc[k * E + c] += sum[0][c] + sum[1][c];
+        }
+      };
+#pragma unroll
+      for (int k = 0; k < NL; ++k)
+        if (all || fx_lstm_stage_time(d, k, T) >= 0) multiply(k == 0 ? s_in[place][own] : below[k > 0 ? k - 1 : 0], w_ih[k], k);
+#pragma unroll
+      for (int i = 0; i < NL * E; ++i) asm volatile("" : "+v"(acc[i]));   // (they are not to sink behind the wait)
+      if (aborted != 0u) return;   // uniform
+      bool need[NL];
+      float hv[NL];
+#pragma unroll
+      for (int k = 0; k < NL; ++k) {
+        const int t = all ? 1 : fx_lstm_stage_time(d, k, T);
+        need[k] = all || (d > 0 && fx_lstm_stage_time(d - 1, k, T) >= 0 && (t >= 0 || k + 1 < NL));
+        hv[k] = !all && t == 0 && a.h0 ? a.h0[((size_t)(j0 + k) * B + b) * HH + own] : 0.0f;
+      }
+      const uint32_t want = fx_lstm_tag_read(base, d);
+      if constexpr (K::sleep > 0) __builtin_amdgcn_s_sleep(K::sleep);
+      for (uint32_t polls = 0;;) {
+        uint64_t el[NL];
+        bool ready = true;
+#pragma unroll
+        for (int k = 0; k < NL; ++k)
+          el[k] = __hip_atomic_load(from[k] + ((d + 1) & 1) * parity, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int k = 0; k < NL; ++k) ready = ready && (!need[k] || fx_lstm_tag_of(el[k]) == want);
+#pragma unroll
+        for (int k = 0; k < NL; ++k) hv[k] = need[k] ? __uint_as_float((uint32_t)el[k]) : hv[k];
+        if (!wave_any(!ready)) break;
+        if (too_long(++polls)) {
+          give_up();
+          break;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NL; ++k) {
+        if (all || fx_lstm_stage_time(d, k, T) >= 0) multiply(hv[k], w_hh[k], k);
+        below[k] = hv[k];
+      }
+      constexpr int left = fx_die_left(NL * E);
+      int first = 0;
+      float sum[left];
+      fx_die_sum<NL * E, 5>(acc, lane, &first, sum);
+#pragma unroll
+      for (int i = 0; i < left; ++i) {
+        const int v = first + i, k = v / E, unit = (cl & 1) * E + v % E;
+        s_part[d & 1][wave][k * C + unit * 4 + (cl >> 1)] = sum[i];
+      }
+      __syncthreads();
+      aborted = s_abort;   // (looked at behind the next products)
+    };
+    int place = 0;
+    for (int d = 0; d < n_steps && aborted == 0u; ++d) {
+      if (d > 2 * (NL - 1) && d < T) step(fx_const<1>(), d, place);
+      else step(fx_const<0>(), d, place);
+      place = place == 2 ? 0 : place + 1;
+    }
+    if (aborted != 0u) {   // the results are not to be used: say so in the data
+      fx_lstm_poison(a, L, (uint32_t)tid, (uint32_t)(NW * 64));
+      return;
+    }
+    __syncthreads();   // the last step's values
+    return;
+  }
+
+  // ---- cells: lane f = (layer of the stage, unit, gate) ----
+  const int cw = wave - NW, f = min(cw * 64 + lane, NC - 1), fk = f / C, gate = f & 3, u = u0 + ((f % C) >> 2), j = j0 + fk;
+  const float bias_ih = a.bih[(size_t)(j * 4 + gate) * HH + u], bias_hh = a.bhh[(size_t)(j * 4 + gate) * HH + u];
+  float cell = a.c0 ? a.c0[((size_t)j * B + b) * HH + u] : 0.0f;
+  __builtin_amdgcn_s_setprio(3);   // (the waves that multiply share the SIMDs: ahead of them)
+  const bool owner = gate == 0 && cw * 64 + lane < NC;
+  const bool last = fk == NL - 1;
+  uint64_t* const h_to = a.hbuf + fx_lstm_hoff(0, j, b, u, L, B, HH);
+  // the stage's input: x, or what the stage before puts into its ring
+  const int link = (stage - 1) * B + b;
+  const uint64_t* const ring_in = a.hbuf + area.ring + (size_t)(link < 0 ? 0 : link) * (FX_LSTM_RING * HH);
+  uint64_t* const ring_out = a.hbuf + area.ring + (size_t)(stage * B + b) * (FX_LSTM_RING * HH);
+  uint64_t* const read_in = a.hbuf + area.read + (link < 0 ? 0 : link) * FX_LSTM_DIE_WG + gi;
+  const uint64_t* const read_out = a.hbuf + area.read + (stage * B + b) * FX_LSTM_DIE_WG;
+  float in[E];
+  auto fetch = [&](int t) {   // x of step t, asked for
+    if (stage == 0 && t < T) fx_die_load<E>(a.x + ((size_t)t * B + b) * HH + lane * E, in);
+  };
+  auto park = [&](int t) {
+    if (t >= T) return;
+    if (stage > 0) {
+      for (uint32_t polls = 0;;) {
+        bool ready = true;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const uint64_t el = __hip_atomic_load(ring_in + (t % FX_LSTM_RING) * HH + e * 64 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          ready = ready && fx_lstm_tag_of(el) == base + (uint32_t)t + 1u;
+          in[e] = __uint_as_float((uint32_t)el);
+        }
+        if (!wave_any(!ready)) break;
+        if (too_long(++polls)) {
+          give_up();
+          break;
+        }
+      }
+      if (lane == 0) DevAtomics::store64(read_in, (uint64_t)(base + (uint32_t)t + 1u));
+#pragma unroll
+      for (int e = 0; e < E; ++e) s_in[t % 3][e * 64 + lane] = in[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) s_in[t % 3][lane * E + e] = in[e];
+    }
+  };
+  bool same_die = true;
+  for (uint32_t polls = 0;;) {
+    const uint64_t el = __hip_atomic_load(where + (lane & (FX_LSTM_DIE_WG - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!wave_any(fx_lstm_tag_of(el) != base + 1u)) {
+      same_die = !wave_any((uint32_t)el != fx_die_of_wave());
+      break;
+    }
+    if (too_long(++polls)) {
+      give_up();
+      break;
+    }
+  }
+  if (cw == 0) {
+    for (int t = 0; t < 2; ++t) {
+      fetch(t);
+      park(t);
+    }
+    fetch(2);
+  }
+  __syncthreads();
+  if (s_abort != 0u) return;
+  for (int d = 0; d < n_steps; ++d) {
+    __syncthreads();
+    const uint32_t aborted = s_abort;
+    float part[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) part[w] = s_part[d & 1][w][f];
+#pragma unroll
+    for (int span = 1; span < NW; span *= 2)
+#pragma unroll
+      for (int w = 0; w + span < NW; w += 2 * span) part[w] += part[w + span];
+    const float pre = (part[0] + bias_ih) + bias_hh;
+    const float act = fx_die_gate(pre, gate == 2);
+    const float fg = quad_lane<1>(act), gg = quad_lane<2>(act), og = quad_lane<3>(act);
+    const int t = fx_lstm_stage_time(d, fk, T);
+    if (owner && t >= 0 && aborted == 0u) {
+      cell = (fg * cell) + (act * gg);
+      const float h = og * fx_tanh(cell);
+      uint64_t* const to = h_to + (d & 1) * parity;
+      const uint64_t el = fx_lstm_pack(__float_as_uint(h), fx_lstm_tag_written(base, d));
+      if (same_die) __hip_atomic_store(to, el, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      else DevAtomics::store64(to, el);
+      if (last && stage + 1 < stages) DevAtomics::store64(ring_out + (t % FX_LSTM_RING) * HH + u, fx_lstm_pack(__float_as_uint(h), base + (uint32_t)t + 1u));
+      if (j == L - 1) a.out[((size_t)t * B + b) * HH + u] = h;
+      if (t == T - 1) {
+        a.state_h[((size_t)j * B + b) * HH + u] = h;
+        a.state_c[((size_t)j * B + b) * HH + u] = cell;
+      }
+    }
+    if (aborted != 0u) return;   // uniform, and nothing was stored
+    // between the barriers of steps d and d + 1 the others read the input of step d + 1; the place of step
+    // d + 2 was last read in step d - 1
+    if (cw == 0) {
+      park(d + 2);
+      fetch(d + 3);
+    }
+    // every half ring: the next half may be written (the next stage is never that far behind but at the start)
+    if (stage + 1 < stages && d % (FX_LSTM_RING / 2) == FX_LSTM_RING / 2 - 1) {
+      const int seen = d + 1 - FX_LSTM_RING / 2;   // vectors that have to be read before vector d + RING / 2 is written
+      for (uint32_t polls = 0; seen > 0;) {
+        const uint32_t n = (uint32_t)__hip_atomic_load(read_out + (lane & (FX_LSTM_DIE_WG - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (!wave_any((int32_t)(n - (base + (uint32_t)seen)) < 0)) break;
+        if (too_long(++polls)) {
+          give_up();
+          break;
+        }
+      }
+    }
+  }
+  __syncthreads();   // the waves that multiply are done
+  if (cw == 0 && lane == 0) fx_lstm_leave<DevAtomics>(a.ctl, gridDim.x, base, advance, a.hbuf, area.words);
+}
+
 typedef void (*fx_lstm_kernel_t)(const FxLstmArgs);
 template <int L>
 static fx_lstm_kernel_t pick_rows(int hpt, int tiles) {
@@ -709,20 +1103,34 @@ static fx_lstm_kernel_t pick_serial(int hpt) {
     default: return nullptr;
   }
 }
-struct LstmLaunch { fx_lstm_kernel_t kernel; int grid, threads, tiles; };   // tiles of rows a workgroup; 0: row by row
+typedef void (*fx_lstm_die_kernel_t)(const FxLstmArgs, int);
+template <int L>
+static fx_lstm_die_kernel_t pick_die(int hpt, int* threads) {
+  switch (hpt) {
+    case 2: *threads = FxLstmDie<1, L>::threads; return fx_lstm_die_kernel<1, L>;
+    case 4: *threads = FxLstmDie<2, L>::threads; return fx_lstm_die_kernel<2, L>;
+    case 8: *threads = FxLstmDie<4, L == 4 ? 2 : L>::threads; return fx_lstm_die_kernel<4, L == 4 ? 2 : L>;
+    case 16: *threads = FxLstmDie<8, 1>::threads; return fx_lstm_die_kernel<8, 1>;
+    default: return nullptr;
+  }
+}
+enum LstmHandOver { LSTM_TAGS, LSTM_WORDS, LSTM_DIE };   // which area of the workspace
+struct LstmLaunch { const void* kernel; int grid, threads, tiles; LstmHandOver over; };   // tiles of rows a workgroup; 0: row by row
 // the forms that serve these sizes, the fastest first
 template <int L>
-static int lstm_forms(const FxLstmArgs& a, LstmLaunch (&f)[3]) {
+static int lstm_forms(const FxLstmArgs& a, LstmLaunch (&f)[4]) {
   const int hpt = a.H / 32;
-  int n = 0;
+  int n = 0, threads = 0;
+  if (fx_lstm_die_fits(a.B, a.H, L))
+    if (fx_lstm_die_kernel_t k = pick_die<L>(hpt, &threads)) f[n++] = LstmLaunch{(const void*)k, FX_LSTM_DIES * FX_LSTM_DIE_WG, threads, 0, LSTM_DIE};
   if (a.B > 1)
     for (int tiles = 1; tiles <= 2; ++tiles) {
       const int groups = (a.B + 4 * tiles - 1) / (4 * tiles), cells = L * tiles < 4 ? L * tiles : 4;   // FxLstmRows
-      if (fx_lstm_kernel_t k = pick_rows<L>(hpt, tiles)) f[n++] = LstmLaunch{k, (a.H / 4) * groups, ((a.H >= 128 ? 8 : a.H / 16) + cells) * 64, tiles};
+      if (fx_lstm_kernel_t k = pick_rows<L>(hpt, tiles)) f[n++] = LstmLaunch{(const void*)k, (a.H / 4) * groups, ((a.H >= 128 ? 8 : a.H / 16) + cells) * 64, tiles, LSTM_WORDS};
     }
   // two hidden units per workgroup: every workgroup fetches the step's vectors from the memory
   // side once, so fewer, larger workgroups fetch less, and sixteen gate sums fill the butterfly
-  if (fx_lstm_kernel_t k = pick_serial<L>(hpt)) f[n++] = LstmLaunch{k, a.H / FX_LSTM_UPW, FX_LSTM_BLOCK * FX_LSTM_UPW, 0};
+  if (fx_lstm_kernel_t k = pick_serial<L>(hpt)) f[n++] = LstmLaunch{(const void*)k, a.H / FX_LSTM_UPW, FX_LSTM_BLOCK * FX_LSTM_UPW, 0, LSTM_TAGS};
   return n;
 }
 
@@ -734,7 +1142,7 @@ static std::set<int> g_lstm_captured;               // devices on which a launch
 struct LstmFit { int per_cu, sure; };
 static std::map<std::pair<int, const void*>, LstmFit> g_lstm_fit;
 static hipError_t lstm_fit(int dev, const LstmLaunch& f, LstmFit* fit) {
-  const void* k = (const void*)f.kernel;
+  const void* k = f.kernel;
   auto it = g_lstm_fit.find({dev, k});
   if (it == g_lstm_fit.end()) {
     LstmFit v{};
@@ -752,10 +1160,10 @@ static hipError_t lstm_fit(int dev, const LstmLaunch& f, LstmFit* fit) {
 
 // 0: launched; 1: shape outside what the kernel is built for; 2: the grid would not be resident
 // all at once (every workgroup waits for values that all the others write); otherwise a HIP error code + 100.
-int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uint64_t* words_hbuf, hipStream_t stream) {
+int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uint32_t* die_ctl, hipStream_t stream) {
   FxLstmArgs a = args;
   if (a.H < 32 || a.H % 32 != 0 || a.B < 1 || a.B > FX_LSTM_MAXB || L < 1 || L * a.B > FX_LSTM_BLOCK) return 1;
-  LstmLaunch f[3];
+  LstmLaunch f[4];
   const int n = L == 1 ? lstm_forms<1>(a, f) : L == 2 ? lstm_forms<2>(a, f) : L == 3 ? lstm_forms<3>(a, f) : L == 4 ? lstm_forms<4>(a, f) : 0;
   if (n == 0) return 1;
   int dev = 0, cus = 0;
@@ -773,6 +1181,10 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
   // A captured launch is replayed whenever the program likes, beside any other: from the first one on,
   // every launch leaves half of the device free where a form of it can.
   const uint32_t device = (uint32_t)cus * FX_LSTM_CU / (g_lstm_captured.count(dev) ? 2u : 1u);
+  const bool legacy = stream == nullptr || stream == hipStreamLegacy;
+  const uint64_t id = legacy ? 0u : (uint64_t)(uintptr_t)stream;
+  const uint64_t thread = stream == hipStreamPerThread ? (uint64_t)std::hash<std::thread::id>()(std::this_thread::get_id()) : 0u;
+  FxLstmGroups& groups = g_lstm_groups[dev];
   const LstmLaunch* l = nullptr;
   uint32_t need = 0;
   for (int i = 0; i < n; ++i) {
@@ -784,27 +1196,26 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     if (e != hipSuccess) return 100 + (int)e;
     if ((long)fit.per_cu * cus < f[i].grid) continue;
     const uint32_t want = fx_lstm_need((uint32_t)f[i].grid, (uint32_t)fit.sure);
+    // (a sequence on one die holds every die: not where a stack on another stream would have to wait for it)
+    if (f[i].over == LSTM_DIE && !capturing && want + groups.beside(id, thread) > device) continue;
     if (l && want >= need) continue;
     l = &f[i];
     need = want;
     if (need <= device) break;
   }
   if (!l) return 2;
-  if (l->tiles > 0) {   // the hand-over through words
-    std::swap(a.ctl, words_ctl);
-    a.hbuf = words_hbuf;
-  }
-  a.ctl_other = words_ctl;
-  void* kargs[1] = {(void*)&a};
+  uint32_t* areas[3] = {a.ctl, words_ctl, die_ctl ? die_ctl : a.ctl};
+  std::swap(areas[0], areas[(int)l->over]);
+  a.ctl = areas[0];
+  a.ctl_other = areas[1];
+  a.ctl_third = areas[2];
+  a.hbuf = (uint64_t*)(a.ctl + FX_LSTM_CTL_WORDS);
+  void* kargs[2] = {(void*)&a, (void*)&L};
   const dim3 grid((uint32_t)l->grid), block((uint32_t)l->threads);
   if (capturing) {
-    e = hipLaunchKernel((const void*)l->kernel, grid, block, kargs, 0, stream);
+    e = hipLaunchKernel(l->kernel, grid, block, kargs, 0, stream);
     return e == hipSuccess ? 0 : 100 + (int)e;
   }
-  const bool legacy = stream == nullptr || stream == hipStreamLegacy;
-  const uint64_t id = legacy ? 0u : (uint64_t)(uintptr_t)stream;
-  const uint64_t thread = stream == hipStreamPerThread ? (uint64_t)std::hash<std::thread::id>()(std::this_thread::get_id()) : 0u;
-  FxLstmGroups& groups = g_lstm_groups[dev];
   auto record = [&](FxLstmGroups::Member& m) {
     if (!m.done) m.done = groups.event_to_use();
     if (!m.done) e = hipEventCreateWithFlags((hipEvent_t*)&m.done, hipEventDisableTiming);
@@ -817,12 +1228,13 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
   };
   bool joins = false;
   FxLstmGroups::Member& m = groups.admit(id, thread, need, device, legacy, &joins);
+  m.last = ++groups.launches;
   if (joins && !(groups.close_late(record) && groups.wait(id, thread, wait_for))) {
     groups.withdraw();
     (void)hipGetLastError();
     return 100 + (int)e;
   }
-  e = hipLaunchKernel((const void*)l->kernel, grid, block, kargs, 0, stream);
+  e = hipLaunchKernel(l->kernel, grid, block, kargs, 0, stream);
   // (a record costs launches in a row 1.3 - 2.5 us each; a completion event given to the kernel itself costs them
   // nothing, but some thousand such launches make every later call of the program, torch's as well, 5 us slower)
   if (e == hipSuccess && !m.late) (void)record(m);

@@ -39,8 +39,10 @@ struct FxLstmGroups {
     uint32_t need;             // the largest of the stream's launches in the group: one of them runs at a time
     void* done;                // event behind the last of them (null: none was made yet)
     bool late;                 // ... which is recorded when the group has closed (close_late), not behind every launch
+    uint64_t last = 0;         // number of its last launch
   };
   std::vector<Member> now, before;
+  uint64_t launches = 0;
   std::vector<void*> spare;    // events to use again
 
   static bool same(const Member& m, uint64_t stream, uint64_t thread) { return m.stream == stream && m.thread == thread; }
@@ -67,6 +69,15 @@ struct FxLstmGroups {
     }
     now.push_back(Member{stream, thread, need, nullptr, late});
     return now.back();
+  }
+  // What other streams' launches of the group need that have launched lately: a launch that does not fit beside
+  // them makes the streams take turns, and takes another form instead where it has one.  (Counted in launches
+  // and not asked of the device: queries are not allowed beside a capture.)
+  uint32_t beside(uint64_t stream, uint64_t thread) const {
+    uint32_t total = 0;
+    for (const Member& m : now)
+      if (!same(m, stream, thread) && launches - m.last < 64u) total += m.need;
+    return total;
   }
   void* event_to_use() {
     if (spare.empty()) return nullptr;

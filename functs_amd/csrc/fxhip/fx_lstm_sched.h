@@ -59,6 +59,7 @@ struct FxLstmArgs {
   uint64_t* hbuf;      // [2][L][B][H] (value, tag): h of the cells of the last two steps
   uint32_t* ctl;       // FX_LSTM_CTL_WORDS control words
   uint32_t* ctl_other; // those of the other hand-over: a wait that was given up in either refuses both
+  uint32_t* ctl_third; // and those of the third one (its own again where there is none)
   uint32_t* err_host;  // pinned word that a given-up wait reports to as well (may be null)
   int T, B, H;
   uint32_t spin_limit;
@@ -126,4 +127,39 @@ FX_LSTM_HD inline void fx_lstm_leave_slots(uint32_t* ctl, uint32_t n_wg, uint32_
   if (A::add(ctl + FX_LSTM_W_LEAVE) + 1u != n_wg) return;
   A::store(ctl + FX_LSTM_W_BASE, (base + n_steps) & 3u);
   A::store(ctl + FX_LSTM_W_LEAVE, 0u);
+}
+
+// The third hand-over, of the kernel that keeps a sequence on one die (fx_lstm_die_kernel): its layers, or as
+// many of them as the die's registers hold (a STAGE), run on the compute units that share a cache.
+//   Steps of a stage are its own: in step d its layer k computes t = d - 2 k, so that what a layer needs of
+//   the layer below was written two steps ago, and was read in the step before as that layer's own state.
+//   The h of (stage's layer, t) travels as above, with its tag, through hbuf[d & 1][j]; the two parities suffice
+//   for the same reason.
+//   From stage to stage h travels through a ring of FX_LSTM_RING vectors with tags base + t + 1.  A stage runs
+//   ahead of the next one, and overwrites vector t - FX_LSTM_RING of the ring only when all workgroups of the
+//   next stage have published that they have read it (counts: base + vectors read).
+#define FX_LSTM_RING 16
+#define FX_LSTM_DIES 8        // dies of the chip, and
+#define FX_LSTM_DIE_WG 32     // workgroups on each, one per compute unit
+FX_LSTM_HD inline int fx_lstm_stage_steps(int T, int n_layers) { return T > 0 ? T + 2 * (n_layers - 1) : 0; }
+FX_LSTM_HD inline int fx_lstm_stage_time(int d, int k, int T) {
+  const int t = d - 2 * k;
+  return (t >= 0 && t < T) ? t : -1;
+}
+// layers of a stage: all of them up to 256 units (their weights are at most 96 registers a lane), one of 512
+FX_LSTM_HD inline int fx_lstm_stage_layers(int H, int L) { return H > 256 ? 1 : H == 256 && L == 4 ? 2 : L; }
+FX_LSTM_HD inline bool fx_lstm_die_fits(int B, int H, int L) {
+  return (H == 64 || H == 128 || H == 256 || H == 512) && L >= 1 && L <= 4 && B >= 1 && B * (L / fx_lstm_stage_layers(H, L)) <= FX_LSTM_DIES;
+}
+// 64-bit words behind the control words: h [2][L][B][H]; rings [stages - 1][B][FX_LSTM_RING][H]; counts of read
+// vectors [stages - 1][B][FX_LSTM_DIE_WG]; the die that every workgroup runs on [FX_LSTM_DIES][FX_LSTM_DIE_WG]
+struct FxLstmDieArea { uint32_t ring, read, where, words; };
+FX_LSTM_HD inline FxLstmDieArea fx_lstm_die_area(int B, int H, int L) {
+  const uint32_t links = (uint32_t)(L / fx_lstm_stage_layers(H, L) - 1) * (uint32_t)B;
+  FxLstmDieArea a;
+  a.ring = (uint32_t)(2 * L * B * H);
+  a.read = a.ring + links * (uint32_t)(FX_LSTM_RING * H);
+  a.where = a.read + links * FX_LSTM_DIE_WG;
+  a.words = a.where + FX_LSTM_DIES * FX_LSTM_DIE_WG;
+  return a;
 }

@@ -423,8 +423,8 @@ int fx_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* co
  * persistent kernel: a workgroup per two hidden units keeps their columns of the weights in
  * registers for the whole sequence (thread k row k of them, and element k of the step's vectors);
  * the diagonals t + j follow each other without a barrier between workgroups, every h value
- * travels with the tag of the step that wrote it (a batch of several rows: as a word that is clear
- * until it is written) and readers poll for it, with bounded waits.  A wait that is given up reports FX_ASYNC_BARRIER through fx_async_error, fills
+ * travels with the tag of the step that wrote it (several rows that do not find dies of their own: as a word
+ * that is clear until it is written) and readers poll for it, with bounded waits.  A wait that is given up reports FX_ASYNC_BARRIER through fx_async_error, fills
  * out / state_h / state_c with NaN and ends the kernel; its workspace stays marked, and every
  * later launch on it does no step, reports the error again and returns NaN, until the caller has
  * cleared the workspace.  A caller must therefore look at fx_async_error after synchronising and
@@ -432,9 +432,12 @@ int fx_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* co
  * Contiguous fp32: x [T, B, H]; wih, whh [L, 4, H, H]; bih, bhh [L, 4, 1, H]; h0, c0, state_h,
  * state_c [L, B, H]; out [T, B, H]; h0 / c0 may be null (zero initial state).  H is 32, 64, ...
  * 1024 (a power of two), L <= 4, B <= 16 (FX_E_UNSUPPORTED otherwise), and the
- * workgroups (H / 2 of 512 threads, or H / 4 of up to 768 for every four or eight rows) must be resident
+ * workgroups (256 of up to 640 threads, 32 on each of the chip's dies, where H is 64 to 512 and the sequences
+ * with their layers, or at H = 512 each layer of theirs, find dies of their own; H / 2 of 512 threads, or H / 4
+ * of up to 768 for every four or eight rows) must be resident
  * together (FX_E_LIMIT if no form's are).  Launches on several streams of a device overlap when all their
- * workgroups find places together (two stacks of 512 units with one sequence each, for instance);
+ * workgroups find places together (two stacks of 512 units with one sequence each, for instance, which leave
+ * the dies' form to a stream that launches alone);
  * one that does not fit waits, in its stream, for the launches before it (a launch on another stream than the
  * legacy default one records an event behind it for that).  A captured launch cannot be
  * made to wait: it, and from then on every launch on that device, takes a form for half of the device

@@ -1,0 +1,168 @@
+// TEST INFRASTRUCTURE ONLY - never linked into or loaded by the product.
+//
+// CPU build of the schedule and hand-over of fx_lstm_die_kernel (fx_lstm_sched.h: a sequence on one die): one
+// host thread per workgroup, stages of layers whose steps are their own, the two parities of the h buffer, the
+// ring between stages with its counts of read vectors, tags from launch to launch.
+#include <math.h>
+#include <string.h>
+
+#include <functional>
+#include <thread>
+#include <vector>
+
+#include "../../functs_amd/csrc/fxhip/fx_lstm_groups.h"
+#include "../../functs_amd/csrc/fxhip/fx_lstm_sched.h"
+
+namespace {
+struct HostAtomics {
+  static uint32_t add(uint32_t* p) { return __atomic_fetch_add(p, 1u, __ATOMIC_ACQ_REL); }
+  static uint32_t load(uint32_t* p) { return __atomic_load_n(p, __ATOMIC_ACQUIRE); }
+  static void store(uint32_t* p, uint32_t v) { __atomic_store_n(p, v, __ATOMIC_RELEASE); }
+  static void store64(uint64_t* p, uint64_t v) { __atomic_store_n(p, v, __ATOMIC_RELEASE); }
+};
+float sigmoidf(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+// n_wg workgroups a stage (at most FX_LSTM_DIE_WG), H / n_wg units each; slow: (stage, workgroup) that dawdles
+struct Run {
+  FxLstmArgs a;
+  int L, n_wg, total, slow_stage, slow_wg;
+  bool give_up(uint32_t polls) const {
+    if (polls <= a.spin_limit && !((polls & 255u) == 0u && HostAtomics::load(a.ctl + FX_LSTM_W_ERR) != 0u)) return false;
+    HostAtomics::store(a.ctl + FX_LSTM_W_ERR, 1u);
+    return true;
+  }
+  template <class F>
+  bool wait(F&& there) const {
+    for (uint32_t polls = 0; !there();) {
+      if (give_up(++polls)) return false;
+      std::this_thread::yield();
+    }
+    return true;
+  }
+  void workgroup(int b, int stage, int gi) const {
+    const int H = a.H, B = a.B, T = a.T, NL = fx_lstm_stage_layers(H, L), stages = L / NL, U = H / n_wg, u0 = gi * U, j0 = stage * NL;
+    const uint32_t base = HostAtomics::load(a.ctl + FX_LSTM_W_BASE);
+    const FxLstmDieArea area = fx_lstm_die_area(B, H, L);
+    const int n_steps = fx_lstm_stage_steps(T, NL);
+    uint64_t* ring_in = a.hbuf + area.ring + (size_t)((stage - 1) * B + b) * (FX_LSTM_RING * H);
+    uint64_t* ring_out = a.hbuf + area.ring + (size_t)(stage * B + b) * (FX_LSTM_RING * H);
+    uint64_t* read_in = a.hbuf + area.read + ((stage - 1) * B + b) * FX_LSTM_DIE_WG + gi;
+    uint64_t* read_out = a.hbuf + area.read + (stage * B + b) * FX_LSTM_DIE_WG;
+    std::vector<std::vector<float>> in(3, std::vector<float>(H)), below(NL, std::vector<float>(H)), hv(NL, std::vector<float>(H));
+    std::vector<float> c((size_t)NL * U);
+    for (int k = 0; k < NL; ++k)
+      for (int u = 0; u < U; ++u) c[k * U + u] = a.c0 ? a.c0[((size_t)(j0 + k) * B + b) * H + u0 + u] : 0.0f;
+    // element i of the vector p, once it carries `tag`
+    auto tagged = [&](uint64_t* p, uint32_t tag, float* to) {
+      return wait([&] {
+        const uint64_t e = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+        const uint32_t bits = (uint32_t)e;
+        memcpy(to, &bits, 4);
+        return fx_lstm_tag_of(e) == tag;
+      });
+    };
+    auto park = [&](int t) {
+      if (t >= T) return true;
+      for (int i = 0; i < H; ++i) {
+        if (stage == 0) in[t % 3][i] = a.x[((size_t)t * B + b) * H + i];
+        else if (!tagged(ring_in + (size_t)(t % FX_LSTM_RING) * H + i, base + (uint32_t)t + 1u, &in[t % 3][i])) return false;
+      }
+      if (stage > 0) HostAtomics::store64(read_in, (uint64_t)(base + (uint32_t)t + 1u));
+      return true;
+    };
+    if (!park(0) || !park(1)) return;
+    for (int d = 0; d < n_steps; ++d) {
+      if (stage == slow_stage && gi == slow_wg && d % 5 == 0) std::this_thread::sleep_for(std::chrono::milliseconds(2));
+      for (int k = 0; k < NL; ++k) {
+        const int t = fx_lstm_stage_time(d, k, T);
+        const bool need = d > 0 && fx_lstm_stage_time(d - 1, k, T) >= 0 && (t >= 0 || k + 1 < NL);
+        for (int i = 0; i < H; ++i) {
+          hv[k][i] = t == 0 && a.h0 ? a.h0[((size_t)(j0 + k) * B + b) * H + i] : 0.0f;
+          if (need && !tagged(a.hbuf + fx_lstm_hoff((d + 1) & 1, j0 + k, b, i, L, B, H), fx_lstm_tag_read(base, d), &hv[k][i])) return;
+        }
+      }
+      for (int k = 0; k < NL; ++k) {
+        const int t = fx_lstm_stage_time(d, k, T), j = j0 + k;
+        if (t < 0) continue;
+        const std::vector<float>& x = k == 0 ? in[d % 3] : below[k - 1];
+        for (int u = 0; u < U; ++u) {
+          float g[4];
+          for (int q = 0; q < 4; ++q) {
+            float s = 0.f;
+            for (int i = 0; i < H; ++i) {
+              const size_t w = ((size_t)(j * 4 + q) * H + i) * H + u0 + u;
+              s += a.wih[w] * x[i] + a.whh[w] * hv[k][i];
+            }
+            g[q] = s + a.bih[(size_t)(j * 4 + q) * H + u0 + u] + a.bhh[(size_t)(j * 4 + q) * H + u0 + u];
+          }
+          float& cell = c[k * U + u];
+          cell = sigmoidf(g[1]) * cell + sigmoidf(g[0]) * tanhf(g[2]);
+          const float h = sigmoidf(g[3]) * tanhf(cell);
+          uint32_t bits;
+          memcpy(&bits, &h, 4);
+          HostAtomics::store64(a.hbuf + fx_lstm_hoff(d & 1, j, b, u0 + u, L, B, H), fx_lstm_pack(bits, fx_lstm_tag_written(base, d)));
+          if (k == NL - 1 && stage + 1 < stages) HostAtomics::store64(ring_out + (size_t)(t % FX_LSTM_RING) * H + u0 + u, fx_lstm_pack(bits, base + (uint32_t)t + 1u));
+          if (j == L - 1) a.out[((size_t)t * B + b) * H + u0 + u] = h;
+          if (t == T - 1) {
+            a.state_h[((size_t)j * B + b) * H + u0 + u] = h;
+            a.state_c[((size_t)j * B + b) * H + u0 + u] = cell;
+          }
+        }
+      }
+      below = hv;
+      if (!park(d + 2)) return;
+      if (stage + 1 < stages && d % (FX_LSTM_RING / 2) == FX_LSTM_RING / 2 - 1) {
+        const int seen = d + 1 - FX_LSTM_RING / 2;
+        for (int w = 0; w < n_wg && seen > 0; ++w)
+          if (!wait([&] { return (int32_t)((uint32_t)__atomic_load_n(read_out + w, __ATOMIC_ACQUIRE) - (base + (uint32_t)seen)) >= 0; })) return;
+      }
+    }
+    fx_lstm_leave<HostAtomics>(a.ctl, (uint32_t)total, base, (uint32_t)n_steps + 1u, a.hbuf, area.words);
+  }
+};
+}  // namespace
+
+// `launches` runs on one workspace that is cleared once; the error word, or -1 when the workspace was not left
+// as the next launch needs it
+extern "C" int fx_lstm_die_emul(const float* x, const float* wih, const float* whh, const float* bih, const float* bhh, const float* h0,
+                                const float* c0, float* out, float* state_h, float* state_c, int T, int B, int H, int L, int n_wg,
+                                uint32_t spin_limit, int launches, uint32_t base0, int slow_stage, int slow_wg) {
+  if (!fx_lstm_die_fits(B, H, L)) return -2;
+  std::vector<uint32_t> ctl(FX_LSTM_CTL_WORDS, 0u);
+  std::vector<uint64_t> area(fx_lstm_die_area(B, H, L).words, 0ull);
+  ctl[FX_LSTM_W_BASE] = base0;
+  Run r;
+  r.a = FxLstmArgs{x, wih, whh, bih, bhh, h0, c0, out, state_h, state_c, area.data(), ctl.data(), nullptr, nullptr, nullptr, T, B, H, spin_limit};
+  const int stages = L / fx_lstm_stage_layers(H, L);
+  r.L = L; r.n_wg = n_wg; r.total = stages * B * n_wg; r.slow_stage = slow_stage; r.slow_wg = slow_wg;
+  uint32_t base = base0;
+  for (int n = 0; n < launches; ++n) {
+    for (size_t i = 0; i < (size_t)T * B * H; ++i) out[i] = NAN;
+    std::vector<std::thread> th;
+    for (int b = 0; b < B; ++b)
+      for (int s = 0; s < stages; ++s)
+        for (int g = 0; g < n_wg; ++g) th.emplace_back(&Run::workgroup, std::cref(r), b, s, g);
+    for (auto& t : th) t.join();
+    if (ctl[FX_LSTM_W_ERR]) return (int)ctl[FX_LSTM_W_ERR];
+    base += (uint32_t)fx_lstm_stage_steps(T, fx_lstm_stage_layers(H, L)) + 1u;
+    if (base >= FX_LSTM_TAG_WRAP) {
+      base = 0u;
+      for (uint64_t e : area)
+        if (e != 0ull) return -1;
+    }
+    if (ctl[FX_LSTM_W_BASE] != base || ctl[FX_LSTM_W_LEAVE] != 0u) return -1;
+  }
+  return 0;
+}
+
+// needs of the launches that streams 0, 1, 2 ... have made (one each, in that order, then `more` of stream 0),
+// as stream 0 sees them beside its own
+extern "C" uint32_t fx_lstm_beside_emul(const uint32_t* needs, int n, int more) {
+  FxLstmGroups g;
+  bool joins;
+  for (int s = 0; s < n + more; ++s) {
+    const uint64_t stream = s < n ? (uint64_t)s : 0u;
+    g.admit(stream, 0u, needs[stream], 0xffffffffu, true, &joins).last = ++g.launches;
+  }
+  return g.beside(0u, 0u);
+}

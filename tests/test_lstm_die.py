@@ -1,0 +1,89 @@
+"""A sequence's layers on one die (fx_lstm_die_kernel): the schedule, the ring between stages and the tags on
+host threads, and the kernel against the oracle.  Tolerances as for the other forms of fx_lstm_stack
+(tests/test_lstm_kernel.py)."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+import torch
+
+from tests.test_lstm_kernel import _close, _gpu, _inputs, _reference
+
+
+@pytest.fixture(scope="module")
+def emul(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("lstm_die") / "liblstm_die_emul.so")
+    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "support", "lstm_die_emul.cpp")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-pthread", src, "-o", so])
+    lib = ctypes.CDLL(so)
+    lib.fx_lstm_die_emul.argtypes = [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.c_uint32, ctypes.c_int, ctypes.c_uint32, ctypes.c_int, ctypes.c_int]
+    lib.fx_lstm_beside_emul.restype = ctypes.c_uint32
+    return lib
+
+
+def _run(lib, args, n_wg=4, launches=1, base0=0, slow=(-1, -1), spin=1 << 30):
+    T, B, H = args[0].shape
+    L = args[1].size(0)
+    out, sh, sc = torch.zeros(T, B, H), torch.zeros(L, B, H), torch.zeros(L, B, H)
+    ts = [t.contiguous() for t in args]
+    rc = lib.fx_lstm_die_emul(*[t.data_ptr() for t in ts + [out, sh, sc]], T, B, H, L, n_wg, spin, launches, base0, *slow)
+    return (out, sh, sc), rc
+
+
+# one and two stages of two layers, stages of one layer whose rings go round more than twice
+@pytest.mark.parametrize("T,H,L,B,launches", [(1, 64, 1, 1, 3), (1, 64, 4, 2, 2), (2, 128, 3, 2, 2), (7, 64, 2, 3, 3), (20, 256, 4, 1, 2), (40, 512, 2, 1, 1), (1, 512, 3, 1, 3)])
+def test_schedule_and_ring_on_host_threads(emul, T, H, L, B, launches):
+    args = _inputs(T + H + L, T, H, L, B)
+    got, rc = _run(emul, args, launches=launches)
+    assert rc == 0
+    _close(got, _reference(*args), "emul T=%d H=%d L=%d B=%d" % (T, H, L, B))
+
+
+@pytest.mark.parametrize("slow", [(0, 1), (1, 0), (2, 3)])
+def test_a_stage_that_lags_is_not_overrun(emul, slow):
+    """One workgroup of the first, second or third stage dawdles: the ring holds the stage before it up."""
+    args = _inputs(3, 45, 512, 3, 1)
+    got, rc = _run(emul, args, slow=slow)
+    assert rc == 0
+    _close(got, _reference(*args), "slow %r" % (slow,))
+
+
+def test_tags_start_over_before_they_wrap(emul):
+    args = _inputs(4, 5, 512, 2, 1)
+    got, rc = _run(emul, args, launches=3, base0=0x80000000 - 8)
+    assert rc == 0
+    _close(got, _reference(*args), "after the tags were cleared")
+
+
+def test_streams_that_launched_lately_are_counted(emul):
+    needs = (ctypes.c_uint32 * 3)(10, 20, 30)
+    assert emul.fx_lstm_beside_emul(needs, 3, 0) == 50
+    assert emul.fx_lstm_beside_emul(needs, 3, 63) == 30    # stream 1 launched 64 launches ago
+    assert emul.fx_lstm_beside_emul(needs, 3, 64) == 0
+    assert emul.fx_lstm_beside_emul(needs, 1, 5) == 0
+
+
+# every width and depth of a stage, one to eight sequences, rings that go round, shorter sequences than the lag
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,L,B", [(1, 64, 1, 1), (2, 64, 3, 8), (33, 64, 4, 5), (1, 128, 4, 8), (19, 128, 2, 3), (1, 256, 1, 8), (30, 256, 3, 8),
+                                     (50, 256, 4, 4), (21, 256, 2, 1), (1, 512, 3, 2), (3, 512, 2, 4), (70, 512, 2, 4), (40, 512, 4, 2), (9, 512, 1, 8)])
+def test_kernel_against_the_oracle(T, H, L, B):
+    args = _inputs(T + H + L + B, T, H, L, B)
+    _close(_gpu(*args, launches=3), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
+
+
+@pytest.mark.gpu
+def test_operands_of_any_float_alignment():
+    from functs_amd._lib import check, lib
+    args = _inputs(8, 6, 256, 2, 2)
+    odd = [torch.cat([t.new_zeros(1), t.reshape(-1)]).cuda()[1:] for t in args]
+    assert all(t.data_ptr() % 16 == 4 for t in odd)
+    T, B, H, L = 6, 2, 256, 2
+    n = lib.fx_lstm_stack_workspace_bytes(B, H, L)
+    ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    out = [torch.empty(T, B, H, device="cuda"), torch.empty(L, B, H, device="cuda"), torch.empty(L, B, H, device="cuda")]
+    check(lib.fx_lstm_stack(*[t.data_ptr() for t in odd + out], T, B, H, L, ws.data_ptr(), n, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    assert lib.fx_async_error(1) == 0
+    _close([t.cpu() for t in out], _reference(*args), "odd alignment")
