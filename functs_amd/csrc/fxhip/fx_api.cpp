@@ -432,8 +432,10 @@ static const FxRsKernel* rs_of(const fx::Plan* pl);
 static void rs_fill_params(const fx::Plan* pl, FxRsLaunch* rl, const FxRsKernel* kern);
 static bool head_active(const fx::Plan* pl) {
   // (with compiled kernels switched off, fx_set_specialization(0), everything runs in the interpreter)
-  return pl->mode == FX_MODE_COMPACT && pl->head.ok && g_head_mode.load(std::memory_order_relaxed) != 0 &&
-         g_specialize.load(std::memory_order_relaxed) != 0;
+  if (pl->mode != FX_MODE_COMPACT || g_head_mode.load(std::memory_order_relaxed) == 0 || g_specialize.load(std::memory_order_relaxed) == 0) return false;
+  // Class scores in whole groups of four; any other number of classes stands for the row-stream kernel that would
+  // have to be generated for it, and goes with those.
+  return pl->head.ok || (pl->head.ragged && g_rs_mode.load(std::memory_order_relaxed) != 0);
 }
 static bool cmap_active(const fx::Plan* pl) {
   return pl->mode == FX_MODE_COMPACT && pl->cmap.ok && g_head_mode.load(std::memory_order_relaxed) != 0 &&
@@ -824,7 +826,7 @@ static int head_launch_info(fx::Plan* pl, FxHeadLaunch* hl) {
   hl->sub_rows = head_sub_rows(hi);
   hl->S = hi.S;
   hl->C = hi.C;
-  fx_fastdiv_make(hi.C / 4u, &hl->g_magic, &hl->g_shift);
+  fx_fastdiv_make(hi.C % 4u ? hi.C : hi.C / 4u, &hl->g_magic, &hl->g_shift);
   hl->thr_bits = hi.thr_bits;
   hl->spin_limit = g_stream_spin.load(std::memory_order_relaxed);
   hl->n_sptr = (uint32_t)pl->sptr.size();

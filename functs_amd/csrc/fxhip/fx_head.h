@@ -28,6 +28,7 @@
 // What the matcher found (host).
 struct FxHeadInfo {
   bool ok = false;
+  bool ragged = false;           // as ok, but rows of class scores that are no whole groups of four
   uint64_t norm_hash = 0;        // hash of the normalised programs (reported also when they do not match)
   uint32_t pred_slot = 0, anc_slot = 0, strd_slot = 0;   // pointer slots (FX_SLOT_TASK: per-task table)
   int32_t pred_tcoef = 0, anc_tcoef = 0, strd_tcoef = 0; // element offset per task
@@ -48,7 +49,7 @@ struct FxHeadLaunch {
   uint32_t chunks, chunk_rows;   // workgroups per task and rows of each (<= FX_BLOCK)
   uint32_t sub_rows;             // rows of a sub-tile (<= FX_HEAD_SUB; the window holds them)
   uint32_t S, C;
-  uint32_t g_magic, g_shift;     // fast division by C / 4 (groups of four class scores per row)
+  uint32_t g_magic, g_shift;     // fast division by C / 4 (groups of four class scores per row); C % 4 != 0: by C
   uint32_t thr_bits;
   uint32_t epoch, spin_limit;
   uint32_t n_sptr, n_tptr;

@@ -236,8 +236,39 @@ __global__ __launch_bounds__(FX_BLOCK) void fx_head_stream(const FxHeadLaunch hl
       __builtin_nontemporal_store(ob, (FX_AS1 fx_u32x4_a4*)(box + (size_t)(orow + r) * 4u));
       __builtin_nontemporal_store(fx_sigmoid(p4), obj + orow + r);
     }
-    // ---- class scores: four per lane
-    {
+    // ---- class scores: four per lane.  Rows that are no whole groups of four: what the sub-tile's rows put out
+    // is one run, which leaves in its 16-byte lines, a line's elements from up to four rows.
+    if ((hl.C & 3u) != 0u) {
+      const uint32_t n = n_kept * hl.C;
+      FX_AS1 float* cls = (FX_AS1 float*)fxh_ptr(hl, hl.out_slot[2], task) + (size_t)hl.out_tstride[2] * task + (size_t)orow * hl.C;
+      const uint32_t skew = ((uint32_t)(uint64_t)cls >> 2) & 3u;   // elements between the line and the run
+      const uint32_t lines = n ? (n + skew + 3u) >> 2 : 0u;
+      for (uint32_t g = threadIdx.x; g < lines; g += NT) {
+        const int32_t e0 = (int32_t)(4u * g - skew);
+        uint32_t r = fx_fastdiv((uint32_t)max(e0, 0), hl.g_magic, hl.g_shift);
+        uint32_t c = (uint32_t)max(e0, 0) - r * hl.C;
+        float v[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+          const uint32_t e = (uint32_t)(e0 + (int32_t)j);   // (ahead of the run: beyond n, as unsigned)
+          const bool live = e < n;
+          v[j] = fx_sigmoid(u2f(W[(live ? s_rowmap[r] * S + 5u + c : 0u)]));
+          if (live && ++c == hl.C) {
+            c = 0u;
+            ++r;
+          }
+        }
+        if (e0 >= 0 && (uint32_t)e0 + 4u <= n) {
+          fx_u32x4 o4;
+          o4.x = f2u(v[0]); o4.y = f2u(v[1]); o4.z = f2u(v[2]); o4.w = f2u(v[3]);
+          __builtin_nontemporal_store(o4, (FX_AS1 fx_u32x4_a4*)(cls + e0));
+        } else {
+#pragma unroll
+          for (uint32_t j = 0; j < 4; ++j)
+            if ((uint32_t)(e0 + (int32_t)j) < n) __builtin_nontemporal_store(v[j], cls + (e0 + (int32_t)j));
+        }
+      }
+    } else {
       const uint32_t G = hl.C >> 2, ng = n_kept * G;
       FX_AS1 float* cls = (FX_AS1 float*)fxh_ptr(hl, hl.out_slot[2], task) + (size_t)hl.out_tstride[2] * task + (size_t)orow * hl.C;
 #pragma unroll 2

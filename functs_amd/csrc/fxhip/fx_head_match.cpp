@@ -47,11 +47,15 @@ void match_head(Plan* P) {
   const FxInsn* ins = (const FxInsn*)(sb + cl.off_insn);
   const FxAffine* aff = (const FxAffine*)(sb + cl.off_aff);
   const FxOut* outs = (const FxOut*)(sb + cl.off_outs);
-  // the output table is sorted by row length: objectness [K], boxes [K, 4], class scores [K, C]
-  const FxOut &o_obj = outs[0], &o_box = outs[1], &o_cls = outs[2];
+  // objectness [K], boxes [K, 4], class scores [K, C]: the output table is sorted by row length, so fewer
+  // than four classes lie ahead of the boxes, and one class may lie ahead of the objectness
+  int role[3] = {0, 1, 2};
+  if (outs[0].rank != 1) std::swap(role[0], role[1]);
+  if (outs[2].rowlen == 4 && outs[role[1]].rowlen < 4) std::swap(role[1], role[2]);
+  const FxOut &o_obj = outs[role[0]], &o_box = outs[role[1]], &o_cls = outs[role[2]];
   if (o_obj.rank != 1 || o_obj.rowlen != 1) return;
   if (o_box.rank != 2 || o_box.rowlen != 4 || o_box.inner != 4) return;
-  if (o_cls.rank != 2 || o_cls.rowlen < 4 || o_cls.rowlen % 4 != 0 || o_cls.inner != o_cls.rowlen) return;
+  if (o_cls.rank != 2 || o_cls.rowlen < 1 || o_cls.inner != o_cls.rowlen) return;
   for (int k = 0; k < 3; ++k)
     if (outs[k].dtype != FX_F32 || outs[k].vt != FX_VT_F) return;
   const uint32_t C = o_cls.rowlen, S = C + 5;
@@ -117,9 +121,10 @@ void match_head(Plan* P) {
   walk(cl.mask_begin, cl.mask_end, true);
   hs.mix(cl.mask_vt);
   for (int k = 0; k < 3 && !bad; ++k) {
-    hs.mix(outs[k].lead);
-    hs.mix(outs[k].pure);
-    walk(outs[k].prog_begin, outs[k].prog_end, false);
+    const FxOut& o = outs[role[k]];
+    hs.mix(o.lead);
+    hs.mix(o.pure);
+    walk(o.prog_begin, o.prog_end, false);
   }
   hi.norm_hash = hs.h;
   if (bad) return;
@@ -150,11 +155,12 @@ void match_head(Plan* P) {
   hi.n_rows = cl.n_rows;
   hi.n_tasks = cl.n_tasks;
   for (int k = 0; k < 3; ++k) {
-    hi.out_slot[k] = outs[k].ptr_slot;
-    hi.out_tstride[k] = outs[k].task_stride;
+    hi.out_slot[k] = outs[role[k]].ptr_slot;
+    hi.out_tstride[k] = outs[role[k]].task_stride;
   }
   hi.slot_total = h->slot_total;
-  hi.ok = true;
+  hi.ok = C % 4 == 0;
+  hi.ragged = !hi.ok;
 }
 
 }  // namespace fx
