@@ -12,8 +12,8 @@
 
 #include "fx_bytecode.h"
 
-#define FX_HEAD_SUB 64u        // most rows of a sub-tile (one ballot)
-#define FX_HEAD_NSUB 4u        // most sub-tiles of a chunk: a chunk holds at most FX_BLOCK rows
+#define FX_HEAD_SUB 256u       // most rows of a sub-tile (FX_BLOCK: one kept row a lane)
+#define FX_HEAD_NSUB 4u        // ballots of a chunk: it holds at most FX_BLOCK rows
 #define FX_HEAD_KV 6u          // 128-bit loads per lane that carry a sub-tile
 #define FX_HEAD_STATUS_BITS 9u // a chunk's count is at most FX_BLOCK
 #define FX_HEAD_FLOOD_BYTES (8u << 20)   // first sub-tiles of a launch from which on the counts are sent ahead of the rows

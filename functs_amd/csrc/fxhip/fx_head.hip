@@ -7,8 +7,9 @@
 //   1. Wave 0 gathers the objectness of every row of the chunk (one float per row, issued before
 //      anything else), evaluates the threshold and publishes the chunk's kept-row count in a
 //      status word tagged with the call's epoch.
-//   2. Meanwhile all waves ask for the rows of the first sub-tile (up to 64 rows: one contiguous
-//      run of memory, coalesced 128-bit loads; the lines travel in registers and are parked in an
+//   2. Meanwhile all waves ask for the rows of the first sub-tile (as many as six 128-bit loads a
+//      lane carry: 72 rows of 85 floats, a whole chunk of up to 24; one contiguous
+//      run of memory, coalesced; the lines travel in registers and are parked in an
 //      LDS window; the next sub-tile is requested as soon as the current one is parked).
 //   3. One look-back per workgroup (wave 1): the write offset of the chunk is the sum of the
 //      counts of the earlier chunks of its image, read from their status words as they appear.
@@ -170,10 +171,14 @@ __global__ __launch_bounds__(FX_BLOCK) void fx_head_stream(const FxHeadLaunch hl
     if (s + 1u < n_sub) request(s + 1u);
     const uint32_t t_r0 = s * sub_rows, t_rows = min(sub_rows, c_rows - t_r0);
     if (wave == 0) {
-      const bool keep = lane < t_rows && s_keep[t_r0 + lane] != 0u;
-      const uint64_t bal = __builtin_amdgcn_ballot_w64(keep);
-      if (keep) s_rowmap[__popcll(bal & ((1ull << lane) - 1ull))] = lane;
-      if (lane == 0) s_nk = (uint32_t)__popcll(bal);
+      uint32_t n = 0;
+      for (uint32_t r0 = 0; r0 < t_rows; r0 += 64u) {
+        const bool keep = r0 + lane < t_rows && s_keep[t_r0 + r0 + lane] != 0u;
+        const uint64_t bal = __builtin_amdgcn_ballot_w64(keep);
+        if (keep) s_rowmap[n + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = r0 + lane;
+        n += (uint32_t)__popcll(bal);
+      }
+      if (lane == 0) s_nk = n;
     } else if (wave == 1 && s == 0) {
       look_back();
     }
