@@ -331,10 +331,12 @@ def main():
                     help="what to capture: benchmark programs, variants (other spellings of the detection head), "
                          "coverage, stream")
     ap.add_argument("--plan-only", action="store_true", help="plan the regions without running them: needs no GPU")
+    ap.add_argument("--boxes", action="store_true", help="also the programs of outputs in boxes: one table serves all shapes of a program "
+                    "whose whole form asks for them (box regression, the YOLO head; captured on a GPU, where constants fold as they do in a call)")
     args = ap.parse_args()
     names = [n for n in args.programs.split(",") if n]
     before = set(os.listdir(args.out)) if os.path.isdir(args.out) else set()
-    with capture(args.out):
+    with capture(args.out, boxes=args.boxes):
         if args.plan_only:
             _plan_benchmark_programs(names)
         else:

@@ -362,6 +362,9 @@ int fx_region_plan(fx_region* reg, const fx_arg* args, int n_args, const fx_plan
 // The plan that a handle stands for now: outputs are computed whole where the region has compiled kernels
 // for that (one store of whole groups an item, temporaries in registers; the lean kernel), in boxes
 // otherwise.  Kernels may be switched off and on or loaded later, so a handle keeps both forms.
+// In boxes, interpreted against compiled (a box's program does not depend on the sizes, so one table serves them
+// all): box regression of 8 732 x 21 boxes 23.6 : 11.6 us a call, the dense part of the YOLO head on four images
+// of 608 55 : 46.
 // Compiled and whole against interpreted and in boxes, the kernel alone: SSD decode and softmax (53
 // instructions) 6.7 us against 18.0; the YOLO head of 16 images (1 697 instructions) 114.5 against 69.8:
 // for programs of that length the line lies on the wrong side.
