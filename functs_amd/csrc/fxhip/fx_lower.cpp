@@ -2403,8 +2403,10 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
         for (uint32_t pc = od.prog_begin; pc < od.prog_end; ++pc) heavy = heavy || cb.code[pc].op == FX_RBEGIN;
         od.unit_items = (!heavy && od.numel >= (8u << 20)) ? 4u : 1u;
         // a pure tail is evaluated once per four items: worth it as soon as the device still gets
-        // four units per CU (a copy of 4 MB takes 2.9 us as 1024 workgroups and 4.4 us as 256)
-        if (od.pure && od.numel >= (4u << 20)) od.unit_items = 4u;
+        // four units per CU (a copy of 4 MB takes 2.9 us as 1024 workgroups and 4.4 us as 256); the leading loads of four
+        // items of a box travel together (YOLO head, four images of 608, its boxes of 5.5 M elements: the kernel 46 -> 36 us,
+        // eight columns of 3 M 258 -> 244; below 2 M the corner decode of 1 M rows is slower, 46 : 50)
+        if ((od.pure && od.numel >= (4u << 20)) || (od.box && !heavy && od.numel >= (2u << 20))) od.unit_items = 4u;
         if (od.rowwave) {
           const uint32_t rows = od.rowlen ? od.numel / od.rowlen : 0;
           const uint32_t rows_per_item = 64u / od.rowseg;
