@@ -262,6 +262,8 @@ struct FxHeader {
 #define FX_FAST_OUTS 2
 #define FX_LEAN_P 24     // pointers and
 #define FX_LEAN_S 16     // scalars of a region that the lean kernel's argument block holds
+#define FX_LEAN_LEAD 1u
+#define FX_LEAN_HALF 2u
 // One output of the region: the fields of FxOut that place a work item, the leading load's
 // affine map, and the two buffers.  160 bytes, laid out so that a kernel for rank <= 3 reads the
 // first 128 only; the records start at a multiple of 64 bytes in the argument segment.
@@ -269,7 +271,7 @@ struct FxLeanOut {
   uint64_t out_ptr;             // the output's buffer and the leading load's, resolved at launch when
   uint64_t lead_ptr;            // they do not change with the task (0: look the slot up in p[])
   uint32_t ptr_slot, lead_slot; // may carry FX_SLOT_TASK
-  uint32_t lead;                // as FxOut::lead
+  uint32_t lead;                // FX_LEAN_LEAD: as FxOut::lead; FX_LEAN_HALF: elements of the leading load's 16-bit type
   uint32_t block_begin, task_stride, unit_items, inner, vd, gpr, gp_magic, gp_shift, n_groups;   // as in FxOut
   int32_t lead_base, lead_tcoef;
   int32_t lead_cf[FX_MAXR];

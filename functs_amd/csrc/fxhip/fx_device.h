@@ -155,6 +155,15 @@ __device__ __forceinline__ uint16_t fx_bf16(float f) {
   return f != f ? (uint16_t)0x7fc0u : (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 
+// the same for two values, by the instruction that rounds two (it would keep a NaN's payload); the same bits for every float
+__device__ __forceinline__ uint32_t fx_bf16_pair(float a, float b) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  const float nan = u2f(0x7fc00000u);
+  const f2 f = {a != a ? nan : a, b != b ? nan : b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, b2));
+}
+
 __device__ __forceinline__ void fx_store(uint64_t base_, uint32_t o, uint32_t dt, uint32_t vt, uint32_t v) {
   FX_AS1 uint8_t* base = (FX_AS1 uint8_t*)base_;
   switch (dt) {
@@ -406,7 +415,11 @@ __device__ __forceinline__ void fx_store_vec(uint64_t base_, uint32_t obase, con
       for (int j = 0; j < FX_V; ++j) v[j] = __half_as_ushort(__float2half(u2f(A[j])));
     } else {
 #pragma unroll
-      for (int j = 0; j < FX_V; ++j) v[j] = fx_bf16(u2f(A[j]));
+      for (int j = 0; j < FX_V; j += 2) {
+        const uint32_t w = fx_bf16_pair(u2f(A[j]), u2f(A[j + 1]));
+        v[j] = (uint16_t)w;
+        v[j + 1] = (uint16_t)(w >> 16);
+      }
     }
     *(FX_AS1 fx_u16x4_a2*)((FX_AS1 uint8_t*)base_ + ((obase + e[0]) << 1)) = v;
   } else {

@@ -337,7 +337,7 @@ hipError_t fx_launch_dense(int rank, const uint32_t* sb, const FxLaunchInfo& li,
     for (uint32_t o = 0; o < a.n_outs; ++o) {
       FxLeanOut& lo = a.out[o];
       lo.out_ptr = (lo.ptr_slot & FX_SLOT_TASK) ? 0 : dyn->p[lo.ptr_slot & 0xffffu];
-      lo.lead_ptr = (!lo.lead || (lo.lead_slot & FX_SLOT_TASK)) ? 0 : dyn->p[lo.lead_slot & 0xffffu];
+      lo.lead_ptr = (!(lo.lead & FX_LEAN_LEAD) || (lo.lead_slot & FX_SLOT_TASK)) ? 0 : dyn->p[lo.lead_slot & 0xffffu];
     }
     memcpy(a.p, dyn->p, sizeof(uint64_t) * a.n_p);
     memcpy(a.s, dyn->s, sizeof(uint32_t) * a.n_s);

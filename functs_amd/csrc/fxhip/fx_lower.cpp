@@ -2581,7 +2581,7 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
   hp->off_taskmap = off_taskmap;
   hp->total_words = (uint32_t)blob.size();
 
-  // One class of at most FX_FAST_OUTS outputs of 32-bit elements, tasks numbered in order, few
+  // One class of at most FX_FAST_OUTS outputs of 32-bit or 16-bit elements, tasks numbered in order, few
   // enough pointers and scalars: the region fits the lean
   // dense kernel's argument block (the kernel itself exists only for compiled programs).
   memset(&P->lean, 0, sizeof(P->lean));
@@ -2592,8 +2592,14 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
     const ClassBuild& cb = classes[0];
     bool fits = taskmap.size() == (size_t)T;
     for (size_t i = 0; fits && i < taskmap.size(); ++i) fits = taskmap[i] == (uint32_t)i;
+    // (16-bit elements of the type that the leading load has: what a loop over 16-bit tensors stores; a bfloat16 + 1 of
+    // 8192 x 4096 31.9 us in the general kernel, 25.1 in the lean one, of 300 x 301 5.3 : 4.9)
+    auto half_out = [&](const FxOut& od) {
+      return (od.dtype == FX_F16 || od.dtype == FX_BF16) && od.vt == FX_VT_F && od.lead && cb.code[od.prog_begin].dt == od.dtype;
+    };
     for (const FxOut& od : cb.outs)
-      fits = fits && od.box == 0 && ((od.dtype == FX_F32 && od.vt == FX_VT_F) || (od.dtype == FX_I32 && od.vt == FX_VT_I));
+      fits = fits && od.box == 0 &&
+             ((od.dtype == FX_F32 && od.vt == FX_VT_F) || (od.dtype == FX_I32 && od.vt == FX_VT_I) || half_out(od));
     if (fits) {
       FxLeanArgs& f = P->lean;
       f.blob_words = (uint32_t)blob.size();
@@ -2612,7 +2618,7 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
         const FxOut& od = cb.outs[o];
         FxLeanOut& lo = f.out[o];
         lo.ptr_slot = od.ptr_slot;
-        lo.lead = od.lead;
+        lo.lead = (od.lead ? FX_LEAN_LEAD : 0u) | (half_out(od) ? FX_LEAN_HALF : 0u);
         lo.block_begin = od.block_begin;
         lo.task_stride = od.task_stride;
         lo.unit_items = od.unit_items;

@@ -379,7 +379,8 @@ struct FxSpec {
 // program it is still tens of kilobytes of code that a workgroup jumps through: on a small
 // region the kernel's time is the start of its workgroups (argument segment, descriptor
 // staging, instruction fetch), not the data.  Regions of one task class with one or two
-// outputs of 32-bit elements (FxLeanArgs, decided at plan time) run this
+// outputs of 32-bit elements, or of the 16-bit elements that the output's leading load has
+// (FxLeanArgs, decided at plan time), run this
 // kernel instead: unit, output record, leading load and pointers come from a short argument
 // block through scalar loads, the leading loads of the unit are issued first, and the
 // descriptor is staged into LDS behind them, and only if a program of the region reads it
@@ -401,7 +402,11 @@ __device__ __forceinline__ void fx_lean_out(const FX_AS4 uint32_t* od, const uin
   constexpr FxSpecEntry en = P::entries[E];
   static_assert(en.kind == 0, "dense regions have output programs only");
   constexpr FxInsn LI = P::code[en.begin > 0 ? en.begin - 1 : 0];   // the leading load, if the output has one
-  const bool lead = en.begin > 0 && LI.op == FX_LDA && od[FX_W(FxLeanOut, lead)] != 0;
+  const uint32_t lead_word = od[FX_W(FxLeanOut, lead)];
+  const bool lead = en.begin > 0 && LI.op == FX_LDA && (lead_word & FX_LEAN_LEAD) != 0;
+  // 16-bit outputs are those of the leading load's type (FX_LEAN_HALF): a region that loads no 16-bit elements has none
+  constexpr bool halves = en.begin > 0 && LI.op == FX_LDA && (LI.dt == FX_F16 || LI.dt == FX_BF16);
+  const uint32_t odt = halves && (lead_word & FX_LEAN_HALF) ? (uint32_t)LI.dt : (uint32_t)FX_F32;
   // a buffer that does not change with the task was resolved by the host; else its slot is looked up
   auto arg_ptr = [&](uint32_t word, uint32_t slot) -> uint64_t {
     if (slot & FX_SLOT_TASK) return gp[tp_off + (slot & 0xffffu)];
@@ -476,7 +481,42 @@ __device__ __forceinline__ void fx_lean_out(const FX_AS4 uint32_t* od, const uin
   };
 
   uint32_t A[FX_K][FX_V];
-  if (have && lead) {
+  bool batch = halves && have && lead && kmax == FX_K && inner >= FX_V && !rowseg;
+  if (batch) {
+    int32_t cfv = ld.cf[0];
+#pragma unroll
+    for (int k = 1; k < R; ++k) cfv = vd == (uint32_t)k ? ld.cf[k] : cfv;
+    batch = cfv == 1;
+  }
+  if (batch) {
+    // FX_K items of 16-bit elements along rows of at least FX_V: their loads without a branch between them (an item without
+    // a live lane loads the buffer's first elements), the conversions behind all of them.  A group at the end of a row that
+    // holds fewer than FX_V elements loads the row's last FX_V: its own sit `gone` places too high.  The bound is memory:
+    // a bfloat16 + 1 of 8192 x 4096 25.1 us (fx_region_dense 31.9, with a branch and a conversion behind each load 31.7; a
+    // copy of its 134 MB takes 23), of 4096 x 4095 13.4 (21.3), of 1000 x 4000, one item a wave, 7.0 (13.4).
+    static_assert(FX_K == 4 && FX_V == 4, "four loads of 64 bits");
+    uint64_t raw[FX_K];
+    uint32_t gone[FX_K];
+#pragma unroll
+    for (uint32_t k = 0; k < FX_K; ++k) {
+      uint32_t e[FX_V], M;
+      FxCoord<R> q;
+      make_item(k, e, M, q);
+      int32_t off[FX_V];
+      fx_offsets<R>(q, ld.cf, ld.base, off);
+      gone[k] = M ? (uint32_t)__builtin_clz(M) - (32u - FX_V) : 0u;   // (M: the low bits, as many as the group has elements)
+      raw[k] = __builtin_bit_cast(uint64_t, *(const FX_AS1 fx_u16x4_a2*)((const FX_AS1 uint8_t*)ld.p +
+                                                                         ((M ? (uint32_t)off[0] - gone[k] : 0u) << 1)));
+    }
+    asm volatile("" : "+v"(raw[0]), "+v"(raw[1]), "+v"(raw[2]), "+v"(raw[3]));
+#pragma unroll
+    for (uint32_t k = 0; k < FX_K; ++k) {
+      const fx_u16x4_a2 v = __builtin_bit_cast(fx_u16x4_a2, raw[k] >> (16u * gone[k]));
+#pragma unroll
+      for (int j = 0; j < FX_V; ++j)
+        A[k][j] = LI.dt == FX_F16 ? f2u(__half2float(__ushort_as_half(v[j]))) : (uint32_t)v[j] << 16;
+    }
+  } else if (have && lead) {
 #pragma unroll
     for (uint32_t k = 0; k < FX_K; ++k) {
       if (k < kmax && item0 + k < n_items) {
@@ -499,7 +539,7 @@ __device__ __forceinline__ void fx_lean_out(const FX_AS4 uint32_t* od, const uin
         FxCoord<R> q;
         make_item(k, e, M, q);
         fx_spec_pure<P, en.begin, en.end, FX_V>(A[k]);
-        fx_store_vec(op, obase, e, M, true, FX_F32, FX_VT_F, A[k]);
+        fx_store_vec(op, obase, e, M, true, odt, FX_VT_F, A[k]);
       }
     }
   } else {
@@ -522,7 +562,7 @@ __device__ __forceinline__ void fx_lean_out(const FX_AS4 uint32_t* od, const uin
         fx_regs_init(rg);
         FxRegTemps<P::n_temps, fx_spec_n_insn<P>()> ts;
         fx_spec_range<P, R, en.begin, en.end>(cx, q, ts, M, B, rg);
-        fx_store_vec(op, obase, e, M, true, FX_F32, FX_VT_F, B);
+        fx_store_vec(op, obase, e, M, true, odt, FX_VT_F, B);
       }
     }
   }
