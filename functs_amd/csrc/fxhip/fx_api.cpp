@@ -53,7 +53,7 @@ uint32_t fx_cmap_chunk_rows();
 int fx_launch_lstm_stack(const FxLstmArgs& a, int L, uint32_t* words_ctl, uint32_t* die_ctl, hipStream_t stream);
 int fx_launch_sort_nms(const fx_nms_desc& d, uint32_t key_cap, void* workspace, uint32_t* err_host, hipStream_t stream);
 size_t fx_nms_pairs_ws_bytes(int n_tasks, uint32_t rows);
-int fx_launch_nms_pairs(const fx_nms_desc& d, hipStream_t stream);
+int fx_launch_nms_pairs(const fx_nms_desc& d, uint32_t spin_limit, hipStream_t stream);
 size_t fx_nms_workspace_bytes(int n_tasks, uint32_t key_cap);
 size_t fx_nms_workspace_clear_bytes(int n_tasks);
 hipError_t fx_launch_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* cols, void* const* outs,
@@ -1711,7 +1711,7 @@ int fx_nms_pairs(const fx_nms_desc* desc, void* stream_) {
   if (need == 0) return fail(FX_E_LIMIT, "fx_nms_pairs: rows must be 1.." + std::to_string(FX_NMS_PAIRS_MAX_ROWS));
   if (!d.workspace || ((uintptr_t)d.workspace & 255u) != 0 || d.workspace_bytes < need)
     return fail(FX_E_INVALID, "fx_nms_pairs: workspace must be 256-byte aligned and hold fx_nms_pairs_workspace_bytes()");
-  const int rc = fx_launch_nms_pairs(d, (hipStream_t)stream_);
+  const int rc = fx_launch_nms_pairs(d, g_stream_spin.load(std::memory_order_relaxed), (hipStream_t)stream_);
   if (rc != 0) return fail(FX_E_HIP, std::string("fx_nms_pairs: ") + hipGetErrorString((hipError_t)(rc - 100)));
   g_launches.fetch_add(3, std::memory_order_relaxed);
   g_spec_launches.fetch_add(3, std::memory_order_relaxed);

@@ -8,14 +8,25 @@
 //      writes their moved boxes, areas and indices to their places in score order;
 //   2. fx_nms_pairs_kernel   a wave per 64 x 32 pairs: one word per box with its overlaps among 32 boxes
 //      ahead of it in score order;
-//   3. fx_nms_walk_kernel    a workgroup per task takes 64 boxes at a time in score order.  Which of a
-//      chunk's boxes are overlapped by boxes kept before is, per earlier chunk, "word of the box and
-//      kept boxes of that chunk": fifteen waves do that for the next chunk, as far as the kept boxes
-//      are known, while the first wave adds the chunk just before its own and resolves it in rounds of
-//      ballots.  The words come straight to registers, several chunks ahead.
-// 2 000 boxes, 260 kept: rank 5.5, pairs 5.6, walk 21 us (0.5 us a chunk: barrier, the far boxes' bits out of
-// LDS, two rounds, barrier), the call 157 -> 47 us.  Results are those of fx_sort_nms bit for bit: the same keys,
-// the same overlap decisions, the same order of decisions.
+//   3. up to 16 chunks of 64 boxes, and where few are to be kept, fx_nms_walk_kernel: a workgroup per task
+//      takes a chunk at a time in score order.  Which of a chunk's boxes are overlapped by boxes kept before is, per earlier chunk,
+//      "word of the box and kept boxes of that chunk": fifteen waves do that for the next chunk, as far as
+//      the kept boxes are known, while the first wave adds the chunk just before its own and resolves it in
+//      rounds of ballots.  The words come straight to registers, several chunks ahead.
+//      Otherwise fx_nms_resolve_kernel, a workgroup per chunk.  A box is dead when a kept box ahead of it
+//      overlaps it, and kept when every overlapping box ahead of it is dead; chunks publish what they have
+//      decided as soon as they have, and look at what the chunks ahead have published, so the chunks are
+//      resolved side by side: the wait is for as many exchanges as a chain of overlaps has links, at most
+//      one a chunk, not for every chunk in turn.
+// Microseconds of the three launches back to back, walk : resolve, one image (2 000 boxes: rank 5.6, pairs 5.4, walk
+// 21 or resolve 10): 2 000 proposals of 60 objects 31.6 : 27.1, dense crowd 26.4 : 23.8, apart from each other
+// 24.2 : 17.3, each overlapping the next 23.3 : 17.1; 4 096: 73 : 44, 40 : 38, 37 : 30, 36 : 30; 8 images of 2 000:
+// 53 : 51, 47 : 47, 45 : 39, 44 : 39.  What is left of resolve is its exchanges, some 1.1 us each: a store's way to
+// the other dies, half a look, the words through LDS.  At 1 000 boxes the two are level (19.6 : 19.7), at 500 the
+// walk is faster (15.1 : 16.3); where max_num is reached early the walk ends early (crowd of 2 000, 300 kept of the
+// first 450: 17.1 : 19.0), hence the rule on max_num.  Call of 2 000 boxes, 260 kept: 46.5 -> 37.5 us.
+// Results are those of fx_sort_nms bit for bit: the same keys, the same overlap decisions, and the one result
+// that decisions in score order have.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -28,17 +39,19 @@ namespace {
 
 // Workspace of a task: [np] moved boxes, [np] areas, [np] rows, 64 words (the first: how many are
 // candidates), [nw][np] 64-bit words of overlaps (of box j among the boxes of chunk c, c <= j / 64; the
-// boxes of a chunk lie side by side); np = n rounded up to 64, nw = np / 64.
+// boxes of a chunk lie side by side), [64] pairs of 64-bit words (the boxes of a chunk that are kept, those that
+// are dead, as far as they are decided); np = n rounded up to 64, nw = np / 64.
 struct PairsWs {
   float4* box;
   float* area;
   uint32_t* row;
   uint32_t* count;
   uint64_t* over;
+  uint64_t* state;
 };
 __host__ __device__ inline size_t pairs_ws_bytes(uint32_t n) {
   const size_t np = (n + 63u) & ~63u;
-  return np * 24u + 256u + np * (np / 64u) * 8u;
+  return np * 24u + 256u + 1024u + np * (np / 64u) * 8u;
 }
 __device__ __forceinline__ PairsWs pairs_ws(void* ws, uint32_t n, uint32_t task) {
   const uint32_t np = (n + 63u) & ~63u;
@@ -49,6 +62,7 @@ __device__ __forceinline__ PairsWs pairs_ws(void* ws, uint32_t n, uint32_t task)
   w.area = (float*)((uint8_t*)w.over + (size_t)np * (np / 64u) * 8u);
   w.row = (uint32_t*)(w.area + np);
   w.count = w.row + np;
+  w.state = (uint64_t*)(w.count + 64u);
   return w;
 }
 
@@ -128,6 +142,20 @@ __global__ __launch_bounds__(256) void fx_nms_pairs_kernel(const fx_nms_desc d) 
   const uint32_t n = d.rows, nw = (n + 63u) >> 6;
   const uint32_t chunk = blockIdx.y, col = blockIdx.x * 4u + wave;
   const PairsWs ws = pairs_ws(d.workspace, n, blockIdx.z);
+  {
+    // the results start out as zeros (rows past the kept ones stay so: the outputs have a fixed shape), the
+    // chunks as undecided; the next launch is the first to touch either
+    const uint32_t at = (chunk * gridDim.x + blockIdx.x) * 256u + threadIdx.x, step = gridDim.x * gridDim.y * 256u;
+    float* dets = d.dets + (size_t)blockIdx.z * d.max_num * 5u;
+    int64_t* out_labels = d.out_labels + (size_t)blockIdx.z * d.max_num;
+    int64_t* out_index = d.out_index ? d.out_index + (size_t)blockIdx.z * d.max_num : nullptr;
+    for (uint32_t k = at; k < d.max_num * 5u; k += step) dets[k] = 0.0f;
+    for (uint32_t k = at; k < d.max_num; k += step) {
+      out_labels[k] = 0;
+      if (out_index) out_index[k] = 0;
+    }
+    if (at < 128u) ws.state[at] = 0ull;
+  }
   if (col > 2u * chunk + 1u) return;   // (waves share nothing)
   // every row has a box, those behind the candidates too: nothing waits for their number
   const uint32_t i = chunk * 64u + lane, j0 = col * 32u;
@@ -259,16 +287,201 @@ __global__ __launch_bounds__(FX_PAIRS_THREADS) void fx_nms_walk_kernel(const fx_
   float* dets = d.dets + (size_t)task * d.max_num * 5u;
   int64_t* out_labels = d.out_labels + (size_t)task * d.max_num;
   int64_t* out_index = d.out_index ? d.out_index + (size_t)task * d.max_num : nullptr;
-  for (uint32_t k = tid; k < d.max_num; k += FX_PAIRS_THREADS) {   // rows past the kept ones are zero: the outputs have a fixed shape
-    const bool live = k < nk;
-    const uint32_t i = live ? ws.row[s_kept[live ? k : 0u]] : 0u;
-    const float4 b = live ? *(const float4*)(boxes + (size_t)i * 4u) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (uint32_t k = tid; k < nk; k += FX_PAIRS_THREADS) {   // (nk <= max_num; rows past the kept ones are zero already)
+    const uint32_t i = ws.row[s_kept[k]];
+    const float4 b = *(const float4*)(boxes + (size_t)i * 4u);
     float* o = dets + (size_t)k * 5u;
     o[0] = b.x; o[1] = b.y; o[2] = b.z; o[3] = b.w;
-    o[4] = live ? scores[i] : 0.0f;
-    out_labels[k] = live && labels ? (int64_t)(uint32_t)labels[i] : 0;
-    if (out_index) out_index[k] = live ? (int64_t)i : 0;
+    o[4] = scores[i];
+    out_labels[k] = labels ? (int64_t)(uint32_t)labels[i] : 0;
+    if (out_index) out_index[k] = (int64_t)i;
   }
+}
+
+__device__ __forceinline__ uint64_t uni64(uint64_t v) { return ((uint64_t)uni((uint32_t)(v >> 32)) << 32) | (uint64_t)uni((uint32_t)v); }
+
+// The boxes of a chunk that can be decided, round after round: one with a kept overlapping predecessor (`in`:
+// those in the chunk) is dead, one whose overlapping predecessors are all dead and that waits for none outside
+// the chunk is kept.
+__device__ __forceinline__ void resolve_chunk(uint64_t in, uint64_t waits, uint32_t lane, uint64_t& kept, uint64_t& dead) {
+  for (;;) {
+    const bool open = (((kept | dead) >> lane) & 1ull) == 0ull;
+    const bool is_dead = open && (in & kept) != 0ull;
+    const bool is_kept = open && !is_dead && ((waits >> lane) & 1ull) == 0ull && (in & ~dead) == 0ull;
+    const uint64_t nd = __ballot(is_dead), nk = __ballot(is_kept);
+    if ((nd | nk) == 0ull) return;
+    dead |= nd;
+    kept |= nk;
+  }
+}
+
+// Wave 0 decides the chunk's boxes; waves 1 .. 15 hold the words of the chunk's boxes among the chunks ahead,
+// W each, look at the state of those and tell wave 0 which boxes are dead for it (s_dead) and which still wait
+// (s_wait).  A wave writes the former before the latter and wave 0 reads them the other way round: LDS serves a
+// wave's accesses in order, so a box that waits no more is known to be dead if it is.
+// A workgroup waits for workgroups of lower number only.  All waits are bounded: one that is given up after
+// spin_limit looks makes wave 0 resolve the chunks from the first on by itself, from the words alone.
+// max_num boxes kept ahead of a chunk end it: none of its boxes would be among the results, whatever it is that the
+// boxes of the chunks ahead still wait for.
+#define FX_GAVE_UP 1u
+#define FX_FULL 2u
+template <uint32_t W>
+__global__ __launch_bounds__(FX_PAIRS_THREADS) void fx_nms_resolve_kernel(const fx_nms_desc d, const uint32_t spin_limit) {
+  __shared__ uint64_t s_keep[64];   // kept boxes of the chunks up to this one
+  __shared__ uint64_t s_wait[16];
+  __shared__ uint32_t s_dead[2];
+  __shared__ uint32_t s_ahead[16];   // boxes that a wave has seen kept
+  __shared__ uint32_t s_stop;        // FX_GAVE_UP, FX_FULL
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uni(tid >> 6);
+  const uint32_t n = d.rows, nw = (n + 63u) >> 6, np = nw * 64u, task = blockIdx.x / nw, c = blockIdx.x - task * nw;
+  const PairsWs ws = pairs_ws(d.workspace, n, task);
+  // asked for together: how many are candidates, the words (written for every row), the rows of this chunk
+  const uint32_t mine = c * 64u + (tid >> 4), part = tid & 15u;
+  const uint32_t n_cand = *ws.count, row = ws.row[min(mine, n - 1u)];
+  uint64_t word[W];
+#pragma unroll
+  for (uint32_t k = 0; k < W; ++k) {
+    const uint32_t l = wave == 0u ? c : wave - 1u + 15u * k;
+    word[k] = (wave == 0u ? k == 0u : l < c) ? ws.over[(size_t)l * np + c * 64u + lane] : 0ull;
+  }
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  const uint32_t count = uni(n_cand), chunks = (count + 63u) >> 6;
+  if (c >= chunks) {
+    // (system scope: a count in pinned host memory goes through to the host, which may be polling it)
+    if (count == 0u && c == 0u && tid == 0u) __hip_atomic_store(d.n_out + task, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  // what the rows of this chunk will hold, sixteen threads a box, asked for ahead of the wait
+  uint32_t label = 0u;
+  float value = 0.0f;
+  if (mine < count) {
+    if (part < 4u) value = d.boxes[(int64_t)task * d.boxes_task_stride + (size_t)row * 4u + part];
+    if (part == 4u) value = d.scores[(int64_t)task * d.scores_task_stride + row];
+    if (part == 5u && d.labels) label = (uint32_t)d.labels[(int64_t)task * d.labels_task_stride + row];
+  }
+  if (tid < 16u) s_wait[tid] = tid != 0u && tid - 1u < c ? ~0ull : 0ull;
+  if (tid < 2u) s_dead[tid] = 0u;
+  if (tid < 16u) s_ahead[tid] = 0u;
+  if (tid == 0u) s_stop = 0u;
+  __syncthreads();
+  uint64_t* state = ws.state;
+  if (wave == 0u) {
+    __builtin_amdgcn_s_setprio(3);   // what this wave decides is what others wait for
+    const uint64_t in = word[0] & ((1ull << lane) - 1ull);
+    const uint32_t m = min(64u, count - c * 64u);
+    uint64_t kept = 0ull, dead = m >= 64u ? 0ull : ~((1ull << m) - 1ull);
+    for (;;) {
+      uint64_t w = __hip_atomic_load(&s_wait[lane & 15u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      const uint32_t d0 = __hip_atomic_load(&s_dead[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const uint32_t d1 = __hip_atomic_load(&s_dead[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      uint32_t ahead = __hip_atomic_load(&s_ahead[lane & 15u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (uni(__hip_atomic_load(&s_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != 0u) break;
+      ahead += fx_lane_xor<1u>(ahead, lane);
+      ahead += fx_lane_xor<2u>(ahead, lane);
+      ahead += fx_lane_xor<4u>(ahead, lane);
+      ahead += fx_lane_xor<8u>(ahead, lane);
+      if (uni(ahead) >= d.max_num) {
+        if (lane == 0u) __hip_atomic_store(&s_stop, FX_FULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        break;
+      }
+      uint32_t w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32);
+      w0 |= fx_lane_xor<1u>(w0, lane); w1 |= fx_lane_xor<1u>(w1, lane);
+      w0 |= fx_lane_xor<2u>(w0, lane); w1 |= fx_lane_xor<2u>(w1, lane);
+      w0 |= fx_lane_xor<4u>(w0, lane); w1 |= fx_lane_xor<4u>(w1, lane);
+      w0 |= fx_lane_xor<8u>(w0, lane); w1 |= fx_lane_xor<8u>(w1, lane);
+      const uint64_t waits = ((uint64_t)uni(w1) << 32) | (uint64_t)uni(w0), was = kept | dead;
+      dead |= (((uint64_t)uni(d1) << 32) | (uint64_t)uni(d0)) & ~kept;
+      resolve_chunk(in, waits, lane, kept, dead);
+      if ((kept | dead) != was && lane < 2u)
+        __hip_atomic_store(state + 2u * c + lane, lane == 0u ? kept : dead, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (~(kept | dead) == 0ull) break;
+    }
+    if (lane == 0u) s_keep[c] = kept;
+  } else {
+    uint32_t open = 0u;   // chunks of this wave that are not decided to the last box
+#pragma unroll
+    for (uint32_t k = 0; k < W; ++k) open |= wave - 1u + 15u * k < c ? 1u << k : 0u;
+    uint64_t waited = ~0ull;
+    uint32_t closed_kept = 0u, counted = 0u;
+    bool dead = false;
+    for (uint32_t polls = 0; open != 0u; ++polls) {
+      if (uni(__hip_atomic_load(&s_stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != 0u) break;
+      if (polls >= spin_limit) {
+        if (lane == 0u) __hip_atomic_store(&s_stop, FX_GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        break;
+      }
+      uint64_t kept[W], gone[W];
+#pragma unroll
+      for (uint32_t k = 0; k < W; ++k) {
+        const uint64_t* at = state + 2u * ((open >> k) & 1u ? wave - 1u + 15u * k : 0u);
+        kept[k] = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        gone[k] = __hip_atomic_load(at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      bool waits = false;
+      uint32_t seen = closed_kept;
+#pragma unroll
+      for (uint32_t k = 0; k < W; ++k) {
+        if (((open >> k) & 1u) == 0u) continue;
+        // (what one lane has seen: were some to see an earlier state than the one that closes the chunk, they would not look again)
+        kept[k] = uni64(kept[k]);
+        gone[k] = uni64(gone[k]);
+        dead = dead || (word[k] & kept[k]) != 0ull;
+        waits = waits || (word[k] & ~(kept[k] | gone[k])) != 0ull;
+        seen += (uint32_t)__popcll(kept[k]);
+        if (~(kept[k] | gone[k]) == 0ull) {
+          open &= ~(1u << k);
+          closed_kept += (uint32_t)__popcll(kept[k]);
+          if (lane == 0u) s_keep[wave - 1u + 15u * k] = kept[k];
+        }
+      }
+      if (seen != counted) {
+        counted = seen;
+        if (lane == 0u) __hip_atomic_store(&s_ahead[wave], seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      const uint64_t now = __ballot(waits && !dead);
+      if (now != waited) {
+        waited = now;
+        const uint64_t x = __ballot(dead);
+        if (lane < 2u) __hip_atomic_fetch_or(&s_dead[lane], (uint32_t)(x >> (32u * lane)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if (lane == 0u) __hip_atomic_store(&s_wait[wave], now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t stop = uni(s_stop);
+  if (stop == FX_FULL) {
+    // (the other boxes of this chunk are no results either way: nobody is to wait for them)
+    if (tid == 0u) __hip_atomic_store(state + 2u * c + 1u, ~0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (c + 1u == chunks && tid == 0u) __hip_atomic_store(d.n_out + task, d.max_num, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  if (stop == FX_GAVE_UP) {
+    if (wave == 0u) {
+      for (uint32_t e = 0; e <= c; ++e) {
+        uint64_t over = 0ull;
+        for (uint32_t l = 0; l < e; ++l) over |= ws.over[(size_t)l * np + e * 64u + lane] & s_keep[l];
+        const uint32_t m = min(64u, count - e * 64u);
+        uint64_t kept = 0ull, dead = __ballot(over != 0ull) | (m >= 64u ? 0ull : ~((1ull << m) - 1ull));
+        resolve_chunk(ws.over[(size_t)e * np + e * 64u + lane] & ((1ull << lane) - 1ull), 0ull, lane, kept, dead);
+        if (lane == 0u) s_keep[e] = kept;
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if (e == c && lane < 2u)
+          __hip_atomic_store(state + 2u * c + lane, lane == 0u ? kept : ~kept, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __syncthreads();
+  }
+  const uint64_t keep = uni64(s_keep[c]);
+  const uint32_t ahead = uni(fx_wave_sum(lane < c ? (uint32_t)__popcll(s_keep[lane]) : 0u, lane));
+  if (c + 1u == chunks && tid == 0u)
+    __hip_atomic_store(d.n_out + task, min(ahead + (uint32_t)__popcll(keep), d.max_num), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  const uint32_t box = tid >> 4, at = ahead + (uint32_t)__popcll(keep & ((1ull << box) - 1ull));
+  if (((keep >> box) & 1ull) == 0ull || at >= d.max_num) return;
+  if (part < 5u) d.dets[((size_t)task * d.max_num + at) * 5u + part] = value;
+  if (part == 5u) d.out_labels[(size_t)task * d.max_num + at] = (int64_t)label;
+  if (part == 6u && d.out_index) d.out_index[(size_t)task * d.max_num + at] = (int64_t)row;
 }
 
 }  // namespace
@@ -276,12 +489,18 @@ __global__ __launch_bounds__(FX_PAIRS_THREADS) void fx_nms_walk_kernel(const fx_
 size_t fx_nms_pairs_ws_bytes(int n_tasks, uint32_t rows) { return (size_t)n_tasks * pairs_ws_bytes(rows); }
 
 // d: mode 0 without counts, 1 .. FX_NMS_PAIRS_MAX_ROWS rows; 0: launched; otherwise a HIP error code + 100
-int fx_launch_nms_pairs(const fx_nms_desc& d, hipStream_t stream) {
+int fx_launch_nms_pairs(const fx_nms_desc& d, uint32_t spin_limit, hipStream_t stream) {
   const uint32_t nw = (d.rows + 63u) / 64u;
   hipLaunchKernelGGL(fx_nms_rank_kernel, dim3((uint32_t)d.n_tasks * 4u * nw), dim3(FX_PAIRS_THREADS), (size_t)nw * 64u * 8u, stream, d);
   hipLaunchKernelGGL(fx_nms_pairs_kernel, dim3((2u * nw + 3u) / 4u, nw, (uint32_t)d.n_tasks), dim3(256), 0, stream, d);
-  auto* walk = nw <= 31u ? fx_nms_walk_kernel<2> : nw <= 46u ? fx_nms_walk_kernel<3> : fx_nms_walk_kernel<5>;
-  hipLaunchKernelGGL(walk, dim3((uint32_t)d.n_tasks), dim3(FX_PAIRS_THREADS), 0, stream, d);
+  // level at 16 chunks, and ahead of each other on either side of it; with few to be kept the walk may end early (top)
+  if (nw > 16u && (uint64_t)d.max_num * 4u >= d.rows) {
+    auto* resolve = nw <= 31u ? fx_nms_resolve_kernel<2> : nw <= 46u ? fx_nms_resolve_kernel<3> : fx_nms_resolve_kernel<5>;
+    hipLaunchKernelGGL(resolve, dim3((uint32_t)d.n_tasks * nw), dim3(FX_PAIRS_THREADS), 0, stream, d, spin_limit);
+  } else {
+    auto* walk = nw <= 31u ? fx_nms_walk_kernel<2> : nw <= 46u ? fx_nms_walk_kernel<3> : fx_nms_walk_kernel<5>;
+    hipLaunchKernelGGL(walk, dim3((uint32_t)d.n_tasks), dim3(FX_PAIRS_THREADS), 0, stream, d);
+  }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : 100 + (int)e;
 }
