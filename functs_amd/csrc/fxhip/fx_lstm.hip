@@ -1196,8 +1196,10 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     if (e != hipSuccess) return 100 + (int)e;
     if ((long)fit.per_cu * cus < f[i].grid) continue;
     const uint32_t want = fx_lstm_need((uint32_t)f[i].grid, (uint32_t)fit.sure);
-    // (a sequence on one die holds every die: not where a stack on another stream would have to wait for it)
-    if (f[i].over == LSTM_DIE && !capturing && want + groups.beside(id, thread) > device) continue;
+    // A sequence on one die holds every die: not one that needs more than half of it where a stack on another stream
+    // would have to wait for it.  One that needs no more is taken in every case, so that what a captured launch computes is, to
+    // the bit, what the calls beside it compute.
+    if (f[i].over == LSTM_DIE && 2u * want > (uint32_t)cus * FX_LSTM_CU && (capturing || want > device || groups.others(id, thread))) continue;
     if (l && want >= need) continue;
     l = &f[i];
     need = want;

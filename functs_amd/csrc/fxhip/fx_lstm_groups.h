@@ -22,6 +22,7 @@
 #pragma once
 #include <stdint.h>
 
+#include <initializer_list>
 #include <vector>
 
 #define FX_LSTM_CU 64u
@@ -70,14 +71,14 @@ struct FxLstmGroups {
     now.push_back(Member{stream, thread, need, nullptr, late});
     return now.back();
   }
-  // What other streams' launches of the group need that have launched lately: a launch that does not fit beside
-  // them makes the streams take turns, and takes another form instead where it has one.  (Counted in launches
-  // and not asked of the device: queries are not allowed beside a capture.)
-  uint32_t beside(uint64_t stream, uint64_t thread) const {
-    uint32_t total = 0;
-    for (const Member& m : now)
-      if (!same(m, stream, thread) && launches - m.last < 64u) total += m.need;
-    return total;
+  // Whether other streams than this one have launched lately: a form that holds more than half of the device
+  // would make the streams take turns.  (Counted in launches and not asked of the device: queries are not allowed
+  // beside a capture.)
+  bool others(uint64_t stream, uint64_t thread) const {
+    for (const std::vector<Member>* group : {&now, &before})
+      for (const Member& m : *group)
+        if (!same(m, stream, thread) && launches - m.last < 64u) return true;
+    return false;
   }
   void* event_to_use() {
     if (spare.empty()) return nullptr;

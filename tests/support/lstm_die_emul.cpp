@@ -155,14 +155,11 @@ extern "C" int fx_lstm_die_emul(const float* x, const float* wih, const float* w
   return 0;
 }
 
-// needs of the launches that streams 0, 1, 2 ... have made (one each, in that order, then `more` of stream 0),
-// as stream 0 sees them beside its own
-extern "C" uint32_t fx_lstm_beside_emul(const uint32_t* needs, int n, int more) {
+// Streams 0 .. n - 1 launch once each, in that order, then stream 0 `more` times, in groups that hold `device`: have
+// others than `stream` launched lately?
+extern "C" int fx_lstm_others_emul(int n, int more, uint32_t need, uint32_t device, int stream) {
   FxLstmGroups g;
   bool joins;
-  for (int s = 0; s < n + more; ++s) {
-    const uint64_t stream = s < n ? (uint64_t)s : 0u;
-    g.admit(stream, 0u, needs[stream], 0xffffffffu, true, &joins).last = ++g.launches;
-  }
-  return g.beside(0u, 0u);
+  for (int s = 0; s < n + more; ++s) g.admit(s < n ? (uint64_t)s : 0u, 0u, need, device, true, &joins).last = ++g.launches;
+  return g.others((uint64_t)stream, 0u) ? 1 : 0;
 }

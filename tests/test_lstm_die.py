@@ -18,7 +18,7 @@ def emul(tmp_path_factory):
     subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-pthread", src, "-o", so])
     lib = ctypes.CDLL(so)
     lib.fx_lstm_die_emul.argtypes = [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.c_uint32, ctypes.c_int, ctypes.c_uint32, ctypes.c_int, ctypes.c_int]
-    lib.fx_lstm_beside_emul.restype = ctypes.c_uint32
+    lib.fx_lstm_others_emul.argtypes = [ctypes.c_int] * 2 + [ctypes.c_uint32] * 2 + [ctypes.c_int]
     return lib
 
 
@@ -56,12 +56,35 @@ def test_tags_start_over_before_they_wrap(emul):
     _close(got, _reference(*args), "after the tags were cleared")
 
 
-def test_streams_that_launched_lately_are_counted(emul):
-    needs = (ctypes.c_uint32 * 3)(10, 20, 30)
-    assert emul.fx_lstm_beside_emul(needs, 3, 0) == 50
-    assert emul.fx_lstm_beside_emul(needs, 3, 63) == 30    # stream 1 launched 64 launches ago
-    assert emul.fx_lstm_beside_emul(needs, 3, 64) == 0
-    assert emul.fx_lstm_beside_emul(needs, 1, 5) == 0
+def test_streams_that_launched_lately_are_told_apart(emul):
+    others = emul.fx_lstm_others_emul
+    for device in (1 << 20, 64):      # launches that overlap, launches that take turns
+        assert others(1, 5, 64, device, 0) == 0
+        assert others(2, 0, 64, device, 0) == others(2, 62, 64, device, 0) == 1
+        assert others(2, 64, 64, device, 0) == 0    # stream 1 launched 64 launches ago
+        assert others(1, 5, 64, device, 7) == 1     # a second stream's first launch
+
+
+@pytest.mark.gpu
+def test_a_captured_stack_computes_what_the_calls_beside_it_compute():
+    """To the bit, whether or not another stream has launched stacks lately."""
+    from functs_amd import jit as fj
+    from functs_amd.benchmark import PROGRAMS
+    from oracle import configs as oc
+    args = oc.c4_inputs(3, 9, 64, 2, 1)
+    gpu = [a.cuda() if isinstance(a, torch.Tensor) else a for a in args]
+    eager = fj.build(fj.script(PROGRAMS["c4"]), list(args))
+    for other in (False, True):
+        if other:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                eager(*gpu)
+            torch.cuda.synchronize()
+        graphed = fj.build(fj.script(PROGRAMS["c4"]), list(args), hip_graph=True)
+        for _ in range(3):
+            want = eager(*gpu)
+            torch.cuda.synchronize()
+            for g, w in zip(graphed(*gpu), want):
+                assert torch.equal(g, w), "after launches on another stream: %s" % other
 
 
 # every width and depth of a stage, one to eight sequences, rings that go round, shorter sequences than the lag
