@@ -205,6 +205,8 @@ _sig("fx_attention_steps_fits", ctypes.c_int, _i, _i)
 _sig("fx_attention_steps", _i, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _i, _i, _i, _i, _i, _i, ctypes.c_float, ctypes.c_float,
      ctypes.c_float, _vp)
 _sig("fx_set_lstm_spin_limit", None, ctypes.c_uint32)
+_sig("fx_set_lstm_form", ctypes.c_int, ctypes.c_int)
+_sig("fx_lstm_form", ctypes.c_int)
 _sig("fx_set_totals_spin_us", None, ctypes.c_uint32)
 _sig("fx_device_count", _i)
 _sig("fx_copy_bytes", _i, _vp, _vp, ctypes.c_size_t, _vp)

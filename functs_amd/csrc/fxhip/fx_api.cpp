@@ -51,6 +51,8 @@ uint32_t fx_cmap_chunk_rows();
 #include "fx_attn.h"
 #include "fx_lstm_sched.h"
 int fx_launch_lstm_stack(const FxLstmArgs& a, int L, uint32_t* words_ctl, uint32_t* die_ctl, hipStream_t stream);
+int fx_lstm_ask(int form);
+int fx_lstm_taken();
 int fx_launch_sort_nms(const fx_nms_desc& d, uint32_t key_cap, void* workspace, uint32_t* err_host, hipStream_t stream);
 size_t fx_nms_pairs_ws_bytes(int n_tasks, uint32_t rows);
 int fx_launch_nms_pairs(const fx_nms_desc& d, uint32_t spin_limit, hipStream_t stream);
@@ -1601,7 +1603,7 @@ int fx_lstm_stack(const float* x, const float* wih, const float* whh, const floa
   uint32_t* words_ctl = (uint32_t*)((char*)workspace + lstm_area_bytes(batch, hidden, layers));
   uint32_t* die_ctl = fx_lstm_die_fits(batch, hidden, layers) ? (uint32_t*)((char*)workspace + 2 * lstm_area_bytes(batch, hidden, layers)) : nullptr;
   const int rc = fx_launch_lstm_stack(a, layers, words_ctl, die_ctl, (hipStream_t)stream_);
-  if (rc == 1) return fail(FX_E_UNSUPPORTED, "fx_lstm_stack: no kernel for these sizes");
+  if (rc == 1) return fail(FX_E_UNSUPPORTED, "fx_lstm_stack: no kernel for these sizes (in the form that was asked for)");
   if (rc == 2)
     return fail(FX_E_LIMIT, "fx_lstm_stack: the workgroups for hidden " + std::to_string(hidden) + " and batch " + std::to_string(batch) + " would not be resident together on this device");
   if (rc != 0) return fail(FX_E_HIP, std::string("fx_lstm_stack: ") + hipGetErrorString((hipError_t)(rc - 100)));
@@ -1611,6 +1613,11 @@ int fx_lstm_stack(const float* x, const float* wih, const float* whh, const floa
   FX_CATCH
 }
 void fx_set_totals_spin_us(uint32_t us) { g_totals_spin_us.store(us, std::memory_order_relaxed); }
+int fx_set_lstm_form(int form) {
+  if (form < FX_LSTM_FORM_ANY || form > FX_LSTM_FORM_DIE) return fail(FX_E_INVALID, "fx_set_lstm_form: no such form");
+  return fx_lstm_ask(form);
+}
+int fx_lstm_form(void) { return fx_lstm_taken(); }
 void fx_set_lstm_spin_limit(uint32_t polls) { g_lstm_spin.store(polls, std::memory_order_relaxed); }
 
 // ---- attention over a growing cache (fx_attn.hip) ----

@@ -1115,24 +1115,32 @@ static fx_lstm_die_kernel_t pick_die(int hpt, int* threads) {
   }
 }
 enum LstmHandOver { LSTM_TAGS, LSTM_WORDS, LSTM_DIE };   // which area of the workspace
-struct LstmLaunch { const void* kernel; int grid, threads, tiles; LstmHandOver over; };   // tiles of rows a workgroup; 0: row by row
+struct LstmLaunch { const void* kernel; int grid, threads, tiles; LstmHandOver over; int form; };   // tiles of rows a workgroup; 0: row by row
 // the forms that serve these sizes, the fastest first
 template <int L>
 static int lstm_forms(const FxLstmArgs& a, LstmLaunch (&f)[4]) {
   const int hpt = a.H / 32;
   int n = 0, threads = 0;
   if (fx_lstm_die_fits(a.B, a.H, L))
-    if (fx_lstm_die_kernel_t k = pick_die<L>(hpt, &threads)) f[n++] = LstmLaunch{(const void*)k, FX_LSTM_DIES * FX_LSTM_DIE_WG, threads, 0, LSTM_DIE};
+    if (fx_lstm_die_kernel_t k = pick_die<L>(hpt, &threads)) f[n++] = LstmLaunch{(const void*)k, FX_LSTM_DIES * FX_LSTM_DIE_WG, threads, 0, LSTM_DIE, FX_LSTM_FORM_DIE};
   if (a.B > 1)
     for (int tiles = 1; tiles <= 2; ++tiles) {
       const int groups = (a.B + 4 * tiles - 1) / (4 * tiles), cells = L * tiles < 4 ? L * tiles : 4;   // FxLstmRows
-      if (fx_lstm_kernel_t k = pick_rows<L>(hpt, tiles)) f[n++] = LstmLaunch{(const void*)k, (a.H / 4) * groups, ((a.H >= 128 ? 8 : a.H / 16) + cells) * 64, tiles, LSTM_WORDS};
+      if (fx_lstm_kernel_t k = pick_rows<L>(hpt, tiles)) f[n++] = LstmLaunch{(const void*)k, (a.H / 4) * groups, ((a.H >= 128 ? 8 : a.H / 16) + cells) * 64, tiles, LSTM_WORDS, tiles == 1 ? FX_LSTM_FORM_ROWS : FX_LSTM_FORM_ROWS2};
     }
   // two hidden units per workgroup: every workgroup fetches the step's vectors from the memory
   // side once, so fewer, larger workgroups fetch less, and sixteen gate sums fill the butterfly
-  if (fx_lstm_kernel_t k = pick_serial<L>(hpt)) f[n++] = LstmLaunch{(const void*)k, a.H / FX_LSTM_UPW, FX_LSTM_BLOCK * FX_LSTM_UPW, 0, LSTM_TAGS};
+  if (fx_lstm_kernel_t k = pick_serial<L>(hpt)) f[n++] = LstmLaunch{(const void*)k, a.H / FX_LSTM_UPW, FX_LSTM_BLOCK * FX_LSTM_UPW, 0, LSTM_TAGS, FX_LSTM_FORM_SINGLE};
   return n;
 }
+
+static thread_local int t_lstm_asked = FX_LSTM_FORM_ANY, t_lstm_taken = FX_LSTM_FORM_ANY;   // fx_set_lstm_form, fx_lstm_form
+int fx_lstm_ask(int form) {
+  const int before = t_lstm_asked;
+  t_lstm_asked = form;
+  return before;
+}
+int fx_lstm_taken() { return t_lstm_taken; }
 
 static std::mutex g_lstm_mu;
 static std::map<int, FxLstmGroups> g_lstm_groups;   // by device
@@ -1187,10 +1195,12 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
   FxLstmGroups& groups = g_lstm_groups[dev];
   const LstmLaunch* l = nullptr;
   uint32_t need = 0;
+  const int asked = t_lstm_asked;
   for (int i = 0; i < n; ++i) {
+    if (asked != FX_LSTM_FORM_ANY && asked != f[i].form) continue;
     // one tile of four rows a workgroup while that makes at most one workgroup for each CU, whose registers the
     // weights fill
-    if (f[i].tiles == 1 && f[i].grid > cus) continue;
+    if (f[i].tiles == 1 && f[i].grid > cus && asked == FX_LSTM_FORM_ANY) continue;
     LstmFit fit;
     e = lstm_fit(dev, f[i], &fit);
     if (e != hipSuccess) return 100 + (int)e;
@@ -1199,13 +1209,14 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     // A sequence on one die holds every die: not one that needs more than half of it where a stack on another stream
     // would have to wait for it.  One that needs no more is taken in every case, so that what a captured launch computes is, to
     // the bit, what the calls beside it compute.
-    if (f[i].over == LSTM_DIE && 2u * want > (uint32_t)cus * FX_LSTM_CU && (capturing || want > device || groups.others(id, thread))) continue;
+    if (f[i].over == LSTM_DIE && 2u * want > (uint32_t)cus * FX_LSTM_CU && (capturing || (asked == FX_LSTM_FORM_ANY && (want > device || groups.others(id, thread))))) continue;
     if (l && want >= need) continue;
     l = &f[i];
     need = want;
     if (need <= device) break;
   }
-  if (!l) return 2;
+  if (!l) return asked == FX_LSTM_FORM_ANY ? 2 : 1;
+  t_lstm_taken = l->form;
   uint32_t* areas[3] = {a.ctl, words_ctl, die_ctl ? die_ctl : a.ctl};
   std::swap(areas[0], areas[(int)l->over]);
   a.ctl = areas[0];

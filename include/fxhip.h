@@ -457,6 +457,17 @@ int fx_lstm_stack(const float* x, const float* wih, const float* whh, const floa
                   const float* c0, float* out, float* state_h, float* state_c, int seq_len, int batch, int hidden,
                   int layers, void* workspace, size_t workspace_bytes, void* stream);
 void fx_set_lstm_spin_limit(uint32_t polls); /* barrier polls before a wait is given up (default 1000000; tests) */
+/* The forms of fx_lstm_stack, and the one that the calling thread's launches are to take (FX_LSTM_FORM_ANY, the
+ * default: the fastest that the sizes and what else may run allow).  Returns the one asked for before, or FX_E_INVALID.
+ * A form that is not built for the sizes, or that a captured launch must not take: FX_E_UNSUPPORTED from the launch.
+ * fx_lstm_form: the form of the calling thread's last launch (FX_LSTM_FORM_ANY: none yet). */
+#define FX_LSTM_FORM_ANY 0
+#define FX_LSTM_FORM_SINGLE 1 /* row by row, tagged values */
+#define FX_LSTM_FORM_ROWS 2   /* four rows a workgroup, values as words */
+#define FX_LSTM_FORM_ROWS2 3  /* eight rows a workgroup, values as words */
+#define FX_LSTM_FORM_DIE 4    /* a sequence on one die */
+int fx_set_lstm_form(int form);
+int fx_lstm_form(void);
 
 /* ---- single-query attention over a growing cache as one launch ----
  * The decoding loop of functs/benchmark/simpleops/attention/attention.py:38-58

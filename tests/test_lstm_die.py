@@ -8,7 +8,7 @@ import subprocess
 import pytest
 import torch
 
-from tests.test_lstm_kernel import _close, _gpu, _inputs, _reference
+from tests.test_lstm_kernel import _close, _gpu, _inputs, _reference, lstm_form
 
 
 @pytest.fixture(scope="module")
@@ -93,7 +93,7 @@ def test_a_captured_stack_computes_what_the_calls_beside_it_compute():
                                      (50, 256, 4, 4), (21, 256, 2, 1), (1, 512, 3, 2), (3, 512, 2, 4), (70, 512, 2, 4), (40, 512, 4, 2), (9, 512, 1, 8)])
 def test_kernel_against_the_oracle(T, H, L, B):
     args = _inputs(T + H + L + B, T, H, L, B)
-    _close(_gpu(*args, launches=3), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
+    _close(_gpu(*args, launches=3, form="DIE"), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
 
 
 @pytest.mark.gpu
@@ -106,7 +106,8 @@ def test_operands_of_any_float_alignment():
     n = lib.fx_lstm_stack_workspace_bytes(B, H, L)
     ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
     out = [torch.empty(T, B, H, device="cuda"), torch.empty(L, B, H, device="cuda"), torch.empty(L, B, H, device="cuda")]
-    check(lib.fx_lstm_stack(*[t.data_ptr() for t in odd + out], T, B, H, L, ws.data_ptr(), n, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    with lstm_form("DIE"):
+        check(lib.fx_lstm_stack(*[t.data_ptr() for t in odd + out], T, B, H, L, ws.data_ptr(), n, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
     torch.cuda.synchronize()
     assert lib.fx_async_error(1) == 0
     _close([t.cpu() for t in out], _reference(*args), "odd alignment")

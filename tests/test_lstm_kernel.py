@@ -8,6 +8,7 @@ with the result when that happens to be near zero.
 On the CPU, the kernel's schedule (diagonals t + j, two parities of the h buffer) and its
 hand-over protocol (values tagged with their step, bounded polls, the tag base carried from launch
 to launch) run with one host thread per workgroup (tests/support/lstm_emul.cpp)."""
+import contextlib
 import ctypes
 
 import pytest
@@ -198,9 +199,25 @@ def test_workgroups_that_share_a_compute_unit_fit_however_their_waves_are_dealt(
             assert sum(most) <= 8 and most[0] * registers + most[1] * v <= 512, (w, v, n, m)
 
 
-def _gpu(x, wih, whh, bih, bhh, h0, c0, launches=1):
+@contextlib.contextmanager
+def lstm_form(form):
+    """Launches of this thread take `form` (FX_LSTM_FORM_..., without the prefix), whatever ran before."""
+    from functs_amd._lib import C, lib
+    before = lib.fx_set_lstm_form(C["FX_LSTM_FORM_" + form])
+    try:
+        yield
+    finally:
+        lib.fx_set_lstm_form(before)
+
+
+def _gpu(x, wih, whh, bih, bhh, h0, c0, launches=1, form="ANY"):
     """`launches` calls in a row on one workspace that is cleared once; the last call's results."""
-    from functs_amd._lib import check, lib
+    with lstm_form(form):
+        return _gpu_launches(x, wih, whh, bih, bhh, h0, c0, launches, form)
+
+
+def _gpu_launches(x, wih, whh, bih, bhh, h0, c0, launches, form):
+    from functs_amd._lib import C, check, lib
     dev = torch.device("cuda:0")
     T, B, H = x.shape
     L = wih.size(0)
@@ -217,6 +234,7 @@ def _gpu(x, wih, whh, bih, bhh, h0, c0, launches=1):
                                 sc.data_ptr(), T, B, H, L, ws.data_ptr(), nbytes, stream))
         torch.cuda.synchronize()
         assert lib.fx_async_error(1) == 0
+        assert form == "ANY" or lib.fx_lstm_form() == C["FX_LSTM_FORM_" + form]
     return out.cpu(), sh.cpu(), sc.cpu()
 
 
@@ -224,26 +242,47 @@ def _gpu(x, wih, whh, bih, bhh, h0, c0, launches=1):
 @pytest.mark.parametrize("T,H,L,B", [(1, 32, 1, 1), (5, 64, 2, 1), (9, 128, 3, 2), (4, 32, 4, 3), (16, 256, 2, 1),
                                      (64, 512, 2, 1), (6, 512, 4, 16), (8, 1024, 1, 2), (7, 1024, 2, 1)])
 def test_kernel_against_the_oracle(T, H, L, B):
+    """Row by row, the form that serves every size."""
     args = _inputs(T + H + L, T, H, L, B)
-    _close(_gpu(*args), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
+    _close(_gpu(*args, form="SINGLE"), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,L,B", [(5, 64, 2, 1), (7, 64, 4, 2), (8, 64, 1, 3), (9, 128, 1, 1), (6, 128, 4, 2), (6, 256, 3, 2), (5, 256, 4, 1),
+                                     (7, 512, 1, 1), (70, 512, 3, 1), (4, 512, 4, 2)])
+def test_row_by_row_at_the_sizes_that_fit_a_die(T, H, L, B):
+    """What captured launches and launches beside others may take there."""
+    args = _inputs(T + H + L, T, H, L, B)
+    _close(_gpu(*args, launches=2, form="SINGLE"), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,H,L,B", [(1, 64, 1, 16), (3, 32, 1, 2), (4, 32, 4, 5), (5, 64, 2, 4), (4, 128, 4, 3), (7, 256, 3, 8),
-                                     (3, 256, 2, 16), (3, 256, 4, 13), (5, 512, 2, 9), (4, 512, 3, 16), (3, 512, 4, 7), (3, 512, 1, 16)])
+                                     (3, 256, 2, 16), (3, 256, 4, 13), (5, 512, 2, 9), (4, 512, 3, 16), (3, 512, 4, 7), (3, 512, 1, 16),
+                                     (5, 64, 1, 9), (6, 64, 2, 12), (5, 64, 4, 16), (7, 128, 1, 10), (5, 128, 2, 16), (6, 128, 3, 11), (5, 128, 4, 9),
+                                     (5, 512, 2, 8), (6, 512, 3, 2), (5, 512, 1, 4), (5, 512, 1, 6)])
 def test_rows_of_a_batch_share_a_step(T, H, L, B):
     """The form for several sequences: groups of four rows, full and ragged, one and two tiles of rows
     a workgroup, every depth, two to eight waves, more finishing (layer, tile) pairs than waves; two
     launches on one workspace."""
     args = _inputs(T + H + L + B, T, H, L, B)
-    _close(_gpu(*args, launches=2), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
+    want, ran = _reference(*args), []
+    # one tile of rows a workgroup and two, where the form is built and resident
+    for form in ("ROWS", "ROWS2"):
+        if form == "ROWS2" and (H < 512 or L == 4) or form == "ROWS" and H == 512 and (L == 4 or B > 8):
+            continue
+        _close(_gpu(*args, launches=2, form=form), want, "gpu %s T=%d H=%d L=%d B=%d" % (form, T, H, L, B))
+        ran.append(form)
+    if not ran:   # four layers of 512 units
+        _close(_gpu(*args, launches=2, form="SINGLE"), want, "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
 
 
 @pytest.mark.gpu
 def test_launches_in_a_row_on_one_workspace_and_no_initial_state():
     x, wih, whh, bih, bhh, _, _ = _inputs(21, 10, 128, 2, 2)
     z = torch.zeros(2, 2, 128)
-    _close(_gpu(x, wih, whh, bih, bhh, None, None, launches=3), _reference(x, wih, whh, bih, bhh, z, z), "third launch")
+    for form in ("SINGLE", "ROWS", "DIE"):
+        _close(_gpu(x, wih, whh, bih, bhh, None, None, launches=3, form=form), _reference(x, wih, whh, bih, bhh, z, z), "third launch, " + form)
 
 
 @pytest.mark.gpu
@@ -251,7 +290,7 @@ def test_benchmark_configuration_against_nn_lstm():
     """T = 64, H = 512, two layers, zero initial states: the library routine as a second opinion."""
     x, wih, whh, bih, bhh = oc.c4_inputs(0)
     z = torch.zeros(2, 1, 512)
-    out, sh, sc = _gpu(x, wih, whh, bih, bhh, z, z)
+    results = [_gpu(x, wih, whh, bih, bhh, z, z, form=form) for form in ("DIE", "SINGLE")]
     lstm = torch.nn.LSTM(512, 512, 2)
     with torch.no_grad():
         for l in range(2):
@@ -260,7 +299,8 @@ def test_benchmark_configuration_against_nn_lstm():
             getattr(lstm, "bias_ih_l%d" % l).copy_(bih[l].reshape(2048))
             getattr(lstm, "bias_hh_l%d" % l).copy_(bhh[l].reshape(2048))
         ref, (hn, cn) = lstm(x)
-    _close((out, sh, sc), (ref, hn, cn), "nn.LSTM")
+    for got in results:
+        _close(got, (ref, hn, cn), "nn.LSTM")
 
 
 @pytest.mark.gpu
@@ -274,6 +314,22 @@ def test_unsupported_shapes_are_refused():
     assert rc == C["FX_E_UNSUPPORTED"]
     rc = lib.fx_lstm_stack(p, p, p, p, p, p, p, p, p, p, 4, 1, 64, 5, ws.data_ptr(), 1 << 20, None)   # five layers
     assert rc == C["FX_E_UNSUPPORTED"]
+
+
+@pytest.mark.gpu
+def test_a_form_that_is_not_built_for_the_sizes_is_refused():
+    from functs_amd._lib import C, lib
+    st = _Stack(4, 32, 2, 2)
+    with lstm_form("DIE"):
+        assert st.rc() == C["FX_E_UNSUPPORTED"]
+    with lstm_form("ROWS2"):
+        assert st.rc() == C["FX_E_UNSUPPORTED"]
+    assert lib.fx_set_lstm_form(99) == C["FX_E_INVALID"] and lib.fx_set_lstm_form(-1) == C["FX_E_INVALID"]
+    assert lib.fx_set_lstm_form(0) == 0
+    st.launch()
+    torch.cuda.synchronize()
+    st.check("any form")
+    assert lib.fx_lstm_form() == C["FX_LSTM_FORM_ROWS"]
 
 
 def test_sizes_the_kernel_is_built_for():
@@ -295,10 +351,14 @@ class _Stack:
         self.ws = torch.zeros(lib.fx_lstm_stack_workspace_bytes(B, H, L), dtype=torch.uint8, device=self.dev)
         self.out = [torch.empty(T, B, H, device=self.dev)] + [torch.empty(L, B, H, device=self.dev) for _ in range(2)]
 
+    def rc(self):
+        from functs_amd._lib import lib
+        return lib.fx_lstm_stack(*[t.data_ptr() for t in self.args + self.out], self.T, self.B, self.H, self.L, self.ws.data_ptr(),
+                                 self.ws.numel(), ctypes.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream))
+
     def launch(self):
-        from functs_amd._lib import check, lib
-        check(lib.fx_lstm_stack(*[t.data_ptr() for t in self.args + self.out], self.T, self.B, self.H, self.L, self.ws.data_ptr(),
-                                self.ws.numel(), ctypes.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream)))
+        from functs_amd._lib import check
+        check(self.rc())
 
     def check(self, what):
         _close(tuple(t.cpu() for t in self.out), self.want, what)
