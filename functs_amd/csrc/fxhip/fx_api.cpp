@@ -1614,7 +1614,7 @@ int fx_lstm_stack(const float* x, const float* wih, const float* whh, const floa
 }
 void fx_set_totals_spin_us(uint32_t us) { g_totals_spin_us.store(us, std::memory_order_relaxed); }
 int fx_set_lstm_form(int form) {
-  if (form < FX_LSTM_FORM_ANY || form > FX_LSTM_FORM_DIE) return fail(FX_E_INVALID, "fx_set_lstm_form: no such form");
+  if (form < FX_LSTM_FORM_ANY || form > FX_LSTM_FORM_SPREAD) return fail(FX_E_INVALID, "fx_set_lstm_form: no such form");
   return fx_lstm_ask(form);
 }
 int fx_lstm_form(void) { return fx_lstm_taken(); }

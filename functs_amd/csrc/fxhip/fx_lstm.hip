@@ -716,7 +716,12 @@ __global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_row
 // us a launch, T = 64, this : the forms above: 512 units, one sequence, one to three layers 80 : 110, 92 : 119, 98 : 188;
 // two layers, four sequences 98 : 219; 256 units, four layers, four sequences 89 : 207; 128, three, eight 71 : 125;
 // 64, one, one 47 : 105.  T = 100, 256 units, three layers, eight sequences 131 : 269.  T = 8: 27 : 28 (512, two
-// layers), 12 : 16 (64, one), 20 : 20 (64, three, eight sequences).  A step of two layers of 512 units is 1.1 us:
+// layers), 12 : 16 (64, one), 20 : 20 (64, three, eight sequences).
+// The same workgroups spread over the chip (spread: slot after slot, every slot on all dies; only those that have a
+// sequence are launched) compute the same bits with values that go to the memory side, for launches that must
+// not hold a die: 512 units, two layers, one sequence 93 on dies, 110 spread, 122 row by row; three layers of 256, four
+// sequences 92, 114, 178 (tiles of rows); 128, three, eight 72, 101, 126; 64, three, eight 63, 95, 105; 64, one, one 48, 77, 108.
+// A step of two layers of 512 units is 1.1 us:
 // 0.3 from the barrier to the cells' stores, 0.3 until they are seen, 0.35 products, 0.1 sums (on the SIMD that also
 // finishes cells, the others wait for it); of 64 units 0.65.
 template <int CTRL>
@@ -806,9 +811,13 @@ struct FxLstmDie {
   // barrier, and looks slow down the stores that they wait for.  Longer products are long enough.  (One layer of 64
   // units, T = 64: 0 to 4 units 52 us, 6 48, 8 46.7, 9 47; 128 units: 2 to 9 within 4 %.)
   static constexpr int sleep = E == 1 ? 9 - NL : E == 2 ? 2 : E * NL == 4 ? 1 : 0;
+  // The same where the workgroups are spread over the dies and a value takes a microsecond (T = 64, units : us.  64 units, one
+  // layer: 0 129, 8 98, 16 77, 24 85; 128, three layers, eight sequences: 0 147, 16 101; 256, three, four: 0 134, 14 114;
+  // 512, two, one: 0 112, 8 110, 16 120)
+  static constexpr int sleep_spread = E == 1 ? 16 : E == 2 ? 15 : E == 4 ? 14 : 8;
 };
 template <int E, int NL>
-__global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kernel(const FxLstmArgs a, int L) {
+__global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kernel(const FxLstmArgs a, int L, int spread) {
   using K = FxLstmDie<E, NL>;
   constexpr int HH = K::HH, C = K::C, NW = K::NW, NC = NL * C;
   __shared__ float s_part[2][NW][NC];   // the waves' sums, by parity of the step: [layer][unit][gate]
@@ -816,7 +825,8 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
   __shared__ uint32_t s_abort;
   const int B = a.B, T = a.T;
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int slot = (int)blockIdx.x % FX_LSTM_DIES, gi = (int)blockIdx.x / FX_LSTM_DIES;
+  const int slot = spread ? (int)blockIdx.x / FX_LSTM_DIE_WG : (int)blockIdx.x % FX_LSTM_DIES;
+  const int gi = spread ? (int)blockIdx.x % FX_LSTM_DIE_WG : (int)blockIdx.x / FX_LSTM_DIES;
   const int stages = L / NL, b = slot / stages, stage = slot % stages, j0 = stage * NL;
   const int u0 = gi * K::U;
   const int n_steps = fx_lstm_stage_steps(T, NL);
@@ -908,7 +918,8 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
         hv[k] = !all && t == 0 && a.h0 ? a.h0[((size_t)(j0 + k) * B + b) * HH + own] : 0.0f;
       }
       const uint32_t want = fx_lstm_tag_read(base, d);
-      if constexpr (K::sleep > 0) __builtin_amdgcn_s_sleep(K::sleep);
+      if (spread) __builtin_amdgcn_s_sleep(K::sleep_spread);
+      else if constexpr (K::sleep > 0) __builtin_amdgcn_s_sleep(K::sleep);
       for (uint32_t polls = 0;;) {
         uint64_t el[NL];
         bool ready = true;
@@ -1103,7 +1114,7 @@ static fx_lstm_kernel_t pick_serial(int hpt) {
     default: return nullptr;
   }
 }
-typedef void (*fx_lstm_die_kernel_t)(const FxLstmArgs, int);
+typedef void (*fx_lstm_die_kernel_t)(const FxLstmArgs, int, int);
 template <int L>
 static fx_lstm_die_kernel_t pick_die(int hpt, int* threads) {
   switch (hpt) {
@@ -1118,11 +1129,14 @@ enum LstmHandOver { LSTM_TAGS, LSTM_WORDS, LSTM_DIE };   // which area of the wo
 struct LstmLaunch { const void* kernel; int grid, threads, tiles; LstmHandOver over; int form; };   // tiles of rows a workgroup; 0: row by row
 // the forms that serve these sizes, the fastest first
 template <int L>
-static int lstm_forms(const FxLstmArgs& a, LstmLaunch (&f)[4]) {
+static int lstm_forms(const FxLstmArgs& a, LstmLaunch (&f)[5]) {
   const int hpt = a.H / 32;
   int n = 0, threads = 0;
   if (fx_lstm_die_fits(a.B, a.H, L))
-    if (fx_lstm_die_kernel_t k = pick_die<L>(hpt, &threads)) f[n++] = LstmLaunch{(const void*)k, FX_LSTM_DIES * FX_LSTM_DIE_WG, threads, 0, LSTM_DIE, FX_LSTM_FORM_DIE};
+    if (fx_lstm_die_kernel_t k = pick_die<L>(hpt, &threads)) {
+      f[n++] = LstmLaunch{(const void*)k, FX_LSTM_DIES * FX_LSTM_DIE_WG, threads, 0, LSTM_DIE, FX_LSTM_FORM_DIE};
+      f[n++] = LstmLaunch{(const void*)k, a.B * (L / fx_lstm_stage_layers(a.H, L)) * FX_LSTM_DIE_WG, threads, 0, LSTM_DIE, FX_LSTM_FORM_SPREAD};
+    }
   if (a.B > 1)
     for (int tiles = 1; tiles <= 2; ++tiles) {
       const int groups = (a.B + 4 * tiles - 1) / (4 * tiles), cells = L * tiles < 4 ? L * tiles : 4;   // FxLstmRows
@@ -1171,7 +1185,7 @@ static hipError_t lstm_fit(int dev, const LstmLaunch& f, LstmFit* fit) {
 int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uint32_t* die_ctl, hipStream_t stream) {
   FxLstmArgs a = args;
   if (a.H < 32 || a.H % 32 != 0 || a.B < 1 || a.B > FX_LSTM_MAXB || L < 1 || L * a.B > FX_LSTM_BLOCK) return 1;
-  LstmLaunch f[4];
+  LstmLaunch f[5];
   const int n = L == 1 ? lstm_forms<1>(a, f) : L == 2 ? lstm_forms<2>(a, f) : L == 3 ? lstm_forms<3>(a, f) : L == 4 ? lstm_forms<4>(a, f) : 0;
   if (n == 0) return 1;
   int dev = 0, cus = 0;
@@ -1206,10 +1220,13 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     if (e != hipSuccess) return 100 + (int)e;
     if ((long)fit.per_cu * cus < f[i].grid) continue;
     const uint32_t want = fx_lstm_need((uint32_t)f[i].grid, (uint32_t)fit.sure);
-    // A sequence on one die holds every die: not one that needs more than half of it where a stack on another stream
-    // would have to wait for it.  One that needs no more is taken in every case, so that what a captured launch computes is, to
-    // the bit, what the calls beside it compute.
-    if (f[i].over == LSTM_DIE && 2u * want > (uint32_t)cus * FX_LSTM_CU && (capturing || (asked == FX_LSTM_FORM_ANY && (want > device || groups.others(id, thread))))) continue;
+    // A sequence on one die holds every die while its workgroups find their places: only where nothing else is about.
+    // The same kernel spread over the chip holds what it uses and computes the same bits, so a size whose spread form needs
+    // at most half of the device is computed by this kernel in every case: what a captured launch, or a call beside others,
+    // computes is, to the bit, what a call by itself computes.
+    const bool half = 2u * want <= (uint32_t)cus * FX_LSTM_CU;
+    if (f[i].form == FX_LSTM_FORM_DIE && (capturing || (asked == FX_LSTM_FORM_ANY && (want > device || groups.others(id, thread))))) continue;
+    if (f[i].form == FX_LSTM_FORM_SPREAD && !half && (capturing || asked == FX_LSTM_FORM_ANY)) continue;
     if (l && want >= need) continue;
     l = &f[i];
     need = want;
@@ -1223,7 +1240,8 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
   a.ctl_other = areas[1];
   a.ctl_third = areas[2];
   a.hbuf = (uint64_t*)(a.ctl + FX_LSTM_CTL_WORDS);
-  void* kargs[2] = {(void*)&a, (void*)&L};
+  int spread = l->form == FX_LSTM_FORM_SPREAD ? 1 : 0;
+  void* kargs[3] = {(void*)&a, (void*)&L, (void*)&spread};
   const dim3 grid((uint32_t)l->grid), block((uint32_t)l->threads);
   if (capturing) {
     e = hipLaunchKernel(l->kernel, grid, block, kargs, 0, stream);

@@ -14,7 +14,7 @@
 // workgroup is not there yet, so less than the device is taken.
 // Launches come in groups that fit together, and a group starts when the one before it has ended: a
 // stream's first launch of a group waits for the last launches of the group before (events, on the
-// device).  A program with one stream never waits; on two streams two stacks of 512 units, one sequence
+// device).  A program with one stream never waits; on four streams four stacks of 512 units, two layers, one sequence
 // each, run at the same time, and two that take the whole device run one after the other.
 // Events: the legacy default stream always exists and is never captured, so its event is recorded when a group
 // closes, from whichever thread that is, and launches on it cost nothing.  On any other stream an event is
@@ -71,8 +71,8 @@ struct FxLstmGroups {
     now.push_back(Member{stream, thread, need, nullptr, late});
     return now.back();
   }
-  // Whether other streams than this one have launched lately: a form that holds more than half of the device
-  // would make the streams take turns.  (Counted in launches and not asked of the device: queries are not allowed
+  // Whether other streams than this one have launched lately: a form that holds every die would make the streams
+  // take turns.  (Counted in launches and not asked of the device: queries are not allowed
   // beside a capture.)
   bool others(uint64_t stream, uint64_t thread) const {
     for (const std::vector<Member>* group : {&now, &before})

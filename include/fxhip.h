@@ -436,12 +436,18 @@ int fx_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* co
  * with their layers, or at H = 512 each layer of theirs, find dies of their own; H / 2 of 512 threads, or H / 4
  * of up to 768 for every four or eight rows) must be resident
  * together (FX_E_LIMIT if no form's are).  Launches on several streams of a device overlap when all their
- * workgroups find places together (two stacks of 512 units with one sequence each, for instance, which leave
- * the dies' form to a stream that launches alone);
+ * workgroups find places together (four stacks of 512 units, two layers, one sequence each, for instance);
  * one that does not fit waits, in its stream, for the launches before it (a launch on another stream than the
- * legacy default one records an event behind it for that).  A captured launch cannot be
+ * legacy default one records an event behind it for that).  Dies of their own are for launches while no other stream
+ * launches; beside others (within 64 launches) and in captures the same kernel takes 32 workgroups a sequence
+ * and stage anywhere on the chip.  A captured launch cannot be
  * made to wait: it, and from then on every launch on that device, takes a form for half of the device
  * where there is one, so that ONE replay and the calls, or two replays, may run at the same time.
+ * Results: the two placements give the same bits, so what a launch computes depends on the operands and the device
+ * only, unless that kernel's workgroups spread over the chip would take more than half of it (more than four sequences
+ * of 256 units and two or three layers, or of 128 units and four; of 512 units when sequences times layers are
+ * more than four; more than two of 256 units and four layers): captured launches and launches beside others then sum
+ * in the order of another form, which may differ in the last bits (FX_LSTM_FORM_... pins one).
  * workspace: fx_lstm_stack_workspace_bytes() of device memory, 256-byte aligned, all zero when it
  * is used for the first time.  A launch that ends without error leaves it ready for the next one,
  * so one workspace, cleared once, serves launch after launch on one stream as long as batch,
@@ -466,6 +472,7 @@ void fx_set_lstm_spin_limit(uint32_t polls); /* barrier polls before a wait is g
 #define FX_LSTM_FORM_ROWS 2   /* four rows a workgroup, values as words */
 #define FX_LSTM_FORM_ROWS2 3  /* eight rows a workgroup, values as words */
 #define FX_LSTM_FORM_DIE 4    /* a sequence on one die */
+#define FX_LSTM_FORM_SPREAD 5 /* the same kernel with its workgroups all over the chip: the same bits */
 int fx_set_lstm_form(int form);
 int fx_lstm_form(void);
 

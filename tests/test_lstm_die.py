@@ -65,13 +65,16 @@ def test_streams_that_launched_lately_are_told_apart(emul):
         assert others(1, 5, 64, device, 7) == 1     # a second stream's first launch
 
 
+# sizes whose workgroups, spread over the chip, take at most half of it
 @pytest.mark.gpu
-def test_a_captured_stack_computes_what_the_calls_beside_it_compute():
+@pytest.mark.parametrize("T,H,L,B", [(9, 64, 2, 1), (5, 64, 3, 8), (6, 128, 3, 8), (6, 128, 4, 3), (7, 256, 3, 4), (9, 256, 4, 2), (20, 512, 2, 1), (8, 512, 4, 1), (6, 512, 1, 4)])
+def test_a_captured_stack_computes_what_the_calls_beside_it_compute(T, H, L, B):
     """To the bit, whether or not another stream has launched stacks lately."""
     from functs_amd import jit as fj
+    from functs_amd._lib import C, lib
     from functs_amd.benchmark import PROGRAMS
     from oracle import configs as oc
-    args = oc.c4_inputs(3, 9, 64, 2, 1)
+    args = oc.c4_inputs(3, T, H, L, B)
     gpu = [a.cuda() if isinstance(a, torch.Tensor) else a for a in args]
     eager = fj.build(fj.script(PROGRAMS["c4"]), list(args))
     for other in (False, True):
@@ -80,11 +83,44 @@ def test_a_captured_stack_computes_what_the_calls_beside_it_compute():
                 eager(*gpu)
             torch.cuda.synchronize()
         graphed = fj.build(fj.script(PROGRAMS["c4"]), list(args), hip_graph=True)
+        graphed(*gpu)
+        assert lib.fx_lstm_form() == C["FX_LSTM_FORM_SPREAD"]
         for _ in range(3):
             want = eager(*gpu)
             torch.cuda.synchronize()
             for g, w in zip(graphed(*gpu), want):
                 assert torch.equal(g, w), "after launches on another stream: %s" % other
+    with torch.cuda.stream(torch.cuda.Stream()):   # and beside the other stream's
+        beside = eager(*gpu)
+        assert lib.fx_lstm_form() == C["FX_LSTM_FORM_SPREAD"]
+    torch.cuda.synchronize()
+    assert all(torch.equal(b, w) for b, w in zip(beside, want))
+
+
+@pytest.mark.gpu
+def test_small_stacks_on_many_streams_and_replays_hold_little():
+    """Three graphs of small stacks at once beside calls on three streams: a launch that is not alone claims the
+    workgroups that it has, on no die in particular."""
+    from tests.test_lstm_kernel import _Stack
+    from functs_amd._lib import C, lib
+    stacks = [_Stack(12, 64, 1, 1) for _ in range(6)]
+    graphs, streams = [], [torch.cuda.Stream() for _ in stacks]
+    torch.cuda.synchronize()
+    print("fx_lstm_stack on six streams", flush=True)
+    for st in stacks[:3]:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            st.launch()
+        assert lib.fx_lstm_form() == C["FX_LSTM_FORM_SPREAD"]
+        graphs.append(g)
+    for _ in range(5):
+        for i, (st, s) in enumerate(zip(stacks, streams)):
+            with torch.cuda.stream(s):
+                graphs[i].replay() if i < 3 else st.launch()
+    torch.cuda.synchronize()
+    assert lib.fx_async_error(1) == 0
+    for st in stacks:
+        st.check("side by side")
 
 
 # every width and depth of a stage, one to eight sequences, rings that go round, shorter sequences than the lag
@@ -93,7 +129,12 @@ def test_a_captured_stack_computes_what_the_calls_beside_it_compute():
                                      (50, 256, 4, 4), (21, 256, 2, 1), (1, 512, 3, 2), (3, 512, 2, 4), (70, 512, 2, 4), (40, 512, 4, 2), (9, 512, 1, 8)])
 def test_kernel_against_the_oracle(T, H, L, B):
     args = _inputs(T + H + L + B, T, H, L, B)
-    _close(_gpu(*args, launches=3, form="DIE"), _reference(*args), "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
+    want, got = _reference(*args), _gpu(*args, launches=3, form="DIE")
+    _close(got, want, "gpu T=%d H=%d L=%d B=%d" % (T, H, L, B))
+    # spread over the dies, where values go by the memory side: the same sums in the same order
+    spread = _gpu(*args, launches=3, form="SPREAD")
+    _close(spread, want, "gpu, spread, T=%d H=%d L=%d B=%d" % (T, H, L, B))
+    assert all(torch.equal(a, b) for a, b in zip(got, spread))
 
 
 @pytest.mark.gpu
