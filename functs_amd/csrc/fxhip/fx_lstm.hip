@@ -1225,8 +1225,11 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     // at most half of the device is computed by this kernel in every case: what a captured launch, or a call beside others,
     // computes is, to the bit, what a call by itself computes.
     const bool half = 2u * want <= (uint32_t)cus * FX_LSTM_CU;
-    if (f[i].form == FX_LSTM_FORM_DIE && (capturing || (asked == FX_LSTM_FORM_ANY && (want > device || groups.others(id, thread))))) continue;
-    if (f[i].form == FX_LSTM_FORM_SPREAD && !half && (capturing || asked == FX_LSTM_FORM_ANY)) continue;
+    if (asked != FX_LSTM_FORM_ANY) {
+      if (capturing && !half) continue;   // (a replay may run beside any other)
+    } else if (f[i].form == FX_LSTM_FORM_DIE ? capturing || want > device || groups.others(id, thread) : f[i].form == FX_LSTM_FORM_SPREAD && !half) {
+      continue;
+    }
     if (l && want >= need) continue;
     l = &f[i];
     need = want;

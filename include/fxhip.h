@@ -465,7 +465,8 @@ int fx_lstm_stack(const float* x, const float* wih, const float* whh, const floa
 void fx_set_lstm_spin_limit(uint32_t polls); /* barrier polls before a wait is given up (default 1000000; tests) */
 /* The forms of fx_lstm_stack, and the one that the calling thread's launches are to take (FX_LSTM_FORM_ANY, the
  * default: the fastest that the sizes and what else may run allow).  Returns the one asked for before, or FX_E_INVALID.
- * A form that is not built for the sizes, or that a captured launch must not take: FX_E_UNSUPPORTED from the launch.
+ * A form that is not built for the sizes, or a captured launch in one that needs more than half of the device:
+ * FX_E_UNSUPPORTED from the launch.
  * fx_lstm_form: the form of the calling thread's last launch (FX_LSTM_FORM_ANY: none yet). */
 #define FX_LSTM_FORM_ANY 0
 #define FX_LSTM_FORM_SINGLE 1 /* row by row, tagged values */

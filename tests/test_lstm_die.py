@@ -111,6 +111,36 @@ def test_small_stacks_on_many_streams_and_replays_hold_little():
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
             st.launch()
+@pytest.mark.gpu
+def test_a_pinned_form_gives_the_same_bits_to_calls_and_captures():
+    """Sizes whose workgroups on dies take the whole device: calls and captures differ in form, unless one is asked for."""
+    from tests.test_lstm_kernel import _Stack
+    from functs_amd._lib import C, lib
+    st = _Stack(9, 256, 3, 8)
+    with lstm_form("ROWS"):
+        st.launch()
+        torch.cuda.synchronize()
+        call = [t.clone() for t in st.out]
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            st.launch()
+    for t in st.out:
+        t.fill_(float("nan"))
+    g.replay()
+    torch.cuda.synchronize()
+    assert lib.fx_async_error(1) == 0
+    st.check("replay")
+    assert all(torch.equal(a, b) for a, b in zip(call, st.out))
+    for form in ("DIE", "SPREAD"):   # (in a capture these would starve a second replay)
+        with lstm_form(form):
+            st.launch()
+            torch.cuda.synchronize()
+            st.check(form)
+            with torch.cuda.graph(torch.cuda.CUDAGraph()):
+                torch.zeros(1, device="cuda")
+                assert st.rc() == C["FX_E_UNSUPPORTED"]
+
+
         assert lib.fx_lstm_form() == C["FX_LSTM_FORM_SPREAD"]
         graphs.append(g)
     for _ in range(5):
