@@ -713,6 +713,9 @@ __global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_row
 // Where a workgroup runs is the hardware's choice (dies in turn).  Loads are device-scope either way; whether a
 // value may be stored to the die's cache only, the workgroups of a stage find out while they load their
 // weights: each publishes its die, and unless all agree they store to the memory side.
+// That a value stored at workgroup scope is seen by a device-scope load of another unit of the die is how this chip
+// is built (first-level caches write through; device-scope loads pass them and find what lies in the die's cache,
+// written back or not), not what the memory model promises: between workgroups it is relied on only where the die is the same.
 // us a launch, T = 64, this : the forms above: 512 units, one sequence, one to three layers 80 : 110, 92 : 119, 98 : 188;
 // two layers, four sequences 98 : 219; 256 units, four layers, four sequences 89 : 207; 128, three, eight 71 : 125;
 // 64, one, one 47 : 105.  T = 100, 256 units, three layers, eight sequences 131 : 269.  T = 8: 27 : 28 (512, two
@@ -822,7 +825,10 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
   constexpr int HH = K::HH, C = K::C, NW = K::NW, NC = NL * C;
   __shared__ float s_part[2][NW][NC];   // the waves' sums, by parity of the step: [layer][unit][gate]
   __shared__ __align__(16) float s_in[3][HH];   // the stage's input of a step and of the two behind it
-  __shared__ uint32_t s_abort;
+  // A wait that is given up between the barriers of steps d - 1 and d sets word d & 1, which is read behind barrier d
+  // and not set again before barrier d + 1: all waves of the workgroup see the same and leave at the same place.
+  // (Ahead of step 0's barrier there is one more, of step -1.)
+  __shared__ uint32_t s_abort[2];
   const int B = a.B, T = a.T;
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int slot = spread ? (int)blockIdx.x / FX_LSTM_DIE_WG : (int)blockIdx.x % FX_LSTM_DIES;
@@ -838,13 +844,15 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
     if (tid == 0) fx_lstm_leave<DevAtomics>(a.ctl, gridDim.x, base, advance, a.hbuf, area.words);
     return;
   }
-  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) || fx_lstm_refused<DevAtomics>(a.ctl_third) ? 1u : 0u;
+  if (tid < 2) s_abort[tid] = 0u;
+  __syncthreads();
+  if (tid == 0 && (fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) || fx_lstm_refused<DevAtomics>(a.ctl_third))) s_abort[1] = 1u;
   uint64_t* const where = a.hbuf + area.where + slot * FX_LSTM_DIE_WG;
   if (tid == 0) DevAtomics::store64(where + gi, fx_lstm_pack(fx_die_of_wave(), base + 1u));
-  auto give_up = [&]() {   // the workgroup leaves behind the next barrier
+  auto give_up = [&](int d) {   // the workgroup leaves behind the barrier of step d, the next one
     DevAtomics::store(a.ctl + FX_LSTM_W_ERR, 1u);
     if (a.err_host) __hip_atomic_store(a.err_host, (uint32_t)FX_ASYNC_BARRIER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    s_abort = 1u;
+    s_abort[d & 1] = 1u;
   };
   // polls so far of a wait: is it to be given up?
   auto too_long = [&](uint32_t polls) {
@@ -869,7 +877,7 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
     for (int k = 0; k < NL; ++k) from[k] = a.hbuf + fx_lstm_hoff(0, j0 + k, b, own, L, B, HH);
     __builtin_amdgcn_s_waitcnt(0);   // (the weights are here: otherwise the loop waits for them, and for looks behind them)
     __syncthreads();
-    if (s_abort != 0u) {   // uniform: written ahead of the barrier
+    if (s_abort[1] != 0u) {
       if (tid == 0 && a.err_host) __hip_atomic_store(a.err_host, (uint32_t)FX_ASYNC_BARRIER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       fx_lstm_poison(a, L, (uint32_t)tid, (uint32_t)(NW * 64));
       return;
@@ -932,7 +940,7 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
         for (int k = 0; k < NL; ++k) hv[k] = need[k] ? __uint_as_float((uint32_t)el[k]) : hv[k];
         if (!wave_any(!ready)) break;
         if (too_long(++polls)) {
-          give_up();
+          give_up(d);
           break;
         }
       }
@@ -951,7 +959,7 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
         s_part[d & 1][wave][k * C + unit * 4 + (cl >> 1)] = sum[i];
       }
       __syncthreads();
-      aborted = s_abort;   // (looked at behind the next products)
+      aborted = s_abort[d & 1];   // (looked at behind the next products)
     };
     int place = 0;
     for (int d = 0; d < n_steps && aborted == 0u; ++d) {
@@ -985,7 +993,7 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
   auto fetch = [&](int t) {   // x of step t, asked for
     if (stage == 0 && t < T) fx_die_load<E>(a.x + ((size_t)t * B + b) * HH + lane * E, in);
   };
-  auto park = [&](int t) {
+  auto park = [&](int t, int d) {   // d: whose barrier is next
     if (t >= T) return;
     if (stage > 0) {
       for (uint32_t polls = 0;;) {
@@ -998,7 +1006,7 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
         }
         if (!wave_any(!ready)) break;
         if (too_long(++polls)) {
-          give_up();
+          give_up(d);
           break;
         }
       }
@@ -1018,22 +1026,22 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
       break;
     }
     if (too_long(++polls)) {
-      give_up();
+      give_up(-1);
       break;
     }
   }
   if (cw == 0) {
     for (int t = 0; t < 2; ++t) {
       fetch(t);
-      park(t);
+      park(t, -1);
     }
     fetch(2);
   }
   __syncthreads();
-  if (s_abort != 0u) return;
+  if (s_abort[1] != 0u) return;
   for (int d = 0; d < n_steps; ++d) {
     __syncthreads();
-    const uint32_t aborted = s_abort;
+    const uint32_t aborted = s_abort[d & 1];
     float part[NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) part[w] = s_part[d & 1][w][f];
@@ -1059,21 +1067,21 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
         a.state_c[((size_t)j * B + b) * HH + u] = cell;
       }
     }
-    if (aborted != 0u) return;   // uniform, and nothing was stored
+    if (aborted != 0u) return;   // uniform, and nothing of this step was stored
     // between the barriers of steps d and d + 1 the others read the input of step d + 1; the place of step
     // d + 2 was last read in step d - 1
     if (cw == 0) {
-      park(d + 2);
+      park(d + 2, d + 1);
       fetch(d + 3);
     }
     // every half ring: the next half may be written (the next stage is never that far behind but at the start)
-    if (stage + 1 < stages && d % (FX_LSTM_RING / 2) == FX_LSTM_RING / 2 - 1) {
+    if (stage + 1 < stages && d + 1 < n_steps && d % (FX_LSTM_RING / 2) == FX_LSTM_RING / 2 - 1) {
       const int seen = d + 1 - FX_LSTM_RING / 2;   // vectors that have to be read before vector d + RING / 2 is written
       for (uint32_t polls = 0; seen > 0;) {
         const uint32_t n = (uint32_t)__hip_atomic_load(read_out + (lane & (FX_LSTM_DIE_WG - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (!wave_any((int32_t)(n - (base + (uint32_t)seen)) < 0)) break;
         if (too_long(++polls)) {
-          give_up();
+          give_up(d + 1);
           break;
         }
       }

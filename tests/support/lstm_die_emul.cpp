@@ -22,10 +22,11 @@ struct HostAtomics {
 };
 float sigmoidf(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-// n_wg workgroups a stage (at most FX_LSTM_DIE_WG), H / n_wg units each; slow: (stage, workgroup) that dawdles
+// n_wg workgroups a stage (at most FX_LSTM_DIE_WG), H / n_wg units each; slow: (stage, workgroup) that dawdles, stop: that
+// leaves after four steps
 struct Run {
   FxLstmArgs a;
-  int L, n_wg, total, slow_stage, slow_wg;
+  int L, n_wg, total, slow_stage, slow_wg, stop_stage = -1, stop_wg = -1;
   bool give_up(uint32_t polls) const {
     if (polls <= a.spin_limit && !((polls & 255u) == 0u && HostAtomics::load(a.ctl + FX_LSTM_W_ERR) != 0u)) return false;
     HostAtomics::store(a.ctl + FX_LSTM_W_ERR, 1u);
@@ -40,6 +41,12 @@ struct Run {
     return true;
   }
   void workgroup(int b, int stage, int gi) const {
+    const bool refused = fx_lstm_refused<HostAtomics>(a.ctl) || fx_lstm_refused<HostAtomics>(a.ctl_other) || fx_lstm_refused<HostAtomics>(a.ctl_third);
+    const bool done = !refused && steps(b, stage, gi);
+    if (refused) *a.err_host = 2u;
+    if (!done && !(stage == stop_stage && gi == stop_wg)) fx_lstm_poison(a, L, 0u, 1u);
+  }
+  bool steps(int b, int stage, int gi) const {
     const int H = a.H, B = a.B, T = a.T, NL = fx_lstm_stage_layers(H, L), stages = L / NL, U = H / n_wg, u0 = gi * U, j0 = stage * NL;
     const uint32_t base = HostAtomics::load(a.ctl + FX_LSTM_W_BASE);
     const FxLstmDieArea area = fx_lstm_die_area(B, H, L);
@@ -70,15 +77,16 @@ struct Run {
       if (stage > 0) HostAtomics::store64(read_in, (uint64_t)(base + (uint32_t)t + 1u));
       return true;
     };
-    if (!park(0) || !park(1)) return;
+    if (!park(0) || !park(1)) return false;
     for (int d = 0; d < n_steps; ++d) {
+      if (stage == stop_stage && gi == stop_wg && d == 4) return false;
       if (stage == slow_stage && gi == slow_wg && d % 5 == 0) std::this_thread::sleep_for(std::chrono::milliseconds(2));
       for (int k = 0; k < NL; ++k) {
         const int t = fx_lstm_stage_time(d, k, T);
         const bool need = d > 0 && fx_lstm_stage_time(d - 1, k, T) >= 0 && (t >= 0 || k + 1 < NL);
         for (int i = 0; i < H; ++i) {
           hv[k][i] = t == 0 && a.h0 ? a.h0[((size_t)(j0 + k) * B + b) * H + i] : 0.0f;
-          if (need && !tagged(a.hbuf + fx_lstm_hoff((d + 1) & 1, j0 + k, b, i, L, B, H), fx_lstm_tag_read(base, d), &hv[k][i])) return;
+          if (need && !tagged(a.hbuf + fx_lstm_hoff((d + 1) & 1, j0 + k, b, i, L, B, H), fx_lstm_tag_read(base, d), &hv[k][i])) return false;
         }
       }
       for (int k = 0; k < NL; ++k) {
@@ -110,14 +118,15 @@ struct Run {
         }
       }
       below = hv;
-      if (!park(d + 2)) return;
-      if (stage + 1 < stages && d % (FX_LSTM_RING / 2) == FX_LSTM_RING / 2 - 1) {
+      if (!park(d + 2)) return false;
+      if (stage + 1 < stages && d + 1 < n_steps && d % (FX_LSTM_RING / 2) == FX_LSTM_RING / 2 - 1) {
         const int seen = d + 1 - FX_LSTM_RING / 2;
         for (int w = 0; w < n_wg && seen > 0; ++w)
-          if (!wait([&] { return (int32_t)((uint32_t)__atomic_load_n(read_out + w, __ATOMIC_ACQUIRE) - (base + (uint32_t)seen)) >= 0; })) return;
+          if (!wait([&] { return (int32_t)((uint32_t)__atomic_load_n(read_out + w, __ATOMIC_ACQUIRE) - (base + (uint32_t)seen)) >= 0; })) return false;
       }
     }
     fx_lstm_leave<HostAtomics>(a.ctl, (uint32_t)total, base, (uint32_t)n_steps + 1u, a.hbuf, area.words);
+    return true;
   }
 };
 }  // namespace
@@ -132,7 +141,7 @@ extern "C" int fx_lstm_die_emul(const float* x, const float* wih, const float* w
   std::vector<uint64_t> area(fx_lstm_die_area(B, H, L).words, 0ull);
   ctl[FX_LSTM_W_BASE] = base0;
   Run r;
-  r.a = FxLstmArgs{x, wih, whh, bih, bhh, h0, c0, out, state_h, state_c, area.data(), ctl.data(), nullptr, nullptr, nullptr, T, B, H, spin_limit};
+  r.a = FxLstmArgs{x, wih, whh, bih, bhh, h0, c0, out, state_h, state_c, area.data(), ctl.data(), ctl.data(), ctl.data(), nullptr, T, B, H, spin_limit};
   const int stages = L / fx_lstm_stage_layers(H, L);
   r.L = L; r.n_wg = n_wg; r.total = stages * B * n_wg; r.slow_stage = slow_stage; r.slow_wg = slow_wg;
   uint32_t base = base0;
@@ -153,6 +162,56 @@ extern "C" int fx_lstm_die_emul(const float* x, const float* wih, const float* w
     if (ctl[FX_LSTM_W_BASE] != base || ctl[FX_LSTM_W_LEAVE] != 0u) return -1;
   }
   return 0;
+}
+
+// A workgroup (stop_stage, stop_wg) leaves in the middle; then, with whatever that left, another launch; then, on a
+// cleared workspace, one with the error word of control area `marked` set (0: its own, 1, 2: the other forms'); then one with
+// all clear.  Bits: 1 the first gave up; 2 with NaN for results; 4 the second was refused; 8 with NaN; 16 the marked one
+// was refused, 32 with NaN; 64 the last one ran.
+extern "C" int fx_lstm_die_emul_give_up(const float* x, const float* wih, const float* whh, const float* bih, const float* bhh, const float* h0,
+                                        const float* c0, float* out, float* state_h, float* state_c, int T, int B, int H, int L, int n_wg,
+                                        uint32_t spin_limit, int stop_stage, int stop_wg, int marked) {
+  std::vector<uint32_t> ctl[3];
+  for (auto& c : ctl) c.assign(FX_LSTM_CTL_WORDS, 0u);
+  std::vector<uint64_t> area(fx_lstm_die_area(B, H, L).words, 0ull);
+  uint32_t err = 0u;
+  Run r;
+  r.a = FxLstmArgs{x, wih, whh, bih, bhh, h0, c0, out, state_h, state_c, area.data(), ctl[0].data(), ctl[1].data(), ctl[2].data(), &err, T, B, H, spin_limit};
+  const int stages = L / fx_lstm_stage_layers(H, L);
+  r.L = L; r.n_wg = n_wg; r.total = stages * B * n_wg; r.slow_stage = r.slow_wg = -1;
+  auto launch = [&] {
+    err = 0u;
+    for (size_t i = 0; i < (size_t)T * B * H; ++i) out[i] = 1.0f;
+    std::vector<std::thread> th;
+    for (int b = 0; b < B; ++b)
+      for (int s = 0; s < stages; ++s)
+        for (int g = 0; g < n_wg; ++g) th.emplace_back(&Run::workgroup, std::cref(r), b, s, g);
+    for (auto& t : th) t.join();
+  };
+  // (the workgroup that left in the middle, or others ahead of it, may have written steps of theirs behind the NaNs: the last step
+  // nobody has reached)
+  auto all_nan = [&] {
+    for (int i = 0; i < B * H; ++i)
+      if (!isnan(out[(size_t)(T - 1) * B * H + i])) return false;
+    return true;
+  };
+  int bits = 0;
+  r.stop_stage = stop_stage; r.stop_wg = stop_wg;
+  launch();
+  bits |= (ctl[0][FX_LSTM_W_ERR] ? 1 : 0) | (all_nan() ? 2 : 0);
+  r.stop_stage = r.stop_wg = -1;
+  launch();
+  bits |= (err == 2u ? 4 : 0) | (all_nan() ? 8 : 0);
+  for (auto& c : ctl) c.assign(FX_LSTM_CTL_WORDS, 0u);
+  area.assign(area.size(), 0ull);
+  r.a.ctl = ctl[0].data(); r.a.ctl_other = ctl[1].data(); r.a.ctl_third = ctl[2].data(); r.a.hbuf = area.data();
+  ctl[marked][FX_LSTM_W_ERR] = 1u;
+  launch();
+  bits |= (err == 2u ? 16 : 0) | (all_nan() ? 32 : 0);
+  ctl[marked][FX_LSTM_W_ERR] = 0u;
+  r.a.spin_limit = 1u << 30;
+  launch();
+  return bits | (err == 0u && ctl[0][FX_LSTM_W_ERR] == 0u ? 64 : 0);
 }
 
 // Streams 0 .. n - 1 launch once each, in that order, then stream 0 `more` times, in groups that hold `device`: have

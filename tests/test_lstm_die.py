@@ -18,6 +18,7 @@ def emul(tmp_path_factory):
     subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-pthread", src, "-o", so])
     lib = ctypes.CDLL(so)
     lib.fx_lstm_die_emul.argtypes = [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.c_uint32, ctypes.c_int, ctypes.c_uint32, ctypes.c_int, ctypes.c_int]
+    lib.fx_lstm_die_emul_give_up.argtypes = [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.c_uint32] + [ctypes.c_int] * 3
     lib.fx_lstm_others_emul.argtypes = [ctypes.c_int] * 2 + [ctypes.c_uint32] * 2 + [ctypes.c_int]
     return lib
 
@@ -54,6 +55,19 @@ def test_tags_start_over_before_they_wrap(emul):
     got, rc = _run(emul, args, launches=3, base0=0x80000000 - 8)
     assert rc == 0
     _close(got, _reference(*args), "after the tags were cleared")
+
+
+# a stage's own h, the ring to the next stage (whose reader or writer is gone), and the three areas of a workspace
+@pytest.mark.parametrize("H,L,B,stop,marked", [(64, 2, 1, (0, 1), 0), (64, 2, 2, (0, 0), 1), (512, 3, 1, (0, 2), 2), (512, 3, 1, (1, 0), 0), (512, 2, 2, (1, 3), 1), (256, 4, 1, (1, 1), 2)])
+def test_a_wait_that_cannot_end_is_given_up_and_its_workspace_refused(emul, H, L, B, stop, marked):
+    args = [t.contiguous() for t in _inputs(H + L, 40, H, L, B)]
+    out, sh, sc = torch.zeros(40, B, H), torch.zeros(L, B, H), torch.zeros(L, B, H)
+    bits = emul.fx_lstm_die_emul_give_up(*[t.data_ptr() for t in args + [out, sh, sc]], 40, B, H, L, 4, 3000, *stop, marked)
+    for bit, what in ((1, "the launch with a workgroup less did not give up"), (2, "it left values that look like results"),
+                      (4, "the workspace of a given-up wait was used again"), (8, "and its results are no NaN"),
+                      (16, "a launch that another form's error word refuses ran"), (32, "and its results are no NaN"), (64, "the cleared workspace failed")):
+        assert bits & bit, what
+    _close((out, sh, sc), _reference(*args), "on the cleared workspace")
 
 
 def test_streams_that_launched_lately_are_told_apart(emul):
@@ -98,20 +112,6 @@ def test_a_captured_stack_computes_what_the_calls_beside_it_compute(T, H, L, B):
 
 
 @pytest.mark.gpu
-def test_small_stacks_on_many_streams_and_replays_hold_little():
-    """Three graphs of small stacks at once beside calls on three streams: a launch that is not alone claims the
-    workgroups that it has, on no die in particular."""
-    from tests.test_lstm_kernel import _Stack
-    from functs_amd._lib import C, lib
-    stacks = [_Stack(12, 64, 1, 1) for _ in range(6)]
-    graphs, streams = [], [torch.cuda.Stream() for _ in stacks]
-    torch.cuda.synchronize()
-    print("fx_lstm_stack on six streams", flush=True)
-    for st in stacks[:3]:
-        g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
-            st.launch()
-@pytest.mark.gpu
 def test_a_pinned_form_gives_the_same_bits_to_calls_and_captures():
     """Sizes whose workgroups on dies take the whole device: calls and captures differ in form, unless one is asked for."""
     from tests.test_lstm_kernel import _Stack
@@ -141,6 +141,20 @@ def test_a_pinned_form_gives_the_same_bits_to_calls_and_captures():
                 assert st.rc() == C["FX_E_UNSUPPORTED"]
 
 
+@pytest.mark.gpu
+def test_small_stacks_on_many_streams_and_replays_hold_little():
+    """Three graphs of small stacks at once beside calls on three streams: a launch that is not alone claims the
+    workgroups that it has, on no die in particular."""
+    from tests.test_lstm_kernel import _Stack
+    from functs_amd._lib import C, lib
+    stacks = [_Stack(12, 64, 1, 1) for _ in range(6)]
+    graphs, streams = [], [torch.cuda.Stream() for _ in stacks]
+    torch.cuda.synchronize()
+    print("fx_lstm_stack on six streams", flush=True)
+    for st in stacks[:3]:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            st.launch()
         assert lib.fx_lstm_form() == C["FX_LSTM_FORM_SPREAD"]
         graphs.append(g)
     for _ in range(5):
@@ -165,6 +179,31 @@ def test_kernel_against_the_oracle(T, H, L, B):
     spread = _gpu(*args, launches=3, form="SPREAD")
     _close(spread, want, "gpu, spread, T=%d H=%d L=%d B=%d" % (T, H, L, B))
     assert all(torch.equal(a, b) for a, b in zip(got, spread))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["DIE", "SPREAD"])
+@pytest.mark.parametrize("H,L,B", [(64, 1, 1), (256, 3, 2), (256, 4, 2), (512, 2, 1)])
+def test_a_given_up_wait_ends_the_kernel_and_marks_the_workspace(H, L, B, form):
+    from tests.test_lstm_kernel import _Stack
+    from functs_amd._lib import C, lib
+    st = _Stack(20, H, L, B)
+    with lstm_form(form):
+        lib.fx_set_lstm_spin_limit(1)   # (no value is there at the first two looks)
+        try:
+            st.launch()
+            torch.cuda.synchronize()
+        finally:
+            lib.fx_set_lstm_spin_limit(1000000)
+        assert lib.fx_async_error(1) == C["FX_ASYNC_BARRIER"] and bool(st.out[0][-1].isnan().all())
+        st.launch()   # refused
+        torch.cuda.synchronize()
+        assert lib.fx_async_error(1) == C["FX_ASYNC_BARRIER"] and all(bool(t.isnan().all()) for t in st.out)
+        st.ws.zero_()
+        st.launch()
+        torch.cuda.synchronize()
+        assert lib.fx_async_error(1) == 0
+        st.check("on the cleared workspace")
 
 
 @pytest.mark.gpu
