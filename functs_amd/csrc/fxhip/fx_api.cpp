@@ -807,28 +807,19 @@ static int stream_status(fx_region* reg, fx::Plan* pl, hipStream_t stream, int d
 }
 
 // ---- detection-head kernel: geometry of a launch ----
-// Rows of a sub-tile: what FX_HEAD_KV 128-bit loads per lane carry, at most FX_HEAD_SUB.
-static uint32_t head_sub_rows(const FxHeadInfo& hi) {
-  const uint32_t cap = (FX_HEAD_KV * FX_BLOCK * 4u - 6u) / hi.S;
-  return std::min<uint32_t>(FX_HEAD_SUB, cap);
-}
 static size_t head_status_words(const FxHeadInfo& hi) {
   const uint32_t min_chunk = std::min<uint32_t>(FX_HEAD_MIN_CHUNK, std::max<uint32_t>(hi.n_rows, 1u));
   return (size_t)hi.n_tasks * ((hi.n_rows + min_chunk - 1) / min_chunk);
 }
 static bool head_fits(const fx::Plan* pl) {
   // a sub-tile of at least 8 rows, and counts of up to FX_BLOCK rows in a status word
-  return head_active(pl) && head_sub_rows(pl->head) >= 8u;
+  return head_active(pl) && fx_head_carried(pl->head.S) >= 8u;
 }
-// Every image's rows are dealt to its workgroups in equal runs, as few workgroups as give every
-// resident slot of the device one (more only when a chunk would exceed FX_BLOCK rows, fewer when
-// it would fall below FX_HEAD_MIN_CHUNK).
 static int head_launch_info(fx::Plan* pl, FxHeadLaunch* hl) {
   const FxHeadInfo& hi = pl->head;
   memset(hl, 0, sizeof(*hl));
   hl->n_rows = hi.n_rows;
   hl->n_tasks = hi.n_tasks;
-  hl->sub_rows = head_sub_rows(hi);
   hl->S = hi.S;
   hl->C = hi.C;
   fx_fastdiv_make(hi.C % 4u ? hi.C : hi.C / 4u, &hl->g_magic, &hl->g_shift);
@@ -849,25 +840,25 @@ static int head_launch_info(fx::Plan* pl, FxHeadLaunch* hl) {
     hl->out_slot[k] = hi.out_slot[k];
     hl->out_tstride[k] = hi.out_tstride[k];
   }
-  if (pl->head_resident == 0) {
-    // One slot per CU is left free: a launch that needs every slot the occupancy rule allows does
-    // not get all of its workgroups placed at once, and the stragglers cost a second round.
-    uint32_t wg = 0, per_cu = 1;
-    HIP_OK(fx_head_resident(fx_head_lds_bytes(*hl), &wg, &per_cu));
-    if (per_cu >= 3) wg -= wg / per_cu;
-    pl->head_resident = std::max<uint32_t>(wg, 1u);
+  uint32_t packed = pl->head_rows;
+  if (packed == 0) {
+    hipError_t e = hipSuccess;
+    const FxHeadGeometry g = fx_head_geometry(hi.n_rows, hi.n_tasks, hi.S, [&](uint32_t window) {
+      // One slot per CU is left free: a launch that needs every slot the occupancy rule allows does
+      // not get all of its workgroups placed at once, and the stragglers cost a second round.
+      uint32_t wg = 0, per_cu = 1;
+      const hipError_t q = fx_head_resident(fx_head_window_bytes(window, hi.S), &wg, &per_cu);
+      if (q != hipSuccess) e = q;
+      return per_cu >= 3 ? wg - wg / per_cu : wg;
+    });
+    HIP_OK(e);
+    packed = pl->head_rows = g.chunk_rows << 16 | g.sub_rows;
   }
-  const uint32_t per_task = std::max<uint32_t>(1u, pl->head_resident / std::max<uint32_t>(hi.n_tasks, 1u));
-  uint32_t cr = (hi.n_rows + per_task - 1) / per_task;
-  const uint32_t min_chunk = std::min<uint32_t>(FX_HEAD_MIN_CHUNK, std::max<uint32_t>(hi.n_rows, 1u));
-  cr = std::min<uint32_t>(FX_BLOCK, std::max<uint32_t>(cr, min_chunk));
+  const uint32_t cr = packed >> 16;
+  hl->sub_rows = packed & 0xffffu;
   hl->chunk_rows = cr;
   hl->chunks = (hi.n_rows + cr - 1) / cr;
-  // A launch whose first sub-tiles alone are megabytes of requests floods the memory system: there
-  // the counts get a head start (fx_head.hip; neutral on some boxes, 5 us of 26 on others).  A
-  // small launch would only lose the time.
-  const uint64_t first_bytes = (uint64_t)hl->chunks * hi.n_tasks * std::min<uint32_t>(cr, hl->sub_rows) * hi.S * 4u;
-  hl->bulk_delay = first_bytes >= FX_HEAD_FLOOD_BYTES ? FX_HEAD_BULK_DELAY : 0u;
+  hl->bulk_delay = fx_head_hold_back(hi.n_rows, hi.n_tasks, hi.S);
   return FX_OK;
 }
 

@@ -294,7 +294,7 @@ __global__ __launch_bounds__(FX_BLOCK) void fx_head_stream(const FxHeadLaunch hl
 }  // namespace
 
 uint32_t fx_head_lds_bytes(const FxHeadLaunch& hl) {
-  return (((hl.sub_rows * hl.S + 3u + 3u) >> 2) + 1u) * 16u;
+  return fx_head_window_bytes(hl.sub_rows, hl.S);
 }
 
 // Workgroups of the kernel that the current device holds at once.

@@ -146,6 +146,7 @@ struct Plan {
   // the same for the chunks of the detection-head kernel, and the workgroups of it the device holds at once
   std::vector<Status> head_status;
   uint32_t head_resident = 0;
+  uint32_t head_rows = 0;            // head kernel: rows of a chunk << 16 | rows of a sub-tile (0: not worked out yet)
   uint32_t cmap_resident_wide = 0;   // class-map head kernel: workgroups of its wide form
   FxLeanArgs lean{};           // dense regions that fit the lean kernel: its argument block but for the per-call parts (n_outs 0: none)
   uint32_t lean_slot_err = 0;  // as FxHeader::slot_err
