@@ -135,6 +135,10 @@ __global__ __launch_bounds__(FX_PAIRS_THREADS) void fx_nms_rank_kernel(const fx_
 }
 
 // grid: (columns of 32, four to a workgroup; chunks of 64 boxes; tasks)
+// RESOLVE: fx_nms_resolve_kernel follows, whose workgroups find the results cleared (the walk's one workgroup fills them to
+// the end itself: of few boxes this launch has few threads for it.  200 boxes, three launches: 12.8 us so, 13.0 cleared here,
+// the call 29.0 against 29.5 to 31)
+template <bool RESOLVE>
 __global__ __launch_bounds__(256) void fx_nms_pairs_kernel(const fx_nms_desc d) {
   __shared__ float4 s_box[4][32];
   __shared__ float s_area[4][32];
@@ -142,7 +146,7 @@ __global__ __launch_bounds__(256) void fx_nms_pairs_kernel(const fx_nms_desc d) 
   const uint32_t n = d.rows, nw = (n + 63u) >> 6;
   const uint32_t chunk = blockIdx.y, col = blockIdx.x * 4u + wave;
   const PairsWs ws = pairs_ws(d.workspace, n, blockIdx.z);
-  {
+  if constexpr (RESOLVE) {
     // the results start out as zeros (rows past the kept ones stay so: the outputs have a fixed shape), the
     // chunks as undecided; the next launch is the first to touch either
     const uint32_t at = (chunk * gridDim.x + blockIdx.x) * 256u + threadIdx.x, step = gridDim.x * gridDim.y * 256u;
@@ -287,14 +291,15 @@ __global__ __launch_bounds__(FX_PAIRS_THREADS) void fx_nms_walk_kernel(const fx_
   float* dets = d.dets + (size_t)task * d.max_num * 5u;
   int64_t* out_labels = d.out_labels + (size_t)task * d.max_num;
   int64_t* out_index = d.out_index ? d.out_index + (size_t)task * d.max_num : nullptr;
-  for (uint32_t k = tid; k < nk; k += FX_PAIRS_THREADS) {   // (nk <= max_num; rows past the kept ones are zero already)
-    const uint32_t i = ws.row[s_kept[k]];
-    const float4 b = *(const float4*)(boxes + (size_t)i * 4u);
+  for (uint32_t k = tid; k < d.max_num; k += FX_PAIRS_THREADS) {   // rows past the kept ones are zero: the outputs have a fixed shape
+    const bool live = k < nk;
+    const uint32_t i = live ? ws.row[s_kept[live ? k : 0u]] : 0u;
+    const float4 b = live ? *(const float4*)(boxes + (size_t)i * 4u) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float* o = dets + (size_t)k * 5u;
     o[0] = b.x; o[1] = b.y; o[2] = b.z; o[3] = b.w;
-    o[4] = scores[i];
-    out_labels[k] = labels ? (int64_t)(uint32_t)labels[i] : 0;
-    if (out_index) out_index[k] = (int64_t)i;
+    o[4] = live ? scores[i] : 0.0f;
+    out_labels[k] = live && labels ? (int64_t)(uint32_t)labels[i] : 0;
+    if (out_index) out_index[k] = live ? (int64_t)i : 0;
   }
 }
 
@@ -492,9 +497,11 @@ size_t fx_nms_pairs_ws_bytes(int n_tasks, uint32_t rows) { return (size_t)n_task
 int fx_launch_nms_pairs(const fx_nms_desc& d, uint32_t spin_limit, hipStream_t stream) {
   const uint32_t nw = (d.rows + 63u) / 64u;
   hipLaunchKernelGGL(fx_nms_rank_kernel, dim3((uint32_t)d.n_tasks * 4u * nw), dim3(FX_PAIRS_THREADS), (size_t)nw * 64u * 8u, stream, d);
-  hipLaunchKernelGGL(fx_nms_pairs_kernel, dim3((2u * nw + 3u) / 4u, nw, (uint32_t)d.n_tasks), dim3(256), 0, stream, d);
   // level at 16 chunks, and ahead of each other on either side of it; with few to be kept the walk may end early (top)
-  if (nw > 16u && (uint64_t)d.max_num * 4u >= d.rows) {
+  const bool by_chunks = nw > 16u && (uint64_t)d.max_num * 4u >= d.rows;
+  auto* pairs = by_chunks ? fx_nms_pairs_kernel<true> : fx_nms_pairs_kernel<false>;
+  hipLaunchKernelGGL(pairs, dim3((2u * nw + 3u) / 4u, nw, (uint32_t)d.n_tasks), dim3(256), 0, stream, d);
+  if (by_chunks) {
     auto* resolve = nw <= 31u ? fx_nms_resolve_kernel<2> : nw <= 46u ? fx_nms_resolve_kernel<3> : fx_nms_resolve_kernel<5>;
     hipLaunchKernelGGL(resolve, dim3((uint32_t)d.n_tasks * nw), dim3(FX_PAIRS_THREADS), 0, stream, d, spin_limit);
   } else {

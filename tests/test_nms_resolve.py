@@ -62,3 +62,32 @@ def test_waits_that_are_given_up(n):
         finally:
             lib.fx_set_stream_spin_limit(4000)
         assert kept == _same(b, s, lab, iou_threshold=0.4, max_num=1024) and kept[2] == 0
+
+
+# both third launches, and rows of which fewer are kept than the outputs hold
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,max_num", [(129, 1024), (1024, 1024), (1025, 1024), (1025, 256), (4096, 1023)])
+def test_rows_past_the_kept_ones_are_zero_whatever_the_outputs_held(n, max_num):
+    import ctypes
+    from functs_amd._lib import FxNmsDesc, check
+    b, s, lab = (t.cuda() for t in _crowd(2, n, 60.0, seed=n))
+    print("n=%d max_num=%d" % (n, max_num), flush=True)
+    results = []
+    for fn, ws in ((lib.fx_nms_pairs, torch.empty(lib.fx_nms_pairs_workspace_bytes(2, n), dtype=torch.uint8, device="cuda")),
+                   (lib.fx_sort_nms, torch.zeros(lib.fx_sort_nms_workspace_bytes(2, 4096), dtype=torch.uint8, device="cuda"))):
+        out = (torch.full((2, max_num, 5), float("nan"), device="cuda"), torch.full((2, max_num), -7, dtype=torch.long, device="cuda"),
+               torch.full((2, max_num), -7, dtype=torch.long, device="cuda"), torch.full((2,), -7, dtype=torch.int32, device="cuda"))
+        d = FxNmsDesc()
+        d.n_tasks, d.rows, d.max_num, d.key_capacity, d.score_thr, d.iou_thr = 2, n, max_num, 4096, float("-inf"), 0.3
+        d.boxes, d.boxes_task_stride, d.scores, d.scores_task_stride = b.data_ptr(), b.stride(0), s.data_ptr(), s.stride(0)
+        d.labels, d.labels_task_stride = lab.data_ptr(), lab.stride(0)
+        d.dets, d.out_labels, d.out_index, d.n_out = (t.data_ptr() for t in out)
+        d.workspace, d.workspace_bytes = ws.data_ptr(), ws.numel()
+        check(fn(ctypes.byref(d), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        results.append(out)
+    (dets, labels, index, kept), want = results
+    assert all(torch.equal(a, w) for a, w in zip(results[0], want))
+    for t in range(2):
+        k = int(kept[t])
+        assert 0 < k < max_num and not bool(dets[t, k:].any()) and not bool(labels[t, k:].any()) and not bool(index[t, k:].any())
