@@ -204,7 +204,7 @@ __global__ __launch_bounds__(W * 64) void fx_attention_kernel(const FxAttnArgs a
     top = wave_max(top);
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-      e[j] = expf(e[j] - top);
+      e[j] = expf(e[j] - top) * (1.0f / (R * 64));   // (a power of two: the weights add up to no more than 1, so y is no larger than V)
       sum += e[j];
     }
 #pragma unroll

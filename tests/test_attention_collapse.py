@@ -189,3 +189,18 @@ def test_a_nan_stays_in_its_head():
     cuda = [a.cuda() if isinstance(a, Tensor) else a for a in args]
     x = fj.build(fj.script(PROGRAMS["attention"]), cuda)(*cuda)[2].cpu()
     assert bool(x[1, 2].isnan().all()) and int(x.isnan().sum()) == 64
+
+
+# largest finite values: the weights add up to one, so what the loop computes is no larger than they are
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [20, 100, 250, 500])
+def test_the_largest_values_do_not_overflow_ahead_of_the_normalisation(rows):
+    args = _args(rows, 1, 2, rows, rows - 3)
+    args[2].fill_(3e38)
+    for w in args[3:6]:
+        w.zero_()
+    args[6].copy_(torch.eye(64) * 0.25)
+    cuda = [a.cuda() if isinstance(a, Tensor) else a for a in args]
+    got = fj.build(fj.script(PROGRAMS["attention"]), cuda)(*cuda)
+    assert bool(got[2].isfinite().all())
+    _compare(got, _in_64_bits(*args), rows)
