@@ -1281,7 +1281,7 @@ void runLstmStack(Stack& stack) {
 //     k[:, :, row] = x @ wk; v[:, :, row] = x @ wv
 //     x = softmax((k @ (x @ wq)^T)^T * scale) @ v @ wo
 // in functional form: the results are new tensors.  Operands that the kernel is not made for (a
-// gradient wanted, autocast, other types or sizes than the graph was built for) run it as ATen's operators.
+// gradient or tangent wanted, autocast, other types or sizes than the graph was built for) run it as ATen's operators.
 void runAttentionSteps(Stack& stack) {
   auto in = last(stack, 12);
   at::Tensor t[7];
@@ -1298,7 +1298,8 @@ void runAttentionSteps(Stack& stack) {
     const int64_t B = x0.size(0), H = x0.size(1), D = x0.size(3), rows = k0.size(2);
     const std::vector<int64_t> cache{B, H, rows, D}, weight{H, D, D};
     for (size_t i = 0; i < 7; ++i) {
-      kernel = kernel && t[i].scalar_type() == at::kFloat && t[i].device() == x0.device() && !t[i].is_neg() && !(at::GradMode::is_enabled() && t[i].requires_grad());
+      kernel = kernel && t[i].scalar_type() == at::kFloat && t[i].device() == x0.device() && !t[i].is_neg() && !(at::GradMode::is_enabled() && t[i].requires_grad()) &&
+               !t[i]._fw_grad(0).defined();
       if (i > 0) kernel = kernel && t[i].sizes() == at::IntArrayRef(i < 3 ? cache : weight);
     }
     kernel = kernel && D <= INT32_MAX && rows <= INT32_MAX && fx_attention_steps_fits((int)D, (int)rows) && B * H <= INT32_MAX / 512;

@@ -204,3 +204,20 @@ def test_the_largest_values_do_not_overflow_ahead_of_the_normalisation(rows):
     got = fj.build(fj.script(PROGRAMS["attention"]), cuda)(*cuda)
     assert bool(got[2].isfinite().all())
     _compare(got, _in_64_bits(*args), rows)
+
+
+@pytest.mark.gpu
+def test_tangents_pass_through():
+    import torch.autograd.forward_ad as fwd
+    args = _args(8, 1, 2, 24, 20)
+    cuda = [a.cuda() if isinstance(a, Tensor) else a for a in args]
+    fn = fj.build(fj.script(PROGRAMS["attention"]), cuda)
+    _compare(fn(*cuda), _in_64_bits(*args), "no tangent")
+    along = torch.randn(cuda[0].shape, generator=torch.Generator().manual_seed(9))
+    with fwd.dual_level():
+        out = [fwd.unpack_dual(o) for o in fn(fwd.make_dual(cuda[0], along.cuda()), *cuda[1:])]
+        want = [fwd.unpack_dual(o) for o in _in_64_bits(fwd.make_dual(args[0].double(), along.double()), *args[1:])]
+        assert all(o.tangent is not None for o in out)
+        _compare([o.primal for o in out], [w.primal for w in want], "values")
+        for name, o, w in zip("kvx", out, want):   # (a derivative passes through the same products)
+            assert float((o.tangent.double().cpu() - w.tangent).abs().max()) <= 1e-4 * float(w.tangent.abs().max()), name
