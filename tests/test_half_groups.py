@@ -34,3 +34,20 @@ def test_one_operation(dtype, rows, cols, lo):
     one, three = run_region("hip", r, x)
     _same(one, x + 1.0)
     _same(three, x.t() * 3.0)
+
+
+# Whole groups are rounded two values at a time, the rest one by one (fx_bf16_pair, fx_bf16): every upper half of a float with lower
+# halves below, at and above a tie.  Subnormal results, results that round up to infinity and every kind of NaN are among them.
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [3, 4, 6, 4096])
+def test_bfloat16_rounding_of_every_upper_half(cols):
+    low = torch.tensor([0, 1, 0x7fff, 0x8000, 0x8001, 0xffff, 0x8000, 0x4000], dtype=torch.int64)
+    bits = (torch.arange(1 << 16).view(-1, 1) << 16 | low).view(-1)
+    bits = bits[:bits.numel() // (2 * cols) * 2 * cols].to(torch.uint32).view(torch.float32)
+    x = torch.cat([bits, bits.flip(0)]).view(-1, cols)      # (either place of a pair)
+    r = Region()
+    a = r.tensor_input(torch.float32, 2)
+    r.output(a.to(torch.bfloat16))
+    r.finalize()
+    (got,) = run_region("hip", r, x)
+    _same(got, x.to(torch.bfloat16))
