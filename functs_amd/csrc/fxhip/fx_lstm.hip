@@ -134,7 +134,7 @@ __global__ __launch_bounds__(FX_LSTM_BLOCK * UPW, HPT >= 32 ? 4 : 2) void fx_lst
   const int wg = (n_wg % 8 == 0) ? ((int)blockIdx.x % 8) * (n_wg / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
   const int u0 = wg * UPW;
   // a workspace that still carries a given-up wait is refused (below, behind the first barrier)
-  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) || fx_lstm_refused<DevAtomics>(a.ctl_third) ? 1u : 0u;
+  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a) ? 1u : 0u;
   // tags of this launch start behind those of every launch before it
   const uint32_t base = DevAtomics::load(a.ctl + FX_LSTM_W_BASE);
 
@@ -447,7 +447,7 @@ __global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_row
   const int wg = (n_wg % 8 == 0) ? (gi % 8) * (n_wg / 8) + gi / 8 : gi;
   const int u0 = wg * 4;
   const int b0 = group * 4 * MT, nb = min(4 * MT, B - b0);
-  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) || fx_lstm_refused<DevAtomics>(a.ctl_third) ? 1u : 0u;
+  if (tid == 0) s_abort = fx_lstm_refused<DevAtomics>(a) ? 1u : 0u;
   const uint32_t base = DevAtomics::load(a.ctl + FX_LSTM_W_BASE);
   const int n_steps = fx_lstm_steps(T, L);
   const uint32_t BH = (uint32_t)(B * HH);               // elements of one vector of all rows
@@ -846,7 +846,7 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
   }
   if (tid < 2) s_abort[tid] = 0u;
   __syncthreads();
-  if (tid == 0 && (fx_lstm_refused<DevAtomics>(a.ctl) || fx_lstm_refused<DevAtomics>(a.ctl_other) || fx_lstm_refused<DevAtomics>(a.ctl_third))) s_abort[1] = 1u;
+  if (tid == 0 && fx_lstm_refused<DevAtomics>(a)) s_abort[1] = 1u;
   uint64_t* const where = a.hbuf + area.where + slot * FX_LSTM_DIE_WG;
   if (tid == 0) DevAtomics::store64(where + gi, fx_lstm_pack(fx_die_of_wave(), base + 1u));
   auto give_up = [&](int d) {   // the workgroup leaves behind the barrier of step d, the next one

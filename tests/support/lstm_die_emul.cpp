@@ -41,7 +41,7 @@ struct Run {
     return true;
   }
   void workgroup(int b, int stage, int gi) const {
-    const bool refused = fx_lstm_refused<HostAtomics>(a.ctl) || fx_lstm_refused<HostAtomics>(a.ctl_other) || fx_lstm_refused<HostAtomics>(a.ctl_third);
+    const bool refused = fx_lstm_refused<HostAtomics>(a);
     const bool done = !refused && steps(b, stage, gi);
     if (refused) *a.err_host = 2u;
     if (!done && !(stage == stop_stage && gi == stop_wg)) fx_lstm_poison(a, L, 0u, 1u);
