@@ -719,7 +719,7 @@ __global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_row
 // us a launch, T = 64, this : the forms above: 512 units, one sequence, one to three layers 80 : 110, 92 : 119, 98 : 188;
 // two layers, four sequences 98 : 219; 256 units, four layers, four sequences 89 : 207; 128, three, eight 71 : 125;
 // 64, one, one 47 : 105.  T = 100, 256 units, three layers, eight sequences 131 : 269.  T = 8: 27 : 28 (512, two
-// layers), 12 : 16 (64, one), 20 : 20 (64, three, eight sequences).
+// layers), 12 : 16 (64, one); shorter sequences: fx_lstm_die_from.
 // The same workgroups spread over the chip (spread: slot after slot, every slot on all dies; only those that have a
 // sequence are launched) compute the same bits with values that go to the memory side, for launches that must
 // not hold a die: 512 units, two layers, one sequence 93 on dies, 110 spread, 122 row by row; three layers of 256, four
@@ -832,7 +832,9 @@ __global__ __launch_bounds__((FxLstmDie<E, NL>::threads)) void fx_lstm_die_kerne
   const int B = a.B, T = a.T;
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int slot = spread ? (int)blockIdx.x / FX_LSTM_DIE_WG : (int)blockIdx.x % FX_LSTM_DIES;
-  const int gi = spread ? (int)blockIdx.x % FX_LSTM_DIE_WG : (int)blockIdx.x / FX_LSTM_DIES;
+  // (spread: workgroups of one die, every eighth, take neighbouring units, whose weights share lines)
+  const int gi = spread ? ((int)blockIdx.x % FX_LSTM_DIES) * (FX_LSTM_DIE_WG / FX_LSTM_DIES) + (int)blockIdx.x % FX_LSTM_DIE_WG / FX_LSTM_DIES
+                        : (int)blockIdx.x / FX_LSTM_DIES;
   const int stages = L / NL, b = slot / stages, stage = slot % stages, j0 = stage * NL;
   const int u0 = gi * K::U;
   const int n_steps = fx_lstm_stage_steps(T, NL);
@@ -1235,8 +1237,9 @@ int fx_launch_lstm_stack(const FxLstmArgs& args, int L, uint32_t* words_ctl, uin
     const bool half = 2u * want <= (uint32_t)cus * FX_LSTM_CU;
     if (asked != FX_LSTM_FORM_ANY) {
       if (capturing && !half) continue;   // (a replay may run beside any other)
-    } else if (f[i].form == FX_LSTM_FORM_DIE ? capturing || want > device || groups.others(id, thread) : f[i].form == FX_LSTM_FORM_SPREAD && !half) {
-      continue;
+    } else if (f[i].over == LSTM_DIE) {
+      if (a.T < fx_lstm_die_from(a.B, a.H, L)) continue;
+      if (f[i].form == FX_LSTM_FORM_DIE ? capturing || want > device || a.T < fx_lstm_die_alone(a.B, a.H, L) || groups.others(id, thread) : !half) continue;
     }
     if (l && want >= need) continue;
     l = &f[i];

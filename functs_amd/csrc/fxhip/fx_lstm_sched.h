@@ -158,6 +158,24 @@ FX_LSTM_HD inline int fx_lstm_stage_layers(int H, int L) { return H > 256 ? 1 : 
 FX_LSTM_HD inline bool fx_lstm_die_fits(int B, int H, int L) {
   return (H == 64 || H == 128 || H == 256 || H == 512) && L >= 1 && L <= 4 && B >= 1 && B * (L / fx_lstm_stage_layers(H, L)) <= FX_LSTM_DIES;
 }
+// A launch's start costs more on dies (one die fetches a layer's weights) and a step less, so the shortest sequences are the other
+// forms', in calls and in captures.  The fewest steps that the kernel is taken for; speed of the best other form = 1, one step ahead of
+// the line and at it (weights in the caches; from further away the kernel is ahead sooner): 64 units, three layers, eight sequences
+// 0.94, 0.99, two layers, four 0.92, 1.06, one, one 0.89, 1.08; 128, four layers, four 1.00, 1.04; 256, three, four 0.97, 1.01; 512, one,
+// eight 0.89, 0.96.  (Spread over the chip, 64 and 128 units lose up to a fifth between this line and some 16 steps: what is captured
+// there has the bits of the calls instead.)
+FX_LSTM_HD inline int fx_lstm_die_from(int B, int H, int L) {
+  if (H <= 128 && B == 1) return 2;
+  if (H == 64) return (L > 2 ? 5 : 3) + (B > 3) + (B > 5);
+  if (H == 128) return L > 2 ? 5 : 3 + (B > 5);
+  if (H == 256) return L == 4 ? 1 : L == 3 ? 5 : L + 1;
+  return L == 1 && B > 4 ? 5 : L == 2 && B > 2 ? 3 : 1;
+}
+// The fewest steps for which its workgroups are placed on dies while nothing else is about; below, spread.  512 units, call
+// on dies : spread : row by row, one sequence, one layer: 8 steps 23.0 : 18.6 : 21.6, 24 steps 40.3 : 40.1, 32 steps 49.0 : 50.9; two
+// layers: 8 steps 27.7 : 27.4 : 30.0, 12 steps 32.1 : 33.0; two sequences: 16 steps 39.6 : 37.9, 24 steps 48.8 : 49.5; three
+// layers: 8 steps 32.0 : 31.7, 12 steps 37.0 : 37.3.
+FX_LSTM_HD inline int fx_lstm_die_alone(int B, int H, int L) { return H < 512 || L * B > 4 || L > 3 ? 1 : L == 1 ? 24 : L == 2 ? 10 * B : 10; }
 // 64-bit words behind the control words: h [2][L][B][H]; rings [stages - 1][B][FX_LSTM_RING][H]; counts of read
 // vectors [stages - 1][B][FX_LSTM_DIE_WG]; the die that every workgroup runs on [FX_LSTM_DIES][FX_LSTM_DIE_WG]
 struct FxLstmDieArea { uint32_t ring, read, where, words; };

@@ -79,9 +79,9 @@ def test_streams_that_launched_lately_are_told_apart(emul):
         assert others(1, 5, 64, device, 7) == 1     # a second stream's first launch
 
 
-# sizes whose workgroups, spread over the chip, take at most half of it
+# sizes whose workgroups, spread over the chip, take at most half of it; (5, 64, 3, 8): fewer steps than the kernel is taken for
 @pytest.mark.gpu
-@pytest.mark.parametrize("T,H,L,B", [(9, 64, 2, 1), (5, 64, 3, 8), (6, 128, 3, 8), (6, 128, 4, 3), (7, 256, 3, 4), (9, 256, 4, 2), (20, 512, 2, 1), (8, 512, 4, 1), (6, 512, 1, 4)])
+@pytest.mark.parametrize("T,H,L,B", [(9, 64, 2, 1), (12, 64, 3, 8), (5, 64, 3, 8), (6, 128, 3, 8), (6, 128, 4, 3), (7, 256, 3, 4), (9, 256, 4, 2), (20, 512, 2, 1), (8, 512, 4, 1), (6, 512, 1, 4)])
 def test_a_captured_stack_computes_what_the_calls_beside_it_compute(T, H, L, B):
     """To the bit, whether or not another stream has launched stacks lately."""
     from functs_amd import jit as fj
@@ -90,6 +90,7 @@ def test_a_captured_stack_computes_what_the_calls_beside_it_compute(T, H, L, B):
     from oracle import configs as oc
     args = oc.c4_inputs(3, T, H, L, B)
     gpu = [a.cuda() if isinstance(a, torch.Tensor) else a for a in args]
+    form = C["FX_LSTM_FORM_ROWS" if (T, H) == (5, 64) else "FX_LSTM_FORM_SPREAD"]
     eager = fj.build(fj.script(PROGRAMS["c4"]), list(args))
     for other in (False, True):
         if other:
@@ -98,7 +99,7 @@ def test_a_captured_stack_computes_what_the_calls_beside_it_compute(T, H, L, B):
             torch.cuda.synchronize()
         graphed = fj.build(fj.script(PROGRAMS["c4"]), list(args), hip_graph=True)
         graphed(*gpu)
-        assert lib.fx_lstm_form() == C["FX_LSTM_FORM_SPREAD"]
+        assert lib.fx_lstm_form() == form
         for _ in range(3):
             want = eager(*gpu)
             torch.cuda.synchronize()
@@ -106,7 +107,7 @@ def test_a_captured_stack_computes_what_the_calls_beside_it_compute(T, H, L, B):
                 assert torch.equal(g, w), "after launches on another stream: %s" % other
     with torch.cuda.stream(torch.cuda.Stream()):   # and beside the other stream's
         beside = eager(*gpu)
-        assert lib.fx_lstm_form() == C["FX_LSTM_FORM_SPREAD"]
+        assert lib.fx_lstm_form() == form
     torch.cuda.synchronize()
     assert all(torch.equal(b, w) for b, w in zip(beside, want))
 
@@ -221,3 +222,16 @@ def test_operands_of_any_float_alignment():
     torch.cuda.synchronize()
     assert lib.fx_async_error(1) == 0
     _close([t.cpu() for t in out], _reference(*args), "odd alignment")
+
+
+# either side of the fewest steps that the kernel is taken for, whatever else the process has launched or captured
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,L,B,other", [(1, 64, 1, 1, "SINGLE"), (2, 64, 1, 1, None), (3, 64, 2, 4, "ROWS"), (4, 64, 2, 4, None), (6, 64, 3, 8, "ROWS"),
+                                           (7, 64, 3, 8, None), (2, 128, 2, 3, "ROWS"), (3, 128, 2, 3, None), (4, 128, 3, 8, "ROWS"), (5, 128, 3, 8, None),
+                                           (4, 256, 3, 4, "ROWS"), (5, 256, 3, 4, None), (1, 256, 4, 2, None), (5, 512, 1, 4, "SPREAD"), (23, 512, 1, 1, "SPREAD"),
+                                           (9, 512, 2, 1, "SPREAD"), (19, 512, 2, 2, "SPREAD"), (1, 512, 3, 1, "SPREAD")])
+def test_short_sequences_take_the_forms_that_start_sooner(T, H, L, B, other):
+    from functs_amd._lib import C, lib
+    args = _inputs(T + H + L + B, T, H, L, B)
+    _close(_gpu(*args, launches=2), _reference(*args), "T=%d H=%d L=%d B=%d" % (T, H, L, B))
+    assert lib.fx_lstm_form() in ([C["FX_LSTM_FORM_" + other]] if other else [C["FX_LSTM_FORM_DIE"], C["FX_LSTM_FORM_SPREAD"]])
