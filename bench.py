@@ -639,12 +639,12 @@ def main():
                 "torchscript_route_functors": n_functors, "torchscript_route_compiled_share": round(spec_share, 3),
                 "loops_collapsed": collapsed,
                 "launches_per_call": (l1 - l0) / n_rep,
-                "dependent_steps": seq_len + layers - 1,
-                "us_per_dependent_step": round(dev_us / (seq_len + layers - 1), 2),
+                "dependent_steps": seq_len + 2 * (layers - 1),
+                "us_per_dependent_step": round(dev_us / (seq_len + 2 * (layers - 1)), 2),
                 "algorithmic_bytes": alg, "gbps_call": round(alg / (cold_us * 1e-6) / 1e9, 1),
                 "frac_hbm_peak": round(alg / (cold_us * 1e-6) / 1e9 / HBM_PEAK_GBPS, 5),
-                "bound": "latency of %d dependent steps (each one hand-over of the h vectors between all workgroups through the "
-                         "memory side of the caches), not HBM" % (seq_len + layers - 1)}
+                "bound": "latency of %d dependent steps (each one hand-over of a layer's h between the 32 workgroups of a die through "
+                         "its cache, a layer two steps behind the one below), not HBM" % (seq_len + 2 * (layers - 1))}
 
     def run_tail():
         """The step behind the hot path: c5's compaction followed by the detection tail

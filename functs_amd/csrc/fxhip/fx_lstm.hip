@@ -722,8 +722,9 @@ __global__ __launch_bounds__((FxLstmRows<L, HPT, MT>::threads)) void fx_lstm_row
 // layers), 12 : 16 (64, one); shorter sequences: fx_lstm_die_from.
 // The same workgroups spread over the chip (spread: slot after slot, every slot on all dies; only those that have a
 // sequence are launched) compute the same bits with values that go to the memory side, for launches that must
-// not hold a die: 512 units, two layers, one sequence 93 on dies, 110 spread, 122 row by row; three layers of 256, four
-// sequences 92, 114, 178 (tiles of rows); 128, three, eight 72, 101, 126; 64, three, eight 63, 95, 105; 64, one, one 48, 77, 108.
+// not hold a die: 512 units, two layers, one sequence 93 on dies, 101 spread (110 before neighbouring units were one die's), 119 row
+// by row; three layers of 256, four sequences 91, 111, 178 (tiles of rows); 128, three, eight 70, 102, 125; 64, three, eight 60, 94, 106;
+// 64, one, one 46, 73, 106.
 // A step of two layers of 512 units is 1.1 us:
 // 0.3 from the barrier to the cells' stores, 0.3 until they are seen, 0.35 products, 0.1 sums (on the SIMD that also
 // finishes cells, the others wait for it); of 64 units 0.65.

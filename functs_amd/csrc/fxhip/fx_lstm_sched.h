@@ -32,7 +32,7 @@
 #define FX_LSTM_W_LEAVE (1u * FX_LSTM_LINE)       // workgroups that have left
 #define FX_LSTM_W_ERR (2u * FX_LSTM_LINE)         // a wait was given up
 #define FX_LSTM_CTL_WORDS (3u * FX_LSTM_LINE)
-#define FX_LSTM_TAG_WRAP 0x80000000u              // the base starts over (and the tags are cleared) beyond this
+#define FX_LSTM_TAG_WRAP 0x80000000u              // the base starts over (and the tags are cleared, fx_lstm_leave) beyond this
 
 // The second hand-over, of the kernel for groups of rows (one row at a time goes by tags): an element is ONE
 // 32-bit word, its value with all bits inverted, and 0 says that it has not been written yet (the
@@ -111,9 +111,12 @@ FX_LSTM_HD inline void fx_lstm_poison(const FxLstmArgs& a, int L, uint32_t first
 // A workgroup that has finished its last step checks out; the last one to do so (nobody reads
 // or writes hbuf any more) moves the tag base past this launch's tags and puts the counter back
 // to zero, so the same workspace serves the next launch on the stream without a clear in
-// between.  Past FX_LSTM_TAG_WRAP the base starts over at zero and the tags in hbuf are cleared
-// first.  A workgroup that gave up a wait does not check out: the error word stays set and the
-// host clears the whole workspace before it is used again.
+// between.  Past FX_LSTM_TAG_WRAP the base starts over at zero, and the tags in hbuf are cleared
+// first: at the memory side.  What the kernel on dies has stored to a die's cache only may be written
+// back on top of that when the launch ends, and is overwritten by the next launch that waits for that
+// place: a tag left over would have to lie untouched for 2^31 steps to be one that is waited for.
+// A workgroup that gave up a wait does not check out: the error word stays set and the host clears the
+// whole workspace before it is used again.
 //   A: atomics policy { add(uint32_t*) -> old value, load(uint32_t*), store(uint32_t*, v), store64(uint64_t*, v) }
 template <class A>
 FX_LSTM_HD inline void fx_lstm_leave(uint32_t* ctl, uint32_t n_wg, uint32_t base, uint32_t n_steps, uint64_t* hbuf,

@@ -439,8 +439,8 @@ int fx_compact_rows_static(const uint8_t* mask, int64_t n, const void* const* co
  * workgroups find places together (four stacks of 512 units, two layers, one sequence each, for instance);
  * one that does not fit waits, in its stream, for the launches before it (a launch on another stream than the
  * legacy default one records an event behind it for that).  Dies of their own are for launches while no other stream
- * launches; beside others (within 64 launches) and in captures the same kernel takes 32 workgroups a sequence
- * and stage anywhere on the chip.  A captured launch cannot be
+ * launches; beside others (within 64 launches), in captures, and for few steps of 512 units the same kernel takes 32
+ * workgroups a sequence and stage anywhere on the chip; the shortest sequences are other forms', whatever else runs.  A captured launch cannot be
  * made to wait: it, and from then on every launch on that device, takes a form for half of the device
  * where there is one, so that ONE replay and the calls, or two replays, may run at the same time.
  * Results: the two placements give the same bits, so what a launch computes depends on the operands and the device
@@ -572,18 +572,19 @@ int fx_nms_pairs(const fx_nms_desc* desc, void* stream);
  * overlap tests and tasks * rows^2 / 16 keys read, whatever is kept; fx_sort_nms gives every task a CU of its
  * own (up to 256 tasks take the time of one) and walks what it keeps, at most max_num boxes, and only a call's
  * candidates: a score threshold is its case (16 tasks of 4 096 rows, 1 in 10 above it: 32 us, fx_nms_pairs 206).
- * Microseconds a call, launches back to back, fx_sort_nms (300 kept; max_num and as many kept 1 024) : fx_nms_pairs
- *     rows     1 task          4 tasks          8 tasks          16 tasks         32 tasks         128 tasks
- *     200      24 : 30         24 : 29          24 : 29          25 : 30          25 : 30          25 : 34
- *     500      40 : 30         40 : 29          40 : 30          40 : 29          41 : 29          38 : 56
- *     1 000    39, 117 : 30    38, 118 : 29     39, 118 : 29     39, 119 : 31     39, 119 : 46     41 : 139
- *     2 000    44, 199 : 29    44, 211 : 29     44, 211 : 41-51  44, 211 : 67-76  45, 223 : 117-127
- *     4 096    53, 194 : 30    54, 195 : 64-76  54, 196 : 111+   54, 196 : 204+   54, 198 : 391+
- * (since then resolving chunks side by side takes 7 us off one image of 2 000 rows that keeps up to 1 024, 29 off
- * 4 096 proposals of 60 objects, fx_nms_pairs.hip)
- * Hence bounds on tasks * rows and on tasks * rows^2, the latter moved by what may be kept.  Few rows are
- * bound by three launches against one when nobody waits for them; a caller of one image that does is served
- * faster from FX_NMS_PAIRS_MIN_ROWS on (129 rows 33 : 31, 200: 39 : 31, 400: 56 : 33; 64: 25.6 : 27.0). */
+ * Microseconds a call, launched back to back from one descriptor, fx_sort_nms : fx_nms_pairs; boxes apart from
+ * each other, the first 300 or 1 024 kept / proposals of 60 objects, at most 300 (walked from 1 200 rows on) or 1 024 kept
+ *     rows     1 task                      4 tasks                     8 tasks                     16 tasks                    32 tasks
+ *     200      21:13 22:13 / 18:13 19:13   22:13 22:13 / 19:13 19:13   23:14 23:14 / 19:14 19:14   23:14 23:14 / 19:14 19:14   23:15 24:15 / 19:15 20:15
+ *     500      28:14 48:15 / 30:15 30:15   29:14 48:15 / 30:15 30:15   29:15 48:16 / 30:16 30:16   29:17 49:18 / 30:18 30:18   29:22 49:23 / 30:23 31:23
+ *     1 000    30:15 135:20 / 50:19 50:19  31:16 137:21 / 49:20 50:20  31:20 137:25 / 50:24 50:25  31:28 138:33 / 50:33 51:33  31:44 138:49 / 50:49 50:49
+ *     2 000    36:17 142:17 / 91:32 91:20  36:26 143:27 / 92:41 92:30  37:40 144:41 / 92:54 92:46  37:65 144:70 / 92:80 92:76  37:114 144:127 / 93:128 93:136
+ *     4 096    51:29 157:31 / 178:73 179:31  52:64 158:67 / 180:109 180:68  52:110 159:117 / 181:154 181:121  52:202 159:223 / 181:249 182:231  52:389 159:436 / 182:434 182:452
+ * (128 tasks of 200 rows 22 : 25, of 500 29 : 50.)  Hence bounds on tasks * rows and on tasks * rows^2, the latter moved by what may
+ * be kept.  They lie on the safe side, where the first of the four columns turns: 16 tasks of 2 000 proposals, and four to
+ * eight of 4 096, would be faster as three launches and are not sent there.  (8 tasks of 2 000 rows apart, of which 300 are kept, lie
+ * just beyond it: 37 : 40.)  Few rows: a caller that prepares every call (functs_amd.detection, 24 us of host work) pays for three
+ * launches instead of one when it does not wait, 200 rows 24 : 30, and gains when it does, 39 : 31; so one to four images are sent there. */
 int fx_nms_pairs_pays(int n_tasks, uint32_t rows, uint32_t max_num, float score_thr);
 
 /* ---- device utilities ---- */
