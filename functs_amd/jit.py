@@ -41,9 +41,12 @@ class AotScriptFunction(object):
 
     def __call__(self, *args, **kwargs):
         if kwargs:   # by name: through the ScriptFunction, which knows the argument names
-            if self._variants is not None or self._lazy_lists:
+            if self._lazy_lists:
                 raise TypeError("this built function takes positional arguments only")
-            return self._aot_script_fn(*args, **kwargs)
+            names = [a.name for a in self._aot_script_fn.schema.arguments][len(args):]
+            if self._variants is None or set(names) != set(kwargs):   # (which reports names that do not fit)
+                return self._aot_script_fn(*args, **kwargs)
+            args = args + tuple(kwargs[n] for n in names)
         if self._variants is None:
             return self._call(*args)
         key = _shape_key(args)

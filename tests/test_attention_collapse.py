@@ -47,6 +47,19 @@ def other_order(x: Tensor, k: Tensor, v: Tensor, wq: Tensor, wk: Tensor, wv: Ten
     return x, k, v
 
 
+def sizes_in_the_text(x: Tensor, k: Tensor, v: Tensor, wq: Tensor, wk: Tensor, wv: Tensor, wo: Tensor, start_len: int):
+    k = k.clone()
+    v = v.clone()
+    gen = start_len
+    for i in range(20 - start_len):
+        k[:, :, gen, :] = torch.matmul(x, wk).view(2, 3, 64)
+        v[:, :, gen, :] = torch.matmul(x, wv).view(2, 3, 64)
+        a = torch.softmax(torch.matmul(k, torch.matmul(x, wq).transpose(2, 3)).transpose(2, 3) * 0.125, dim=3)
+        x = torch.matmul(torch.matmul(a, v), wo)
+        gen = gen + 1
+    return k, v, x
+
+
 def softmax_over_the_depth(x: Tensor, k: Tensor, v: Tensor, wq: Tensor, wk: Tensor, wv: Tensor, wo: Tensor, start_len: int):
     gen = start_len
     for i in range(k.size(2) - start_len):
@@ -204,6 +217,19 @@ def test_the_largest_values_do_not_overflow_ahead_of_the_normalisation(rows):
     got = fj.build(fj.script(PROGRAMS["attention"]), cuda)(*cuda)
     assert bool(got[2].isfinite().all())
     _compare(got, _in_64_bits(*args), rows)
+
+
+@pytest.mark.gpu
+def test_arguments_by_name():
+    args = _args(11, 2, 3, 20, 14)
+    cuda = [a.cuda() if isinstance(a, Tensor) else a for a in args]
+    fn = fj.build(fj.script(sizes_in_the_text), cuda)
+    names = ["x", "k", "v", "wq", "wk", "wv", "wo", "start_len"]
+    before = aot.launch_stats()[0]
+    got = fn(*cuda[:3], **dict(zip(names[3:], cuda[3:])))
+    torch.cuda.synchronize()
+    assert aot.launch_stats()[0] - before == 1
+    _compare(got, _in_64_bits(*args), "by name")
 
 
 @pytest.mark.gpu

@@ -21,6 +21,18 @@ def _cuda(args):
 
 
 # ---- CPU ----------------------------------------------------------------------------------------
+def test_arguments_by_name_of_a_function_built_for_its_shapes():
+    def rows_times(x: torch.Tensor, n: int):
+        return x.size(0) * n
+
+    fn = fj.build(fj.script(rows_times), [torch.zeros(3, 2), 2])
+    assert fn._variants is not None
+    assert fn(x=torch.zeros(4, 2), n=5) == fn(torch.zeros(4, 2), n=5) == fn(torch.zeros(4, 2), 5) == 20
+    for wrong in ({"x": torch.zeros(4, 2)}, {"x": torch.zeros(4, 2), "m": 5}, {"x": torch.zeros(4, 2), "n": 5, "m": 5}):
+        with pytest.raises(RuntimeError):
+            fn(**wrong)
+
+
 def test_a_single_functor_graph_is_called_directly_and_others_through_the_interpreter():
     for name, small in (("c2", dict(grids=[2, 3, 4])), ("c5", dict(grids=[2, 3, 4], batch=3)), ("c1", dict(size=16, n=8))):
         args = INPUTS[name](0, **small)
