@@ -64,6 +64,20 @@ class FxNmsDesc(ctypes.Structure):
     ]
 
 
+class FxHeadDesc(ctypes.Structure):
+    """fx_head_desc of include/fxhip.h."""
+    _fields_ = [
+        ("n_levels", ctypes.c_int32),
+        ("keep_thr", ctypes.c_float),
+        ("maps", ctypes.c_void_p * 4),
+        ("bases", ctypes.c_void_p * 4),
+        ("shifts", ctypes.c_void_p * 4),
+        ("cells", ctypes.c_uint32 * 4),
+        ("anchors", ctypes.c_uint32 * 4),
+        ("strides", ctypes.c_void_p),
+    ]
+
+
 def _parse_header():
     """Opcode / dtype / error constants straight from the C header, so that the
     Python side can never drift from the ABI."""
@@ -193,6 +207,7 @@ _sig("fx_async_error_take", _i, _i)
 _sig("fx_async_error_report", None, _i)
 _fp = ctypes.c_void_p
 _sig("fx_sort_nms", ctypes.c_int, ctypes.POINTER(FxNmsDesc), ctypes.c_void_p)
+_sig("fx_head_nms", ctypes.c_int, ctypes.POINTER(FxHeadDesc), ctypes.POINTER(FxNmsDesc), ctypes.c_void_p)
 _sig("fx_nms_pairs", ctypes.c_int, ctypes.POINTER(FxNmsDesc), ctypes.c_void_p)
 _sig("fx_nms_pairs_pays", ctypes.c_int, ctypes.c_int, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_float)
 _sig("fx_nms_pairs_workspace_bytes", ctypes.c_size_t, ctypes.c_int, ctypes.c_uint32)

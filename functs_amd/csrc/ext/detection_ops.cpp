@@ -77,6 +77,24 @@ Tensor imagesContiguous(const Tensor& t, const char* op, const char* name) {
 struct Batched { Tensor dets, labels, index, n; };
 constexpr int32_t kPending = INT32_MIN + 1;   // no count and not FX_NMS_OVERFLOW (-1)
 
+// Memory for the results of a launch, and its places in the descriptor
+Batched resultsOf(fx_nms_desc& d, c10::Device dev, int64_t T, int64_t max_num, bool index) {
+  Batched r;
+  const auto f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
+  r.dets = at::empty({T, max_num, 5}, f32);
+  r.labels = at::empty({T, max_num}, f32.dtype(at::kLong));
+  if (index) r.index = at::empty({T, max_num}, f32.dtype(at::kLong));
+  // the kept counts land in pinned host memory, marked pending until the kernel stores them: the
+  // one wait of the tail is a poll of these words, not a synchronisation of the stream
+  r.n = at::empty({T}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  for (int64_t t = 0; t < T; ++t) r.n.data_ptr<int32_t>()[t] = kPending;
+  d.dets = r.dets.data_ptr<float>();
+  d.out_labels = r.labels.data_ptr<int64_t>();
+  d.out_index = index ? r.index.data_ptr<int64_t>() : nullptr;
+  d.n_out = (uint32_t*)r.n.data_ptr<int32_t>();
+  return r;
+}
+
 // One launch for all images.  boxes [T, K, 4]; mode 1: scores [T, K, row], of which the first
 // n_classes columns are class scores, factors [T, K] or undefined; mode 0: scores [T, K], labels
 // [T, K] int64 or undefined.  counts: int32 [T] on the device or in pinned host memory, or undefined.
@@ -130,19 +148,7 @@ Batched launch(const char* op, int mode, const Tensor& boxes_, const Tensor& sco
   d.iou_thr = (float)iou_thr;
   d.max_num = (uint32_t)max_num;
   d.key_capacity = FX_NMS_MAX_CANDIDATES;
-  Batched r;
-  const auto f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
-  r.dets = at::empty({T, max_num, 5}, f32);
-  r.labels = at::empty({T, max_num}, f32.dtype(at::kLong));
-  r.index = at::empty({T, max_num}, f32.dtype(at::kLong));
-  // the kept counts land in pinned host memory, marked pending until the kernel stores them: the
-  // one wait of the tail is a poll of these words, not a synchronisation of the stream
-  r.n = at::empty({T}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-  for (int64_t t = 0; t < T; ++t) r.n.data_ptr<int32_t>()[t] = kPending;
-  d.dets = r.dets.data_ptr<float>();
-  d.out_labels = r.labels.data_ptr<int64_t>();
-  d.out_index = r.index.data_ptr<int64_t>();
-  d.n_out = (uint32_t*)r.n.data_ptr<int32_t>();
+  Batched r = resultsOf(d, dev, T, max_num, true);
   if (T > 0) {
     auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
     const bool pays = mode == 0 && !counts.defined() && fx_nms_pairs_pays((int)T, (uint32_t)K, d.max_num, d.score_thr);
@@ -466,6 +472,29 @@ bool fuseTailsIn(Block* b) {
 }
 
 }  // namespace
+
+std::array<Tensor, 3> launchHeadTail(const fx_head_desc& head, c10::Device dev, int64_t images, int64_t rows, int64_t classes,
+                                     double score_thr, double iou_thr, int64_t max_num) {
+  c10::DeviceGuard guard(dev);
+  fx_nms_desc d;
+  memset(&d, 0, sizeof d);
+  d.mode = 1;
+  d.n_tasks = (int32_t)images;
+  d.rows = (uint32_t)rows;
+  d.n_classes = (uint32_t)classes;
+  d.score_thr = (float)score_thr;
+  d.iou_thr = (float)iou_thr;
+  d.max_num = (uint32_t)max_num;
+  d.key_capacity = FX_NMS_MAX_CANDIDATES;
+  Batched r = resultsOf(d, dev, images, max_num, false);
+  auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
+  const Tensor ws = nmsWorkspaces().get(dev, (void*)stream.stream(), images, d.key_capacity);
+  d.workspace = ws.data_ptr();
+  d.workspace_bytes = (size_t)ws.numel();
+  FX_OK_OR_THROW(fx_head_nms(&head, &d, (void*)stream.stream()));
+  at::getHostAllocator(at::kCUDA)->record_event(r.n.data_ptr(), r.n.storage().data_ptr().get_context(), stream.unwrap());
+  return {r.dets, r.labels, r.n};
+}
 
 bool FuseDetectionTail(std::shared_ptr<Graph> graph) { return fuseTailsIn(graph->block()); }
 

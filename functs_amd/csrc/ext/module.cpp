@@ -223,6 +223,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("_plan_functors", PlanFunctors);
   m.def("_jit_pass_infer_static_shapes", InferStaticShapes);
   m.def("_jit_pass_fuse_detection_tail", FuseDetectionTail);
+  m.def("_jit_pass_fuse_detection_head", FuseDetectionHead);
   m.def("_jit_pass_pad_compacted_results", PadCompactedResults);
   m.def("_functor_host_timing", functorHostTiming);
   m.def("_functor_host_times", []() {

@@ -4,10 +4,13 @@
 #pragma once
 #include <torch/csrc/jit/ir/ir.h>
 
+#include <array>
 #include <memory>
 #include <string>
 #include <unordered_map>
 #include <vector>
+
+struct fx_head_desc;   // include/fxhip.h
 
 namespace functs {
 
@@ -92,6 +95,16 @@ void setSinkProducers(bool on);
 // per image, as ATen and torchvision kernels with host synchronisations in between
 // (yolov3_bbox.py:104-179, 233-243).  True if the graph changed.
 bool FuseDetectionTail(std::shared_ptr<torch::jit::Graph> graph);
+
+// The chain of functors behind which a YOLO-style head's tail runs batched gets a launch beside it that takes the
+// candidates from the head's maps (detection_head.cpp).  Behind FaitPipeline, for functions that are built from examples on a
+// GPU (functs_amd/jit.py).  True if the graph changed: it serves arguments of the example's shapes only.
+bool FuseDetectionHead(std::shared_ptr<torch::jit::Graph> graph);
+// that launch: (dets [images, max_num, 5], labels [images, max_num], kept counts [images], which land in pinned host memory)
+std::array<at::Tensor, 3> launchHeadTail(const fx_head_desc& head, c10::Device device, int64_t images, int64_t rows, int64_t classes,
+                                         double score_thr, double iou_thr, int64_t max_num);
+// raises what earlier launches reported (fx_async_error), as every functor does before it launches
+void raiseAsyncErrors();
 
 // Opt-in (functs_amd.jit.build(..., padded_outputs=True)): every compacting functor whose results
 // are only returned gets padded_outputs=1, i.e. it returns each result at its full size (a map:

@@ -51,6 +51,9 @@ FUNCTS_SYM(ForallSelectRev, "fx::forall_select_rev")
 FUNCTS_SYM(LstmStack, "fx::lstm_stack")
 // a decoding loop of single-query attention collapsed to one node (attention.cpp)
 FUNCTS_SYM(AttentionSteps, "fx::attention_steps")
+// a detection head with its tail as one node, and whether the node serves its operands (detection_head.cpp)
+FUNCTS_SYM(DetectionHead, "fx::detection_head")
+FUNCTS_SYM(DetectionHeadFits, "fx::detection_head_fits")
 // attributes of tssa::ParallelFunctor
 FUNCTS_SYM(parallel_degree, "attr::parallel_degree")
 FUNCTS_SYM(is_parallel_args, "attr::is_parallel_args")

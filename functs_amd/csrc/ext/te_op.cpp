@@ -1881,6 +1881,8 @@ std::vector<std::string> PlanFunctors(std::shared_ptr<Graph> graph) {
   return report;
 }
 
+void raiseAsyncErrors() { checkAsyncError(); }
+
 void setEarlyResultsHook(EarlyResultsHook* hook) { t_early_hook = hook; }
 
 void functorHostTiming(bool on) {

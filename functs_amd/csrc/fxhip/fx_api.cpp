@@ -54,6 +54,7 @@ int fx_launch_lstm_stack(const FxLstmArgs& a, int L, uint32_t* words_ctl, uint32
 int fx_lstm_ask(int form);
 int fx_lstm_taken();
 int fx_launch_sort_nms(const fx_nms_desc& d, uint32_t key_cap, void* workspace, uint32_t* err_host, hipStream_t stream);
+int fx_launch_head_nms(const fx_head_desc& head, const fx_nms_desc& d, uint32_t key_cap, void* workspace, uint32_t* err_host, hipStream_t stream);
 size_t fx_nms_pairs_ws_bytes(int n_tasks, uint32_t rows);
 int fx_launch_nms_pairs(const fx_nms_desc& d, uint32_t spin_limit, hipStream_t stream);
 size_t fx_nms_workspace_bytes(int n_tasks, uint32_t key_cap);
@@ -1676,6 +1677,38 @@ int fx_sort_nms(const fx_nms_desc* desc, void* stream_) {
     return fail(FX_E_INVALID, "fx_sort_nms: workspace must be 256-byte aligned and hold fx_sort_nms_workspace_bytes()");
   const int rc = fx_launch_sort_nms(d, cap, d.workspace, err_word(true), (hipStream_t)stream_);
   if (rc != 0) return fail(FX_E_HIP, std::string("fx_sort_nms: ") + hipGetErrorString((hipError_t)(rc - 100)));
+  g_launches.fetch_add(1, std::memory_order_relaxed);
+  g_spec_launches.fetch_add(1, std::memory_order_relaxed);
+  return FX_OK;
+}
+
+int fx_head_nms(const fx_head_desc* head, const fx_nms_desc* desc, void* stream_) {
+  if (!head || !desc) return fail(FX_E_INVALID, "fx_head_nms: null descriptor");
+  const fx_nms_desc& d = *desc;
+  if (d.mode != 1 || d.n_tasks < 0 || d.n_classes < 1) return fail(FX_E_INVALID, "fx_head_nms: mode 1, classes and a number of tasks");
+  if (head->n_levels < 1 || head->n_levels > FX_HEAD_LEVELS)
+    return fail(FX_E_LIMIT, "fx_head_nms: 1.." + std::to_string(FX_HEAD_LEVELS) + " levels");
+  if (!head->strides || !d.dets || !d.out_labels || !d.n_out) return fail(FX_E_INVALID, "fx_head_nms: null argument");
+  if (d.max_num < 1 || d.max_num > FX_NMS_MAX_OUT) return fail(FX_E_LIMIT, "fx_head_nms: max_num must be 1.." + std::to_string(FX_NMS_MAX_OUT));
+  uint64_t rows = 0;
+  for (int l = 0; l < head->n_levels; ++l) {
+    if (!head->maps[l] || !head->bases[l] || !head->shifts[l]) return fail(FX_E_INVALID, "fx_head_nms: null argument");
+    const uint64_t cells = head->cells[l], anchors = head->anchors[l];
+    if (cells < 1 || anchors < 1 || cells * d.n_classes < 4) return fail(FX_E_LIMIT, "fx_head_nms: fewer than 4 class scores to a run of a level");
+    if (cells >= (1ull << 31) || anchors >= (1ull << 31) || cells * anchors * (5ull + d.n_classes) >= (1ull << 31) ||
+        (uint64_t)d.n_tasks * anchors >= (1ull << 31))
+      return fail(FX_E_LIMIT, "fx_head_nms: a level beyond 31 bits");
+    rows += cells * anchors;
+  }
+  if (rows != d.rows || rows * (5ull + d.n_classes) >= (1ull << 31)) return fail(FX_E_LIMIT, "fx_head_nms: rows must be the levels' and rows * attributes fit 31 bits");
+  if (d.key_capacity < 1 || d.key_capacity > FX_NMS_MAX_CANDIDATES)
+    return fail(FX_E_LIMIT, "fx_head_nms: key_capacity must be 1.." + std::to_string(FX_NMS_MAX_CANDIDATES));
+  if (d.n_tasks == 0) return FX_OK;
+  const uint32_t cap = nms_key_cap(d.key_capacity);
+  if (!d.workspace || ((uintptr_t)d.workspace & 255u) != 0 || d.workspace_bytes < fx_nms_workspace_bytes(d.n_tasks, cap))
+    return fail(FX_E_INVALID, "fx_head_nms: workspace must be 256-byte aligned and hold fx_sort_nms_workspace_bytes()");
+  const int rc = fx_launch_head_nms(*head, d, cap, d.workspace, err_word(true), (hipStream_t)stream_);
+  if (rc != 0) return fail(FX_E_HIP, std::string("fx_head_nms: ") + hipGetErrorString((hipError_t)(rc - 100)));
   g_launches.fetch_add(1, std::memory_order_relaxed);
   g_spec_launches.fetch_add(1, std::memory_order_relaxed);
   return FX_OK;

@@ -27,9 +27,10 @@ class AotScriptFunction(object):
     only.  Such a function keeps the functionalized script it was built from and builds a graph
     per set of argument shapes, the first one from the example; ``graph`` is that first one."""
 
-    def __init__(self, aot_script_fn, source=None, key=None, lazy_lists=False, padded_outputs=False, **kwargs):
+    def __init__(self, aot_script_fn, source=None, key=None, lazy_lists=False, padded_outputs=False, heads=False, **kwargs):
         self._aot_script_fn = aot_script_fn
         self._source = source
+        self._heads = heads
         self._lazy_lists = lazy_lists
         self._padded_outputs = padded_outputs
         self._call = _direct(aot_script_fn, lazy_lists)
@@ -52,7 +53,7 @@ class AotScriptFunction(object):
         key = _shape_key(args)
         fn = self._variants.get(key)
         if fn is None:
-            fn = self._variants[key] = _direct(_compile(self._source, args, self._padded_outputs)[0], self._lazy_lists)
+            fn = self._variants[key] = _direct(_compile(self._source, args, self._padded_outputs, self._heads)[0], self._lazy_lists)
         return fn(*args)
 
 
@@ -122,8 +123,8 @@ class GraphedFunction(AotScriptFunction):
     region cannot be captured: its output shapes need a synchronisation per call.
     """
 
-    def __init__(self, aot_script_fn, source=None, key=None):
-        super().__init__(aot_script_fn, source=source, key=key)
+    def __init__(self, aot_script_fn, source=None, key=None, heads=False):
+        super().__init__(aot_script_fn, source=source, key=key, heads=heads)
         if "compact_rows=1" in str(aot_script_fn.graph):
             raise ValueError("a function with a row-compacting region cannot run as a HIP graph")
         self._captures = {}
@@ -205,7 +206,9 @@ def build(fn, example_input: List[object], hip_graph: bool = False, lazy_lists: 
     switches it on for code that calls ``build`` the reference's way."""
     if not isinstance(fn, (torch.jit.ScriptFunction, torch.jit.ScriptModule)):
         raise AttributeError("only a functionalized jit script can be built")
-    aot, specialized = _compile(fn, example_input, padded_outputs)
+    # a function built from host examples stays the functors that its ``graph`` shows, also where it is called on a GPU
+    heads = any(t.is_cuda for a in example_input for t in (a if isinstance(a, (list, tuple)) else (a,)) if isinstance(t, torch.Tensor))
+    aot, specialized = _compile(fn, example_input, padded_outputs, heads)
     source, key = (fn, _shape_key(example_input)) if specialized else (None, None)
     if compile_kernels is None:
         env = os.environ.get("FUNCTS_AMD_COMPILE_KERNELS", "0").strip().lower()
@@ -214,17 +217,20 @@ def build(fn, example_input: List[object], hip_graph: bool = False, lazy_lists: 
         from . import aot as _aot
         _aot.compile_missing(aot, tables=compile_kernels if isinstance(compile_kernels, str) else "auto")
     if hip_graph:
-        return GraphedFunction(aot, source, key)
-    return AotScriptFunction(aot, source, key, lazy_lists=lazy_lists, padded_outputs=padded_outputs)
+        return GraphedFunction(aot, source, key, heads)
+    return AotScriptFunction(aot, source, key, lazy_lists=lazy_lists, padded_outputs=padded_outputs, heads=heads)
 
 
-def _compile(fn, example_input, padded_outputs=False):
-    """(compiled function, whether its graph holds constants of the example's shapes)"""
+def _compile(fn, example_input, padded_outputs=False, heads=False):
+    """(compiled function, whether its graph holds constants of the example's shapes); ``heads``: a detection head
+    with its tail may become one launch beside its functors"""
     g = fn.graph.copy()
     if isinstance(fn, torch.jit.ScriptModule):
         _strip_self(g)
     hints = [extract_type_hint_from_tensor(i) for i in example_input]
     specialized = bool(_C._jit_pass_fait_pipeline(g, hints))
+    if heads and _C._jit_pass_fuse_detection_head(g):
+        specialized = True
     if padded_outputs:
         _C._jit_pass_pad_compacted_results(g)
     return _C._create_function_from_graph("forward", g), specialized

@@ -559,6 +559,27 @@ typedef struct fx_nms_desc {
 size_t fx_sort_nms_workspace_bytes(int n_tasks, uint32_t key_capacity);
 size_t fx_sort_nms_workspace_clear_bytes(int n_tasks);
 int fx_sort_nms(const fx_nms_desc* desc, void* stream);
+/* The same tail behind a whole detection head, taken from its maps in the same one launch (functs/benchmark/ai_model/
+ * yolov3/yolov3_bbox.py:12-23, 78-101, 194-243): no row is permuted, decoded, filtered or written that is no candidate.
+ * A level's map is [n_tasks, anchors * (5 + n_classes), cells], its attributes the centre (squashed by a sigmoid), the
+ * logarithms of the sizes, the objectness and the class logits; row number first_row + cell * anchors + anchor.  A row is
+ * kept when sigmoid(objectness) >= keep_thr; its box is the decode of anchor bases[anchor] + shifts[cell] (corners) and
+ * strides[row], its scores the sigmoids of its class logits.  Candidates are then as in mode 1 of fx_nms_desc, of
+ * which boxes, scores, factors, labels and counts are not read and rows must be the levels' rows.  Results are those of the
+ * same program in separate launches, bit for bit; out_index counts rows before the filter.
+ * 4 or more class scores to a run of a level (n_classes * cells); workspace as for fx_sort_nms. */
+#define FX_HEAD_LEVELS 4
+typedef struct fx_head_desc {
+  int32_t n_levels;
+  float keep_thr;
+  const float* maps[FX_HEAD_LEVELS];
+  const float* bases[FX_HEAD_LEVELS];  /* [anchors, 4] */
+  const float* shifts[FX_HEAD_LEVELS]; /* [cells, 4] */
+  uint32_t cells[FX_HEAD_LEVELS];
+  uint32_t anchors[FX_HEAD_LEVELS];
+  const float* strides;                /* [rows] */
+} fx_head_desc;
+int fx_head_nms(const fx_head_desc* head, const fx_nms_desc* desc, void* stream);
 /* The same results for boxes that are all candidates (mode 0, counts null), up to FX_NMS_PAIRS_MAX_ROWS
  * rows, as three launches that spread the ranking, the overlap tests and, of many chunks, the decisions over the chip.  Its workspace is
  * scratch memory (256-byte aligned, nothing is expected in it or left in it); key_capacity is not read.

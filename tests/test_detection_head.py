@@ -1,0 +1,180 @@
+"""The detection head taken from its maps in one launch (fx_head_nms, ext/detection_head.cpp): the same bits as the chain of
+functors that a function built from host examples keeps."""
+import ctypes
+from typing import List, Tuple
+
+import pytest
+import torch
+from torch import Tensor
+
+import functs_amd.jit as fj
+from functs_amd import _lib, aot
+from functs_amd.benchmark import PROGRAMS
+from functs_amd.benchmark.inputs import yolov3_head
+from functs_amd.benchmark.programs import _yolov3_head_scores
+
+
+def no_threshold(pred_maps: List[Tensor], base_anchors: List[Tensor]):
+    """Every class of every kept row is a candidate."""
+    bboxes, cls_scores, objectness = _yolov3_head_scores(pred_maps, base_anchors)
+    det_results: List[Tuple[Tensor, Tensor]] = []
+    for i in range(bboxes.size(0)):
+        o = objectness[i]
+        keep = o >= 0.4
+        det_results.append(torch.ops.functs.multiclass_nms(bboxes[i][keep, :], cls_scores[i][keep, :], o[keep], 0.0, 0.45, 100, True))
+    return det_results
+
+
+def strict(pred_maps: List[Tensor], base_anchors: List[Tensor]):
+    """Only a score that rounds to 1 passes, more results than candidates."""
+    bboxes, cls_scores, objectness = _yolov3_head_scores(pred_maps, base_anchors)
+    det_results: List[Tuple[Tensor, Tensor]] = []
+    for i in range(bboxes.size(0)):
+        o = objectness[i]
+        keep = o >= 0.4
+        det_results.append(torch.ops.functs.multiclass_nms(bboxes[i][keep, :], cls_scores[i][keep, :], o[keep], 0.99999994, 0.3, 300, True))
+    return det_results
+
+
+def _kinds(block):
+    for n in block.nodes():
+        yield n.kind()
+        for b in n.blocks():
+            yield from _kinds(b)
+
+
+def _both(program, args):
+    """(function with the one launch, function with the chain: its examples lie on the host), built for the same shapes"""
+    gargs = [[t.cuda() for t in a] for a in args]
+    one, chain = fj.build(fj.script(program), gargs), fj.build(fj.script(program), args)
+    assert list(_kinds(one.graph.block())).count("fx::detection_head") == 1
+    assert "fx::detection_head" not in list(_kinds(chain.graph.block()))
+    return one, chain, gargs
+
+
+def _launches(fn, args):
+    before = aot.launch_stats()[0]
+    out = fn(*args)
+    torch.cuda.synchronize()
+    return out, aot.launch_stats()[0] - before
+
+
+def _assert_same(got, ref):
+    assert len(got) == len(ref)
+    for (d, l), (rd, rl) in zip(got, ref):
+        assert torch.equal(l, rl) and torch.equal(d, rd)
+
+
+def test_a_function_built_from_host_examples_keeps_the_chain():
+    fn = fj.build(fj.script(PROGRAMS["yolo_head_nms"]), list(yolov3_head(0, 2, (2, 4, 8), 5)))
+    assert "fx::detection_head" not in list(_kinds(fn.graph.block()))
+
+
+# Runs of class scores that end inside a vector, inside a group of 256 and with one; one cell; up to 16 and one to three images
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,grids,classes", [(1, (1, 2, 3), 4), (3, (2, 4, 8), 5), (2, (4, 8, 16), 16), (16, (7, 14, 28), 10), (1, (13, 26, 52), 80),
+                                                 (3, (19, 38, 76), 37), (300, (1, 2, 3), 4)])
+def test_same_bits_as_the_chain(batch, grids, classes):
+    args = list(yolov3_head(batch + classes, batch, grids, classes))
+    for m in args[0]:
+        m.view(batch, 3, 5 + classes, -1)[:, :, 5:] -= 1.0 if grids[0] < 4 else 3.5 if grids[0] < 8 else 6.0
+    print("head", batch, grids, classes, flush=True)
+    one, chain, gargs = _both(PROGRAMS["yolo_head_nms"], args)
+    got, launches = _launches(one, gargs)
+    ref, n_chain = _launches(chain, gargs)
+    assert launches == 1 and n_chain > 1
+    _assert_same(got, ref)
+    assert sum(d.size(0) for d, _ in got) > 0
+
+
+@pytest.mark.gpu
+def test_other_thresholds_and_special_values():
+    args = list(yolov3_head(3, 2, (3, 6, 12), 6))
+    flat = args[0][2].view(2, 3, 11, 144)
+    for k, x in enumerate((float("nan"), float("inf"), -float("inf"))):
+        flat[:, k, 5, 3::7] = x          # class logits
+        flat[:, k, 4, 5::11] = x         # objectness
+    flat[0, 0, 0, 7] = flat[1, 2, 2, 9] = 95.0
+    flat[:, 1, 7, 2::9] = 40.0           # scores that are 1
+    for program in (no_threshold, strict, PROGRAMS["yolo_head_nms"]):
+        print(program.__name__, flush=True)
+        one, chain, gargs = _both(program, args)
+        (got, n_one), (ref, n_chain) = _launches(one, gargs), _launches(chain, gargs)
+        assert n_one == 1 and n_chain > 1
+        _assert_same(got, ref)
+        assert sum(d.size(0) for d, _ in got) > 0
+
+
+@pytest.mark.gpu
+def test_rows_that_are_not_kept_do_not_count_as_candidates():
+    """More class scores above the threshold than there is room for, of rows that the objectness drops: nothing is refused,
+    the share of a workgroup is read again.  The same with rows that are kept is refused, and the next call works."""
+    args = list(yolov3_head(4, 1, (19, 38, 76), 80))
+    for m in args[0]:
+        v = m.view(1, 3, 85, -1)
+        v[:, :, 5:] = v[:, :, 5:].abs()
+        v[:, :, 4] = -9.0
+        v[:, :, 4, 5::200] = 2.0         # 117 rows of 80 candidates
+    one, chain, gargs = _both(PROGRAMS["yolo_head_nms"], args)
+    print("again", flush=True)
+    got, launches = _launches(one, gargs)
+    assert launches == 1
+    _assert_same(got, chain(*gargs))
+    full = [[m.clone() for m in gargs[0]], gargs[1]]
+    for m in full[0]:
+        m.view(1, 3, 85, -1)[:, :, 4:] = 1.0
+    print("refused", flush=True)
+    with pytest.raises(RuntimeError, match="more than 16384 candidates"):
+        one(*full)
+    _assert_same(one(*gargs), got)
+
+
+@pytest.mark.gpu
+def test_operands_that_the_launch_does_not_take_run_the_chain():
+    args = list(yolov3_head(5, 2, (4, 8, 16), 20))
+    for m in args[0]:
+        m.view(2, 3, 25, -1)[:, :, 5:] -= 4.0
+    one, chain, gargs = _both(PROGRAMS["yolo_head_nms"], args)
+    ref, n_chain = _launches(chain, gargs)
+    assert n_chain > 1
+    last = [[m.contiguous(memory_format=torch.channels_last) for m in gargs[0]], gargs[1]]
+    print("channels last", flush=True)
+    got, n = _launches(one, last)
+    assert n == n_chain
+    _assert_same(got, ref)
+    grad = [[m.clone().requires_grad_() for m in gargs[0]], gargs[1]]
+    print("gradients", flush=True)
+    got, n = _launches(one, grad)
+    assert n == n_chain
+    _assert_same(got, ref)
+    with torch.no_grad():
+        got, n = _launches(one, grad)
+    assert n == 1
+    _assert_same(got, ref)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    print("another stream", flush=True)
+    with torch.cuda.stream(side):
+        got, n = _launches(one, gargs)
+    assert n == 1
+    _assert_same(got, ref)
+
+
+def test_descriptors_that_do_not_fit_are_refused():
+    """(nothing is launched: every descriptor is refused on the host)"""
+    one = (ctypes.c_float * 4)()
+    at = ctypes.cast(one, ctypes.c_void_p).value
+
+    def call(levels=1, cells=4, anchors=3, rows=12, classes=5, max_num=10, cap=128, maps=at, mode=1):
+        h = _lib.FxHeadDesc()
+        h.n_levels, h.keep_thr, h.strides = levels, 0.1, at
+        for k in range(4):
+            h.maps[k], h.bases[k], h.shifts[k], h.cells[k], h.anchors[k] = maps, at, at, cells, anchors
+        d = _lib.FxNmsDesc()
+        d.mode, d.n_tasks, d.rows, d.n_classes, d.max_num, d.key_capacity = mode, 1, rows, classes, max_num, cap
+        d.dets = d.out_labels = d.n_out = at
+        return _lib.lib.fx_head_nms(ctypes.byref(h), ctypes.byref(d), None)
+
+    for bad in (dict(levels=0), dict(levels=5), dict(cells=0, rows=0), dict(rows=11), dict(cells=1, rows=3, classes=3), dict(max_num=0), dict(max_num=1025),
+                dict(cap=0), dict(cap=16385), dict(maps=None), dict(mode=0), dict(classes=0), dict(cells=1 << 20, rows=3 << 20, classes=1 << 10), dict()):
+        assert call(**bad) < 0, bad
