@@ -40,4 +40,22 @@ __device__ __forceinline__ void overlaps_fast(const Box& a, float area_a, const 
   sure = thr > 0.0f && t > 1e-30f && t < 1e30f && (over || inter < t * 0.999998f);
 }
 
+// The lanes of the wave in which the two may overlap: boxes apart from each other are told by four comparisons (no overlap
+// passes a positive threshold, whatever the areas), and most waves hold no others.  Masks, not a branch a lane: what the
+// compiler makes of the latter is four times the instructions.
+__device__ __forceinline__ uint64_t near_lanes(const float4& a, const float4& b, float thr) {
+  const uint64_t near = __ballot(a.z > b.x) & __ballot(b.z > a.x) & __ballot(a.w > b.y) & __ballot(b.w > a.y);
+  return thr > 0.0f ? near : ~0ull;
+}
+// of those lanes the ones in which they do: the decisions of overlaps(), by the division for waves in which a lane needs it
+__device__ __forceinline__ uint64_t overlap_lanes(uint64_t near, const float4& a, float area_a, const float4& b, float area_b, float thr) {
+  const Box p{a.x, a.y, a.z, a.w}, q{b.x, b.y, b.z, b.w};
+  bool over, sure;
+  overlaps_fast(p, area_a, q, area_b, thr, over, sure);
+  uint64_t lanes = __ballot(over);
+  const uint64_t open = __ballot(!sure) & near;
+  if (open != 0ull) lanes = (lanes & ~open) | (__ballot(overlaps(p, area_a, q, area_b, thr)) & open);
+  return lanes & near;
+}
+
 }  // namespace

@@ -10,13 +10,17 @@
 //      bits : candidate index), collected in LDS by each workgroup and appended to the task's
 //      key buffer in the workspace - their order of arrival does not matter, the index in the
 //      key restores it;
-//   2. bitonic sort of the keys: descending score, equal scores by ascending index (a stable
-//      descending sort);
+//   2. keys in ascending order: descending score, equal scores by ascending index (a stable descending sort): by
+//      buckets of the score for up to FX_NMS_FEW candidates, whose boxes come with their keys, else a bitonic sort;
 //   3. candidates are taken 64 at a time in that order.  Each is tested against the kept list
-//      (16 threads per candidate), the 64 x 64 overlaps inside the chunk become one 64-bit word
+//      (16 waves, every 16th kept box each), the overlaps inside the chunk become one 64-bit word
 //      per candidate (its overlapping predecessors), and one wave resolves the chunk: all
 //      candidates decide together in rounds, as many as the longest chain of overlaps.  The
 //      walk ends when max_num boxes are kept: later candidates cannot change earlier decisions.
+// What is left behind the scan runs on one CU an image and is bound by what that CU issues and by the trips between its
+// steps.  16 images of 8 500 rows, 80 classes, about 760 candidates each: 23.8 us; 27.9 with the sort for all, factors and
+// boxes gathered by the last workgroup, the rows written in the walk (whose barriers then wait for the stores) and
+// the walk's overlaps by the division.  128 boxes of one image, one workgroup, nothing handed over: 12.1 us, 13.1.
 // The workspace counters are zero when a launch starts and zero again when it ends.
 // The number of valid rows per task is read from memory (device or pinned host), so the count a
 // preceding compaction produced never has to reach the host.
@@ -43,6 +47,14 @@
 
 #define FX_NMS_THREADS 1024u
 #define FX_NMS_CHUNK 64u
+#define FX_NMS_OWN 2u           // candidates a thread of the finishing workgroup holds where it orders by buckets
+#define FX_NMS_FEW (FX_NMS_OWN * FX_NMS_THREADS)
+#define FX_NMS_BUCKET_BITS 11u
+#define FX_NMS_BUCKETS (1u << FX_NMS_BUCKET_BITS)
+#define FX_NMS_CROWD 48u        // candidates in a bucket that compare themselves with each other
+// key capacity from which LDS holds what a walk of FX_NMS_FEW candidates needs
+#define FX_NMS_ROOMY 16384u
+static_assert(FX_NMS_ROOMY * 8u >= FX_NMS_BUCKETS * 4u + FX_NMS_FEW * 56u, "the finishing workgroup's arrays lie in the keys' memory");
 
 namespace {
 
@@ -56,7 +68,8 @@ __device__ __forceinline__ uint64_t bitonic_step(uint64_t key, bool up, uint32_t
 }
 
 // workspace: per task FX_NMS_WS_WORDS counters (candidates, finished slices, largest coordinate,
-// row count + 1; zero between launches) in front of all tasks' key buffers
+// row count + 1; zero between launches) in front of all tasks' key buffers, behind which lie FX_NMS_FEW boxes a task
+// (of the first candidates, in the keys' order of arrival)
 #define FX_NMS_WS_WORDS 64u
 
 // ---- a detection head's maps as the source of the rows ----
@@ -64,9 +77,9 @@ __device__ __forceinline__ uint64_t bitonic_step(uint64_t key, bool up, uint32_t
 // puts them (yolov3_bbox.py:211-220).  Class scores of one (level, anchor) are C * cells consecutive elements of an
 // image's map; a wave reads them in groups of 256 that never span two of these runs, so what a wave needs to know
 // about its group is uniform.
-// Four 608 x 608 images, 80 classes, about 700 candidates each, cold lines: 28.0 us, of which some 8 are the scan (31 MB);
-// the functors and the tail this stands for (rows across their order 38.5, row stream 16.8, tail 26.1) 81.4, and the
-// call 97 -> 45 us.  One image 27.6, two of 416 x 416 and 37 classes 26.0: what follows the scan is the same.
+// Four 608 x 608 images, 80 classes, about 700 candidates each, cold lines: 21.9 us, of which the scan's 28 MB are 6.7 behind
+// 2 of start; the functors and the tail this stands for (rows across their order 38.5, row stream 16.8, tail 26.1) 81.4,
+// and the call 97 -> 38 us.  One image 19.8 (128 workgroups scan it; 64: 20.5, 256: 21.7, they queue up for the ticket).
 struct HeadLevel {
   const float *map, *base, *shift;
   uint32_t cells, anchors, row0;     // row0: rows of the levels before it
@@ -81,34 +94,40 @@ struct HeadMaps {
   const float* strides;
 };
 struct NoMaps {};
+__device__ __forceinline__ uint32_t divisor_magic(const HeadMaps& h) { return h.c_magic; }
+__device__ __forceinline__ uint32_t divisor_shift(const HeadMaps& h) { return h.c_shift; }
+__device__ __forceinline__ uint32_t divisor_magic(const NoMaps&) { return 0u; }
+__device__ __forceinline__ uint32_t divisor_shift(const NoMaps&) { return 0u; }
 
-// A row's place: level by selects (lanes differ), then its planes and tables.
+// A class score's place, from its number (256 x the groups in front of its run, and its number in the run): level by selects
+// (lanes differ), then the row's planes and tables.
 struct HeadRow {
   const float* at;      // attribute 0; attribute k lies k * cells behind it
-  uint32_t cells;
+  uint32_t cells, row, label;
   const float *base, *shift, *stride;
 };
-__device__ __forceinline__ HeadRow head_row(const HeadMaps& h, uint32_t task, uint32_t row) {
-  const float *map = h.lv[0].map, *base = h.lv[0].base, *shift = h.lv[0].shift;
-  uint32_t cells = h.lv[0].cells, anchors = h.lv[0].anchors, row0 = 0u, am = h.lv[0].anchors_magic, as = h.lv[0].anchors_shift;
+__device__ __forceinline__ HeadRow head_row(const HeadMaps& h, uint32_t task, uint32_t number) {
+  HeadLevel v = h.lv[0];
 #pragma unroll
-  for (uint32_t l = 1; l < FX_HEAD_LEVELS; ++l) {
-    const bool in = l < h.n_levels && row >= h.lv[l].row0;
-    map = in ? h.lv[l].map : map;
-    base = in ? h.lv[l].base : base;
-    shift = in ? h.lv[l].shift : shift;
-    cells = in ? h.lv[l].cells : cells;
-    anchors = in ? h.lv[l].anchors : anchors;
-    row0 = in ? h.lv[l].row0 : row0;
-    am = in ? h.lv[l].anchors_magic : am;
-    as = in ? h.lv[l].anchors_shift : as;
-  }
-  const uint32_t r = row - row0, cell = fx_fastdiv(r, am, as), a = r - cell * anchors;
-  return HeadRow{map + (size_t)(task * anchors + a) * h.width * cells + cell, cells, base + a * 4u, shift + (size_t)cell * 4u, h.strides + row};
+  for (uint32_t l = 1; l < FX_HEAD_LEVELS; ++l)
+    if (l < h.n_levels && (number >> 8) >= h.lv[l].group0) v = h.lv[l];
+  const uint32_t a = fx_fastdiv((number >> 8) - v.group0, v.run_magic, v.run_shift), in_run = number - (v.group0 + a * v.run_groups) * 256u;
+  const uint32_t label = fx_fastdiv(in_run, v.cells_magic, v.cells_shift), cell = in_run - label * v.cells, row = v.row0 + cell * v.anchors + a;
+  return HeadRow{v.map + (size_t)(task * v.anchors + a) * h.width * v.cells + cell, v.cells, row, label, v.base + a * 4u,
+                 v.shift + (size_t)cell * 4u, h.strides + row};
+}
+// the number of (row, label), as above
+__device__ __forceinline__ uint32_t head_number(const HeadMaps& h, uint32_t row, uint32_t label) {
+  HeadLevel v = h.lv[0];
+#pragma unroll
+  for (uint32_t l = 1; l < FX_HEAD_LEVELS; ++l)
+    if (l < h.n_levels && row >= h.lv[l].row0) v = h.lv[l];
+  const uint32_t r = row - v.row0, cell = fx_fastdiv(r, v.anchors_magic, v.anchors_shift), a = r - cell * v.anchors;
+  return (v.group0 + a * v.run_groups) * 256u + label * v.cells + cell;
 }
 // The decode of yolov3_bbox.py:12-23 with the operations of the region it stands for, one by one (nothing is contracted).
 __device__ __forceinline__ float4 head_box(const HeadRow& r) {
-  const float px = r.at[0], py = r.at[r.cells], pw = r.at[2u * r.cells], ph = r.at[3u * (size_t)r.cells];
+  const float px = r.at[0], py = r.at[r.cells], pw = r.at[2u * (size_t)r.cells], ph = r.at[3u * (size_t)r.cells];
   const float4 b = make_float4(r.base[0], r.base[1], r.base[2], r.base[3]), s = make_float4(r.shift[0], r.shift[1], r.shift[2], r.shift[3]);
   const float stride = *r.stride;
   const float a0 = b.x + s.x, a1 = b.y + s.y, a2 = b.z + s.z, a3 = b.w + s.w;
@@ -118,63 +137,51 @@ __device__ __forceinline__ float4 head_box(const HeadRow& r) {
 }
 __device__ __forceinline__ float head_objectness(const HeadRow& r) { return fx_sigmoid(r.at[4u * (size_t)r.cells]); }
 
-// The scan of a head's class scores: the elements whose score passes the threshold become keys in LDS.  Scores are
-// compared as logits first, with a bound below which none passes (launch), so that the sigmoid is paid for by the few
-// that may.  A workgroup with more keys than there is room for reads its share again and drops rows
-// that are not kept on the way; otherwise that is head_filter's, one row a thread, not a gather between the loads here.
-// Eight groups a wave in flight: a workgroup's share of a head (4 images of 22 743 rows, 80 classes: 113 KB) is asked for at once.
+// The scan of a head's class scores: elements that may pass the threshold go to LDS with their numbers.  They are compared as
+// logits, with a bound below which none passes (launch): everything else is gather_own's, one element a thread, not a
+// branch between the loads.  A workgroup with more of them than there is room for reads its share again and takes only those
+// that are candidates.
+// Four groups a wave in flight: with eight the kernel is larger, and its code takes longer to arrive than the loads save (12.0 us
+// from the first workgroup's start to the last one's end of scan, 10.7 with four; 8.7 with the levels' arguments in one trip).
 __device__ __forceinline__ void head_scan(const fx_nms_desc& d, const HeadMaps& h, const uint32_t key_cap, const uint32_t slices,
-                                          const uint32_t task, const uint32_t slice, uint64_t* s_keys, uint32_t* s_count, uint32_t* s_again) {
-  constexpr uint32_t U = 8u, WAVES = FX_NMS_THREADS / 64u;
+                                          const uint32_t task, const uint32_t slice, uint64_t* s_keys, uint32_t* s_count) {
+  constexpr uint32_t U = 4u, WAVES = FX_NMS_THREADS / 64u;
   const uint32_t lane = threadIdx.x & 63u, wave = uni(threadIdx.x >> 6), C = d.n_classes;
   const uint32_t share = (h.groups + slices - 1u) / slices, first = min(slice * share, h.groups), end = min(first + share, h.groups);
   for (uint32_t pass = 0; pass < 2u; ++pass) {
     for (uint32_t g0 = first + wave; g0 < end; g0 += WAVES * U) {
-      float v[U][4];
-      uint32_t e0[U];   // the lane's first element in its run; at the run's end the loads move back to its last four
-      auto level = [&](uint32_t g) -> const HeadLevel& {
-        uint32_t l = 0u;
-#pragma unroll
-        for (uint32_t k = 1; k < FX_HEAD_LEVELS; ++k) l += k < h.n_levels && g >= h.lv[k].group0 ? 1u : 0u;
-        return h.lv[l];
-      };
+      fx_u32x4_a4 v[U];
+      uint32_t number[U], skip[U];   // skip: elements of the lane's four that are not its own (a run's last loads move back to its end)
 #pragma unroll
       for (uint32_t u = 0; u < U; ++u) {
         const uint32_t g = uni(min(g0 + u * WAVES, end - 1u));
-        const HeadLevel& lv = level(g);
-        const uint32_t a = fx_fastdiv(g - lv.group0, lv.run_magic, lv.run_shift), in_run = g - lv.group0 - a * lv.run_groups;
-        const uint32_t n = C * lv.cells;
-        const float* run = lv.map + ((size_t)(task * lv.anchors + a) * h.width + 5u) * lv.cells;
-        e0[u] = in_run * 256u + lane * 4u;
-        const fx_u32x4 q = *(const fx_u32x4_a4*)(run + min(e0[u], n - 4u));
+        HeadLevel lv = h.lv[0];   // (selects, not an index: the arguments come in one trip)
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) v[u][e] = __uint_as_float(q[e]);
+        for (uint32_t k = 1; k < FX_HEAD_LEVELS; ++k)
+          if (k < h.n_levels && g >= h.lv[k].group0) lv = h.lv[k];
+        const uint32_t a = fx_fastdiv(g - lv.group0, lv.run_magic, lv.run_shift), run0 = lv.group0 + a * lv.run_groups;
+        const float* run = lv.map + ((size_t)(task * lv.anchors + a) * h.width + 5u) * lv.cells;
+        const uint32_t own = (g - run0) * 256u + lane * 4u, from = min(own, C * lv.cells - 4u);
+        v[u] = __builtin_nontemporal_load((const fx_u32x4_a4*)(run + from));   // (every line once)
+        number[u] = run0 * 256u + from;
+        skip[u] = g0 + u * WAVES < end ? own - from : 4u;
       }
       uint32_t mine = 0u;
 #pragma unroll
       for (uint32_t u = 0; u < U; ++u)
 #pragma unroll
         for (uint32_t e = 0; e < 4u; ++e)
-          if (v[u][e] > h.logit_lo) mine |= 1u << (u * 4u + e);
+          if (__uint_as_float(v[u][e]) > h.logit_lo && e >= skip[u]) mine |= 1u << (u * 4u + e);
       if (mine == 0u) continue;
 #pragma unroll
-      for (uint32_t u = 0; u < U; ++u) {
-        if (((mine >> (u * 4u)) & 15u) == 0u || g0 + u * WAVES >= end) continue;
-        const uint32_t g = uni(g0 + u * WAVES);
-        const HeadLevel& lv = level(g);
-        const uint32_t a = fx_fastdiv(g - lv.group0, lv.run_magic, lv.run_shift), from = min(e0[u], C * lv.cells - 4u);
+      for (uint32_t u = 0; u < U; ++u)
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) {
-          if (!((mine >> (u * 4u + e)) & 1u) || from + e < e0[u]) continue;
-          const float s = fx_sigmoid(v[u][e]);
-          if (!(s > d.score_thr)) continue;
-          const uint32_t c = fx_fastdiv(from + e, lv.cells_magic, lv.cells_shift), cell = from + e - c * lv.cells;
-          const uint32_t row = lv.row0 + cell * lv.anchors + a;
-          if (pass == 1u && !(head_objectness(head_row(h, task, row)) >= h.keep_thr)) continue;
-          const uint32_t slot = atomicAdd(s_count, 1u);
-          if (slot < key_cap) s_keys[slot] = ((uint64_t)(~orderable(s)) << 32) | (uint64_t)(row * C + c);
-        }
-      }
+        for (uint32_t e = 0; e < 4u; ++e)
+          if ((mine >> (u * 4u + e)) & 1u) {
+            if (pass == 1u && !(fx_sigmoid(__uint_as_float(v[u][e])) > d.score_thr && head_objectness(head_row(h, task, number[u] + e)) >= h.keep_thr)) continue;
+            const uint32_t slot = atomicAdd(s_count, 1u);
+            if (slot < key_cap) s_keys[slot] = ((uint64_t)v[u][e] << 32) | (uint64_t)(number[u] + e);
+          }
     }
     if (pass == 1u) break;
     __syncthreads();
@@ -186,36 +193,57 @@ __device__ __forceinline__ void head_scan(const fx_nms_desc& d, const HeadMaps& 
   }
 }
 
-// The keys of a workgroup: rows that are not kept leave, scores take their row's objectness, and the largest
-// coordinate of the boxes is taken (here, side by side in all workgroups of a task, and not in the one that finishes it).
-__device__ __forceinline__ void head_filter(const fx_nms_desc& d, const HeadMaps& h, const uint32_t key_cap, const uint32_t task,
-                                            uint64_t* s_keys, uint32_t* s_count, uint32_t* s_kept, uint32_t* s_maxc) {
+// What a candidate needs besides its score is gathered here, by every workgroup for its own, one candidate a thread: a
+// gather by the one that finishes the task is bound by the lines a CU gets (700 candidates of a head, seven lines each: 5.5 us),
+// a gather in the scan sits between the rounds of loads.  Scores take their row's factor, a head's rows that are not kept
+// leave, boxes (of few candidates) go to s_box, the largest coordinate to s_maxc.
+template <class Maps>
+__device__ __forceinline__ void gather_own(const fx_nms_desc& d, const Maps& h, const uint32_t C, const uint32_t key_cap, const uint32_t task,
+                                           const float* boxes, const float* factors, uint64_t* s_keys, float4* s_box, uint32_t* s_count,
+                                           uint32_t* s_kept, uint32_t* s_maxc) {
+  constexpr bool HEAD = !std::is_same_v<Maps, NoMaps>;
   const uint32_t n = min(*s_count, key_cap), over = *s_count - n;
-  if (threadIdx.x == 0u) *s_kept = 0u;
-  __syncthreads();
-  uint32_t my_max = 0u;
+  if (HEAD && threadIdx.x == 0u) *s_kept = 0u;
+  if (HEAD) __syncthreads();
+  uint32_t my_max = 0u;   // below orderable() of every value
   for (uint32_t k0 = 0; k0 < n; k0 += FX_NMS_THREADS) {
     const uint32_t k = k0 + threadIdx.x;
     uint64_t key = 0ull;
-    bool keep = false;
-    if (k < n) {
+    float4 b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    bool keep = k < n;
+    if (keep) {
       key = s_keys[k];
-      const HeadRow r = head_row(h, task, fx_fastdiv((uint32_t)key, h.c_magic, h.c_shift));
-      const float o = head_objectness(r);
-      const float4 b = head_box(r);
-      keep = o >= h.keep_thr;
-      key = ((uint64_t)(~orderable(from_orderable(~(uint32_t)(key >> 32)) * o)) << 32) | (uint64_t)(uint32_t)key;
+      float f = 1.0f;
+      if constexpr (HEAD) {
+        const HeadRow r = head_row(h, task, (uint32_t)key);
+        const float score = fx_sigmoid(__uint_as_float((uint32_t)(key >> 32)));
+        f = head_objectness(r);
+        b = head_box(r);
+        keep = score > d.score_thr && f >= h.keep_thr;
+        key = ((uint64_t)(~orderable(score)) << 32) | (uint64_t)(r.row * C + r.label);
+      } else {
+        const uint32_t r = (uint32_t)key / C;
+        if (factors) f = factors[r];
+        b = *(const float4*)(boxes + (size_t)r * 4u);
+      }
+      if (HEAD || factors) key = ((uint64_t)(~orderable(from_orderable(~(uint32_t)(key >> 32)) * f)) << 32) | (uint64_t)(uint32_t)key;
       if (keep) my_max = max(my_max, max(max(orderable(b.x), orderable(b.y)), max(orderable(b.z), orderable(b.w))));
     }
-    __syncthreads();   // (the places that are written lie among those that have been read)
-    if (keep) s_keys[atomicAdd(s_kept, 1u)] = key;
+    if (HEAD) __syncthreads();   // (the places that are written lie among those that have been read)
+    if (keep) {
+      const uint32_t at = HEAD ? atomicAdd(s_kept, 1u) : k;
+      if (HEAD || factors) s_keys[at] = key;
+      if (n <= FX_NMS_FEW && key_cap >= FX_NMS_ROOMY) s_box[at] = b;
+    }
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) my_max = max(my_max, (uint32_t)__shfl_xor((int)my_max, o, 64));
   if ((threadIdx.x & 63u) == 0u && my_max != 0u) atomicMax(s_maxc, my_max);
   __syncthreads();
-  if (threadIdx.x == 0u) *s_count = *s_kept + over;
-  __syncthreads();
+  if (HEAD) {
+    if (threadIdx.x == 0u) *s_count = *s_kept + over;
+    __syncthreads();
+  }
 }
 
 // Maps: NoMaps (boxes and scores as the descriptor has them) or HeadMaps (rows that the kernel takes from a head's maps itself).
@@ -225,21 +253,24 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
                                                                     uint32_t* err_host) {
   constexpr bool HEAD = !std::is_same_v<Maps, NoMaps>;
   extern __shared__ __attribute__((aligned(16))) uint64_t s_keys[];   // key_cap (a power of two)
-  __shared__ float s_kbox[FX_NMS_MAX_OUT][4];
+  __shared__ float4 s_kbox[FX_NMS_MAX_OUT];
   __shared__ float s_karea[FX_NMS_MAX_OUT];
-  __shared__ float s_cbox[FX_NMS_CHUNK][4];     // chunk: original boxes
-  __shared__ float s_obox[FX_NMS_CHUNK][4];     // chunk: boxes moved by their class offset
+  __shared__ uint32_t s_kept[FX_NMS_MAX_OUT];   // places in score order
+  __shared__ float4 s_cbox[FX_NMS_CHUNK];       // chunk: original boxes
+  __shared__ float4 s_obox[FX_NMS_CHUNK];       // chunk: boxes moved by their class offset
   __shared__ float s_carea[FX_NMS_CHUNK];
-  __shared__ uint32_t s_cidx[FX_NMS_CHUNK], s_clabel[FX_NMS_CHUNK];
-  __shared__ float s_cscore[FX_NMS_CHUNK];
-  __shared__ uint32_t s_in[FX_NMS_CHUNK][2];    // earlier candidates of the chunk that overlap candidate j
-  __shared__ uint32_t s_dead[2];                // candidates of the chunk that the kept list overlaps
+  __shared__ uint32_t s_clabel[FX_NMS_CHUNK];
+  __shared__ uint32_t s_in[2][FX_NMS_CHUNK][2]; // by the chunk's parity: earlier candidates of the chunk that overlap candidate j
+  __shared__ uint32_t s_dead[2][2];             // candidates of the chunk that the kept list overlaps
   __shared__ uint32_t s_count, s_maxc, s_nk, s_base, s_ticket;
+  __shared__ uint32_t s_lo, s_hi, s_crowd, s_wave[FX_NMS_THREADS / 64u];
 
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t task = blockIdx.x / slices, slice = blockIdx.x - task * slices;
   uint32_t* const ctr = ws + (size_t)task * FX_NMS_WS_WORDS;   // [0] candidates, [1] finished slices, [2] largest coordinate
   uint64_t* const g_keys = (uint64_t*)(ws + (size_t)d.n_tasks * FX_NMS_WS_WORDS) + (size_t)task * key_cap;
+  const bool roomy = key_cap >= FX_NMS_ROOMY;
+  uint64_t* const g_box = (uint64_t*)(ws + (size_t)d.n_tasks * FX_NMS_WS_WORDS) + (size_t)d.n_tasks * key_cap + (size_t)task * (2u * FX_NMS_FEW);
   // NC classes, in rows of C elements (C > NC: columns behind the class scores that are not candidates)
   const uint32_t NC = d.mode == 1 ? d.n_classes : 1u;
   const uint32_t C = (d.mode == 1 && d.scores_row_stride != 0u) ? d.scores_row_stride : NC;
@@ -251,35 +282,39 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
   int64_t* out_labels = d.out_labels + (size_t)task * d.max_num;
   int64_t* out_index = d.out_index ? d.out_index + (size_t)task * d.max_num : nullptr;
 
-  // The task's row count may lie in host memory, where a read costs a trip over the bus and the
-  // reads of many workgroups queue up: slice 0 reads it and passes it on through the workspace
-  // (count + 1 in ctr[3]); a slice that does not see it within its polls reads it itself.
   if (tid == 0) {
     s_count = 0u;
     s_maxc = 0u;
-    uint32_t rows = d.rows;
-    if (!HEAD && d.counts) {
-      uint32_t seen = 0u;
-      if (slice != 0u)
-        for (uint32_t polls = 0; polls < 4096u && seen == 0u; ++polls) {
-          seen = __hip_atomic_load(&ctr[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (seen == 0u) __builtin_amdgcn_s_sleep(2);
-        }
-      if (seen == 0u) {
-        seen = min(d.rows, __hip_atomic_load(d.counts + task, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)) + 1u;
-        if (slice == 0u) __hip_atomic_store(&ctr[3], seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      rows = seen - 1u;
-    }
-    s_base = rows;
   }
-  __syncthreads();
-  const uint32_t rows = s_base;
+  uint32_t rows = d.rows;
+  if constexpr (!HEAD) {
+    // The task's row count may lie in host memory, where a read costs a trip over the bus and the
+    // reads of many workgroups queue up: slice 0 reads it and passes it on through the workspace
+    // (count + 1 in ctr[3]); a slice that does not see it within its polls reads it itself.
+    if (tid == 0) {
+      if (d.counts) {
+        uint32_t seen = 0u;
+        if (slice != 0u)
+          for (uint32_t polls = 0; polls < 4096u && seen == 0u; ++polls) {
+            seen = __hip_atomic_load(&ctr[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (seen == 0u) __builtin_amdgcn_s_sleep(2);
+          }
+        if (seen == 0u) {
+          seen = min(d.rows, __hip_atomic_load(d.counts + task, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)) + 1u;
+          if (slice == 0u) __hip_atomic_store(&ctr[3], seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        rows = seen - 1u;
+      }
+      s_base = rows;
+    }
+    __syncthreads();
+    rows = s_base;
+  }
   __syncthreads();   // s_base is used again below
 
   FX_NMS_STAMP(0);
   if constexpr (HEAD) {
-    head_scan(d, h, key_cap, slices, task, slice, s_keys, &s_count, &s_base);
+    head_scan(d, h, key_cap, slices, task, slice, s_keys, &s_count);
   } else {
     // 1. candidates: four 128-bit loads per thread in flight
     const uint32_t all_items = rows * C;   // < 2^32 (host)
@@ -335,13 +370,16 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
   }
   __syncthreads();
   FX_NMS_STAMP(1);
-  if constexpr (HEAD) head_filter(d, h, key_cap, task, s_keys, &s_count, &s_base, &s_maxc);
-  {
+  float4* const s_own = (float4*)(s_keys + FX_NMS_FEW);   // (with FX_NMS_ROOMY)
+  gather_own(d, h, C, key_cap, task, boxes, d.mode == 1 ? factors : nullptr, s_keys, s_own, &s_count, &s_base, &s_maxc);
+  uint64_t key[FX_NMS_OWN], corner[FX_NMS_OWN][2];
+  uint32_t count, largest;
+  if (slices > 1u) {
     // hand this workgroup's keys over and take a ticket
     const uint32_t mine = min(s_count, key_cap);
     if (tid == 0) {
       s_base = atomicAdd(&ctr[0], s_count);
-      if (HEAD && mine != 0u) atomicMax(&ctr[2], s_maxc);
+      if (mine != 0u) atomicMax(&ctr[2], s_maxc);
     }
     __syncthreads();
     const uint32_t gbase = s_base;
@@ -353,6 +391,9 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
     // compiler is told the order explicitly: nothing moves across the signal fences.
     for (uint32_t k = tid; k < mine; k += FX_NMS_THREADS)
       if (gbase + k < key_cap) __hip_atomic_store(&g_keys[gbase + k], s_keys[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (roomy)   // (a workgroup with more candidates than that has no boxes: neither has the task need of any)
+      for (uint32_t k = tid; k < 2u * mine && (k >> 1) + gbase < FX_NMS_FEW; k += FX_NMS_THREADS)
+        if (mine <= FX_NMS_FEW) __hip_atomic_store(&g_box[2u * gbase + k], ((const uint64_t*)s_own)[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -360,11 +401,42 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
     if (tid == 0) s_ticket = atomicAdd(&ctr[1], 1u);
     __syncthreads();
     if (s_ticket != slices - 1u) return;   // somebody else finishes the task
+    FX_NMS_STAMP(2);
+    // the last workgroup of the task: everything the others wrote is visible.  The first candidates are asked for
+    // together with their number.
+#pragma unroll
+    for (uint32_t i = 0; i < FX_NMS_OWN; ++i) {
+      const uint32_t k = i * FX_NMS_THREADS + tid;
+      key[i] = __hip_atomic_load(&g_keys[min(k, key_cap - 1u)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      corner[i][0] = corner[i][1] = 0ull;
+      if (roomy) {
+        corner[i][0] = __hip_atomic_load(&g_box[2u * k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        corner[i][1] = __hip_atomic_load(&g_box[2u * k + 1u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    count = uni(__hip_atomic_load(&ctr[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    largest = __hip_atomic_load(&ctr[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    // the only one: its own candidates are all
+    count = uni(s_count);
+    largest = s_maxc;
+#pragma unroll
+    for (uint32_t i = 0; i < FX_NMS_OWN; ++i) {
+      const uint32_t k = i * FX_NMS_THREADS + tid;
+      key[i] = 0ull;
+      corner[i][0] = corner[i][1] = 0ull;
+      if (!roomy || count > FX_NMS_FEW || k >= count) continue;
+      key[i] = s_keys[k];
+      corner[i][0] = ((const uint64_t*)s_own)[2u * k];
+      corner[i][1] = ((const uint64_t*)s_own)[2u * k + 1u];
+    }
   }
-  FX_NMS_STAMP(2);
-  // the last workgroup of the task: everything the others wrote is visible
-  const uint32_t count = __hip_atomic_load(&ctr[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint32_t max_seen = HEAD ? __hip_atomic_load(&ctr[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+  const float class_step = from_orderable(largest) + 1.0f;   // (no candidates: not used)
+  if (tid == 0) {
+    s_lo = ~0u;
+    s_hi = 0u;
+    s_crowd = 0u;
+  }
   __syncthreads();
   if (tid == 0) {   // the counters are zero again for the next launch
     __hip_atomic_store(&ctr[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -374,8 +446,12 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
   }
   if (count > key_cap) {   // more candidates than the launch was sized for: reported, nothing returned
     if (tid == 0) {
-      __hip_atomic_store(d.n_out + task, FX_NMS_OVERFLOW, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      // (a host that polls n_out takes the report back when it sees the overflow: the report has to be there by then)
       if (err_host) __hip_atomic_store(err_host, (uint32_t)FX_ASYNC_NMS_CAPACITY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __hip_atomic_store(d.n_out + task, FX_NMS_OVERFLOW, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     for (uint32_t k = tid; k < d.max_num * 5u; k += FX_NMS_THREADS) dets[k] = 0.0f;
     for (uint32_t k = tid; k < d.max_num; k += FX_NMS_THREADS) {
@@ -384,150 +460,259 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
     }
     return;
   }
-  // The largest coordinate of the candidates' boxes (classes are told apart by moving boxes by a
-  // multiple of it): taken here, one box per thread, not in the scan, where a gather per
-  // candidate would sit between the rounds of loads.
-  uint32_t my_max = 0u;                // below orderable() of every value
-  for (uint32_t k = tid; k < count; k += FX_NMS_THREADS) {
-    uint64_t key = __hip_atomic_load(&g_keys[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if constexpr (HEAD) {   // (factor and largest coordinate: every workgroup for its own, head_filter)
-      s_keys[k] = key;
-      continue;
-    }
-    const uint32_t r = (uint32_t)key / C;
-    if (d.mode == 1 && factors) {
-      const float sc = from_orderable(~(uint32_t)(key >> 32)) * factors[r];
-      key = ((uint64_t)(~orderable(sc)) << 32) | (uint64_t)(uint32_t)key;
-    }
-    s_keys[k] = key;
-    const float4 b = *(const float4*)(boxes + (size_t)r * 4u);
-    my_max = max(my_max, max(max(orderable(b.x), orderable(b.y)), max(orderable(b.z), orderable(b.w))));
-  }
-  if constexpr (!HEAD) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) my_max = max(my_max, (uint32_t)__shfl_xor((int)my_max, o, 64));
-    if (lane == 0u) atomicMax(&s_maxc, my_max);
-  }
-  __syncthreads();
-  const float class_step = from_orderable(HEAD ? max_seen : s_maxc) + 1.0f;
+  // what a key stands for
+  auto row_of = [&](uint32_t idx) { return HEAD ? fx_fastdiv(idx, divisor_magic(h), divisor_shift(h)) : idx / C; };
+  auto label_of = [&](uint32_t idx, uint32_t r) { return d.mode == 1 ? idx - r * C : (labels ? (uint32_t)labels[idx] : 0u); };
+  auto moved_by = [](const float4& b, float off) { return make_float4(b.x + off, b.y + off, b.z + off, b.w + off); };
+  auto area_of = [](const float4& b) { return (b.z - b.x) * (b.w - b.y); };
 
-  // 2. bitonic sort (ascending keys = descending score, ascending index); the tail is padding.
-  // Stages whose partners lie at most 64 apart stay inside aligned blocks of 128 keys: a wave
-  // runs all of them on its blocks without a workgroup barrier (LDS accesses of one wave are
-  // performed in order), so a phase costs one barrier per wider stage plus one.
+  // Of up to FX_NMS_OWN candidates a thread, everything the walk needs lies in LDS in score order (s_keys' memory, whose
+  // keys have been handed over): buckets, keys by bucket, keys in order, moved boxes, boxes, areas, labels.
+  const uint32_t np = (count + 63u) & ~63u;
+  uint32_t* const s_bucket = (uint32_t*)s_keys;
+  uint64_t* const s_part = (uint64_t*)(s_bucket + FX_NMS_BUCKETS);
+  uint64_t* const s_order = s_part + np;
+  float4* const s_moved = (float4*)(s_order + np);
+  float4* const s_box = s_moved + np;
+  float* const s_area = (float*)(s_box + np);
+  uint32_t* const s_label = (uint32_t*)(s_area + np);
+  bool placed = roomy && count <= FX_NMS_FEW;
   FX_NMS_STAMP(3);
-  uint32_t n2 = 128u;
-  while (n2 < count) n2 <<= 1;
-  for (uint32_t i = count + tid; i < n2; i += FX_NMS_THREADS) s_keys[i] = ~0ull;
-  __syncthreads();
-  auto exchange = [&](uint32_t i, uint32_t j, uint32_t k) {
-    const uint32_t l = i | j;
-    const uint64_t a = s_keys[i], b = s_keys[l];
-    const bool up = (i & k) == 0u;
-    if ((a > b) == up) { s_keys[i] = b; s_keys[l] = a; }
-  };
-  auto narrow_stages = [&](uint32_t k_first, uint32_t k_last) {   // every stage j <= 64 of phases k_first .. k_last
-    for (uint32_t blk = wave; blk < (n2 >> 7); blk += FX_NMS_THREADS / 64u) {
-      // the block's 128 keys in registers, two a lane (positions lane and lane + 64): the stages
-      // exchange them between lanes, LDS is read and written once per call
-      const uint32_t p0 = (blk << 7) + lane;
-      uint64_t ka = s_keys[p0], kb = s_keys[p0 + 64u];
-      for (uint32_t k = k_first; k <= k_last; k <<= 1) {
-        const bool up_a = (p0 & k) == 0u, up_b = ((p0 + 64u) & k) == 0u;
-        if (k >= 128u) {   // partners 64 apart: the lane's own two keys (up_a == up_b here)
-          const bool sw = (ka > kb) == up_a;
-          const uint64_t lo = sw ? kb : ka, hi = sw ? ka : kb;
-          ka = lo; kb = hi;
-        }
-        if (k >= 64u) { ka = bitonic_step<32>(ka, up_a, lane); kb = bitonic_step<32>(kb, up_b, lane); }
-        if (k >= 32u) { ka = bitonic_step<16>(ka, up_a, lane); kb = bitonic_step<16>(kb, up_b, lane); }
-        if (k >= 16u) { ka = bitonic_step<8>(ka, up_a, lane); kb = bitonic_step<8>(kb, up_b, lane); }
-        if (k >= 8u) { ka = bitonic_step<4>(ka, up_a, lane); kb = bitonic_step<4>(kb, up_b, lane); }
-        if (k >= 4u) { ka = bitonic_step<2>(ka, up_a, lane); kb = bitonic_step<2>(kb, up_b, lane); }
-        ka = bitonic_step<1>(ka, up_a, lane); kb = bitonic_step<1>(kb, up_b, lane);
-      }
-      s_keys[p0] = ka; s_keys[p0 + 64u] = kb;
+  if (placed) {
+    // 2. order by buckets of the score's bits: a candidate's bucket says how many lie ahead of it but for its
+    // bucket's own, of which there are one or two (700 candidates, 2 048 buckets between the lowest score and the highest).
+    uint32_t label[FX_NMS_OWN], lo = ~0u, hi = 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < FX_NMS_BUCKETS / FX_NMS_THREADS; ++i) s_bucket[i * FX_NMS_THREADS + tid] = 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < FX_NMS_OWN; ++i) {
+      label[i] = 0u;
+      if (i * FX_NMS_THREADS + tid >= count) continue;
+      const uint32_t idx = (uint32_t)key[i];
+      label[i] = label_of(idx, row_of(idx));
+      lo = min(lo, (uint32_t)(key[i] >> 32));
+      hi = max(hi, (uint32_t)(key[i] >> 32));
     }
-  };
-  narrow_stages(2u, 128u);
-  __syncthreads();
-  for (uint32_t k = 256u; k <= n2; k <<= 1) {
-    for (uint32_t j = k >> 1; j >= 128u; j >>= 1) {
-      for (uint32_t p = tid; p < (n2 >> 1); p += FX_NMS_THREADS) exchange(((p & ~(j - 1u)) << 1) | (p & (j - 1u)), j, k);
-      __syncthreads();
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+      hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
     }
-    narrow_stages(k, k);
+    if (lane == 0u && lo <= hi) {
+      atomicMin(&s_lo, lo);
+      atomicMax(&s_hi, hi);
+    }
     __syncthreads();
-  }
-
-  FX_NMS_STAMP(4);
-  // 3. greedy walk
-  if (tid == 0) s_nk = 0u;
-  __syncthreads();
-  uint32_t nk = 0u;
-  for (uint32_t pos = 0; pos < count && nk < d.max_num; pos += FX_NMS_CHUNK) {
-    const uint32_t m = min(FX_NMS_CHUNK, count - pos);
-    if (tid < FX_NMS_CHUNK) {
-      s_in[tid][0] = 0u; s_in[tid][1] = 0u;
-      if (tid < 2u) s_dead[tid] = 0u;
-      if (tid < m) {
-        const uint64_t key = s_keys[pos + tid];
-        const uint32_t idx = (uint32_t)key;
-        const uint32_t r = idx / C;
-        const uint32_t label = d.mode == 1 ? idx - r * C : (labels ? (uint32_t)labels[idx] : 0u);
-        float4 b;
-        if constexpr (HEAD) b = head_box(head_row(h, task, r));
-        else b = *(const float4*)(boxes + (size_t)r * 4u);
-        const float off = (float)label * class_step;
-        const float x1 = b.x + off, y1 = b.y + off, x2 = b.z + off, y2 = b.w + off;
-        s_cbox[tid][0] = b.x; s_cbox[tid][1] = b.y; s_cbox[tid][2] = b.z; s_cbox[tid][3] = b.w;
-        s_obox[tid][0] = x1; s_obox[tid][1] = y1; s_obox[tid][2] = x2; s_obox[tid][3] = y2;
-        s_carea[tid] = (x2 - x1) * (y2 - y1);
-        s_cidx[tid] = d.mode == 1 ? r * NC + label : idx;   // position among the candidates proper
-        s_clabel[tid] = label;
-        s_cscore[tid] = from_orderable(~(uint32_t)(key >> 32));
-      }
+    const uint32_t first = uni(s_lo), range = uni(s_hi) - first;
+    const uint32_t shift = range < FX_NMS_BUCKETS ? 0u : 32u - (uint32_t)__builtin_clz(range) - FX_NMS_BUCKET_BITS;
+    uint32_t bucket[FX_NMS_OWN], slot[FX_NMS_OWN];
+#pragma unroll
+    for (uint32_t i = 0; i < FX_NMS_OWN; ++i) {
+      bucket[i] = 0u;
+      if (i * FX_NMS_THREADS + tid >= count) continue;
+      bucket[i] = ((uint32_t)(key[i] >> 32) - first) >> shift;
+      slot[i] = atomicAdd(&s_bucket[bucket[i]], 1u);
     }
     __syncthreads();
     {
-      // against the kept list: candidate c, every 16th kept box
-      const uint32_t c = tid & 63u, part = tid >> 6;
-      if (c < m) {
-        const Box cb{s_obox[c][0], s_obox[c][1], s_obox[c][2], s_obox[c][3]};
-        const float ca = s_carea[c];
-        bool dead = false;
-        for (uint32_t k = part; k < nk && !dead; k += FX_NMS_THREADS / 64u) {
-          const Box kb{s_kbox[k][0], s_kbox[k][1], s_kbox[k][2], s_kbox[k][3]};
-          dead = overlaps(kb, s_karea[k], cb, ca, d.iou_thr);
-        }
-        if (dead) atomicOr(&s_dead[c >> 5], 1u << (c & 31u));
-      }
-      // inside the chunk: candidate i against four later candidates
-      const uint32_t i = tid >> 4, j0 = (tid & 15u) * 4u;
-      if (i < m) {
-        const Box ib{s_obox[i][0], s_obox[i][1], s_obox[i][2], s_obox[i][3]};
-        const float ia = s_carea[i];
+      const uint2 n = ((const uint2*)s_bucket)[tid];
+      static_assert(FX_NMS_BUCKETS == 2u * FX_NMS_THREADS, "two buckets a thread");
+      uint32_t ahead = n.x + n.y;
 #pragma unroll
-        for (uint32_t jj = 0; jj < 4u; ++jj) {
-          const uint32_t j = j0 + jj;
-          if (j > i && j < m) {
-            const Box jb{s_obox[j][0], s_obox[j][1], s_obox[j][2], s_obox[j][3]};
-            if (overlaps(ib, ia, jb, s_carea[j], d.iou_thr)) atomicOr(&s_in[j][i >> 5], 1u << (i & 31u));
-          }
-        }
+      for (uint32_t o = 1; o < 64u; o <<= 1) {
+        const uint32_t t = (uint32_t)__shfl_up((int)ahead, o, 64);
+        ahead += lane >= o ? t : 0u;
       }
+      if (lane == 63u) s_wave[wave] = ahead;
+      if (max(n.x, n.y) > FX_NMS_CROWD) s_crowd = 1u;
+      __syncthreads();
+      const uint32_t w = s_wave[lane & (FX_NMS_THREADS / 64u - 1u)];
+      ahead += fx_wave_sum(lane < wave ? w : 0u, lane) - n.x - n.y;
+      ((uint2*)s_bucket)[tid] = make_uint2(ahead | (n.x << 16), (ahead + n.x) | (n.y << 16));   // start and number
+    }
+    placed = uni(s_crowd) == 0u;   // many scores in one bucket (all alike, say): the sort below
+    __syncthreads();
+    if (placed) {
+      uint32_t entry[FX_NMS_OWN];
+#pragma unroll
+      for (uint32_t i = 0; i < FX_NMS_OWN; ++i) {
+        if (i * FX_NMS_THREADS + tid >= count) continue;
+        entry[i] = s_bucket[bucket[i]];
+        s_part[(entry[i] & 0xffffu) + slot[i]] = key[i];
+      }
+      __syncthreads();
+#pragma unroll
+      for (uint32_t i = 0; i < FX_NMS_OWN; ++i) {
+        if (i * FX_NMS_THREADS + tid >= count) continue;
+        const uint32_t start = entry[i] & 0xffffu, n = entry[i] >> 16;
+        uint32_t at = start;
+        if (n > 1u)
+          for (uint32_t k = 0; k < n; ++k) at += s_part[start + k] < key[i] ? 1u : 0u;
+        const float4 b = make_float4(__uint_as_float((uint32_t)corner[i][0]), __uint_as_float((uint32_t)(corner[i][0] >> 32)),
+                                     __uint_as_float((uint32_t)corner[i][1]), __uint_as_float((uint32_t)(corner[i][1] >> 32)));
+        const float4 m = moved_by(b, (float)label[i] * class_step);
+        s_order[at] = key[i];
+        s_moved[at] = m;
+        s_box[at] = b;
+        s_area[at] = area_of(m);
+        s_label[at] = label[i];
+      }
+      FX_NMS_STAMP(4);
+    } else {
+#pragma unroll
+      for (uint32_t i = 0; i < FX_NMS_OWN; ++i)
+        if (i * FX_NMS_THREADS + tid < count) s_keys[i * FX_NMS_THREADS + tid] = key[i];
+    }
+  } else {
+    if (slices > 1u)
+      for (uint32_t k = tid; k < count; k += FX_NMS_THREADS) s_keys[k] = __hip_atomic_load(&g_keys[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (!placed) {
+    // 2. bitonic sort (ascending keys = descending score, ascending index); the tail is padding.
+    // Stages whose partners lie at most 64 apart stay inside aligned blocks of 128 keys: a wave
+    // runs all of them on its blocks without a workgroup barrier (LDS accesses of one wave are
+    // performed in order), so a phase costs one barrier per wider stage plus one.
+    uint32_t n2 = 128u;
+    while (n2 < count) n2 <<= 1;
+    for (uint32_t i = count + tid; i < n2; i += FX_NMS_THREADS) s_keys[i] = ~0ull;
+    __syncthreads();
+    auto exchange = [&](uint32_t i, uint32_t j, uint32_t k) {
+      const uint32_t l = i | j;
+      const uint64_t a = s_keys[i], b = s_keys[l];
+      const bool up = (i & k) == 0u;
+      if ((a > b) == up) { s_keys[i] = b; s_keys[l] = a; }
+    };
+    auto narrow_stages = [&](uint32_t k_first, uint32_t k_last) {   // every stage j <= 64 of phases k_first .. k_last
+      for (uint32_t blk = wave; blk < (n2 >> 7); blk += FX_NMS_THREADS / 64u) {
+        // the block's 128 keys in registers, two a lane (positions lane and lane + 64): the stages
+        // exchange them between lanes, LDS is read and written once per call
+        const uint32_t p0 = (blk << 7) + lane;
+        uint64_t ka = s_keys[p0], kb = s_keys[p0 + 64u];
+        for (uint32_t k = k_first; k <= k_last; k <<= 1) {
+          const bool up_a = (p0 & k) == 0u, up_b = ((p0 + 64u) & k) == 0u;
+          if (k >= 128u) {   // partners 64 apart: the lane's own two keys (up_a == up_b here)
+            const bool sw = (ka > kb) == up_a;
+            const uint64_t lo = sw ? kb : ka, hi = sw ? ka : kb;
+            ka = lo; kb = hi;
+          }
+          if (k >= 64u) { ka = bitonic_step<32>(ka, up_a, lane); kb = bitonic_step<32>(kb, up_b, lane); }
+          if (k >= 32u) { ka = bitonic_step<16>(ka, up_a, lane); kb = bitonic_step<16>(kb, up_b, lane); }
+          if (k >= 16u) { ka = bitonic_step<8>(ka, up_a, lane); kb = bitonic_step<8>(kb, up_b, lane); }
+          if (k >= 8u) { ka = bitonic_step<4>(ka, up_a, lane); kb = bitonic_step<4>(kb, up_b, lane); }
+          if (k >= 4u) { ka = bitonic_step<2>(ka, up_a, lane); kb = bitonic_step<2>(kb, up_b, lane); }
+          ka = bitonic_step<1>(ka, up_a, lane); kb = bitonic_step<1>(kb, up_b, lane);
+        }
+        s_keys[p0] = ka; s_keys[p0 + 64u] = kb;
+      }
+    };
+    narrow_stages(2u, 128u);
+    __syncthreads();
+    for (uint32_t k = 256u; k <= n2; k <<= 1) {
+      for (uint32_t j = k >> 1; j >= 128u; j >>= 1) {
+        for (uint32_t p = tid; p < (n2 >> 1); p += FX_NMS_THREADS) exchange(((p & ~(j - 1u)) << 1) | (p & (j - 1u)), j, k);
+        __syncthreads();
+      }
+      narrow_stages(k, k);
+      __syncthreads();
+    }
+    FX_NMS_STAMP(4);
+  }
+
+  auto write_out = [&](uint32_t slot, uint64_t k, const float4& b, uint32_t label) {
+    float* o = dets + (size_t)slot * 5u;
+    o[0] = b.x; o[1] = b.y; o[2] = b.z; o[3] = b.w;
+    o[4] = from_orderable(~(uint32_t)(k >> 32));
+    out_labels[slot] = (int64_t)label;
+    if (out_index) out_index[slot] = (int64_t)(d.mode == 1 ? row_of((uint32_t)k) * NC + label : (uint32_t)k);   // position among the candidates proper
+  };
+
+  // 3. greedy walk
+  if (tid == 0) s_nk = 0u;
+  if (tid < 4u * FX_NMS_CHUNK) ((uint32_t*)s_in)[tid] = 0u;
+  if (tid < 4u) ((uint32_t*)s_dead)[tid] = 0u;
+  __syncthreads();
+  uint32_t nk = 0u, p = 0u;
+  for (uint32_t pos = 0; pos < count && nk < d.max_num; pos += FX_NMS_CHUNK, p ^= 1u) {
+    const uint32_t m = min(FX_NMS_CHUNK, count - pos);
+    if (!placed) {
+      if (tid < m) {
+        const uint32_t idx = (uint32_t)s_keys[pos + tid], r = row_of(idx), label = label_of(idx, r);
+        float4 b;
+        if constexpr (HEAD) b = head_box(head_row(h, task, head_number(h, r, label)));
+        else b = *(const float4*)(boxes + (size_t)r * 4u);
+        const float4 q = moved_by(b, (float)label * class_step);
+        s_cbox[tid] = b;
+        s_obox[tid] = q;
+        s_carea[tid] = area_of(q);
+        s_clabel[tid] = label;
+      }
+      __syncthreads();
+    }
+    const float4* const moved = placed ? s_moved + pos : s_obox;
+    const float* const areas = placed ? s_area + pos : s_carea;
+    {
+      // inside the chunk: pairs (i, j), i < j; lanes behind i take (i, lane), those before it (63 - i, 63 - lane), so that two
+      // rows of pairs fill one wave
+      uint32_t pi[2], pj[2];
+      float4 bi[2], bj[2];
+      float ai[2], aj[2];
+#pragma unroll
+      for (uint32_t e = 0; e < 2u; ++e) {
+        const uint32_t row = uni(wave) * 2u + e;
+        const bool back = lane < row;
+        pi[e] = back ? 63u - row : row;
+        pj[e] = back ? 63u - lane : lane;
+        const uint32_t i = min(pi[e], m - 1u), j = min(pj[e], m - 1u);   // (pairs that are none: not looked at below)
+        bi[e] = moved[i];
+        bj[e] = moved[j];
+        ai[e] = areas[i];
+        aj[e] = areas[j];
+      }
+      const float4 q = moved[min(lane, m - 1u)];
+      const float ca = areas[min(lane, m - 1u)];
+      const uint64_t n0 = near_lanes(bi[0], bj[0], d.iou_thr), n1 = near_lanes(bi[1], bj[1], d.iou_thr);
+#pragma unroll
+      for (uint32_t e = 0; e < 2u; ++e) {
+        const uint64_t near = e == 0u ? n0 : n1;
+        if (near == 0ull) continue;
+        const uint64_t over = overlap_lanes(near, bi[e], ai[e], bj[e], aj[e], d.iou_thr);
+        if (((over >> lane) & 1ull) != 0ull && pi[e] < pj[e] && pj[e] < m) atomicOr(&s_in[p][pj[e]][pi[e] >> 5], 1u << (pi[e] & 31u));
+      }
+      // candidate `lane` against every 16th kept box, four of them at a time (a box that is there twice does not matter)
+      uint64_t dead = 0ull;
+      for (uint32_t k = uni(wave); k < nk; k += FX_NMS_THREADS / 16u) {
+        float4 o[4];
+        float oa[4];
+        uint64_t near[4];
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e) {
+          o[e] = s_kbox[min(k + e * (FX_NMS_THREADS / 64u), nk - 1u)];
+          oa[e] = s_karea[min(k + e * (FX_NMS_THREADS / 64u), nk - 1u)];
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e) near[e] = near_lanes(o[e], q, d.iou_thr);
+        if ((near[0] | near[1] | near[2] | near[3]) == 0ull) continue;
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e)
+          if (near[e] != 0ull) dead |= overlap_lanes(near[e], o[e], oa[e], q, ca, d.iou_thr);
+      }
+      if (dead != 0ull && lane < 2u) atomicOr(&s_dead[p][lane], (uint32_t)(dead >> (32u * lane)));
     }
     __syncthreads();
+    if (wave == 1u) {   // for the chunk after this one; the last to read these has passed a barrier
+      s_in[p ^ 1u][lane][0] = 0u;
+      s_in[p ^ 1u][lane][1] = 0u;
+      if (lane < 2u) s_dead[p ^ 1u][lane] = 0u;
+    }
     if (wave == 0u) {
       // In order, candidate i is kept unless a kept one before it overlaps it.  All candidates
       // decide together, round after round: one with a kept overlapping predecessor is dead, one
       // whose overlapping predecessors are all dead is kept, the others wait; the first undecided
       // candidate always decides, and with few overlaps two or three rounds settle the chunk
       // (a walk from candidate to candidate costs 64 dependent steps).
-      const uint64_t in = ((uint64_t)s_in[lane][1] << 32) | (uint64_t)s_in[lane][0];
+      const uint64_t in = ((uint64_t)s_in[p][lane][1] << 32) | (uint64_t)s_in[p][lane][0];
       const uint64_t valid = m >= 64u ? ~0ull : (1ull << m) - 1ull;
-      uint64_t deadm = (((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)s_dead[1]) << 32) |
-                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)s_dead[0])) | ~valid;
+      uint64_t deadm = (((uint64_t)uni(s_dead[p][1]) << 32) | (uint64_t)uni(s_dead[p][0])) | ~valid;
       uint64_t keptm = 0ull;
       bool decided = ((deadm >> lane) & 1ull) != 0ull;
       for (;;) {
@@ -546,21 +731,20 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
       const uint32_t kept_now = (uint32_t)__popcll(keep);
       if ((keep >> lane) & 1ull) {
         const uint32_t slot = nk + rank;
-        s_kbox[slot][0] = s_obox[lane][0]; s_kbox[slot][1] = s_obox[lane][1];
-        s_kbox[slot][2] = s_obox[lane][2]; s_kbox[slot][3] = s_obox[lane][3];
-        s_karea[slot] = s_carea[lane];
-        float* o = dets + (size_t)slot * 5u;
-        o[0] = s_cbox[lane][0]; o[1] = s_cbox[lane][1]; o[2] = s_cbox[lane][2]; o[3] = s_cbox[lane][3];
-        o[4] = s_cscore[lane];
-        out_labels[slot] = (int64_t)s_clabel[lane];
-        if (out_index) out_index[slot] = (int64_t)s_cidx[lane];
+        s_kbox[slot] = moved[lane];
+        s_karea[slot] = areas[lane];
+        s_kept[slot] = pos + lane;
+        if (!placed) write_out(slot, s_keys[pos + lane], s_cbox[lane], s_clabel[lane]);
       }
       if (lane == 0u) s_nk = nk + kept_now;
     }
     __syncthreads();
-    nk = s_nk;
+    nk = uni(s_nk);
   }
   FX_NMS_STAMP(5);
+  // (behind the walk, not in it: its barriers would wait until the stores have been acknowledged)
+  if (placed)
+    for (uint32_t k = tid; k < nk; k += FX_NMS_THREADS) write_out(k, s_order[s_kept[k]], s_box[s_kept[k]], s_label[s_kept[k]]);
   // rows past the kept ones are zero: the outputs have a fixed shape
   for (uint32_t k = nk * 5u + tid; k < d.max_num * 5u; k += FX_NMS_THREADS) dets[k] = 0.0f;
   for (uint32_t k = nk + tid; k < d.max_num; k += FX_NMS_THREADS) {
@@ -597,7 +781,7 @@ uint32_t fx_nms_slices(const fx_nms_desc& d) {
 }
 
 size_t fx_nms_workspace_bytes(int n_tasks, uint32_t key_cap) {
-  return (size_t)n_tasks * ((size_t)FX_NMS_WS_WORDS * 4 + (size_t)key_cap * 8);
+  return (size_t)n_tasks * ((size_t)FX_NMS_WS_WORDS * 4 + (size_t)key_cap * 8 + (key_cap >= FX_NMS_ROOMY ? FX_NMS_FEW * 16u : 0u));
 }
 size_t fx_nms_workspace_clear_bytes(int n_tasks) { return (size_t)n_tasks * FX_NMS_WS_WORDS * 4; }
 
@@ -667,8 +851,8 @@ int fx_launch_head_nms(const fx_head_desc& head, const fx_nms_desc& d, uint32_t 
     rows += v.cells * v.anchors;
     m.groups += v.run_groups * v.anchors;
   }
-  // a workgroup per CU over all images, at most 64 an image (fx_nms_slices), none without a group for every wave
-  const uint32_t slices = std::min<uint32_t>(std::min<uint32_t>(std::max(device_cus() / (uint32_t)d.n_tasks, 1u), 64u),
+  // a workgroup per CU over all images, at most 128 an image (above HeadLevel), none without a group for every wave
+  const uint32_t slices = std::min<uint32_t>(std::min<uint32_t>(std::max(device_cus() / (uint32_t)d.n_tasks, 1u), 128u),
                                              (m.groups + FX_NMS_THREADS / 64u - 1u) / (FX_NMS_THREADS / 64u));
   return launch_sort_nms(d, m, slices, key_cap, workspace, err_host, stream);
 }
