@@ -37,7 +37,7 @@ hipError_t fx_launch_compact_stream(int rank, const uint32_t* sb, const FxLaunch
                                     hipStream_t stream, const FxSpecKernels* spec);
 uint32_t fx_stream_lds_bytes(const FxLaunchInfo& li, bool compiled);
 bool fx_spec_has_stream(const FxSpecKernels* spec);
-bool fx_spec_has_lean(const FxSpecKernels* spec);
+bool fx_spec_has_lean(const FxSpecKernels* spec, const FxLeanArgs* lean);
 // fx_head.hip
 hipError_t fx_launch_head_stream(const FxHeadLaunch& hl, const FxDyn* dyn, hipStream_t stream);
 hipError_t fx_upload_words(const uint64_t* words, size_t n_words, void* dst, hipStream_t stream);
@@ -723,7 +723,7 @@ static const FxLeanArgs* lean_of(const fx::Plan* pl) {
 int fx_plan_dense_lean(const fx_plan* p) {
   if (!p) return 0;
   const fx::Plan* pl = P(p);
-  return (pl->mode == FX_MODE_DENSE && lean_of(pl) && pl->lean.n_outs != 0 && fx_spec_has_lean(spec_of(pl))) ? 1 : 0;
+  return (pl->mode == FX_MODE_DENSE && fx_spec_has_lean(spec_of(pl), lean_of(pl))) ? 1 : 0;
 }
 void fx_set_dense_lean(int on) { g_dense_lean.store(on ? 1 : 0, std::memory_order_relaxed); }
 

@@ -264,6 +264,8 @@ struct FxHeader {
 #define FX_LEAN_S 16     // scalars of a region that the lean kernel's argument block holds
 #define FX_LEAN_LEAD 1u
 #define FX_LEAN_HALF 2u
+#define FX_LEAN_COLS 4u  // the outputs are the columns of rows of four elements (fx_dense_cols): out[0] is a column,
+                         // its lead_* the place of a row's first element, gp_* division by inner, n_groups the rows
 // One output of the region: the fields of FxOut that place a work item, the leading load's
 // affine map, and the two buffers.  160 bytes, laid out so that a kernel for rank <= 3 reads the
 // first 128 only; the records start at a multiple of 64 bytes in the argument segment.

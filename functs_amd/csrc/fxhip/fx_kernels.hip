@@ -220,7 +220,12 @@ const FxSpecKernels* fx_spec_find(uint64_t hash) {
   return it == spec_table().end() ? nullptr : &it->second;   // entries are never erased
 }
 bool fx_spec_has_stream(const FxSpecKernels* spec) { return spec && spec->stream != nullptr; }
-bool fx_spec_has_lean(const FxSpecKernels* spec) { return spec && spec->lean != nullptr; }
+// the short-argument kernel that serves a plan's FxLeanArgs, if its programs have one
+static const void* lean_kernel(const FxSpecKernels* spec, const FxLeanArgs* lean) {
+  if (!spec || !lean || lean->n_outs == 0) return nullptr;
+  return lean->out[0].lead & FX_LEAN_COLS ? spec->cols : spec->lean;
+}
+bool fx_spec_has_lean(const FxSpecKernels* spec, const FxLeanArgs* lean) { return lean_kernel(spec, lean) != nullptr; }
 int fx_spec_count() {
   std::lock_guard<std::mutex> g(spec_mutex());
   return (int)spec_table().size();
@@ -330,7 +335,7 @@ static hipError_t allow_lds(K kernel, uint32_t bytes) {
 hipError_t fx_launch_dense(int rank, const uint32_t* sb, const FxLaunchInfo& li, const FxDyn* dyn, uint32_t grid,
                            hipStream_t stream, const FxSpecKernels* spec, const FxLeanArgs* lean, uint32_t slot_err) {
   if (grid == 0) return hipSuccess;
-  if (spec && spec->lean && lean && lean->n_outs != 0) {
+  if (const void* kernel = lean_kernel(spec, lean)) {
     // the lean kernel: a short argument block instead of FxLaunch + FxDyn
     FxLeanArgs a = *lean;
     a.err_ptr = slot_err ? dyn->p[slot_err - 1u] : 0;
@@ -342,8 +347,9 @@ hipError_t fx_launch_dense(int rank, const uint32_t* sb, const FxLaunchInfo& li,
     memcpy(a.p, dyn->p, sizeof(uint64_t) * a.n_p);
     memcpy(a.s, dyn->s, sizeof(uint32_t) * a.n_s);
     void* args[2] = {(void*)&sb, (void*)&a};
-    return hipLaunchKernel(spec->lean, dim3(grid), dim3(FX_BLOCK), args, spec->lean_stages ? lds_bytes_compiled(li) : 0u,
-                           stream);
+    const bool cols = (a.out[0].lead & FX_LEAN_COLS) != 0;
+    if (cols) grid = std::min<uint32_t>(a.total_units, 256u * 12u);   // (as many as the other dense kernels take)
+    return hipLaunchKernel(kernel, dim3(grid), dim3(FX_BLOCK), args, cols || spec->lean_stages ? lds_bytes_compiled(li) : 0u, stream);
   }
   const FxLaunch la = make_launch(li);
   const uint32_t lds = fx_lds_bytes(li);

@@ -2644,6 +2644,59 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
       }
     }
   }
+  // An output of rows of four elements that went into boxes column by column (every column a program of its own):
+  // where they have compiled kernels a lane runs the programs side by side on one row and stores the row at once
+  // (fx_dense_cols).
+  if (P->mode == FX_MODE_DENSE && classes.size() == 1 && classes[0].outs.size() == 4 && P->grid > 0 &&
+      P->lean.n_outs == 0 && P->sptr.size() + P->tptr.size() * (size_t)T <= FX_LEAN_P &&
+      P->sscal.size() + P->tscal.size() * (size_t)T <= FX_LEAN_S) {
+    const ClassBuild& cb = classes[0];
+    const FxOut& first = cb.outs[0];
+    bool fits = taskmap.size() == (size_t)T && first.box != 0;
+    for (size_t i = 0; fits && i < taskmap.size(); ++i) fits = taskmap[i] == (uint32_t)i;
+    for (size_t o = 0; fits && o < cb.outs.size(); ++o) {
+      const FxOut& od = cb.outs[o];
+      fits = od.box != 0 && od.dtype == FX_F32 && od.vt == FX_VT_F && od.lead && !od.rowwave && od.ptr_slot == first.ptr_slot &&
+             od.task_stride == first.task_stride && od.inner == first.inner && od.vd == first.vd && od.numel == first.numel && od.inner > 0;
+      for (int k = 1; fits && k < FX_MAXR; ++k) fits = od.dim[k] == first.dim[k] && od.magic[k] == first.magic[k] && od.shift[k] == first.shift[k];
+      if (!fits) break;
+      const FxAffine &a = cb.affs[(size_t)od.box - 1], &a0 = cb.affs[(size_t)first.box - 1];
+      fits = a.base == a0.base + (int32_t)o && a.tcoef == a0.tcoef;
+      for (int k = 0; k < FX_MAXR; ++k) fits = fits && fx_aff_coef(&a, k) == fx_aff_coef(&a0, k);
+      for (int k = 0; k < FX_MAXLOOP; ++k) fits = fits && a.rcoef[k] == 0;
+    }
+    if (fits) {
+      const FxAffine& at = cb.affs[(size_t)first.box - 1];
+      FxLeanArgs& f = P->lean;
+      f.blob_words = (uint32_t)blob.size();
+      f.n_p = (uint32_t)(P->sptr.size() + P->tptr.size() * (size_t)T);
+      f.n_s = (uint32_t)(P->sscal.size() + P->tscal.size() * (size_t)T);
+      f.n_outs = 1;
+      f.bpt = (first.numel + FX_BLOCK - 1u) / FX_BLOCK;
+      f.total_units = f.bpt * (uint32_t)T;
+      fx_fastdiv_make(f.bpt, &f.bpt_magic, &f.bpt_shift);
+      f.n_sptr = h.n_sptr;
+      f.n_tptr = h.n_tptr;
+      f.cls_off = off_class;
+      P->lean_slot_err = h.slot_err;
+      FxLeanOut& lo = f.out[0];
+      lo.ptr_slot = first.ptr_slot;
+      lo.lead = FX_LEAN_COLS;
+      lo.task_stride = first.task_stride;
+      lo.inner = first.inner;
+      lo.vd = first.vd;
+      lo.n_groups = first.numel;
+      fx_fastdiv_make(first.inner, &lo.gp_magic, &lo.gp_shift);
+      for (int k = 1; k < FX_MAXR; ++k) {
+        lo.dms[k - 1][0] = first.dim[k];
+        lo.dms[k - 1][1] = first.magic[k];
+        lo.dms[k - 1][2] = first.shift[k];
+      }
+      for (int k = 0; k < FX_MAXR; ++k) lo.lead_cf[k] = fx_aff_coef(&at, k);
+      lo.lead_base = at.base;
+      lo.lead_tcoef = at.tcoef;
+    }
+  }
 
   P->lds_bytes = (uint32_t)((blob.size() + 2 * (P->sptr.size() + P->tptr.size() * (size_t)T) +
                              (P->sscal.size() + P->tscal.size() * (size_t)T) + 4 +
