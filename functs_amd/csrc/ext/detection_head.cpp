@@ -15,6 +15,7 @@
 //
 // The match is structural and complete, as that of the loop kernels (attention.cpp).  Both forms stay in the graph, behind
 //   if fx::detection_head_fits(operands): fx::detection_head(operands)  else: the chain,
+// (fx::detection_head_pairs and the chain with its functs::unbatch_detection_pairs where that is all that is made of it)
 // because a call may come with operands that only the chain serves (gradients, a capture, other devices).
 #include <ATen/ATen.h>
 #include <ATen/autocast_mode.h>
@@ -299,18 +300,26 @@ bool fuseAt(Node* tail) {
     choice->setSourceRange(tail->sourceRange());
     choice->insertBefore(tail);
     Block *yes = choice->addBlock(), *no = choice->addBlock();
-    Node* head = g->create(sym::DetectionHead(), args, 3);
+    // where nothing but the list of pairs is made of the results, the launch waits for its own counts
+    Node* pairs = tail->output(0)->uses().size() == 1 ? tail->output(0)->uses()[0].user : nullptr;
+    const bool alone = pairs && pairs->kind() == Symbol::fromQualString("functs::unbatch_detection_pairs") && pairs->owningBlock() == tail->owningBlock() &&
+                       pairs->inputs().size() == 3 && pairs->input(0) == tail->output(0) && pairs->input(1) == tail->output(1) &&
+                       pairs->input(2) == tail->output(2) && tail->output(1)->uses().size() == 1 && tail->output(2)->uses().size() == 1;
+    Node* end = alone ? pairs : tail;
+    Node* head = g->create(alone ? sym::DetectionHeadPairs() : sym::DetectionHead(), args, end->outputs().size());
     head->setSourceRange(tail->sourceRange());
     yes->appendNode(head);
-    for (size_t k = 0; k < 3; ++k) {
-      head->output(k)->setType(c10::TensorType::get());
+    for (size_t k = 0; k < end->outputs().size(); ++k) {
+      head->output(k)->setType(end->output(k)->type());
       yes->registerOutput(head->output(k));
-      Value* out = choice->addOutput()->setType(c10::TensorType::get());
-      tail->output(k)->replaceAllUsesWith(out);
+      Value* out = choice->addOutput()->setType(end->output(k)->type());
+      end->output(k)->replaceAllUsesWith(out);
     }
     // the chain, in its order; what else feeds it is defined before it
     Node* last = nullptr;
-    for (Node* n : {dense, filter, tail}) {
+    std::vector<Node*> chain{dense, filter, tail};
+    if (alone) chain.push_back(pairs);
+    for (Node* n : chain) {
       if (last) n->moveAfter(last);
       else {
         Node* mark = g->create(c10::prim::Constant, 0);
@@ -320,20 +329,21 @@ bool fuseAt(Node* tail) {
       }
       last = n;
     }
-    for (Value* o : tail->outputs()) no->registerOutput(o);
+    for (Value* o : end->outputs()) no->registerOutput(o);
     return true;
   }
   return false;
 }
 
 bool fuseIn(Block* b) {
+  // (collected first: what is joined moves nodes behind the tail into another block)
   bool changed = false;
-  for (auto it = b->nodes().begin(); it != b->nodes().end();) {
-    Node* n = *it;
-    ++it;
+  std::vector<Node*> tails;
+  for (Node* n : b->nodes()) {
     for (Block* inner : n->blocks()) changed = fuseIn(inner) || changed;
-    changed = fuseAt(n) || changed;
+    if (n->kind() == Symbol::fromQualString("functs::multiclass_nms_batched")) tails.push_back(n);
   }
+  for (Node* n : tails) changed = fuseAt(n) || changed;
   return changed;
 }
 
@@ -383,39 +393,58 @@ bool fits(const Operands& o) {
   return capture == hipStreamCaptureStatusNone;
 }
 
-void runHead(Stack& stack) {
-  const Operands o = operandsOf(stack);
+// what the launchers take besides the operands
+struct Launch { fx_head_desc h; int64_t rows = 0; };
+Launch launchOf(const Operands& o) {
   TORCH_CHECK(fits(o), "fx::detection_head: operands that the kernel does not serve");
   raiseAsyncErrors();
-  fx_head_desc h;
-  memset(&h, 0, sizeof h);
-  h.n_levels = (int32_t)o.maps.size();
-  h.keep_thr = (float)o.keep_thr;
-  h.strides = o.strides.data_ptr<float>();
-  int64_t rows = 0;
-  for (size_t l = 0; l < o.maps.size(); ++l) {
-    h.maps[l] = o.maps[l].data_ptr<float>();
-    h.bases[l] = o.bases[l].data_ptr<float>();
-    h.shifts[l] = o.shifts[l].data_ptr<float>();
-    h.cells[l] = (uint32_t)(o.maps[l].size(2) * o.maps[l].size(3));
-    h.anchors[l] = (uint32_t)o.bases[l].size(0);
-    rows += (int64_t)h.cells[l] * h.anchors[l];
+  Launch l;
+  memset(&l.h, 0, sizeof l.h);
+  l.h.n_levels = (int32_t)o.maps.size();
+  l.h.keep_thr = (float)o.keep_thr;
+  l.h.strides = o.strides.data_ptr<float>();
+  for (size_t k = 0; k < o.maps.size(); ++k) {
+    l.h.maps[k] = o.maps[k].data_ptr<float>();
+    l.h.bases[k] = o.bases[k].data_ptr<float>();
+    l.h.shifts[k] = o.shifts[k].data_ptr<float>();
+    l.h.cells[k] = (uint32_t)(o.maps[k].size(2) * o.maps[k].size(3));
+    l.h.anchors[k] = (uint32_t)o.bases[k].size(0);
+    l.rows += (int64_t)l.h.cells[k] * l.h.anchors[k];
   }
-  auto r = launchHeadTail(h, o.maps[0].device(), o.images, rows, o.classes, o.score_thr, o.iou, o.max_num);
+  return l;
+}
+void runHead(Stack& stack) {
+  const Operands o = operandsOf(stack);
+  const Launch l = launchOf(o);
+  auto r = launchHeadTail(l.h, o.maps[0].device(), o.images, l.rows, o.classes, o.score_thr, o.iou, o.max_num);
   for (at::Tensor& t : r) push(stack, std::move(t));
 }
+void runHeadPairs(Stack& stack) {
+  const Operands o = operandsOf(stack);
+  const Launch l = launchOf(o);
+  push(stack, launchHeadPairs(l.h, o.maps[0].device(), o.images, l.rows, o.classes, o.score_thr, o.iou, o.max_num));
+}
 
+std::vector<c10::Argument> headArguments() {
+  const auto list = c10::ListType::ofTensors();
+  return {c10::Argument("maps", list), c10::Argument("bases", list), c10::Argument("shifts", list), c10::Argument("strides", c10::TensorType::get()),
+          c10::Argument("images", c10::IntType::get()), c10::Argument("classes", c10::IntType::get()), c10::Argument("keep_thr", c10::FloatType::get()),
+          c10::Argument("score_thr", c10::FloatType::get()), c10::Argument("iou_threshold", c10::FloatType::get()), c10::Argument("max_num", c10::IntType::get())};
+}
+
+// (all conservative: the answer of the first depends on modes and the current stream too)
 RegisterOperators registerHead({
-    Operator("fx::detection_head_fits(Tensor[] maps, Tensor[] bases, Tensor[] shifts, Tensor strides, int images, int classes, float keep_thr, "
-             "float score_thr, float iou_threshold, int max_num) -> bool",
-             [](Stack& stack) {
+    Operator("fx::detection_head_fits", "", headArguments(), {c10::Argument("", c10::BoolType::get())},
+             Operation([](Stack& stack) {
                const Operands o = operandsOf(stack);
                push(stack, fits(o));
-             },
-             c10::AliasAnalysisKind::CONSERVATIVE),   // (what it answers depends on modes and the current stream too)
-    Operator("fx::detection_head(Tensor[] maps, Tensor[] bases, Tensor[] shifts, Tensor strides, int images, int classes, float keep_thr, "
-             "float score_thr, float iou_threshold, int max_num) -> (Tensor dets, Tensor labels, Tensor n)",
-             runHead, c10::AliasAnalysisKind::CONSERVATIVE),
+             }),
+             c10::AliasAnalysisKind::CONSERVATIVE),
+    Operator("fx::detection_head", "", headArguments(),
+             {c10::Argument("dets", c10::TensorType::get()), c10::Argument("labels", c10::TensorType::get()), c10::Argument("n", c10::TensorType::get())},
+             Operation(runHead), c10::AliasAnalysisKind::CONSERVATIVE),
+    Operator("fx::detection_head_pairs", "", headArguments(), {c10::Argument("", detectionPairsType())}, Operation(runHeadPairs),
+             c10::AliasAnalysisKind::CONSERVATIVE),
 });
 
 }  // namespace

@@ -103,6 +103,10 @@ bool FuseDetectionHead(std::shared_ptr<torch::jit::Graph> graph);
 // that launch: (dets [images, max_num, 5], labels [images, max_num], kept counts [images], which land in pinned host memory)
 std::array<at::Tensor, 3> launchHeadTail(const fx_head_desc& head, c10::Device device, int64_t images, int64_t rows, int64_t classes,
                                          double score_thr, double iou_thr, int64_t max_num);
+// that launch and the wait for its counts: per image (dets, labels), as functs::unbatch_detection_pairs makes them; its type
+c10::IValue launchHeadPairs(const fx_head_desc& head, c10::Device device, int64_t images, int64_t rows, int64_t classes, double score_thr,
+                            double iou_thr, int64_t max_num);
+c10::TypePtr detectionPairsType();
 // raises what earlier launches reported (fx_async_error), as every functor does before it launches
 void raiseAsyncErrors();
 

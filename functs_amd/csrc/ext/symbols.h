@@ -53,6 +53,7 @@ FUNCTS_SYM(LstmStack, "fx::lstm_stack")
 FUNCTS_SYM(AttentionSteps, "fx::attention_steps")
 // a detection head with its tail as one node, and whether the node serves its operands (detection_head.cpp)
 FUNCTS_SYM(DetectionHead, "fx::detection_head")
+FUNCTS_SYM(DetectionHeadPairs, "fx::detection_head_pairs")
 FUNCTS_SYM(DetectionHeadFits, "fx::detection_head_fits")
 // attributes of tssa::ParallelFunctor
 FUNCTS_SYM(parallel_degree, "attr::parallel_degree")
