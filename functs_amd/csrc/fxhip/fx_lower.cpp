@@ -2344,6 +2344,24 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
           pure = fx_op_is_pure_unary(in.op) || (fx_op_is_pure_binary(in.op) && (in.flags & FX_F_IMM));
         }
         od.pure = pure ? 1u : 0u;
+        // An elementwise output whose operand lies as the output does is one long row: no group ends inside a row of an odd
+        // length, and every access but the last is whole and aligned (8 191 x 4 095 bfloat16 + 1 25.0 -> 22.5 us,
+        // 3 001 x 1 111 floats 6.2 -> 5.8).
+        if (pure && P->mode == FX_MODE_DENSE && dims.size() > 1 && od.numel > 0 && od.numel < 0x7ffffff0u) {
+          const FxAffine& at = L.affs[(size_t)L.code[p.begin].b];
+          const int64_t step = fx_aff_coef(&at, (int)dims.size() - 1);
+          int64_t stride = 1;
+          bool flat = step != 0 || dims.back() == 1;
+          for (int k = (int)dims.size() - 1; k >= 0; --k) {
+            flat = flat && (dims[(size_t)k] == 1 || fx_aff_coef(&at, k) == step * stride);
+            stride *= dims[(size_t)k];
+          }
+          if (flat && dims.back() > 1) {
+            Shape row(dims.size(), 1);
+            row.back() = (int64_t)od.numel;
+            fillDims(od, row);
+          }
+        }
       }
       if (P->mode == FX_MODE_COMPACT) {
         FX_CHECK(!s.empty() && s[0] == (int64_t)cb.cls.n_rows, FX_E_INVALID,
@@ -2618,7 +2636,9 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
         const FxOut& od = cb.outs[o];
         FxLeanOut& lo = f.out[o];
         lo.ptr_slot = od.ptr_slot;
-        lo.lead = (od.lead ? FX_LEAN_LEAD : 0u) | (half_out(od) ? FX_LEAN_HALF : 0u);
+        // (from 4 MB on: what fits a die's cache may stay there for whoever reads it next)
+        const bool large = od.pure && (uint64_t)od.numel * (half_out(od) ? 2u : 4u) >= (4u << 20);
+        lo.lead = (od.lead ? FX_LEAN_LEAD : 0u) | (half_out(od) ? FX_LEAN_HALF : 0u) | (large ? FX_LEAN_STREAM : 0u);
         lo.block_begin = od.block_begin;
         lo.task_stride = od.task_stride;
         lo.unit_items = od.unit_items;
