@@ -632,53 +632,36 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
   if (tid < 4u) ((uint32_t*)s_dead)[tid] = 0u;
   __syncthreads();
   uint32_t nk = 0u, p = 0u;
+  // (not placed: boxes of a chunk are asked for while the one before is decided)
+  float4 next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  uint32_t next_label = 0u;
+  auto ask = [&](uint32_t pos) {
+    if (tid >= FX_NMS_CHUNK || pos + tid >= count) return;
+    const uint32_t idx = (uint32_t)s_keys[pos + tid], r = row_of(idx);
+    next_label = label_of(idx, r);
+    if constexpr (HEAD) next = head_box(head_row(h, task, head_number(h, r, next_label)));
+    else next = *(const float4*)(boxes + (size_t)r * 4u);
+  };
+  if (!placed) ask(0u);
   for (uint32_t pos = 0; pos < count && nk < d.max_num; pos += FX_NMS_CHUNK, p ^= 1u) {
     const uint32_t m = min(FX_NMS_CHUNK, count - pos);
     if (!placed) {
       if (tid < m) {
-        const uint32_t idx = (uint32_t)s_keys[pos + tid], r = row_of(idx), label = label_of(idx, r);
-        float4 b;
-        if constexpr (HEAD) b = head_box(head_row(h, task, head_number(h, r, label)));
-        else b = *(const float4*)(boxes + (size_t)r * 4u);
-        const float4 q = moved_by(b, (float)label * class_step);
-        s_cbox[tid] = b;
+        const float4 q = moved_by(next, (float)next_label * class_step);
+        s_cbox[tid] = next;
         s_obox[tid] = q;
         s_carea[tid] = area_of(q);
-        s_clabel[tid] = label;
+        s_clabel[tid] = next_label;
       }
       __syncthreads();
+      ask(pos + FX_NMS_CHUNK);
     }
     const float4* const moved = placed ? s_moved + pos : s_obox;
     const float* const areas = placed ? s_area + pos : s_carea;
-    {
-      // inside the chunk: pairs (i, j), i < j; lanes behind i take (i, lane), those before it (63 - i, 63 - lane), so that two
-      // rows of pairs fill one wave
-      uint32_t pi[2], pj[2];
-      float4 bi[2], bj[2];
-      float ai[2], aj[2];
-#pragma unroll
-      for (uint32_t e = 0; e < 2u; ++e) {
-        const uint32_t row = uni(wave) * 2u + e;
-        const bool back = lane < row;
-        pi[e] = back ? 63u - row : row;
-        pj[e] = back ? 63u - lane : lane;
-        const uint32_t i = min(pi[e], m - 1u), j = min(pj[e], m - 1u);   // (pairs that are none: not looked at below)
-        bi[e] = moved[i];
-        bj[e] = moved[j];
-        ai[e] = areas[i];
-        aj[e] = areas[j];
-      }
+    if (nk != 0u) {
+      // candidate `lane` against every 16th kept box, four of them at a time (a box that is there twice does not matter)
       const float4 q = moved[min(lane, m - 1u)];
       const float ca = areas[min(lane, m - 1u)];
-      const uint64_t n0 = near_lanes(bi[0], bj[0], d.iou_thr), n1 = near_lanes(bi[1], bj[1], d.iou_thr);
-#pragma unroll
-      for (uint32_t e = 0; e < 2u; ++e) {
-        const uint64_t near = e == 0u ? n0 : n1;
-        if (near == 0ull) continue;
-        const uint64_t over = overlap_lanes(near, bi[e], ai[e], bj[e], aj[e], d.iou_thr);
-        if (((over >> lane) & 1ull) != 0ull && pi[e] < pj[e] && pj[e] < m) atomicOr(&s_in[p][pj[e]][pi[e] >> 5], 1u << (pi[e] & 31u));
-      }
-      // candidate `lane` against every 16th kept box, four of them at a time (a box that is there twice does not matter)
       uint64_t dead = 0ull;
       for (uint32_t k = uni(wave); k < nk; k += FX_NMS_THREADS / 16u) {
         float4 o[4];
@@ -690,13 +673,33 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
           oa[e] = s_karea[min(k + e * (FX_NMS_THREADS / 64u), nk - 1u)];
         }
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) near[e] = near_lanes(o[e], q, d.iou_thr);
+        for (uint32_t e = 0; e < 4u; ++e) near[e] = near_lanes(o[e], q, d.iou_thr) & ~dead;
         if ((near[0] | near[1] | near[2] | near[3]) == 0ull) continue;
 #pragma unroll
         for (uint32_t e = 0; e < 4u; ++e)
           if (near[e] != 0ull) dead |= overlap_lanes(near[e], o[e], oa[e], q, ca, d.iou_thr);
       }
       if (dead != 0ull && lane < 2u) atomicOr(&s_dead[p][lane], (uint32_t)(dead >> (32u * lane)));
+      __syncthreads();
+    }
+    {
+      // inside the chunk: pairs (i, j), i < j, of candidates that no kept box overlaps; lanes behind i take (i, lane), those
+      // before it (63 - i, 63 - lane), so that two rows of pairs fill one wave
+      const uint64_t gone = ((uint64_t)uni(s_dead[p][1]) << 32) | (uint64_t)uni(s_dead[p][0]);
+#pragma unroll
+      for (uint32_t e = 0; e < 2u; ++e) {
+        const uint32_t row = uni(wave) * 2u + e, other = 63u - row;
+        if (((gone >> row) & (gone >> other) & 1ull) != 0ull) continue;
+        const bool back = lane < row;
+        const uint32_t pi = back ? other : row, pj = back ? 63u - lane : lane, i = min(pi, m - 1u), j = min(pj, m - 1u);   // (pairs that are none: not looked at below)
+        const float4 bi = moved[i], bj = moved[j];
+        const float ai = areas[i], aj = areas[j];
+        const uint64_t pairs = __ballot(pi < pj && pj < m && ((gone >> pi) & 1ull) == 0ull && ((gone >> pj) & 1ull) == 0ull);
+        const uint64_t near = near_lanes(bi, bj, d.iou_thr) & pairs;
+        if (near == 0ull) continue;
+        const uint64_t over = overlap_lanes(near, bi, ai, bj, aj, d.iou_thr);
+        if (((over >> lane) & 1ull) != 0ull) atomicOr(&s_in[p][pj][pi >> 5], 1u << (pi & 31u));
+      }
     }
     __syncthreads();
     if (wave == 1u) {   // for the chunk after this one; the last to read these has passed a barrier

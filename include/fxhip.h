@@ -596,16 +596,18 @@ int fx_nms_pairs(const fx_nms_desc* desc, void* stream);
  * Microseconds a call, launched back to back from one descriptor, fx_sort_nms : fx_nms_pairs; boxes apart from
  * each other, the first 300 or 1 024 kept / proposals of 60 objects, at most 300 (walked from 1 200 rows on) or 1 024 kept
  *     rows     1 task                      4 tasks                     8 tasks                     16 tasks                    32 tasks
- *     200      21:13 22:13 / 18:13 19:13   22:13 22:13 / 19:13 19:13   23:14 23:14 / 19:14 19:14   23:14 23:14 / 19:14 19:14   23:15 24:15 / 19:15 20:15
- *     500      28:14 48:15 / 30:15 30:15   29:14 48:15 / 30:15 30:15   29:15 48:16 / 30:16 30:16   29:17 49:18 / 30:18 30:18   29:22 49:23 / 30:23 31:23
- *     1 000    30:15 135:20 / 50:19 50:19  31:16 137:21 / 49:20 50:20  31:20 137:25 / 50:24 50:25  31:28 138:33 / 50:33 51:33  31:44 138:49 / 50:49 50:49
- *     2 000    36:17 142:17 / 91:32 91:20  36:26 143:27 / 92:41 92:30  37:40 144:41 / 92:54 92:46  37:65 144:70 / 92:80 92:76  37:114 144:127 / 93:128 93:136
- *     4 096    51:29 157:31 / 178:73 179:31  52:64 158:67 / 180:109 180:68  52:110 159:117 / 181:154 181:121  52:202 159:223 / 181:249 182:231  52:389 159:436 / 182:434 182:452
- * (128 tasks of 200 rows 22 : 25, of 500 29 : 50.)  Hence bounds on tasks * rows and on tasks * rows^2, the latter moved by what may
- * be kept.  They lie on the safe side, where the first of the four columns turns: 16 tasks of 2 000 proposals, and four to
- * eight of 4 096, would be faster as three launches and are not sent there.  (8 tasks of 2 000 rows apart, of which 300 are kept, lie
- * just beyond it: 37 : 40.)  Few rows: a caller that prepares every call (functs_amd.detection, 24 us of host work) pays for three
- * launches instead of one when it does not wait, 200 rows 24 : 30, and gains when it does, 39 : 31; so one to four images are sent there. */
+ *     150      13:12 14:12 / 14:12 14:12   14:13 14:12 / 15:13 15:13   14:13 14:13 / 15:13 15:13   14:13 14:13 / 15:13 15:13   14:14 14:14 / 15:14 15:14
+ *     200      17:13 17:13 / 17:13 17:13   17:13 17:13 / 18:13 18:13   17:13 17:13 / 18:13 17:13   17:14 17:14 / 18:14 18:14   17:14 17:14 / 18:15 18:15
+ *     500      20:14 32:15 / 26:15 26:15   21:14 32:15 / 26:15 26:15   21:14 32:16 / 27:15 27:15   21:16 32:17 / 27:17 26:17   21:21 32:23 / 27:22 27:22
+ *     1 000    21:14 80:19 / 40:19 42:19   22:16 81:21 / 42:20 42:20   22:19 81:24 / 41:24 43:24   22:27 81:32 / 43:32 43:32   22:43 81:48 / 43:48 43:48
+ *     2 000    23:17 82:18 / 73:32 73:22   24:25 83:26 / 73:40 74:31   24:39 82:40 / 76:53 76:46   24:63 82:69 / 78:78 76:77   24:113 83:126 / 77:127 76:139
+ *     4 096    44:28 104:30 / 166:73 155:32   44:62 104:66 / 168:108 167:69   44:108 104:117 / 168:154 176:125   44:200 104:222 / 177:247 177:236   44:386 105:435 / 177:432 180:464
+ * Hence bounds on tasks * rows and on tasks * rows^2, the latter moved by what may be kept: of the four columns the first, boxes
+ * apart of which few are kept, turns first, the others far behind it.  Proposals decide: 16 tasks of 1 000 rows and 8 of 2 000 are
+ * sent to three launches (43 : 32, 76 : 53), which boxes apart would not need (22 : 27, 24 : 39).  Calls of functs::batched_nms,
+ * fx_sort_nms : fx_nms_pairs: 128 boxes 19.1 : 20.5, 150 21.6 : 20.7, 200 23.9 : 21.1, 450 33.4 : 23.1.  Few rows of many images
+ * are left where one launch is: a caller that prepares every call (functs_amd.detection, 24 us of host work) pays for three
+ * launches when it does not wait, and gains by them when it does; so one to four images of fewer than 320 rows are sent there. */
 int fx_nms_pairs_pays(int n_tasks, uint32_t rows, uint32_t max_num, float score_thr);
 
 /* ---- device utilities ---- */
