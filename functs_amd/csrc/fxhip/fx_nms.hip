@@ -196,7 +196,7 @@ __device__ __forceinline__ void head_scan(const fx_nms_desc& d, const HeadMaps& 
 // What a candidate needs besides its score is gathered here, by every workgroup for its own, one candidate a thread: a
 // gather by the one that finishes the task is bound by the lines a CU gets (700 candidates of a head, seven lines each: 5.5 us),
 // a gather in the scan sits between the rounds of loads.  Scores take their row's factor, a head's rows that are not kept
-// leave, boxes (of few candidates) go to s_box, the largest coordinate to s_maxc.
+// leave, the largest coordinate goes to s_maxc, and the boxes to s_box where the candidates that are left are at most FX_NMS_FEW.
 template <class Maps>
 __device__ __forceinline__ void gather_own(const fx_nms_desc& d, const Maps& h, const uint32_t C, const uint32_t key_cap, const uint32_t task,
                                            const float* boxes, const float* factors, uint64_t* s_keys, float4* s_box, uint32_t* s_count,
@@ -240,8 +240,16 @@ __device__ __forceinline__ void gather_own(const fx_nms_desc& d, const Maps& h, 
   for (int o = 32; o >= 1; o >>= 1) my_max = max(my_max, (uint32_t)__shfl_xor((int)my_max, o, 64));
   if ((threadIdx.x & 63u) == 0u && my_max != 0u) atomicMax(s_maxc, my_max);
   __syncthreads();
-  if (HEAD) {
-    if (threadIdx.x == 0u) *s_count = *s_kept + over;
+  if constexpr (HEAD) {
+    const uint32_t kept = *s_kept;
+    // Where the scan found more than s_box holds, s_box's memory was full of keys until here.  What is left of them is decided
+    // behind this by its number alone, so if that is small its boxes are made now, from rows and labels.
+    if (n > FX_NMS_FEW && kept <= FX_NMS_FEW && key_cap >= FX_NMS_ROOMY)
+      for (uint32_t k = threadIdx.x; k < kept; k += FX_NMS_THREADS) {
+        const uint32_t idx = (uint32_t)s_keys[k], r = fx_fastdiv(idx, h.c_magic, h.c_shift);
+        s_box[k] = head_box(head_row(h, task, head_number(h, r, idx - r * C)));
+      }
+    if (threadIdx.x == 0u) *s_count = kept + over;
     __syncthreads();
   }
 }
@@ -391,7 +399,7 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
     // compiler is told the order explicitly: nothing moves across the signal fences.
     for (uint32_t k = tid; k < mine; k += FX_NMS_THREADS)
       if (gbase + k < key_cap) __hip_atomic_store(&g_keys[gbase + k], s_keys[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (roomy)   // (a workgroup with more candidates than that has no boxes: neither has the task need of any)
+    if (roomy)   // (a workgroup that keeps more candidates than that has no boxes: neither has the task need of any)
       for (uint32_t k = tid; k < 2u * mine && (k >> 1) + gbase < FX_NMS_FEW; k += FX_NMS_THREADS)
         if (mine <= FX_NMS_FEW) __hip_atomic_store(&g_box[2u * gbase + k], ((const uint64_t*)s_own)[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);

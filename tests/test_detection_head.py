@@ -202,3 +202,55 @@ def test_descriptors_that_do_not_fit_are_refused():
     for bad in (dict(levels=0), dict(levels=5), dict(cells=0, rows=0), dict(rows=11), dict(cells=1, rows=3, classes=3), dict(max_num=0), dict(max_num=1025),
                 dict(cap=0), dict(cap=16385), dict(maps=None), dict(mode=0), dict(classes=0), dict(cells=1 << 20, rows=3 << 20, classes=1 << 10), dict()):
         assert call(**bad) < 0, bad
+
+
+def _elements_of_workgroups(batch, grids, classes):
+    """Class scores that every workgroup of an image scans (fx_launch_head_nms: groups of 256, none across two runs)."""
+    groups = []
+    for g in grids:
+        run = classes * g * g
+        groups += ([256] * (run // 256) + ([run % 256] if run % 256 else [])) * 3
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    slices = min(max(cus // batch, 1), 128, -(-len(groups) // 16))
+    share = -(-len(groups) // slices)
+    return [sum(groups[k * share:(k + 1) * share]) for k in range(slices)]
+
+
+def _few_rows_kept(seed, batch, grids, classes, rows):
+    """Every class score passes the threshold, the objectness of `rows` rows an image does."""
+    g = torch.Generator().manual_seed(seed)
+    args = list(yolov3_head(seed, batch, grids, classes))
+    views = [m.view(batch, 3, 5 + classes, -1) for m in args[0]]
+    starts = [0]
+    for v in views:
+        v[:, :, 5:].clamp_(-2.0, 2.0)
+        v[:, :, 4] = -9.0
+        starts.append(starts[-1] + 3 * v.size(3))
+    for b in range(batch):
+        for row in torch.randperm(starts[-1], generator=g)[:rows].tolist():
+            level = max(k for k in range(len(views)) if row >= starts[k])
+            r = row - starts[level]
+            views[level][b, r // views[level].size(3), 4, r % views[level].size(3)] = 2.0
+    return args
+
+
+# Workgroups with more class scores above the threshold than the 2 048 whose boxes LDS holds, up to 16 384, of which few are
+# left; alone with their image and several to one.  Few, 700 and just up to 2 048 candidates (ordered by buckets), more (sorted).
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,grids,classes,rows,elements", [
+    (1, (3, 6, 12), 5, (1, 140, 409, 410), 2835), (130, (4, 8, 16), 8, (1, 88, 256, 257), 8064), (130, (4, 8, 16), 16, (1, 43, 128, 129), 16128),
+    (8, (19, 38, 76), 10, (1, 70, 204, 205), 7168), (1, (19, 38, 76), 80, (1, 9, 25, 26), 14336), (2, (19, 38, 76), 64, (1, 11, 32, 33), 11520)])
+def test_few_candidates_of_many_scores_above_the_threshold(batch, grids, classes, rows, elements):
+    fullest = max(_elements_of_workgroups(batch, grids, classes))
+    assert 2048 < fullest <= 16384 and fullest == elements
+    one = None
+    for kept in rows:
+        args = _few_rows_kept(kept, batch, grids, classes, kept)
+        print("few of many", batch, grids, classes, kept, flush=True)
+        if one is None:
+            one, chain, _ = _both(PROGRAMS["yolo_head_nms"], args)
+        gargs = [[t.cuda() for t in a] for a in args]
+        (got, launches), (ref, n_chain) = _launches(one, gargs), _launches(chain, gargs)
+        assert launches == 1 and n_chain > 1
+        _assert_same(got, ref)
+        assert min(d.size(0) for d, _ in got) > 0
