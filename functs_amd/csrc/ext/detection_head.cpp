@@ -16,10 +16,12 @@
 // The match is structural and complete, as that of the loop kernels (attention.cpp).  Both forms stay in the graph, behind
 //   if fx::detection_head_fits(operands): fx::detection_head(operands)  else: the chain,
 // (fx::detection_head_pairs and the chain with its functs::unbatch_detection_pairs where that is all that is made of it)
-// because a call may come with operands that only the chain serves (gradients, a capture, other devices).
+// because a call may come with operands that only the chain serves (gradients, a capture, other devices).  They stand
+// where the tail stood: a program that writes to the head's operands in between keeps the chain as it is.
 #include <ATen/ATen.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/jit/ir/alias_analysis.h>
 #include <torch/csrc/jit/ir/constants.h>
 #include <torch/csrc/jit/runtime/custom_operator.h>
 
@@ -244,7 +246,16 @@ bool isFunctor(Node* n, bool map) {
   return compact == map && padded == map && n->g(c10::attr::Subgraph)->inputs().size() == n->inputs().size() + 1;
 }
 
-bool fuseAt(Node* tail) {
+// whether a node from `from` to `to` (neither included) may write to what `from` reads
+bool writtenBetween(const std::shared_ptr<Graph>& graph, Node* from, Node* to) {
+  const AliasDb aliases(graph);
+  const ValueSet reads(from->inputs().begin(), from->inputs().end());
+  for (Node* n = from->next(); n != to; n = n->next())
+    if (aliases.writesToAlias(n, reads)) return true;
+  return false;
+}
+
+bool fuseAt(const std::shared_ptr<Graph>& graph, Node* tail) {
   static const Symbol batched = Symbol::fromQualString("functs::multiclass_nms_batched");
   if (tail->kind() != batched || tail->inputs().size() != 8) return false;
   Node* filter = tail->input(0)->node();
@@ -282,8 +293,10 @@ bool fuseAt(Node* tail) {
     if (!ps || ps->size() != 3 || !matchFilter(*fg, which[0], which[1], which[2], *ps, padded->toBool(), &f_preds, &f_boxes, &keep_thr)) continue;
     if (argumentOf(filter, *fg, f_preds) != dense->output(p) || argumentOf(filter, *fg, f_boxes) != dense->output(1 - p)) continue;
     if (!matchDense(*dg, dg->outputs()[p], dg->outputs()[1 - p], &h) || filter->i(sym::parallel_degree()) != h.images || h.images < 1) continue;
+    // (the filter reads what the dense functor made, which nobody else has, and constants)
+    if (writtenBetween(graph, dense, tail)) return false;
 
-    Graph* g = tail->owningGraph();
+    Graph* g = graph.get();
     WithInsertPoint at(dense);
     auto tensors = [&](const std::vector<Value*>& vs) {
       std::vector<Value*> args;
@@ -335,15 +348,15 @@ bool fuseAt(Node* tail) {
   return false;
 }
 
-bool fuseIn(Block* b) {
+bool fuseIn(const std::shared_ptr<Graph>& graph, Block* b) {
   // (collected first: what is joined moves nodes behind the tail into another block)
   bool changed = false;
   std::vector<Node*> tails;
   for (Node* n : b->nodes()) {
-    for (Block* inner : n->blocks()) changed = fuseIn(inner) || changed;
+    for (Block* inner : n->blocks()) changed = fuseIn(graph, inner) || changed;
     if (n->kind() == Symbol::fromQualString("functs::multiclass_nms_batched")) tails.push_back(n);
   }
-  for (Node* n : tails) changed = fuseAt(n) || changed;
+  for (Node* n : tails) changed = fuseAt(graph, n) || changed;
   return changed;
 }
 
@@ -450,7 +463,7 @@ RegisterOperators registerHead({
 }  // namespace
 
 bool FuseDetectionHead(std::shared_ptr<Graph> graph) {
-  const bool changed = fuseIn(graph->block());
+  const bool changed = fuseIn(graph, graph->block());
   if (changed) Validate(graph);
   return changed;
 }

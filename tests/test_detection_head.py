@@ -8,10 +8,10 @@ import torch
 from torch import Tensor
 
 import functs_amd.jit as fj
-from functs_amd import _lib, aot
+from functs_amd import _C, _lib, aot
 from functs_amd.benchmark import PROGRAMS
 from functs_amd.benchmark.inputs import yolov3_head
-from functs_amd.benchmark.programs import _yolov3_head_scores
+from functs_amd.benchmark.programs import _decode_stack, _yolov3_head_scores
 
 
 def no_threshold(pred_maps: List[Tensor], base_anchors: List[Tensor]):
@@ -48,6 +48,68 @@ def scaled(pred_maps: List[Tensor], base_anchors: List[Tensor]):
     return out
 
 
+def _given(pred_maps: List[Tensor], base_anchors: List[Tensor], shifts: List[Tensor], strides: Tensor):
+    """The head with its tables as arguments (types of what a program makes on a GPU are not known without one)."""
+    num_imgs = pred_maps[0].size(0)
+    num_attrib = pred_maps[0].size(1) // base_anchors[0].size(0)
+    mlvl_anchors: List[Tensor] = []
+    flatten_preds: List[Tensor] = []
+    for lvl in range(3):
+        mlvl_anchors.append((base_anchors[lvl].unsqueeze(0) + shifts[lvl]).reshape(-1, 4))
+        pred = pred_maps[lvl].permute(0, 2, 3, 1).reshape(num_imgs, -1, num_attrib).clone()
+        pred[..., :2].sigmoid_()
+        flatten_preds.append(pred.clone())
+    preds = torch.cat(flatten_preds, dim=1)
+    bboxes = _decode_stack(torch.cat(mlvl_anchors), preds[..., :4], strides)
+    padding = bboxes.new_zeros(num_imgs, bboxes.size(1), 1)
+    return bboxes, torch.cat([preds[..., 5:].sigmoid(), padding], dim=-1), preds[..., 4].sigmoid()
+
+
+def _given_tail(bboxes: Tensor, cls_scores: Tensor, objectness: Tensor):
+    det_results: List[Tuple[Tensor, Tensor]] = []
+    for i in range(bboxes.size(0)):
+        o = objectness[i]
+        keep = o >= 0.005
+        det_results.append(torch.ops.functs.multiclass_nms(bboxes[i][keep, :], cls_scores[i][keep, :], o[keep], 0.05, 0.45, 100, True))
+    return det_results
+
+
+def only_read(pred_maps: List[Tensor], base_anchors: List[Tensor], shifts: List[Tensor], strides: Tensor):
+    bboxes, cls_scores, objectness = _given(pred_maps, base_anchors, shifts, strides)
+    return _given_tail(bboxes, cls_scores, objectness)
+
+
+def written_before(pred_maps: List[Tensor], base_anchors: List[Tensor], shifts: List[Tensor], strides: Tensor):
+    pred_maps[0].mul_(0.5)
+    bboxes, cls_scores, objectness = _given(pred_maps, base_anchors, shifts, strides)
+    return _given_tail(bboxes, cls_scores, objectness)
+
+
+def written_behind(pred_maps: List[Tensor], base_anchors: List[Tensor], shifts: List[Tensor], strides: Tensor):
+    bboxes, cls_scores, objectness = _given(pred_maps, base_anchors, shifts, strides)
+    det_results = _given_tail(bboxes, cls_scores, objectness)
+    pred_maps[0].zero_()
+    return det_results
+
+
+def map_written(pred_maps: List[Tensor], base_anchors: List[Tensor], shifts: List[Tensor], strides: Tensor):
+    bboxes, cls_scores, objectness = _given(pred_maps, base_anchors, shifts, strides)
+    pred_maps[0].zero_()
+    return _given_tail(bboxes, cls_scores, objectness)
+
+
+def anchors_written(pred_maps: List[Tensor], base_anchors: List[Tensor], shifts: List[Tensor], strides: Tensor):
+    bboxes, cls_scores, objectness = _given(pred_maps, base_anchors, shifts, strides)
+    base_anchors[1].zero_()
+    return _given_tail(bboxes, cls_scores, objectness)
+
+
+def strides_written(pred_maps: List[Tensor], base_anchors: List[Tensor], shifts: List[Tensor], strides: Tensor):
+    bboxes, cls_scores, objectness = _given(pred_maps, base_anchors, shifts, strides)
+    strides.zero_()
+    return _given_tail(bboxes, cls_scores, objectness)
+
+
 def _kinds(block):
     for n in block.nodes():
         yield n.kind()
@@ -80,6 +142,50 @@ def _assert_same(got, ref):
 def test_a_function_built_from_host_examples_keeps_the_chain():
     fn = fj.build(fj.script(PROGRAMS["yolo_head_nms"]), list(yolov3_head(0, 2, (2, 4, 8), 5)))
     assert not any("detection_head" in k for k in _kinds(fn.graph.block()))
+
+
+WRITES = (map_written, anchors_written, strides_written)
+
+
+@pytest.mark.parametrize("program", (only_read, written_before, written_behind) + WRITES)
+def test_writes_between_the_head_and_its_tail_keep_the_chain(program):
+    """The launch and the chain beside it stand at the tail: what the program writes before that, they would read."""
+    def hint(*sizes):
+        return torch.TensorType.get().with_dtype(torch.float32).with_sizes(list(sizes)).with_device(torch.device("cuda", 0))
+    grids = (2, 4, 8)
+    g = fj.script(program).graph.copy()
+    _C._jit_pass_fait_pipeline(g, [torch.TupleType([hint(2, 30, f, f) for f in grids]), torch.TupleType([hint(3, 4) for f in grids]),
+                                   torch.TupleType([hint(f * f, 1, 4) for f in grids]), hint(252, 1)])
+    before = list(g.nodes())
+    order = [n.kind() for n in before]
+    assert _C._jit_pass_fuse_detection_head(g) == (program not in WRITES)
+    if program in WRITES:
+        assert [n.kind() for n in g.nodes()] == order
+        write = next(k for k, kind in enumerate(order) if kind == "aten::copy_")
+        assert order.index("tssa::ParallelFunctor") < write < order.index("functs::multiclass_nms_batched")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("program", (written_before, written_behind) + WRITES)
+def test_writes_are_seen_where_the_program_makes_them(program):
+    batch, grids, classes = 2, (4, 8, 16), 5
+    maps, bases = yolov3_head(12, batch, grids, classes)
+    shifts = [torch.rand(f * f, 1, 4) * 100.0 for f in grids]
+    strides = torch.full((3 * sum(f * f for f in grids), 1), 8.0)
+
+    def on_gpu():
+        return [[t.cuda() for t in a] for a in (maps, bases, shifts)] + [strides.cuda()]
+    print(program.__name__, flush=True)
+    plain = fj.build(fj.script(only_read), on_gpu())
+    args = on_gpu()
+    if program is written_before:
+        args[0][0].mul_(0.5)
+    ref = plain(*args)
+    fn, args = fj.build(fj.script(program), on_gpu()), on_gpu()
+    _assert_same(fn(*args), ref)
+    assert sum(d.size(0) for d, _ in ref) > 0
+    same = [torch.equal(t, r) for a, b in zip(args, on_gpu()) for t, r in (zip(a, b) if isinstance(a, list) else [(a, b)])]
+    assert same.count(False) == 1
 
 
 # Runs of class scores that end inside a vector, inside a group of 256 and with one; one cell; up to 16 and one to three images
