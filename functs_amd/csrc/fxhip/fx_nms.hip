@@ -90,7 +90,7 @@ struct HeadMaps {
   HeadLevel lv[FX_HEAD_LEVELS];
   uint32_t n_levels, groups, width;  // groups of an image; attributes of a row (5 + classes)
   uint32_t c_magic, c_shift;         // division by the number of classes
-  float keep_thr, logit_lo;          // no element up to logit_lo passes the score threshold
+  float keep_thr, logit_lo;          // no element below logit_lo passes the score threshold
   const float* strides;
 };
 struct NoMaps {};
@@ -171,7 +171,7 @@ __device__ __forceinline__ void head_scan(const fx_nms_desc& d, const HeadMaps& 
       for (uint32_t u = 0; u < U; ++u)
 #pragma unroll
         for (uint32_t e = 0; e < 4u; ++e)
-          if (__uint_as_float(v[u][e]) > h.logit_lo && e >= skip[u]) mine |= 1u << (u * 4u + e);
+          if (__uint_as_float(v[u][e]) >= h.logit_lo && e >= skip[u]) mine |= 1u << (u * 4u + e);
       if (mine == 0u) continue;
 #pragma unroll
       for (uint32_t u = 0; u < U; ++u)
@@ -826,12 +826,13 @@ int fx_launch_sort_nms(const fx_nms_desc& d, uint32_t key_cap, void* workspace, 
   return launch_sort_nms(d, NoMaps{}, fx_nms_slices(d), key_cap, workspace, err_host, stream);
 }
 
-// below: no logit up to it has a score above thr (the device's sigmoid is off by less than 1e-6, so nothing up to the
-// logit of thr less 1e-5 of it passes; a threshold of 1 or more, or NaN, lets nothing pass)
+// no logit below it has a score above thr (the device's sigmoid is off by less than 1e-6, so nothing up to the logit of
+// thr less 1e-5 of it passes; a threshold of 1 or more, or NaN, lets nothing pass, and one below 0 every number, with -inf,
+// whose score is 0: the bound itself is one of the logits that are looked at)
 static float logit_bound(float thr) {
   const double t = (double)thr * (1.0 - 1e-5);
   if (!(thr < 1.0f)) return std::numeric_limits<float>::infinity();
-  if (!(t > 1e-30)) return -std::numeric_limits<float>::infinity();
+  if (!(t > 1e-30)) return thr < 0.0f ? -std::numeric_limits<float>::infinity() : std::numeric_limits<float>::lowest();
   const double x = std::log(t / (1.0 - t));
   return std::nextafterf((float)x, -std::numeric_limits<float>::infinity());
 }

@@ -360,3 +360,28 @@ def test_few_candidates_of_many_scores_above_the_threshold(batch, grids, classes
         assert launches == 1 and n_chain > 1
         _assert_same(got, ref)
         assert min(d.size(0) for d, _ in got) > 0
+
+
+def below_zero(pred_maps: List[Tensor], base_anchors: List[Tensor]):
+    """Every number is a score above the threshold."""
+    bboxes, cls_scores, objectness = _yolov3_head_scores(pred_maps, base_anchors)
+    det_results: List[Tuple[Tensor, Tensor]] = []
+    for i in range(bboxes.size(0)):
+        o = objectness[i]
+        keep = o >= 0.4
+        det_results.append(torch.ops.functs.multiclass_nms(bboxes[i][keep, :], cls_scores[i][keep, :], o[keep], -0.5, 0.45, 1000, True))
+    return det_results
+
+
+@pytest.mark.gpu
+def test_scores_of_zero_above_a_threshold_below_zero():
+    """(a class that is masked out: its logit is -inf, its score 0)"""
+    args = list(yolov3_head(8, 2, (2, 4, 8), 6))
+    for m in args[0]:
+        m.view(2, 3, 11, -1)[:, :, 6::2] = -float("inf")
+    print("below zero", flush=True)
+    one, chain, gargs = _both(below_zero, args)
+    (got, n_one), (ref, n_chain) = _launches(one, gargs), _launches(chain, gargs)
+    assert n_one == 1 and n_chain > 1
+    assert all(bool((d[:, 4] == 0).any()) for d, _ in ref)
+    _assert_same(got, ref)
