@@ -388,7 +388,7 @@ bool fits(const Operands& o) {
            !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
                                                      c10::DispatchKey::Python, c10::DispatchKey::Functionalize}));
   };
-  int64_t rows = 0;
+  int64_t rows = 0, groups = 0;
   for (size_t l = 0; l < n; ++l) {
     const at::Tensor &m = o.maps[l], &b = o.bases[l], &s = o.shifts[l];
     if (!plain(m) || !plain(b) || !plain(s) || m.dim() != 4 || b.dim() != 2) return false;
@@ -397,7 +397,9 @@ bool fits(const Operands& o) {
         cells * o.classes < 4 || m.numel() / o.images >= ((int64_t)1 << 31) || o.images * anchors >= ((int64_t)1 << 31))
       return false;
     rows += anchors * cells;
+    groups += anchors * ((cells * o.classes + 255) / 256);
   }
+  if (groups > (int64_t)FX_HEAD_MAX_GROUPS) return false;
   if (!plain(o.strides) || o.strides.numel() != rows || rows * width >= ((int64_t)1 << 31)) return false;
   if (at::autocast::is_autocast_enabled(at::kCUDA)) return false;
   // (a graph is left the chain, whose launches of a capture are known)

@@ -1690,7 +1690,7 @@ int fx_head_nms(const fx_head_desc* head, const fx_nms_desc* desc, void* stream_
     return fail(FX_E_LIMIT, "fx_head_nms: 1.." + std::to_string(FX_HEAD_LEVELS) + " levels");
   if (!head->strides || !d.dets || !d.out_labels || !d.n_out) return fail(FX_E_INVALID, "fx_head_nms: null argument");
   if (d.max_num < 1 || d.max_num > FX_NMS_MAX_OUT) return fail(FX_E_LIMIT, "fx_head_nms: max_num must be 1.." + std::to_string(FX_NMS_MAX_OUT));
-  uint64_t rows = 0;
+  uint64_t rows = 0, groups = 0;   // (groups: of the scan, which numbers class scores by them in 32 bits)
   for (int l = 0; l < head->n_levels; ++l) {
     if (!head->maps[l] || !head->bases[l] || !head->shifts[l]) return fail(FX_E_INVALID, "fx_head_nms: null argument");
     const uint64_t cells = head->cells[l], anchors = head->anchors[l];
@@ -1699,7 +1699,9 @@ int fx_head_nms(const fx_head_desc* head, const fx_nms_desc* desc, void* stream_
         (uint64_t)d.n_tasks * anchors >= (1ull << 31))
       return fail(FX_E_LIMIT, "fx_head_nms: a level beyond 31 bits");
     rows += cells * anchors;
+    groups += anchors * ((cells * d.n_classes + 255u) / 256u);
   }
+  if (groups > FX_HEAD_MAX_GROUPS) return fail(FX_E_LIMIT, "fx_head_nms: runs of class scores, each to the next 256, beyond 32 bits");
   if (rows != d.rows || rows * (5ull + d.n_classes) >= (1ull << 31)) return fail(FX_E_LIMIT, "fx_head_nms: rows must be the levels' and rows * attributes fit 31 bits");
   if (d.key_capacity < 1 || d.key_capacity > FX_NMS_MAX_CANDIDATES)
     return fail(FX_E_LIMIT, "fx_head_nms: key_capacity must be 1.." + std::to_string(FX_NMS_MAX_CANDIDATES));

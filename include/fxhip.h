@@ -569,6 +569,7 @@ int fx_sort_nms(const fx_nms_desc* desc, void* stream);
  * same program in separate launches, bit for bit; out_index counts rows before the filter.
  * 4 or more class scores to a run of a level (n_classes * cells); workspace as for fx_sort_nms. */
 #define FX_HEAD_LEVELS 4
+#define FX_HEAD_MAX_GROUPS (1u << 24)  /* over all levels, anchors * ceil(n_classes * cells / 256) */
 typedef struct fx_head_desc {
   int32_t n_levels;
   float keep_thr;

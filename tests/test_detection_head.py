@@ -385,3 +385,37 @@ def test_scores_of_zero_above_a_threshold_below_zero():
     assert n_one == 1 and n_chain > 1
     assert all(bool((d[:, 4] == 0).any()) for d, _ in ref)
     _assert_same(got, ref)
+
+
+def _refusal(fill):
+    """The error of a descriptor of one level, and its message (nothing is launched: there is no workspace)."""
+    at = ctypes.cast((ctypes.c_float * 4)(), ctypes.c_void_p).value
+    h, d = _lib.FxHeadDesc(), _lib.FxNmsDesc()
+    h.n_levels, h.keep_thr, h.strides = 1, 0.1, at
+    h.maps[0], h.bases[0], h.shifts[0] = at, at, at
+    d.mode, d.n_tasks, d.max_num, d.key_capacity = 1, 1, 10, 128
+    d.dets = d.out_labels = d.n_out = at
+    fill(h, d)
+    return _lib.lib.fx_head_nms(ctypes.byref(h), ctypes.byref(d), None), _lib.lib.fx_last_error().decode()
+
+
+# Class scores are numbered with every run rounded up to 256: runs of four are 64 times as many numbers as scores
+@pytest.mark.parametrize("anchors,cells,classes,error", [(1 << 24, 1, 4, "workspace"), ((1 << 24) + 1, 1, 4, "beyond 32 bits"),
+                                                         (1 << 24, 2, 50, "workspace"), ((1 << 24) + 1, 2, 50, "beyond 32 bits")])
+def test_numbers_beyond_32_bits_are_refused(anchors, cells, classes, error):
+    def fill(h, d):
+        h.cells[0], h.anchors[0] = cells, anchors
+        d.rows, d.n_classes = anchors * cells, classes
+    rc, message = _refusal(fill)
+    assert rc < 0 and error in message, message
+
+
+@pytest.mark.gpu
+def test_numbers_beyond_32_bits_run_the_chain():
+    """(asked only, nothing is launched)"""
+    fits = torch._C._jit_get_operation("fx::detection_head_fits")
+    fits = fits[0] if isinstance(fits, tuple) else fits
+    for anchors in (1 << 24, (1 << 24) + 1):
+        maps, bases, shift, strides = (torch.empty(s, device="cuda") for s in ((1, anchors * 9, 1, 1), (anchors, 4), (1, 1, 4), (anchors, 1)))
+        print("fits", anchors, flush=True)
+        assert fits([maps], [bases], [shift], strides, 1, 4, 0.5, 0.05, 0.45, 100) == (anchors <= 1 << 24)
