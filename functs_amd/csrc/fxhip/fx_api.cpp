@@ -1684,7 +1684,8 @@ int fx_sort_nms(const fx_nms_desc* desc, void* stream_) {
 
 int fx_head_nms(const fx_head_desc* head, const fx_nms_desc* desc, void* stream_) {
   if (!head || !desc) return fail(FX_E_INVALID, "fx_head_nms: null descriptor");
-  const fx_nms_desc& d = *desc;
+  fx_nms_desc d = *desc;
+  d.scores_row_stride = 0;   // (of the scores, which are not read: a row's number and label are taken from n_classes)
   if (d.mode != 1 || d.n_tasks < 0 || d.n_classes < 1) return fail(FX_E_INVALID, "fx_head_nms: mode 1, classes and a number of tasks");
   if (head->n_levels < 1 || head->n_levels > FX_HEAD_LEVELS)
     return fail(FX_E_LIMIT, "fx_head_nms: 1.." + std::to_string(FX_HEAD_LEVELS) + " levels");

@@ -565,7 +565,7 @@ int fx_sort_nms(const fx_nms_desc* desc, void* stream);
  * logarithms of the sizes, the objectness and the class logits; row number first_row + cell * anchors + anchor.  A row is
  * kept when sigmoid(objectness) >= keep_thr; its box is the decode of anchor bases[anchor] + shifts[cell] (corners) and
  * strides[row], its scores the sigmoids of its class logits.  Candidates are then as in mode 1 of fx_nms_desc, of
- * which boxes, scores, factors, labels and counts are not read and rows must be the levels' rows.  Results are those of the
+ * which boxes, scores, scores_row_stride, factors, labels and counts are not read and rows must be the levels' rows.  Results are those of the
  * same program in separate launches, bit for bit; out_index counts rows before the filter.
  * 4 or more class scores to a run of a level (n_classes * cells); workspace as for fx_sort_nms. */
 #define FX_HEAD_LEVELS 4

@@ -419,3 +419,36 @@ def test_numbers_beyond_32_bits_run_the_chain():
         maps, bases, shift, strides = (torch.empty(s, device="cuda") for s in ((1, anchors * 9, 1, 1), (anchors, 4), (1, 1, 4), (anchors, 1)))
         print("fits", anchors, flush=True)
         assert fits([maps], [bases], [shift], strides, 1, 4, 0.5, 0.05, 0.45, 100) == (anchors <= 1 << 24)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shift", [4.0, 0.0])   # ordered by buckets, and sorted, where boxes are looked up by their rows
+def test_a_row_stride_of_the_scores_is_not_read(shift):
+    batch, grids, classes, max_num, cap = 2, (4, 8, 16), 5, 100, 16384
+    maps, bases = yolov3_head(21, batch, grids, classes)
+    for m in maps:
+        m.view(batch, 3, 5 + classes, -1)[:, :, 5:] -= shift
+    rows = 3 * sum(f * f for f in grids)
+    maps, bases = [m.cuda() for m in maps], [b.cuda() for b in bases]
+    shifts = [(torch.rand(f * f, 4, generator=torch.Generator().manual_seed(f)) * 100.0).cuda() for f in grids]
+    strides = torch.full((rows,), 8.0, device="cuda")
+    size = _lib.lib.fx_sort_nms_workspace_bytes(batch, cap)
+    results = []
+    for stride in (0, classes + 1):
+        dets, labels = torch.full((batch, max_num, 5), -1.0, device="cuda"), torch.full((batch, max_num), -1, device="cuda")
+        index, n, ws = torch.full_like(labels, -1), torch.full((batch,), -1, dtype=torch.int32, device="cuda"), torch.zeros(size, dtype=torch.uint8, device="cuda")
+        h, d = _lib.FxHeadDesc(), _lib.FxNmsDesc()
+        h.n_levels, h.keep_thr, h.strides = 3, 0.005, strides.data_ptr()
+        for k, f in enumerate(grids):
+            h.maps[k], h.bases[k], h.shifts[k], h.cells[k], h.anchors[k] = maps[k].data_ptr(), bases[k].data_ptr(), shifts[k].data_ptr(), f * f, 3
+        d.mode, d.n_tasks, d.rows, d.n_classes, d.scores_row_stride = 1, batch, rows, classes, stride
+        d.score_thr, d.iou_thr, d.max_num, d.key_capacity = 0.05, 0.45, max_num, cap
+        d.dets, d.out_labels, d.out_index, d.n_out = dets.data_ptr(), labels.data_ptr(), index.data_ptr(), n.data_ptr()
+        d.workspace, d.workspace_bytes = ws.data_ptr(), size
+        print("stride", shift, stride, flush=True)
+        assert _lib.lib.fx_head_nms(ctypes.byref(h), ctypes.byref(d), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        torch.cuda.synchronize()
+        results.append([dets, labels, index, n])
+    assert int(results[0][3].min()) > 0 and (shift > 0.0) == (sum(int((m.view(batch, 3, 5 + classes, -1)[:, :, 5:] > -2.944).sum()) for m in maps) < 2048 * batch)
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
