@@ -264,7 +264,6 @@ struct FxHeader {
 #define FX_LEAN_S 16     // scalars of a region that the lean kernel's argument block holds
 #define FX_LEAN_LEAD 1u
 #define FX_LEAN_HALF 2u
-#define FX_LEAN_STREAM 8u  // a pure output that is large: its stores leave for memory at once
 #define FX_LEAN_COLS 4u  // the outputs are the columns of rows of four elements (fx_dense_cols): out[0] is a column,
                          // its lead_* the place of a row's first element, gp_* division by inner, n_groups the rows
 // One output of the region: the fields of FxOut that place a work item, the leading load's

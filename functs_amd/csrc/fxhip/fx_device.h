@@ -389,7 +389,6 @@ __device__ __forceinline__ uint32_t fx_unflatten(uint32_t rem, uint32_t vd, cons
 
 // Results of one item.  contig (wave-uniform): e[j] == e[0] + j, so a lane whose
 // FX_V elements are all live writes them with one 128-bit store.
-template <bool STREAM = false>
 __device__ __forceinline__ void fx_store_vec(uint64_t base_, uint32_t obase, const uint32_t (&e)[FX_V], uint32_t M,
                                              bool contig, uint32_t dt, uint32_t vt, const uint32_t (&A)[FX_V]) {
   const bool raw32 = (dt == FX_F32 && vt == FX_VT_F) || (dt == FX_I32 && vt == FX_VT_I);
@@ -402,9 +401,7 @@ __device__ __forceinline__ void fx_store_vec(uint64_t base_, uint32_t obase, con
       asm("" : "+v"(t0), "+v"(t1), "+v"(t2), "+v"(t3));
       fx_u32x4 v;
       v.x = t0; v.y = t1; v.z = t2; v.w = t3;
-      FX_AS1 fx_u32x4_a4* to = (FX_AS1 fx_u32x4_a4*)(base + ((obase + e[0]) << 2));
-      if constexpr (STREAM) __builtin_nontemporal_store((fx_u32x4_a4)v, to);
-      else *to = v;
+      *(FX_AS1 fx_u32x4_a4*)(base + ((obase + e[0]) << 2)) = v;
     } else {
 #pragma unroll
       for (int j = 0; j < FX_V; ++j)
@@ -424,9 +421,7 @@ __device__ __forceinline__ void fx_store_vec(uint64_t base_, uint32_t obase, con
         v[j + 1] = (uint16_t)(w >> 16);
       }
     }
-    FX_AS1 fx_u16x4_a2* to = (FX_AS1 fx_u16x4_a2*)((FX_AS1 uint8_t*)base_ + ((obase + e[0]) << 1));
-    if constexpr (STREAM) __builtin_nontemporal_store(v, to);
-    else *to = v;
+    *(FX_AS1 fx_u16x4_a2*)((FX_AS1 uint8_t*)base_ + ((obase + e[0]) << 1)) = v;
   } else {
 #pragma unroll
     for (int j = 0; j < FX_V; ++j)

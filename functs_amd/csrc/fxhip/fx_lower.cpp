@@ -2344,9 +2344,12 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
           pure = fx_op_is_pure_unary(in.op) || (fx_op_is_pure_binary(in.op) && (in.flags & FX_F_IMM));
         }
         od.pure = pure ? 1u : 0u;
-        // An elementwise output whose operand lies as the output does is one long row: no group ends inside a row of an odd
-        // length, and every access but the last is whole and aligned (8 191 x 4 095 bfloat16 + 1 25.0 -> 22.5 us,
-        // 3 001 x 1 111 floats 6.2 -> 5.8).
+        // An elementwise output whose operand lies as the output does (from any offset, at any step) is one long row: no group
+        // ends inside a row of an odd length, and every store but the last is whole and aligned as the output is (inputs not in
+        // the caches, + 1: 3 001 x 1 111 floats 7.4 -> 7.1 us, 8 191 x 4 095 floats 54.0 -> 49.6, bfloat16 26.1 -> 24.2).
+        // Results stay in the caches.  Stored past them (nontemporal) a call on inputs that are there was faster (3 001 x 1 111
+        // floats 6.3 -> 6.0, 8 192 x 4 096 bfloat16 26.3 -> 22.7), one on inputs that are not was slower (67 MB 24.3 -> 25.4), and so was
+        // whatever read the result next: the same loop behind it 46.7 -> 50.7 us the two (8 191 x 2 047 floats), row sums 37 -> 42.
         if (pure && P->mode == FX_MODE_DENSE && dims.size() > 1 && od.numel > 0 && od.numel < 0x7ffffff0u) {
           const FxAffine& at = L.affs[(size_t)L.code[p.begin].b];
           const int64_t step = fx_aff_coef(&at, (int)dims.size() - 1);
@@ -2636,9 +2639,7 @@ static std::unique_ptr<Plan> build_plan(Region& R, const fx_arg* args, int n_arg
         const FxOut& od = cb.outs[o];
         FxLeanOut& lo = f.out[o];
         lo.ptr_slot = od.ptr_slot;
-        // (from 4 MB on: what fits a die's cache may stay there for whoever reads it next)
-        const bool large = od.pure && (uint64_t)od.numel * (half_out(od) ? 2u : 4u) >= (4u << 20);
-        lo.lead = (od.lead ? FX_LEAN_LEAD : 0u) | (half_out(od) ? FX_LEAN_HALF : 0u) | (large ? FX_LEAN_STREAM : 0u);
+        lo.lead = (od.lead ? FX_LEAN_LEAD : 0u) | (half_out(od) ? FX_LEAN_HALF : 0u);
         lo.block_begin = od.block_begin;
         lo.task_stride = od.task_stride;
         lo.unit_items = od.unit_items;

@@ -533,10 +533,6 @@ __device__ __forceinline__ void fx_lean_out(const FX_AS4 uint32_t* od, const uin
   if (!have) return;
   cx.wseg = rowseg ? rowseg : 64u;
   if constexpr (en.pure != 0) {
-    // Results of a large output go past the caches as they are made (FX_LEAN_STREAM): kept there they are written to memory
-    // when the kernel ends, with nothing left to overlap.  8 191 x 2 048 floats + 1 26.1 -> 20.8 us a call, 8 192 x 4 096
-    // bfloat16 26.2 -> 22.5, 3 001 x 1 112 floats 6.3 -> 5.8, all on cold lines.
-    const bool stream = (lead_word & FX_LEAN_STREAM) != 0;
 #pragma unroll
     for (uint32_t k = 0; k < FX_K; ++k) {
       if (k < kmax && item0 + k < n_items) {
@@ -544,8 +540,7 @@ __device__ __forceinline__ void fx_lean_out(const FX_AS4 uint32_t* od, const uin
         FxCoord<R> q;
         make_item(k, e, M, q);
         fx_spec_pure<P, en.begin, en.end, FX_V>(A[k]);
-        if (stream) fx_store_vec<true>(op, obase, e, M, true, odt, FX_VT_F, A[k]);
-        else fx_store_vec(op, obase, e, M, true, odt, FX_VT_F, A[k]);
+        fx_store_vec(op, obase, e, M, true, odt, FX_VT_F, A[k]);
       }
     }
   } else {

@@ -1,5 +1,5 @@
-"""Elementwise outputs whose operand lies as the output does are one long row (fx_lower.cpp); large ones are stored past the
-caches.  Every layout gives what eager mode gives, whether or not it is taken as one row."""
+"""Elementwise outputs whose operand lies as the output does are one long row (fx_lower.cpp).  Every layout gives what eager
+mode gives, whether or not it is taken as one row."""
 import pytest
 import torch
 
@@ -46,7 +46,7 @@ def test_layouts(backend, layout, dtype):
     assert torch.equal(got, x * 2.0 + 1.0 if dtype is torch.float32 else x + 1)
 
 
-# outputs on either side of the size from which stores go past the caches, of odd lengths and with operands that are not one row
+# outputs of some megabytes, of odd lengths and with operands that are not one row
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,rows,cols", [(torch.float32, 1023, 1025), (torch.float32, 1025, 1023), (torch.float32, 4099, 513),
                                              (torch.bfloat16, 2049, 1023), (torch.bfloat16, 2047, 1025), (torch.float16, 3001, 1111)])
