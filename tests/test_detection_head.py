@@ -237,8 +237,9 @@ def test_detections_that_are_used_otherwise():
 
 @pytest.mark.gpu
 def test_rows_that_are_not_kept_do_not_count_as_candidates():
-    """More class scores above the threshold than there is room for, of rows that the objectness drops: nothing is refused,
-    the share of a workgroup is read again.  The same with rows that are kept is refused, and the next call works."""
+    """More class scores of an image above the threshold than there is room for, of rows that the objectness drops: nothing is
+    refused.  The same with rows that are kept is refused, and the next call works.  (A workgroup's share is not read again here: it is
+    14 336 scores; test_shares_that_are_read_again.)"""
     args = list(yolov3_head(4, 1, (19, 38, 76), 80))
     for m in args[0]:
         v = m.view(1, 3, 85, -1)
@@ -452,3 +453,22 @@ def test_a_row_stride_of_the_scores_is_not_read(shift):
     assert int(results[0][3].min()) > 0 and (shift > 0.0) == (sum(int((m.view(batch, 3, 5 + classes, -1)[:, :, 5:] > -2.944).sum()) for m in maps) < 2048 * batch)
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+# More class scores above the threshold in a workgroup than its list has room for (16 384): its share is read again, with the
+# objectness.  Several workgroups to an image, and one; ordered by buckets, and sorted.
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,grids,classes,rows,elements", [(4, (19, 38, 76), 80, (1, 25, 26, 200), 28672), (130, (4, 8, 16), 20, (1, 102, 103, 800), 20160)])
+def test_shares_that_are_read_again(batch, grids, classes, rows, elements):
+    assert max(_elements_of_workgroups(batch, grids, classes)) == elements > 16384
+    one = None
+    for kept in rows:
+        args = _few_rows_kept(kept, batch, grids, classes, kept)
+        print("read again", batch, grids, classes, kept, flush=True)
+        if one is None:
+            one, chain, _ = _both(PROGRAMS["yolo_head_nms"], args)
+        gargs = [[t.cuda() for t in a] for a in args]
+        (got, launches), (ref, n_chain) = _launches(one, gargs), _launches(chain, gargs)
+        assert launches == 1 and n_chain > 1
+        _assert_same(got, ref)
+        assert min(d.size(0) for d, _ in got) > 0
