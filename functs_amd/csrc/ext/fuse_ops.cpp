@@ -250,7 +250,106 @@ bool canSink(Node* n, Node* sink_point, Block* block) {
   return true;
 }
 
-void fuseBlock(Block* block, bool force_group) {
+// What a region may not be moved past or made of, in a graph that still writes to tensors (arguments written in place: what a
+// program owns is functional by now).  A region reads its operands where it stands and returns values, so
+//   - a node that reads what a node in between may write stays where it is;
+//   - a view of what is written, also through the view, is made in a region only if nobody else sees it.
+// Two values may share memory if views lead to one value, or to two that come from outside, out of a container or a block, or go
+// into one (stock AliasDb does not know the nodes that loops have become by now).
+class Writes {
+ public:
+  explicit Writes(Graph& graph) : graph_(graph), any_(!written().empty()) {}
+
+  // whether `n` reads what one of `between` may write
+  bool crossed(Node* n, const std::vector<Node*>& between) const {
+    if (!any_) return false;
+    std::vector<Value*> written;
+    for (Node* w : between) collect(w, written);
+    for (Value* w : written)
+      for (Value* r : n->inputs())
+        if (mayReach(r, w)) return true;
+    return false;
+  }
+  // whether `v` is a view of what the program writes somewhere
+  bool viewOfWritten(Value* v) const {
+    if (!any_ || !isTensorValue(v) || !viewed(v)) return false;
+    for (Value* w : written())
+      if (mayReach(v, w)) return true;
+    return false;
+  }
+
+ private:
+  Graph& graph_;
+  bool any_;
+
+  static bool writesOperand(Node* n, size_t i) {
+    const auto* schema = n->maybeSchema();
+    return schema && i < schema->arguments().size() && isTensorValue(n->input(i)) && schema->is_mutable({c10::SchemaArgType::input, i});
+  }
+  static void collect(Node* n, std::vector<Value*>& written) {
+    for (size_t i = 0; i < n->inputs().size(); ++i)
+      if (writesOperand(n, i)) written.push_back(n->input(i));
+    for (Block* b : n->blocks())
+      for (Node* inner : b->nodes()) collect(inner, written);
+  }
+  std::vector<Value*> written() const {   // (asked anew: joining nodes replaces values)
+    std::vector<Value*> all;
+    for (Node* n : graph_.nodes()) collect(n, all);
+    return all;
+  }
+  // what `v` is a view of, or nullptr
+  static Value* viewed(Value* v) {
+    Node* n = v->node();
+    const auto* schema = n->maybeSchema();
+    if (!schema || n->outputs().size() != 1 || schema->returns().empty() || !schema->returns()[0].alias_info()) return nullptr;
+    for (size_t i = 0; i < n->inputs().size() && i < schema->arguments().size(); ++i)
+      if (schema->arguments()[i].alias_info() && isTensorValue(n->input(i))) return n->input(i);
+    return nullptr;
+  }
+  static Value* root(Value* v) {
+    while (Value* of = viewed(v)) v = of;
+    return v;
+  }
+  // whether a value that is no view has its memory to itself: an operator's result that nothing holds on to
+  static bool alone(Value* v) {
+    Node* n = v->node();
+    if (n->kind() != c10::prim::FusionGroup && n->kind() != sym::ForallSelectRev()) {
+      const auto* schema = n->maybeSchema();
+      if (!schema || n->kind().is_prim() || n->kind() == c10::aten::__getitem__) return false;
+      for (const auto& r : schema->returns())
+        if (r.alias_info()) return false;
+    }
+    for (const Use& u : v->uses()) {
+      Node* by = u.user;
+      if (by->kind() == c10::prim::ListConstruct) {   // (the list of a cat or an index is gone behind it)
+        for (const Use& lu : by->output()->uses())
+          if (lu.user->kind() != c10::aten::cat && lu.user->kind() != c10::aten::stack && !isIndexLike(lu.user)) return false;
+      } else if (by->kind() == c10::prim::Return) {
+        if (by->owningBlock()->owningNode()) return false;
+      } else if (by->kind() == c10::prim::TupleConstruct || by->kind() == c10::aten::append ||
+                 (!by->blocks().empty() && by->kind() != c10::prim::FusionGroup)) {
+        return false;
+      }
+    }
+    return true;
+  }
+  static bool mayReach(Value* read, Value* written) {
+    if (isTensorValue(read)) {
+      Value *a = root(read), *b = root(written);
+      return a == b || (!alone(a) && !alone(b));
+    }
+    if (auto lt = read->type()->cast<c10::ListType>()) {
+      const auto kind = lt->getElementType()->kind();
+      if (kind != c10::TypeKind::TensorType && kind != c10::TypeKind::OptionalType) return false;
+      if (read->node()->kind() != c10::prim::ListConstruct) return true;
+      for (Value* e : read->node()->inputs())
+        if (mayReach(e, written)) return true;
+    }
+    return false;
+  }
+};
+
+void fuseBlock(Block* block, bool force_group, const Writes& writes) {
   Node* tail = block->return_node();
   for (;;) {
     std::vector<Node*> group;          // collected in reverse program order
@@ -258,18 +357,18 @@ void fuseBlock(Block* block, bool force_group) {
     std::unordered_set<Node*> wanted;  // producers of values a member reads
     Node* head = tail;                 // the group occupies [head, sink_point)
     Node* sink_point = tail;           // nodes that stepped aside occupy [sink_point, tail)
-    bool stayed = false;               // a foreign node was left in place above the window
+    std::vector<Node*> stayed;         // foreign nodes that were left in place above the window
     for (Node* n = tail->prev(); n != block->param_node();) {
       Node* prev = n->prev();
       const bool empty = group.empty();
-      bool ok = n->kind() != c10::prim::Constant && isFusableNode(n);
+      bool ok = n->kind() != c10::prim::Constant && isFusableNode(n) && !writes.crossed(n, stayed);
       const bool is_out = !wanted.count(n);
       if (ok) {
         for (Value* o : n->outputs()) {
           bool used_outside = false;
           for (const Use& u : o->uses()) used_outside = used_outside || !members.count(u.user);
           // group outputs must be tensors (fuse_ops.cpp:232-240)
-          if (used_outside && !isTensorValue(o)) ok = false;
+          if (used_outside && (!isTensorValue(o) || writes.viewOfWritten(o))) ok = false;
         }
         if (!is_out && isIndexLike(n)) ok = false;  // only as a group output (fuse_ops.cpp:205-207)
       }
@@ -287,11 +386,11 @@ void fuseBlock(Block* block, bool force_group) {
           tail = n;
           head = n;
           sink_point = n;
-        } else if (!stayed && canSink(n, sink_point, block)) {
+        } else if (stayed.empty() && canSink(n, sink_point, block)) {
           n->moveBefore(sink_point);
           sink_point = n;
         } else if (n->kind() != c10::prim::Constant) {
-          stayed = true;
+          stayed.push_back(n);
         }
         n = prev;
         continue;
@@ -322,6 +421,7 @@ void collectBlocks(Block* b, std::vector<Block*>& out) {
 void FuseOps(std::shared_ptr<Graph> graph) {
   std::vector<Block*> blocks;
   collectBlocks(graph->block(), blocks);
+  const Writes writes(*graph);
   for (Block* b : blocks) {
     // a ParallelMap body that is fusable throughout is fused as a whole, whatever its size
     // (one launch instead of a loop); a mixed body follows the ordinary rule, so that a lone
@@ -330,7 +430,7 @@ void FuseOps(std::shared_ptr<Graph> graph) {
     if (whole_map)
       for (Node* n : b->nodes())
         whole_map = whole_map && (n->kind() == c10::prim::Constant || isFusableNode(n) || isIndexLike(n));
-    fuseBlock(b, whole_map);
+    fuseBlock(b, whole_map, writes);
   }
 }
 
