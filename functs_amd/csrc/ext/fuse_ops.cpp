@@ -649,7 +649,7 @@ bool producesBoolMask(Value* v, int depth = 0) {
 // group(...) -> (.., x, .., m);  x[m] for every other output x, and y[m] for values y
 // that exist before the group  ==>  group[compact_rows](..., y) -> (.., x', .., y')
 // with m as the last block output.
-bool foldMaskedSelect(Node* group) {
+bool foldMaskedSelect(Node* group, const Writes& writes) {
   if (group->hasAttribute(sym::compact_rows())) return false;
   Block* body = group->blocks()[0];
   for (size_t mi = 0; mi < group->outputs().size(); ++mi) {
@@ -681,6 +681,12 @@ bool foldMaskedSelect(Node* group) {
           Node* lifted = liftTo(def->owningBlock(), group);
           if (!lifted || !def->isBefore(lifted)) { ok = false; break; }
         }
+        // ... and to hold there what it holds where it is selected from
+        std::vector<Node*> between;
+        Node* at = liftTo(group->owningBlock(), ix);
+        for (Node* n = group->next(); at && n != at; n = n->next()) between.push_back(n);
+        if (at && at != ix) between.push_back(at);
+        if (!at || writes.crossed(ix, between)) { ok = false; break; }
       }
       if (!selects.count(x)) order.push_back(x);
       selects[x].push_back(ix);
@@ -730,15 +736,15 @@ void collectGroups(Block* b, std::vector<Node*>& out) {
   }
 }
 
-void foldIn(Block* b) {
+void foldIn(Block* b, const Writes& writes) {
   std::vector<Node*> groups;  // folding destroys neighbouring nodes: no live iterators
   collectGroups(b, groups);
-  for (Node* g : groups) foldMaskedSelect(g);
+  for (Node* g : groups) foldMaskedSelect(g, writes);
 }
 
 }  // namespace
 
-void FuseMaskedSelect(std::shared_ptr<Graph> graph) { foldIn(graph->block()); }
+void FuseMaskedSelect(std::shared_ptr<Graph> graph) { foldIn(graph->block(), Writes(*graph)); }
 
 // ---------------------------------------------------------------------------
 // UnrollLoopsWithDeps (fait/passes/unroll_loops.cpp:11-77) and UnrollSimpleMaps

@@ -114,6 +114,21 @@ def in_a_branch(x: Tensor, m: Tensor, flag: bool):
     return y + m + 1.0
 
 
+def rows_by_a_mask(x: Tensor, m: Tensor):
+    s = m * 2.0 + 1.0
+    keep = s[:, 0] > 1.0
+    x.zero_()
+    return x[keep], s[keep]
+
+
+def rows_by_a_mask_written_behind(x: Tensor, m: Tensor):
+    s = m * 2.0 + 1.0
+    keep = s[:, 0] > 1.0
+    y = x[keep]
+    x.zero_()
+    return y, s[keep]
+
+
 def classes_behind(x: Tensor, m: Tensor):
     scores = torch.softmax(x * 2.0 + m, dim=-1)
     x.zero_()
@@ -126,7 +141,7 @@ def classes_behind(x: Tensor, m: Tensor):
 
 
 PROGRAMS = (whole_argument, row, written_ahead, written_in_a_loop, rows_in_a_loop, read_again, columns, loop_behind, view_kept, view_read_behind,
-            from_a_copy, two_arguments_in_a_loop, other_argument, joined, in_a_branch, classes_behind)
+            from_a_copy, two_arguments_in_a_loop, other_argument, joined, in_a_branch, rows_by_a_mask, rows_by_a_mask_written_behind, classes_behind)
 
 
 def _arguments(program):
@@ -145,6 +160,13 @@ def test_no_write_is_lost(program):
     before = _writes(g.block())
     _C._jit_pass_fait_pipeline(g, [fj.extract_type_hint_from_tensor(a) for a in _arguments(program)])
     assert _writes(g.block()) == before > 0
+
+
+def test_rows_selected_ahead_of_a_write_are_compacted():
+    for program, folded in ((rows_by_a_mask, False), (rows_by_a_mask_written_behind, True)):
+        g = fj.script(program).graph.copy()
+        _C._jit_pass_fait_pipeline(g, [fj.extract_type_hint_from_tensor(a) for a in _arguments(program)])
+        assert ("compact_rows=1" in str(g)) == folded, program.__name__
 
 
 @pytest.mark.gpu
