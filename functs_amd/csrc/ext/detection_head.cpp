@@ -21,7 +21,6 @@
 #include <ATen/ATen.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
-#include <torch/csrc/jit/ir/alias_analysis.h>
 #include <torch/csrc/jit/ir/constants.h>
 #include <torch/csrc/jit/runtime/custom_operator.h>
 
@@ -244,15 +243,6 @@ bool isFunctor(Node* n, bool map) {
   const bool compact = n->hasAttribute(sym::compact_rows()) && n->i(sym::compact_rows()) != 0;
   const bool padded = n->hasAttribute(sym::padded_outputs()) && n->i(sym::padded_outputs()) != 0;
   return compact == map && padded == map && n->g(c10::attr::Subgraph)->inputs().size() == n->inputs().size() + 1;
-}
-
-// whether a node from `from` to `to` (neither included) may write to what `from` reads
-bool writtenBetween(const std::shared_ptr<Graph>& graph, Node* from, Node* to) {
-  const AliasDb aliases(graph);
-  const ValueSet reads(from->inputs().begin(), from->inputs().end());
-  for (Node* n = from->next(); n != to; n = n->next())
-    if (aliases.writesToAlias(n, reads)) return true;
-  return false;
 }
 
 bool fuseAt(const std::shared_ptr<Graph>& graph, Node* tail) {

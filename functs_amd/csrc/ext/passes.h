@@ -84,6 +84,8 @@ void ToParallelFunctor(std::shared_ptr<torch::jit::Graph> graph);
 // (fait/passes/te_op.cpp:135-236).  True if the graph changed; setSinkProducers(false) switches
 // the pass off for the process.
 bool SinkProducersIntoMaps(std::shared_ptr<torch::jit::Graph> graph);
+// whether a node from `from` to `to` (neither included; of one block, whose regions are functors by now) may write to what `from` reads
+bool writtenBetween(const std::shared_ptr<torch::jit::Graph>& graph, torch::jit::Node* from, torch::jit::Node* to);
 void setSinkProducers(bool on);
 
 // A per-image loop of functs::multiclass_nms(list_b[i], list_s[i], list_f[i], constants...) over

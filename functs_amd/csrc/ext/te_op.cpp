@@ -18,6 +18,7 @@
 #include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <torch/csrc/jit/ir/alias_analysis.h>
 #include <torch/csrc/jit/ir/constants.h>
 #include <torch/csrc/jit/passes/common_subexpression_elimination.h>
 #include <torch/csrc/jit/passes/constant_propagation.h>
@@ -1482,6 +1483,7 @@ bool trySinkProducer(Node* f2, Node* f1) {
       if (u.user->kind() == c10::prim::device) continue;   // answered by F1's own arguments, below
       return false;
     }
+  if (writtenBetween(g->shared_from_this(), f1, f2)) return false;   // (the map would read F1's arguments as they are by then)
   // where F1's results live is where its tensor arguments live
   {
     Value* some_tensor = nullptr;
@@ -1640,6 +1642,14 @@ bool sinkIn(Block* b) {
 }  // namespace
 
 void ToParallelFunctor(std::shared_ptr<Graph> graph) { toFunctorIn(graph->block()); }
+
+bool writtenBetween(const std::shared_ptr<Graph>& graph, Node* from, Node* to) {
+  const AliasDb aliases(graph);
+  const ValueSet reads(from->inputs().begin(), from->inputs().end());
+  for (Node* n = from->next(); n != to; n = n->next())
+    if (aliases.writesToAlias(n, reads)) return true;
+  return false;
+}
 
 bool SinkProducersIntoMaps(std::shared_ptr<Graph> graph) {
   if (!g_sink_producers.load()) return false;

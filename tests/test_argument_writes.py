@@ -140,6 +140,69 @@ def classes_behind(x: Tensor, m: Tensor):
     return out
 
 
+def decoded_ahead(loc: Tensor, conf: Tensor, priors: Tensor):
+    l0 = loc[0]
+    cxcy = priors[:, :2] + l0[:, :2] * 0.1 * priors[:, 2:]
+    wh = priors[:, 2:] * torch.exp(l0[:, 2:] * 0.2)
+    boxes = torch.zeros_like(priors)
+    boxes[:, :2] = cxcy - wh / 2
+    boxes[:, 2:] = cxcy + wh / 2
+    scores = conf[0].softmax(-1)
+    conf.zero_()
+    out_b: List[Tensor] = []
+    out_s: List[Tensor] = []
+    for c in range(1, scores.size(1)):
+        sc = scores[:, c]
+        m = sc > 0.05
+        out_b.append(boxes[m])
+        out_s.append(sc[m])
+    return out_b, out_s
+
+
+def written_at_the_end(loc: Tensor, conf: Tensor, priors: Tensor):
+    l0 = loc[0]
+    cxcy = priors[:, :2] + l0[:, :2] * 0.1 * priors[:, 2:]
+    wh = priors[:, 2:] * torch.exp(l0[:, 2:] * 0.2)
+    boxes = torch.zeros_like(priors)
+    boxes[:, :2] = cxcy - wh / 2
+    boxes[:, 2:] = cxcy + wh / 2
+    scores = conf[0].softmax(-1)
+    out_b: List[Tensor] = []
+    out_s: List[Tensor] = []
+    for c in range(1, scores.size(1)):
+        sc = scores[:, c]
+        m = sc > 0.05
+        out_b.append(boxes[m])
+        out_s.append(sc[m])
+    conf.zero_()
+    return out_b, out_s
+
+
+def _head_arguments():
+    g = torch.Generator().manual_seed(5)
+    return [0.5 * torch.randn(1, 300, 4, generator=g), torch.randn(1, 300, 21, generator=g), torch.rand(300, 4, generator=g)]
+
+
+def test_a_producer_sinks_into_its_map_unless_its_arguments_are_written():
+    for program, functors in ((written_at_the_end, 1), (decoded_ahead, 2)):
+        g = fj.script(program).graph.copy()
+        _C._jit_pass_fait_pipeline(g, [fj.extract_type_hint_from_tensor(a) for a in _head_arguments()])
+        assert [n.kind() for n in g.nodes()].count("tssa::ParallelFunctor") == functors, program.__name__
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("program", [decoded_ahead, written_at_the_end])
+def test_what_a_map_reads_is_what_the_program_decoded(program):
+    ref_args = _head_arguments()
+    ref = program(*ref_args)
+    print(program.__name__, flush=True)
+    fn, args = fj.build(fj.script(program), [a.cuda() for a in _head_arguments()]), [a.cuda() for a in _head_arguments()]
+    got = fn(*args)
+    assert sum(t.size(0) for t in ref[0]) > 0
+    for a, b in zip(got[0] + got[1] + args, ref[0] + ref[1] + ref_args):
+        torch.testing.assert_close(a.cpu(), b, rtol=1e-5, atol=1e-5)   # (a few operations and sums of 21 in 32 bits)
+
+
 PROGRAMS = (whole_argument, row, written_ahead, written_in_a_loop, rows_in_a_loop, read_again, columns, loop_behind, view_kept, view_read_behind,
             from_a_copy, two_arguments_in_a_loop, other_argument, joined, in_a_branch, rows_by_a_mask, rows_by_a_mask_written_behind, classes_behind)
 
