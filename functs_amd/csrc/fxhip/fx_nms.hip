@@ -205,7 +205,12 @@ __device__ __forceinline__ void gather_own(const fx_nms_desc& d, const Maps& h, 
   const uint32_t n = min(*s_count, key_cap), over = *s_count - n;
   if (HEAD && threadIdx.x == 0u) *s_kept = 0u;
   if (HEAD) __syncthreads();
+  // Where a head's scan found more than s_box holds, its memory is full of keys, of which the objectness may leave few: rows
+  // first, then the boxes of what is left, from rows and labels (one 608 x 608 image, all of its 1.8 M scores above the
+  // threshold, one row kept: the call 45 us, 62 with all boxes made, the chain of functors 57).
+  const bool rows_first = HEAD && n > FX_NMS_FEW;
   uint32_t my_max = 0u;   // below orderable() of every value
+  auto largest_of = [&](const float4& b) { my_max = max(my_max, max(max(orderable(b.x), orderable(b.y)), max(orderable(b.z), orderable(b.w)))); };
   for (uint32_t k0 = 0; k0 < n; k0 += FX_NMS_THREADS) {
     const uint32_t k = k0 + threadIdx.x;
     uint64_t key = 0ull;
@@ -218,7 +223,7 @@ __device__ __forceinline__ void gather_own(const fx_nms_desc& d, const Maps& h, 
         const HeadRow r = head_row(h, task, (uint32_t)key);
         const float score = fx_sigmoid(__uint_as_float((uint32_t)(key >> 32)));
         f = head_objectness(r);
-        b = head_box(r);
+        if (!rows_first) b = head_box(r);
         keep = score > d.score_thr && f >= h.keep_thr;
         key = ((uint64_t)(~orderable(score)) << 32) | (uint64_t)(r.row * C + r.label);
       } else {
@@ -227,7 +232,7 @@ __device__ __forceinline__ void gather_own(const fx_nms_desc& d, const Maps& h, 
         b = *(const float4*)(boxes + (size_t)r * 4u);
       }
       if (HEAD || factors) key = ((uint64_t)(~orderable(from_orderable(~(uint32_t)(key >> 32)) * f)) << 32) | (uint64_t)(uint32_t)key;
-      if (keep) my_max = max(my_max, max(max(orderable(b.x), orderable(b.y)), max(orderable(b.z), orderable(b.w))));
+      if (keep && !rows_first) largest_of(b);
     }
     if (HEAD) __syncthreads();   // (the places that are written lie among those that have been read)
     if (keep) {
@@ -236,20 +241,24 @@ __device__ __forceinline__ void gather_own(const fx_nms_desc& d, const Maps& h, 
       if (n <= FX_NMS_FEW && key_cap >= FX_NMS_ROOMY) s_box[at] = b;
     }
   }
+  if constexpr (HEAD) {
+    if (rows_first) {
+      __syncthreads();
+      const uint32_t kept = *s_kept;
+      for (uint32_t k = threadIdx.x; k < kept; k += FX_NMS_THREADS) {
+        const uint32_t idx = (uint32_t)s_keys[k], r = fx_fastdiv(idx, h.c_magic, h.c_shift);
+        const float4 b = head_box(head_row(h, task, head_number(h, r, idx - r * C)));
+        largest_of(b);
+        if (kept <= FX_NMS_FEW && key_cap >= FX_NMS_ROOMY) s_box[k] = b;
+      }
+    }
+  }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) my_max = max(my_max, (uint32_t)__shfl_xor((int)my_max, o, 64));
   if ((threadIdx.x & 63u) == 0u && my_max != 0u) atomicMax(s_maxc, my_max);
   __syncthreads();
-  if constexpr (HEAD) {
-    const uint32_t kept = *s_kept;
-    // Where the scan found more than s_box holds, s_box's memory was full of keys until here.  What is left of them is decided
-    // behind this by its number alone, so if that is small its boxes are made now, from rows and labels.
-    if (n > FX_NMS_FEW && kept <= FX_NMS_FEW && key_cap >= FX_NMS_ROOMY)
-      for (uint32_t k = threadIdx.x; k < kept; k += FX_NMS_THREADS) {
-        const uint32_t idx = (uint32_t)s_keys[k], r = fx_fastdiv(idx, h.c_magic, h.c_shift);
-        s_box[k] = head_box(head_row(h, task, head_number(h, r, idx - r * C)));
-      }
-    if (threadIdx.x == 0u) *s_count = kept + over;
+  if (HEAD) {
+    if (threadIdx.x == 0u) *s_count = *s_kept + over;
     __syncthreads();
   }
 }
