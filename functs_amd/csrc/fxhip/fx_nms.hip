@@ -77,9 +77,9 @@ __device__ __forceinline__ uint64_t bitonic_step(uint64_t key, bool up, uint32_t
 // puts them (yolov3_bbox.py:211-220).  Class scores of one (level, anchor) are C * cells consecutive elements of an
 // image's map; a wave reads them in groups of 256 that never span two of these runs, so what a wave needs to know
 // about its group is uniform.
-// Four 608 x 608 images, 80 classes, about 700 candidates each, cold lines: 21.9 us, of which the scan's 28 MB are 6.7 behind
+// Four 608 x 608 images, 80 classes, about 700 candidates each, cold lines: 21.7 us, of which the scan's 28 MB are 6.7 behind
 // 2 of start; the functors and the tail this stands for (rows across their order 38.5, row stream 16.8, tail 26.1) 81.4,
-// and the call 97 -> 38 us.  One image 19.8 (128 workgroups scan it; 64: 20.5, 256: 21.7, they queue up for the ticket).
+// and the call 97 -> 35 us.  One image 19.8 (128 workgroups scan it; 64: 20.5, 256: 21.7, they queue up for the ticket).
 struct HeadLevel {
   const float *map, *base, *shift;
   uint32_t cells, anchors, row0;     // row0: rows of the levels before it
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(FX_NMS_THREADS) void fx_sort_nms_kernel(const fx_nm
         for (uint32_t e = 0; e < 4u; ++e) {
           if ((mine >> (u * 4u + e)) & 1u) {
             const uint32_t i = base + (u * FX_NMS_THREADS + tid) * 4u + e;
-            // (the raw score for now: the row's factor is applied by the finishing workgroup)
+            // (the raw score for now: gather_own applies the row's factor)
             if (slot < key_cap) s_keys[slot] = ((uint64_t)(~orderable(v[u][e])) << 32) | (uint64_t)i;
             ++slot;
           }
