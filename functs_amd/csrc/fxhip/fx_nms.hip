@@ -21,6 +21,9 @@
 // steps.  16 images of 8 500 rows, 80 classes, about 760 candidates each: 23.8 us; 27.9 with the sort for all, factors and
 // boxes gathered by the last workgroup, the rows written in the walk (whose barriers then wait for the stores) and
 // the walk's overlaps by the division.  128 boxes of one image, one workgroup, nothing handed over: 12.1 us, 13.1.
+// Few candidates that several workgroups find pay for the buckets and the hand-over: calls of one image of 8 500 rows with 8 / 100 /
+// 200 / 700 candidates 14.3 / 16.7 / 16.8 / 17.6 us, with the sort and the last workgroup's gather 13.0 / 15.8 / 17.3 / 21.2.  (Up to 128
+// candidates ordered by counting, eight threads each, 13.8 / 16.5, was 0.2 to 0.4 slower at 200 to 300: the kernel grows.)
 // The workspace counters are zero when a launch starts and zero again when it ends.
 // The number of valid rows per task is read from memory (device or pinned host), so the count a
 // preceding compaction produced never has to reach the host.
